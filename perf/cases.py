@@ -237,10 +237,162 @@ def work(case):
 def tolerance(case):
     """Largest relative error of another correct implementation: about four times what the path differs by from the
     same formulas in a wider type on the same inputs (fp32 against fp64: 2e-6 at most; 16-bit forward 3.5e-3, with
-    gradients 3.2e-3 to 6e-3; encoder pass 8e-3).  A training step through the encoder differs by up to 2.7e-2 from
-    one with fp32 attention: rounding moves activations across the ReLU's edge."""
+    gradients 3.2e-3 to 9.2e-3, the largest that of the table at head_dim 128; encoder pass 8e-3).  A training step
+    through the encoder is up to 2.6e-2 from the formulas in 64 bits, since rounding moves activations across the
+    ReLU's edge: two such steps, each as far from them on a side of its own, differ by 3.7e-2."""
     if case["kind"] == "encoder":
-        return {"rel": 0.03, "max": 0.9} if case["train"] else {"rel": 0.02, "max": 0.3}
+        return {"rel": 0.08, "max": 0.9} if case["train"] else {"rel": 0.02, "max": 0.3}
     if case["dtype"] == "fp32":
         return {"rel": 1e-5, "max": 1e-3}
-    return {"rel": 0.02, "max": 0.4} if case.get("train") else {"rel": 0.012, "max": 0.2}
+    return {"rel": 0.03, "max": 0.4} if case.get("train") else {"rel": 0.012, "max": 0.2}
+
+
+# ---- the same formulas in 64 bits ----
+
+def _bucket(rel, bidirectional):
+    """T5's bucket of memory position - query position: 32 buckets, logarithmic from a quarter of them to distance
+    128.  The logarithm is T5's own in 32 bits, which is what fixes where the buckets begin."""
+    n = 16 if bidirectional else 32
+    first = (rel > 0).long() * n if bidirectional else torch.zeros_like(rel)
+    dist = rel.abs() if bidirectional else (-rel).clamp(min=0)
+    half = n // 2
+    far = half + (torch.log(dist.float() / half) / math.log(128 / half) * (n - half)).long()
+    return first + torch.where(dist < half, dist, far.clamp(max=n - 1))
+
+
+def _softmax(s):
+    """Over the last dimension; a row without a visible key gives zeros."""
+    return torch.softmax(s, -1).nan_to_num(0.0)
+
+
+def _dense(q, k, v, table, causal, dout=None):
+    """Attention of one sequence over (H, L, D) rows, a few query rows at a time: o, and with ``dout`` the gradients of
+    q, k, v and the table."""
+    H, L, _ = q.shape
+    N = k.shape[1]
+    kT, vT = k.transpose(1, 2).contiguous(), v.transpose(1, 2).contiguous()
+    o = torch.empty_like(q)
+    grads = [torch.zeros_like(t) for t in (q, k, v)] + [torch.zeros_like(table)] if dout is not None else None
+    step = max(1, min(L, (1 << 26) // (H * N)))
+    for r in range(0, L, step):
+        rows = slice(r, min(L, r + step))
+        rel = torch.arange(N, device=q.device)[None, :] - torch.arange(rows.start, rows.stop, device=q.device)[:, None]
+        bucket = _bucket(rel, not causal)
+        s = q[:, rows] @ kT + table[bucket].permute(2, 0, 1)
+        if causal:
+            s.masked_fill_(rel > 0, -math.inf)
+        p = _softmax(s)
+        o[:, rows] = p @ v
+        if dout is None:
+            continue
+        g = dout[:, rows]
+        ds = p * (g @ vT - (g * o[:, rows]).sum(-1, keepdim=True))
+        grads[0][:, rows] = ds @ k
+        grads[1] += ds.transpose(1, 2).contiguous() @ q[:, rows]
+        grads[2] += p.transpose(1, 2).contiguous() @ g
+        for b in range(table.shape[0]):
+            grads[3][b] += (ds * (bucket == b)).sum((1, 2))
+    return (o, *grads) if dout is not None else o
+
+
+def _sparse(case, st):
+    q, k, v = (t.double() for t in st["qkv"])
+    table = st["table"].double()
+    L, w, aux, dev = case["L"], case["block_len"], case["aux"], q.device
+    o = torch.empty_like(q)
+    pos = torch.arange(L, device=dev)
+    for lo in range(0, L, w):
+        i = pos[lo:lo + w, None]
+        if case["pattern"] == "block":
+            # columns: the leading global tokens, then the own block; the last block is filled up with zero keys, and
+            # the first one does not see its last columns
+            pad = (0, 0, 0, lo + w - min(L, lo + w))
+            kk, vv = (torch.cat([t[:, :, :aux], torch.nn.functional.pad(t[:, :, lo:lo + w], pad)], 2) for t in (k, v))
+            col = torch.arange(w + aux, device=dev)[None, :]
+            rel, seen = col - aux - (i - lo), (col < w) | (lo > 0)
+        else:
+            a, b = max(0, lo - w + 1), min(L, lo + 2 * w - 1)
+            kk, vv = k[:, :, a:b], v[:, :, a:b]
+            rel = pos[None, a:b] - i
+            seen = rel.abs() < w
+            if case["pattern"] == "tglobal":
+                side = st["side"][0].shape[2]
+                kk, vv = (torch.cat([t, x.double()], 2) for t, x in zip((kk, vv), st["side"]))
+                srel = torch.arange(side, device=dev)[None, :] - (i // aux).clamp(max=side - 1)
+                rel, seen = torch.cat([rel, srel], 1), torch.cat([seen, torch.ones_like(srel, dtype=torch.bool)], 1)
+        s = q[:, :, lo:lo + w] @ kk.transpose(2, 3).contiguous() + table[_bucket(rel, True)].permute(2, 0, 1)
+        o[:, :, lo:lo + w] = _softmax(s.masked_fill(~seen, -math.inf)) @ vv
+    if case["pattern"] == "block":
+        for b in range(case["B"]):
+            rel = pos[None, :] - pos[:aux, None]
+            s = q[b, :, :aux] @ k[b].transpose(1, 2).contiguous() + table[_bucket(rel, True)].permute(2, 0, 1)
+            o[b, :, :aux] = torch.softmax(s, -1) @ v[b]
+    return o
+
+
+def _encoder(case, st):
+    w = {n: p.detach().double().requires_grad_(case["train"]) for n, p in st["model"].named_parameters()}
+    B, L, H = case["B"], case["L"], case["H"]
+    lens = st["mask"].sum(1).tolist() if st["mask"] is not None else [L] * B
+
+    def norm(x, name):
+        return x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-6) * w[name]
+
+    def attend(q, k, v, table):
+        if not case["train"]:
+            return _dense(q, k, v, table, False)
+        p = torch.arange(q.shape[1], device=q.device)
+        s = q @ k.transpose(1, 2).contiguous() + table[_bucket(p[None, :] - p[:, None], True)].permute(2, 0, 1)
+        return torch.softmax(s, -1) @ v
+
+    table = w["encoder.block.0.layer.0.SelfAttention.relative_attention_bias.weight"]
+    xs = []
+    for b, n in enumerate(lens):
+        x = w["shared.weight"][st["ids"][b, :n]]
+        for j in range(case["layers"]):
+            at, ff = f"encoder.block.{j}.layer.0.", f"encoder.block.{j}.layer.1."
+            y = norm(x, at + "layer_norm.weight")
+            q, k, v = ((y @ w[at + f"SelfAttention.{c}.weight"].T).view(n, H, -1).transpose(0, 1).contiguous() for c in "qkv")
+            x = x + attend(q, k, v, table).transpose(0, 1).reshape(n, -1) @ w[at + "SelfAttention.o.weight"].T
+            y = norm(x, ff + "layer_norm.weight")
+            x = x + torch.relu(y @ w[ff + "DenseReluDense.wi.weight"].T) @ w[ff + "DenseReluDense.wo.weight"].T
+        # positions behind a sequence's end are zero
+        xs.append(torch.nn.functional.pad(norm(x, "encoder.final_layer_norm.weight"), (0, 0, 0, L - n)))
+    hidden = torch.stack(xs)
+    if not case["train"]:
+        return hidden
+    hidden.backward(st["dout"].double())
+    return {"hidden": hidden.detach(), "grads": [w[n].grad for n, _ in st["model"].named_parameters()]}
+
+
+def exact(case, seed):
+    """What ``run`` returns for these inputs, from the formulas in 64 bits."""
+    st = prepare(case, seed)
+    kind = case["kind"]
+    if kind == "encoder":
+        with torch.set_grad_enabled(case["train"]):
+            return _encoder(case, st)
+    with torch.no_grad():
+        if kind == "sparse":
+            return _sparse(case, st)
+        if kind == "decode":
+            q, (k, v) = st["q"].double(), st["kv"]
+            lens = st["lens"].tolist() if st["lens"] is not None else [case["N"]] * case["B"]
+            out = [torch.softmax(q[b] @ k[b, :, :n].double().transpose(1, 2).contiguous(), -1) @ v[b, :, :n].double()
+                   for b, n in enumerate(lens)]
+            return torch.stack(out)
+        rows = [t.detach().double() for t in st["qkv"]] + ([st["dout"].double()] if case["train"] else [])
+        table = st["table"].detach().double()
+        if kind == "attn":
+            each = [[t[b] for t in rows] for b in range(case["B"])]
+        else:
+            cu = st["cu"].tolist()
+            each = [[t[a:b].transpose(0, 1) for t in rows] for a, b in zip(cu, cu[1:])]
+        outs = [_dense(*(t.contiguous() for t in r[:3]), table, case["causal"], *(t.contiguous() for t in r[3:])) for r in each]
+
+        def join(ts):
+            return torch.stack(ts) if kind == "attn" else torch.cat([t.transpose(0, 1) for t in ts])
+
+        if not case["train"]:
+            return join(outs)
+        return [*(join([o[i] for o in outs]) for i in range(4)), sum(o[4] for o in outs)]

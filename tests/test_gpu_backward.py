@@ -116,6 +116,25 @@ def test_16_bit_gradients_at_head_dim_128(gpu_device, dtype, causal, B, H, M, N)
         check(name, g, w, TOL[dtype])
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("B,H,M,N", [(48, 16, 33, 65), (53, 15, 130, 97), (24, 16, 290, 257)])
+def test_16_bit_gradients_of_launches_that_fill_the_chip(gpu_device, causal, D, B, H, M, N):
+    """From 512 (causal 768) blocks of 128 own rows on a workgroup owns 128 rows and walks tiles of 32; below, 64 rows
+    and tiles of 64 whose halves go to two wavefronts each.  Both kinds of placement ((head, batch) pairs that divide by
+    eight and that do not), a tile more than a multiple of 32 and one row more than a tile."""
+    from turbot5_amd import ops
+    dtype = torch.bfloat16
+    q, k, v = rnd(B, H, M, D, seed=91, dtype=dtype), rnd(B, H, N, D, seed=92, dtype=dtype), rnd(B, H, N, D, seed=93, dtype=dtype)
+    table = rnd(32, H, seed=94, scale=1.0)
+    dout = rnd(B, H, M, D, seed=95, scale=1.0, dtype=dtype)
+    _, wq, wk, wv, wt = oracle_grads(q, k, v, table, dout, causal, None)
+    dq, dk, dv, dt = (t.to(gpu_device).requires_grad_(True) for t in (q, k, v, table))
+    ops.flash_attention_with_fusing_bias(dq, dk, dv, dt, causal=causal).backward(dout.to(gpu_device))
+    for name, g, w in (("dq", dq.grad, wq), ("dk", dk.grad, wk), ("dv", dv.grad, wv), ("dtable", dt.grad, wt)):
+        check(name, g, w, TOL[dtype])
+
+
 def test_head_dim_128_backward_refuses_fp32(gpu_device):
     from turbot5_amd import ops
     q, k, v = (rnd(1, 1, 64, 128, seed=86 + i).to(gpu_device).requires_grad_(True) for i in range(3))

@@ -3,14 +3,13 @@
 // (src/turbot5/ops/fused_bias_attention.py:397-820: _bwd_preprocess, _bwd_kv_bias_kernel with its atomics on the
 // table gradient :617-619, _bwd_q_kernel).
 //
-// Three kernels.  The general ones do all arithmetic in fp32 (inputs of any of the three types are widened on their
+// The general kernels do all arithmetic in fp32 (inputs of any of the three types are widened on their
 // way into LDS; the products run on the fp32 matrix cores, v_mfma_f32_32x32x2_f32), so one code path serves fp32 and
-// 16-bit tensors at head_dim 16, 32 and 64; 16-bit tensors at head_dim 64 have a faster pair of their own on the 16-bit
-// matrix cores (bwd16_kernel, further down) unless the caller asks for fp32 arithmetic, and at head_dim 128 three
-// passes of the same kind (bwd16_d128_kernel).  The general kernels:
+// 16-bit tensors at head_dim 16, 32 and 64; 16-bit tensors at head_dim 64 and 128 have kernels of their own on the 16-bit
+// matrix cores (bwd16_kernel, further down) unless the caller asks for fp32 arithmetic.  The general kernels:
 //
-//   bwd_rows_kernel   delta_i = sum_d o_id do_id and the log-sum-exp in base-2 units, per query row; also clears the
-//                     table gradient
+//   bwd_rows_kernel   delta_i = sum_d o_id do_id and the log-sum-exp in base-2 units, per query row, both negated; also
+//                     clears the table gradient
 //   bwd_kernel<KV=0>  a workgroup owns 128 query rows (32 per wavefront) and walks the key tiles of 64:
 //                     S^T = K Q^T, dP^T = V dO^T (key rows from LDS as the A operand, so a lane owns one query and
 //                     its log-sum-exp and delta are lane scalars), P^T = exp2(c1 S^T + bias - lse),
@@ -116,10 +115,10 @@ __global__ __launch_bounds__(256) void bwd_rows_kernel(const BwdParams p) {
 #pragma unroll
     for (int off = 1; off < G::TPR; off <<= 1) acc += __shfl_xor(acc, off, 64);
     if (row >= rows || sub != 0) return;
-    p.delta[row] = acc;
+    p.delta[row] = -acc;     // negated: it is the start value of the dP accumulators
     const float l = p.lse[row];
-    // a row without a visible key: +inf makes every exp2(score - lse2) of the row 0
-    p.lse2[row] = l == -INFINITY ? INFINITY : l * 1.4426950408889634f;
+    // negated as well; a row without a visible key: -inf makes every exp2(score + lse2) of the row 0
+    p.lse2[row] = l == -INFINITY ? -INFINITY : l * -1.4426950408889634f;
 }
 
 template <typename T, int D, bool CAUSAL, bool KV>
@@ -187,7 +186,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
             fb[2 * s4] = hh ? y[1] : y[0]; fb[2 * s4 + 1] = hh ? y[3] : y[2];
         }
     }
-    float lse2_own = INFINITY, delta_own = 0.f;
+    float lse2_own = -INFINITY, delta_own = 0.f;
     if (!KV && own_ok) { lse2_own = p.lse2[stat_base + own_row * stat_sr]; delta_own = p.delta[stat_base + own_row * stat_sr]; }
 
     // tiles of the other kind that can hold a visible pair
@@ -223,7 +222,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
             }
             if (KV && tid < 2 * kBwdOther) {
                 const int row = tid & (kBwdOther - 1);
-                float val = tid < kBwdOther ? INFINITY : 0.f;
+                float val = tid < kBwdOther ? -INFINITY : 0.f;
                 if (o0 + row < n_other)
                     val = tid < kBwdOther ? p.lse2[stat_base + (o0 + row) * stat_sr] : p.delta[stat_base + (o0 + row) * stat_sr];
                 rowstat[tid] = val;
@@ -264,8 +263,8 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
                 const float bias2 = has_bias ? lut_bias[x] : 0.f;
                 const float l2 = KV ? rowstat[ol] : lse2_own;
                 const float dl = KV ? rowstat[kBwdOther + ol] : delta_own;
-                const float pv = valid ? __builtin_amdgcn_exp2f(__builtin_fmaf(p.c1, s[nt][r], bias2) - l2) : 0.f;
-                const float ds = pv * (dp[nt][r] - dl);
+                const float pv = valid ? __builtin_amdgcn_exp2f(__builtin_fmaf(p.c1, s[nt][r], bias2) + l2) : 0.f;
+                const float ds = pv * (dp[nt][r] + dl);
                 s[nt][r] = pv;
                 dp[nt][r] = ds;
                 if constexpr (!KV) {
@@ -332,18 +331,28 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
 
 
 // ------------------------------------------------------------------------------------------------------------------
-// 16-bit inputs at head_dim 64: the same two passes on the 16-bit matrix cores (v_mfma_f32_32x32x16_bf16 / _f16).
+// 16-bit inputs at head_dim 64 and 128: passes of the same kind on the 16-bit matrix cores
+// (v_mfma_f32_32x32x16_bf16 / _f16).  PASS 0: dq and the table gradient; 1: dk and dv; 2: dk; 3: dv.
 //
-// The products over head_dim (S^T = K Q^T, dP^T = V dO^T and their counterparts of the dk / dv pass) take the inputs as
+// The products over head_dim (S^T = K Q^T, dP^T = V dO^T and their counterparts of the dk / dv passes) take the inputs as
 // they are; the probabilities and dS are rounded to the input type for the products over the tile's rows, as the
 // reference does (fused_bias_attention.py:575-590: p.to(Q.dtype), ds.to(Q.dtype)); sums stay in fp32.  A tile of
-// the other kind is 64 rows of 128 bytes in LDS and serves both kinds of product from one copy: rows are read as they
+// the other kind is rows of 128 or 256 bytes in LDS and serves both kinds of product from one copy: rows are read as they
 // lie (A operand, contraction over head_dim), and the contraction over the tile's rows reads it through the
 // transposing LDS read (ds_read_b64_tr_b16: four rows x 16 columns per group of 16 lanes), whose k-slot order --
 // rows 4h .. 4h+3 and 8+4h .. 8+4h+3 of every 16 in lane half h -- is exactly the order in which a lane holds the rows
 // of a 32x32 accumulator, so P and dS go from accumulator registers to B operands with a conversion and no shuffle.
 // The 16-byte chunks of a row are XOR-swizzled with a pattern that keeps both kinds of read free of bank conflicts.
-// The next tile's rows are fetched into registers while the current tile is worked on.
+//
+// What bounds it: no single pipe.  At B16 H12 L1024 D64 bf16 the matrix pipe is busy 40 % of the cycles, the vector
+// port 50 %, LDS 45 %, with three wavefronts per SIMD.  Hence the choices below: one 32 x 32 block of scores per
+// wavefront and step (144-168 registers; two blocks need two wavefronts per SIMD and copies between the code of the
+// block classes), accumulators touched by one piece of code only (a class decides about arguments, never about products:
+// with the products in the classes' branches the compiler kept a copy of every accumulator per branch and spilled), and
+// as few instructions per score as the formulas allow.  Deeper staging (3 or 4 tile buffers) was slower: the LDS it
+// takes costs more than the wait it saves.  Before / after, us, the passes with bwd_rows_kernel, bf16: B16 H12
+// L1024 D64 299 / 248, the same causal 205 / 180, B4 H12 L4096 D64 840 / 762, B4 H6 L4096 D128 1274 / 835, B2 H8
+// L1999 D128 causal 280 / 135.
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x8 __attribute__((ext_vector_type(8)));
@@ -378,29 +387,90 @@ __device__ __forceinline__ void dma_16(u32x4 rs, unsigned lds_addr, int voffset)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
                  :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voffset), "s"(rsrc) : "memory", "m0");
 }
+// the same with 4 bytes per lane (256 consecutive bytes of LDS)
+__device__ __forceinline__ void dma_4(u32x4 rs, unsigned lds_addr, int voffset) {
+    const u32x4 rsrc = {(unsigned)__builtin_amdgcn_readfirstlane((int)rs[0]), (unsigned)__builtin_amdgcn_readfirstlane((int)rs[1]),
+                        (unsigned)__builtin_amdgcn_readfirstlane((int)rs[2]), (unsigned)__builtin_amdgcn_readfirstlane((int)rs[3])};
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
+                 :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voffset), "s"(rsrc) : "memory", "m0");
+}
+// waits until at most N of this wavefront's memory requests are outstanding (they complete in order)
+template <int N> __device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N < 64, "");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
 
-template <typename T, bool CAUSAL, bool KV>
-__global__ __launch_bounds__(kBwdThreads, 2) void bwd16_kernel(const BwdParams p) {
-    constexpr int D = 64, DT = 2, KS = 4, NT = kBwdOther / 32;
+// head_dim 128 (the T5-3B / 11B head shape): rows of 256 bytes, sixteen chunks
+__device__ __forceinline__ int tile_swz128(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+
+// Geometry of a 16-bit backward workgroup: four wavefronts, each on 32 own rows and 32 rows of the tile at a time (one
+// 32 x 32 block of scores: 32 score registers, which is what lets three wavefronts share a SIMD at head_dim 64).
+// SPLIT 1: four groups of own rows, tiles of 32.  SPLIT 2: two groups of own rows, tiles of 64 whose halves go to
+// different wavefronts; the two partial gradients of a row are added through LDS at the end.
+template <int D, int PASS, int SPLIT>
+struct Bwd16Geom {
+    static constexpr bool KV = PASS != 0;
+    static constexpr int OWNW = 4 / SPLIT, OWN = 32 * OWNW, OTHER = 32 * SPLIT;
+    static constexpr int TILE = OTHER * D * 2;                    // bytes of one staged tile
+    static constexpr int SLABS = TILE / 1024 / 4;                 // 1 KB requests per wavefront and tile
+    static constexpr int RPS = 1024 / (2 * D);                    // rows per request
+    static constexpr int STAGES = 2;                               // tile buffers
+    static constexpr int REQS = 2 * SLABS + (KV ? 1 : 0);         // requests per wavefront and tile
+    static constexpr int SKEW_ROWS = (D == 128 && SPLIT == 2) ? 8 : 32;   // queries per round of the table gradient
+    static constexpr int LUT_PAD16 = 64;                          // a 32 x 32 block spans 63 distances
+    static constexpr int STAT = STAGES * 2 * TILE;                // byte offsets
+    static constexpr int LUT = STAT + (KV ? STAGES * 2 * 64 * 4 : 0);
+    static __host__ __device__ int lut_floats(int sat) { return (2 * (sat + LUT_PAD16) + 4) & ~3; }
+    static __host__ __device__ int hist(int sat) { return LUT + 4 * lut_floats(sat); }
+    static __host__ __device__ int skew(int sat) { return hist(sat) + (KV ? 0 : 4 * ((2 * sat + 4) & ~3)); }
+    static __host__ __device__ int bytes(int sat, bool bias) { return skew(sat) + (KV || !bias ? 0 : 4 * SKEW_ROWS * 64 * 4); }
+};
+
+// Workgroup -> (own block, head, sequence).  Workgroups go to the eight XCDs in turn; all own blocks of a (head,
+// sequence) pair go to one XCD, whose L2 then holds the pair's rows of the other kind for all of them.  Where the
+// pairs do not divide by eight they are dealt out in turn instead.  With a causal mask the own blocks differ in length
+// (a query block sees the keys up to its own end, a key block the queries from its own start on), and whatever is
+// dispatched last should be short: the blocks are then the slowest index, longest first.
+template <bool CAUSAL, bool KV>
+__device__ __forceinline__ void bwd_place(int H, int B, int nblk, int& blk, int& h, int& b) {
+    const int pairs = H * B, id = blockIdx.x;
+    int pair, level;
+    if ((pairs & 7) == 0) {
+        const int pp = pairs >> 3, slot = id >> 3;
+        if (CAUSAL) { level = slot / pp; pair = (id & 7) * pp + (slot - level * pp); }
+        else { const int q = slot / nblk; level = slot - q * nblk; pair = (id & 7) * pp + q; }
+    } else {
+        level = id / pairs; pair = id - level * pairs;
+    }
+    blk = (CAUSAL && !KV) ? nblk - 1 - level : level;
+    h = pair / B; b = pair - h * B;
+}
+
+// rows 16 u .. + 15 of a 32-row accumulator as a B operand
+template <typename v8> __device__ __forceinline__ v8 to_frag(const f32x16& x, int u) {
+    f32x8 y;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) y[e] = x[8 * u + e];
+    return __builtin_convertvector(y, v8);
+}
+
+template <int D> __device__ __forceinline__ int row_swz(int row) { return D == 64 ? tile_swz(row) : tile_swz128(row); }
+
+template <typename T, int D, bool CAUSAL, int PASS, int SPLIT>
+__global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ? 3 : 2) void bwd16_kernel(const BwdParams p, int nblk) {
+    constexpr bool KV = PASS != 0, DS = PASS != 3, DA = PASS != 3, DV = PASS == 1 || PASS == 3;   // dS; dq or dk; dv
+    using G = Bwd16Geom<D, PASS, SPLIT>;
+    constexpr int DT = D / 32, KS = D / 16, OTHER = G::OTHER, CH = D / 8;
     using H16 = Half16<T>;
     using v8 = typename H16::v8;
-    // two buffers of each: tile t + 1 is written while tile t is read, one barrier per tile
-    __shared__ __attribute__((aligned(16))) T ta2[2][kBwdOther * D];   // K (dq) / Q (dk, dv) tiles
-    __shared__ __attribute__((aligned(16))) T tb2[2][kBwdOther * D];   // V (dq) / dO (dk, dv) tiles
-    __shared__ __attribute__((aligned(16))) float rowstat2[2][2 * kBwdOther];   // KV: lse2 and delta of the tiles' queries
-    __shared__ float lut_bias[2 * kMaxSaturation + 1];
-    __shared__ int lut_bucket[KV ? 1 : 2 * kMaxSaturation + 1];
-    __shared__ float hist[KV ? 1 : kMaxBuckets];
-    __shared__ float hist_rel[KV ? 1 : 2 * kMaxSaturation + 1];   // dS summed per clamped distance (tiles around the diagonal)
+    extern __shared__ __attribute__((aligned(16))) unsigned char bwd_smem[];
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, hh = lane >> 5;
-    // Grid: (own blocks, heads, batch).  With a causal mask the own blocks differ in length (a query block sees the
-    // keys up to its own end, a key block the queries from its own start on), and whatever is dispatched last should
-    // be short: the launch is then (heads, batch, own blocks), the slowest index walking the blocks longest first.
-    const int h = CAUSAL ? blockIdx.x : blockIdx.y, b = CAUSAL ? blockIdx.y : blockIdx.z;
-    const int own_block = !CAUSAL ? blockIdx.x : (KV ? blockIdx.z : gridDim.z - 1 - blockIdx.z);
-    const int own_base = own_block * kBwdOwn;
-    const int own_row = own_base + wave * 32 + lr;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, hh = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), ow = wave % G::OWNW, sub0 = (wave / G::OWNW) * 32;
+    int own_block, h, b;
+    bwd_place<CAUSAL, KV>(p.H, p.B, nblk, own_block, h, b);
+    const int own_base = own_block * G::OWN;
+    const int w_lo = own_base + ow * 32, own_row = w_lo + lr;     // this wavefront's, this lane's own rows
     int M = p.M, N = p.N;
     int64_t q_first = 0, k_first = 0;
     if (p.cu_q != nullptr) {
@@ -413,6 +483,9 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd16_kernel(const BwdParams p
     const int P = N - M;
     const bool has_bias = p.table != nullptr;
     const int sat = has_bias ? p.bs.sat : 0;
+    float* const lut = reinterpret_cast<float*>(bwd_smem + G::LUT);
+    float* const hist_rel = reinterpret_cast<float*>(bwd_smem + G::hist(sat));   // dS summed per clamped distance
+    float* const skew = reinterpret_cast<float*>(bwd_smem + G::skew(sat)) + wave * G::SKEW_ROWS * 64;
 
     const T* qp = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + q_first * p.q_sr;
     const T* kp = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh + k_first * p.k_sr;
@@ -420,6 +493,43 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd16_kernel(const BwdParams p
     const T* gp = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.do_sb + (int64_t)h * p.do_sh + q_first * p.do_sr;
     const int64_t stat_sr = p.cu_q != nullptr ? p.H : 1;
     const int64_t stat_base = p.cu_q != nullptr ? q_first * p.H + h : ((int64_t)b * p.H + h) * p.M;
+
+    // tiles that can hold a visible pair
+    int t_lo = 0, t_hi = (n_other + OTHER - 1) / OTHER;
+    if (CAUSAL) {
+        if (!KV) t_hi = min(t_hi, max(0, own_base + G::OWN - 1 + P + OTHER) / OTHER);
+        else t_lo = max(0, own_base - P) / OTHER;
+    }
+
+    // staging by LDS-DMA, 1 KB per request; each wavefront requests its share of the slabs of both tiles.  The chunk
+    // swizzle is applied on the source side: the lane that writes physical chunk pc of row r fetches logical chunk
+    // pc ^ swizzle(r).  Rows past the end of the tensor are out of the descriptor's range and arrive as zeros.
+    // (Slices stay below 2 GiB -- checked on the host -- so 32-bit offsets do.)
+    const T* src_a = KV ? qp : kp;
+    const T* src_b = KV ? gp : vp;
+    const int a_srb = (int)(KV ? p.q_sr : p.k_sr) * 2, b_srb = (int)(KV ? p.do_sr : p.v_sr) * 2;     // row strides in bytes
+    const u32x4 rs_a = dma_rsrc(src_a, n_other > 0 ? (unsigned)(n_other - 1) * (unsigned)a_srb + D * 2 : 0u);
+    const u32x4 rs_b = dma_rsrc(src_b, n_other > 0 ? (unsigned)(n_other - 1) * (unsigned)b_srb + D * 2 : 0u);
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)bwd_smem;
+    // dk / dv: minus the log-sum-exp and minus delta of the tile's queries, one request of 64 words each (a tile of 32
+    // leaves the second half unused); wavefronts 2 and 3 repeat those of 0 and 1, so that all have the same count
+    const u32x4 rs_s = dma_rsrc((wave & 1 ? p.delta : p.lse2) + stat_base, n_other > 0 ? (unsigned)(n_other - 1) * (unsigned)(stat_sr * 4) + 4 : 0u);
+    auto request = [&](int t, int buf) {     // tile t into buffer buf
+#pragma unroll
+        for (int c = 0; c < G::SLABS; ++c) {
+            const int slab = G::SLABS * wave + c, row = slab * G::RPS + lane / CH, ch = (lane % CH) ^ row_swz<D>(row);
+            const unsigned at = (unsigned)buf * (2 * G::TILE) + slab * 1024u;
+            const int other = min(t * OTHER + row, n_other);     // (a row past the end: one that cannot wrap around)
+            dma_16(rs_a, lds0 + at, other * a_srb + ch * 16);
+            dma_16(rs_b, lds0 + at + G::TILE, other * b_srb + ch * 16);
+        }
+        if constexpr (KV) dma_4(rs_s, lds0 + G::STAT + buf * 512 + (wave & 1) * 256, (t * OTHER + lane) * (int)stat_sr * 4);
+    };
+    // Tile t + STAGES - 1 is requested when the barrier at the top of tile t has shown that every wavefront is done with
+    // the buffer it goes into (tile t - 1's): it has STAGES - 1 tiles' work to arrive in.
+#pragma unroll
+    for (int c = 0; c < G::STAGES - 1; ++c)
+        if (t_lo + c < t_hi) request(t_lo + c, c);
 
     // own rows as B operands: lane (lr, hh) holds elements 16 s + 8 hh .. + 7 of its row
     const bool own_ok = own_row < n_own;
@@ -433,68 +543,36 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd16_kernel(const BwdParams p
             for (int e = 0; e < 8; ++e) { fa[s][e] = (T)0.0f; fb[s][e] = (T)0.0f; }
             if (own_ok) {
                 fa[s] = *reinterpret_cast<const v8*>(a + 16 * s + 8 * hh);
-                fb[s] = *reinterpret_cast<const v8*>(c + 16 * s + 8 * hh);
+                if constexpr (DS) fb[s] = *reinterpret_cast<const v8*>(c + 16 * s + 8 * hh);
             }
         }
     }
-    float lse2_own = INFINITY, delta_own = 0.f;
-    if (!KV && own_ok) { lse2_own = p.lse2[stat_base + own_row * stat_sr]; delta_own = p.delta[stat_base + own_row * stat_sr]; }
+    // (rows past the end: -inf makes every probability of the row 0)
+    float nlse2_own = -INFINITY, ndelta_own = 0.f;
+    if (!KV && own_ok) { nlse2_own = p.lse2[stat_base + own_row * stat_sr]; ndelta_own = p.delta[stat_base + own_row * stat_sr]; }
 
-    int t_lo = 0, t_hi = (n_other + kBwdOther - 1) / kBwdOther;
-    if (CAUSAL) {
-        if (!KV) t_hi = min(t_hi, max(0, (own_base + kBwdOwn - 1 + P) / kBwdOther + 1));
-        else t_lo = max(0, own_base - P) / kBwdOther;
+    // bias per distance, ascending with the tile's row index in both passes (dk / dv: by -rel), so that consecutive
+    // rows are consecutive words; padded by 64 on both sides, more than the distances of a lane's rows span
+    float bias_lo = 0.f, bias_hi = 0.f;     // ... and of the two saturated sides
+    {
+        auto bias_at = [&](int rel) {
+            return load_table(p.table, p.table_dtype, (int64_t)bucket_of(p.bs, rel) * p.t_sbucket + (int64_t)h * p.t_shead) * 1.4426950408889634f;
+        };
+        const int mid = sat + G::LUT_PAD16;
+        for (int x = tid; x <= 2 * mid; x += kBwdThreads) lut[x] = has_bias ? bias_at(KV ? mid - x : x - mid) : 0.f;
+        if (has_bias) {
+            bias_lo = bias_at(-sat); bias_hi = bias_at(sat);
+            if constexpr (!KV) {
+                for (int x = tid; x <= 2 * sat; x += kBwdThreads) hist_rel[x] = 0.f;
+                for (int x = lane; x < G::SKEW_ROWS * 64; x += 64) skew[x] = 0.f;
+            }
+        }
     }
 
-    // staging by LDS-DMA: a tile is 8 slabs of 1 KB (8 rows); wavefront w requests slabs 2 w and 2 w + 1 of each of
-    // the two tiles.  The chunk swizzle is applied on the source side: the lane that writes physical chunk pc of row r
-    // fetches logical chunk pc ^ swizzle(r).  Rows past the end of the tensor are out of the descriptor's range and
-    // arrive as zeros.  (Slices stay below 2 GiB -- checked on the host -- so 32-bit offsets do.)
-    const T* src_a = KV ? qp : kp;
-    const T* src_b = KV ? gp : vp;
-    const int a_srb = (int)(KV ? p.q_sr : p.k_sr) * 2, b_srb = (int)(KV ? p.do_sr : p.v_sr) * 2;     // row strides in bytes
-    const u32x4 rs_a = dma_rsrc(src_a, n_other > 0 ? (unsigned)(n_other - 1) * (unsigned)a_srb + D * 2 : 0u);
-    const u32x4 rs_b = dma_rsrc(src_b, n_other > 0 ? (unsigned)(n_other - 1) * (unsigned)b_srb + D * 2 : 0u);
-    int dma_a[2], dma_b[2];     // this lane's byte offsets inside a tile, per slab
+    // row reads: element offsets of this lane's chunk (2 s + hh) of row lr; the 32-row halves of a tile differ by a constant
+    int row_off[KS];
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
-        const int row = (2 * wave + c) * 8 + (lane >> 3), ch = (lane & 7) ^ tile_swz(row);
-        dma_a[c] = row * a_srb + ch * 16;
-        dma_b[c] = row * b_srb + ch * 16;
-    }
-    const unsigned lds_a = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&ta2[0][0];
-    const unsigned lds_b = (unsigned)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)&tb2[0][0];
-    float rstat = 0.f;
-    auto request = [&](int t, int buf) {     // tile t into buffer buf: four requests per wavefront
-        const int o0 = t * kBwdOther;
-#pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const unsigned at = (unsigned)buf * (kBwdOther * D * 2) + (2 * wave + c) * 1024u;
-            dma_16(rs_a, lds_a + at, o0 * a_srb + dma_a[c]);
-            dma_16(rs_b, lds_b + at, o0 * b_srb + dma_b[c]);
-        }
-    };
-    auto fetch_stat = [&](int t) {
-        const int o0 = t * kBwdOther;
-        if (KV && tid < 2 * kBwdOther) {
-            const int row = tid & (kBwdOther - 1);
-            rstat = tid < kBwdOther ? INFINITY : 0.f;
-            if (o0 + row < n_other)
-                rstat = tid < kBwdOther ? p.lse2[stat_base + (o0 + row) * stat_sr] : p.delta[stat_base + (o0 + row) * stat_sr];
-        }
-    };
-    auto stage_stat = [&](int buf) {
-        if (KV && tid < 2 * kBwdOther) rowstat2[buf][tid] = rstat;
-    };
-    // row reads: element offsets of this lane's chunk (2 s + hh) of row 32 nt + lr
-    int row_off[NT][KS];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const int row = 32 * nt + lr;
-            row_off[nt][s] = row * D + (((2 * s + hh) ^ tile_swz(row)) * 8);
-        }
+    for (int s = 0; s < KS; ++s) row_off[s] = (sub0 + lr) * D + (((2 * s + hh) ^ row_swz<D>(lr)) * 8);
     // transposing reads: within a group of 16 lanes, lane 4 j + a supplies the address of elements 4 a' .. of row j
     // and receives, for column (lane % 16) of the group's 16 columns, the rows j = 0 .. 3.  Group g covers the
     // columns 32 dt + 16 (g & 1) .. + 15 and the rows 4 (g >> 1) .. + 3 (first read) and 8 more (second read).
@@ -504,186 +582,191 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd16_kernel(const BwdParams p
         const int row = 4 * (g >> 1) + jj, x = 2 * (g & 1) + (aa >> 1);
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) {
-            tr_lo[dt] = row * D + (((4 * dt + x) ^ tile_swz(row)) * 8) + (aa & 1) * 4;
-            tr_hi[dt] = (row + 8) * D + (((4 * dt + x) ^ tile_swz(row + 8)) * 8) + (aa & 1) * 4;
+            tr_lo[dt] = (sub0 + row) * D + (((4 * dt + x) ^ row_swz<D>(row)) * 8) + (aa & 1) * 4;
+            tr_hi[dt] = (sub0 + row + 8) * D + (((4 * dt + x) ^ row_swz<D>(row + 8)) * 8) + (aa & 1) * 4;
         }
     }
-    auto tr_frag = [&](const T* tile, int g16, int dt) {   // columns 32 dt .. + 31 x rows 16 g16 .. + 15 of the tile, as an A operand
+    auto tr_frag = [&](const T* tile, int g16, int dt) {   // columns 32 dt .. + 31 x rows 16 g16 .. + 15 of the block, as an A operand
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + tr_lo[dt] + 16 * g16 * D));
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + tr_hi[dt] + 16 * g16 * D));
         return __builtin_bit_cast(v8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
     };
 
-    f32x16 acc_a[DT], acc_b[DT];     // dQ^T or dK^T; dV^T
+    f32x16 acc_a[DA ? DT : 1], acc_b[DV ? DT : 1];     // dQ^T or dK^T; dV^T
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) { acc_a[dt][r] = 0.f; acc_b[dt][r] = 0.f; }
+        for (int r = 0; r < 16; ++r) { if constexpr (DA) acc_a[dt][r] = 0.f; if constexpr (DV) acc_b[dt][r] = 0.f; }
     float sum_lo = 0.f, sum_hi = 0.f;
+    const float c1 = p.c1;
 
-    // Tile t + 1 is requested when the barrier at the top of tile t has shown that every wavefront is done with the
-    // buffer it goes into, and has all of tile t's work to arrive in.
-    if (t_lo < t_hi) { request(t_lo, 0); fetch_stat(t_lo); stage_stat(0); }
-    // the per-distance bias (and bucket) table, behind the first tile's requests and the loads of the own rows: its
-    // look-ups in the bias table are one more round trip to memory, which now runs beside theirs
-    if (has_bias) {
-        for (int x = tid; x <= 2 * sat; x += kBwdThreads) {
-            const int bk = bucket_of(p.bs, x - sat);
-            lut_bias[x] = load_table(p.table, p.table_dtype, (int64_t)bk * p.t_sbucket + (int64_t)h * p.t_shead) * 1.4426950408889634f;
-            if constexpr (!KV) { lut_bucket[x] = bk; hist_rel[x] = 0.f; }
-        }
-        if constexpr (!KV)
-            for (int x = tid; x < p.n_buckets; x += kBwdThreads) hist[x] = 0.f;
-    }
-
-    for (int t = t_lo; t < t_hi; ++t) {
-        const int o0 = t * kBwdOther;
-        const int buf = (t - t_lo) & 1;
-        __builtin_amdgcn_s_waitcnt(0x0F70);     // vmcnt(0): this wavefront's requests for tile t have landed
-        __syncthreads();                        // ... and everybody's; the other buffer is free (and, first time round, the LUT written)
-        if (t + 1 < t_hi) { request(t + 1, buf ^ 1); fetch_stat(t + 1); }
-        const T* ta = ta2[buf]; const T* tb = tb2[buf];
-        const float* rowstat = rowstat2[buf];
+    for (int t = t_lo, buf = 0; t < t_hi; ++t, buf = buf + 1 == G::STAGES ? 0 : buf + 1) {
+        // this wavefront's requests for tile t have landed (those of the STAGES - 2 tiles behind it may be in flight) ...
+        if (G::STAGES > 2 && t + G::STAGES - 2 < t_hi) wait_vmcnt<(G::STAGES - 2) * G::REQS>(); else wait_vmcnt<0>();
+        __syncthreads();     // ... and everybody's; the buffer of tile t - 1 is free (and, first time round, the LUT written)
+        if (t + G::STAGES - 1 < t_hi) request(t + G::STAGES - 1, buf == 0 ? G::STAGES - 1 : buf - 1);
+        const T* ta = reinterpret_cast<const T*>(bwd_smem + buf * 2 * G::TILE);
+        const T* tb = reinterpret_cast<const T*>(bwd_smem + buf * 2 * G::TILE + G::TILE);
+        const float* rowstat = reinterpret_cast<const float*>(bwd_smem + G::STAT) + buf * 128 + sub0 + 4 * hh;
         (void)rowstat;
 
-        f32x16 s[NT], dp[NT];
+        const int s0 = t * OTHER + sub0;        // first tile row of this wavefront's block
+        // rel = j - (i + P): dq pass j in the tile, i own; dk / dv pass i in the tile, j own
+        const int rel_min = KV ? w_lo - (s0 + 31 + P) : s0 - (w_lo + 31 + P), rel_max = rel_min + 62;
+        if (s0 < n_other && (!CAUSAL || rel_min <= 0)) {
+            f32x16 s, dp;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            // (dP starts at -delta: the matrix core subtracts it for free)
+            for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
+            if constexpr (KV && DS) {      // (dP starts at -delta: the matrix core subtracts it for free)
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                f32x4 d4 = {delta_own, delta_own, delta_own, delta_own};
-                if constexpr (KV) d4 = *reinterpret_cast<const f32x4*>(rowstat + kBwdOther + 32 * nt + 8 * r4 + 4 * hh);
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(rowstat + 64 + 8 * r4);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { s[nt][4 * r4 + e] = 0.f; dp[nt][4 * r4 + e] = -d4[e]; }
+                    for (int e = 0; e < 4; ++e) dp[4 * r4 + e] = d4[e];
+                }
             }
+            // (the two chains in turn: 2 % faster than one behind the other)
 #pragma unroll
             for (int k2 = 0; k2 < KS; ++k2) {
-                s[nt] = H16::mfma(*reinterpret_cast<const v8*>(ta + row_off[nt][k2]), fa[k2], s[nt]);
-                dp[nt] = H16::mfma(*reinterpret_cast<const v8*>(tb + row_off[nt][k2]), fb[k2], dp[nt]);
+                s = H16::mfma(*reinterpret_cast<const v8*>(ta + row_off[k2]), fa[k2], s);
+                if constexpr (DS) dp = H16::mfma(*reinterpret_cast<const v8*>(tb + row_off[k2]), fb[k2], dp);
             }
-        }
 
-        // wavefront-uniform tile classes: every pair at a saturated distance on one side (constant bias); every pair
-        // visible (no per-element test)
-        const int w_lo = own_base + wave * 32, w_hi = w_lo + 31;            // this wavefront's own rows
-        // rel = j - (i + P): dq pass j in the tile, i own; dk/dv pass i in the tile, j own
-        const int rel_min = KV ? w_lo - (o0 + kBwdOther - 1 + P) : o0 - (w_hi + P);
-        const int rel_max = KV ? w_hi - (o0 + P) : o0 + kBwdOther - 1 - (w_lo + P);
-        int side = 0;
-        if (rel_max <= -sat) side = 1; else if (rel_min >= sat) side = 2;
-        const bool all_visible = o0 + kBwdOther <= n_other && w_hi < n_own && (!CAUSAL || rel_max <= 0);
-        const float c1 = p.c1;
-        float tile_sum = 0.f;
-        // Second stage, 16 rows of the tile at a time: probabilities and dS of this lane's eight pairs, rounded to
-        // the input type, then the products that contract over those rows --
-        //   dQ^T += K^T dS^T   /   dK^T += Q^T dS, dV^T += dO^T P
-        // -- so that the matrix cores work on one group while the vector units form the next.
-        auto second_stage = [&](auto check_c, auto lut_c) {
-            constexpr bool CHECK = decltype(check_c)::value, LUT = decltype(lut_c)::value;
-            const float bias_c = (has_bias && !LUT) ? lut_bias[side == 1 ? 0 : 2 * sat] : 0.f;
-            // Table gradient around the diagonal (dq pass, LUT variants): dS summed per distance.  Pairs at one
-            // distance lie on a diagonal of the (key, query) tile, and a lane half walks its keys in ascending order:
-            // each lane adds its dS to a running value that then moves one lane up (one query further) with every
-            // key, so a diagonal's sum travels with it.  A lane half holds the keys 8 k + 4 hh .. + 3: five lanes up
-            // between two groups.  What leaves a half at lane 31 is added to the distance's word in LDS first, and
-            // at the end of the tile every lane adds what it holds: some 190 single-lane atomic adds per tile and
-            // wavefront instead of 2 048 (an LDS floating-point atomic handles about one lane per cycle).
-            float diag = 0.f;
-            int x_last = 0;
-            (void)x_last;
+            // base-2 arguments of the probabilities; two classes of block (wavefront-uniform): every pair at a saturated
+            // distance on one side (one bias), or a look-up per pair
+            const bool sat_lo = rel_max <= -sat, sat_hi = rel_min >= sat;
+            if (sat_lo || sat_hi) {
+                const float bias_c = sat_lo ? bias_lo : bias_hi;
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    f32x4 l4 = {nlse2_own, nlse2_own, nlse2_own, nlse2_own};
+                    if constexpr (KV) l4 = *reinterpret_cast<const f32x4*>(rowstat + 8 * r4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[4 * r4 + e] = __builtin_fmaf(c1, s[4 * r4 + e], bias_c + l4[e]);
+                }
+            } else {
+                const float* lp = lut + (KV ? s0 + P - own_row : s0 - P - own_row) + 4 * hh + sat + G::LUT_PAD16;
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    f32x4 l4 = {nlse2_own, nlse2_own, nlse2_own, nlse2_own};
+                    if constexpr (KV) l4 = *reinterpret_cast<const f32x4*>(rowstat + 8 * r4);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) s[4 * r4 + e] = __builtin_fmaf(c1, s[4 * r4 + e], lp[8 * r4 + e]) + l4[e];
+                }
+            }
+            // blocks with an invisible pair (own rows past the end need no test: a query's probabilities are 0, a
+            // key's gradients are not stored)
+            if (s0 + 32 > n_other || (CAUSAL && rel_max > 0)) {
+                // (row 8 (r >> 2) + (r & 3) of the lane's half: visible from `first` on, up to `last`)
+                const int first = CAUSAL && KV ? own_row - P - s0 - 4 * hh : 0;
+                const int last = min(n_other - 1 - s0 - 4 * hh, CAUSAL && !KV ? own_row + P - s0 - 4 * hh : 32);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int ol = 8 * (r >> 2) + (r & 3);
+                    s[r] = (!(CAUSAL && KV) || ol >= first) && ol <= last ? s[r] : -INFINITY;
+                }
+            }
+            // probabilities and dS, rounded to the input type for the products that contract over the block's rows:
+            //   dQ^T += K^T dS^T   /   dV^T += dO^T P, dK^T += Q^T dS
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = __builtin_amdgcn_exp2f(s[r]);
+                if constexpr (KV) dp[r] *= s[r];
+                else dp[r] = (dp[r] + ndelta_own) * s[r];
+            }
+            if constexpr (DV) {
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
-                    f32x8 ds8, pv8;
+                    const v8 pb = to_frag<v8>(s, u);
 #pragma unroll
-                    for (int half = 0; half < 2; ++half) {
-                        const int r4 = 2 * u + half;
-                        const int ol0 = 32 * nt + 8 * r4 + 4 * hh;     // first of four consecutive rows of the other kind
-                        f32x4 l4 = {lse2_own, lse2_own, lse2_own, lse2_own};
-                        if constexpr (KV) l4 = *reinterpret_cast<const f32x4*>(rowstat + ol0);
-                        f32x4 bl4;   // constant bias minus log-sum-exp
+                    for (int dt = 0; dt < DT; ++dt) acc_b[dt] = H16::mfma(tr_frag(tb, u, dt), pb, acc_b[dt]);
+                }
+            }
+            if constexpr (DA) {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) bl4[e] = bias_c - l4[e];
+                for (int u = 0; u < 2; ++u) {
+                    const v8 dsb = to_frag<v8>(dp, u);
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int r = 4 * r4 + e, ol = ol0 + e;
-                            const int i = KV ? o0 + ol : own_row, j = KV ? own_row : o0 + ol;
-                            const int rel = j - (i + P);
-                            int x = 0;
-                            float bias2 = bias_c;
-                            if constexpr (LUT) {
-                                x = min(max(rel, -sat), sat) + sat;
-                                bias2 = lut_bias[x];
+                    for (int dt = 0; dt < DT; ++dt) acc_a[dt] = H16::mfma(tr_frag(ta, u, dt), dsb, acc_a[dt]);
+                }
+            }
+            if constexpr (!KV) {
+                if (has_bias) {
+                    if (sat_lo || sat_hi) {
+                        const float sum = ((dp[0] + dp[1]) + (dp[2] + dp[3])) + ((dp[4] + dp[5]) + (dp[6] + dp[7])) +
+                                          ((dp[8] + dp[9]) + (dp[10] + dp[11])) + ((dp[12] + dp[13]) + (dp[14] + dp[15]));
+                        if (sat_lo) sum_lo += sum; else sum_hi += sum;
+                    } else {
+                        // Table gradient around the diagonal: dS summed per distance.  The block goes to LDS skewed, the
+                        // pair of key kk and query lr at row lr, column kk - lr + R - 1, so that a column holds one
+                        // distance; a lane then sums a column.  What lies outside the skewed band is zero and never
+                        // written.  16 words written and R read per lane at constant offsets, without bank conflicts.
+                        // (A sum that travels through the lanes and leaves them by LDS atomics took 16 instructions per
+                        // score: the pass at B16 H12 L1024 went from 154 to 131 us, of which 36 are the table's.)
+                        constexpr int R = G::SKEW_ROWS;
+#pragma unroll
+                        for (int round = 0; round < 32 / R; ++round) {
+                            if (R == 32 || lr / R == round) {
+                                float* w = skew + (lr % R) * 63 + (R - 1) + 4 * hh;
+#pragma unroll
+                                for (int r = 0; r < 16; ++r) w[8 * (r >> 2) + (r & 3)] = dp[r];
                             }
-                            float pv = LUT ? __builtin_amdgcn_exp2f(__builtin_fmaf(c1, s[nt][r], bias2) - l4[e])
-                                           : __builtin_amdgcn_exp2f(__builtin_fmaf(c1, s[nt][r], bl4[e]));
-                            if constexpr (CHECK) {
-                                const bool valid = i < M && j < N && (!CAUSAL || rel <= 0);
-                                pv = valid ? pv : 0.f;
-                            }
-                            const float ds = pv * dp[nt][r];
-                            pv8[4 * half + e] = pv;
-                            ds8[4 * half + e] = ds;
-                            if constexpr (!KV) {
-                                // table gradient (no test for a table here: a branch per element would cut the
-                                // loop into pieces; without one the sum is simply not used, and the LUT variants
-                                // run only with one).  Per clamped distance: neighbouring lanes hold neighbouring
-                                // distances, so the adds of one instruction go to different words; a pair that
-                                // is not visible adds 0.
-                                if constexpr (!LUT) {
-                                    tile_sum += ds;
-                                } else {
-                                    diag += ds;      // (a pair that is not visible adds 0)
-                                    x_last = x;
-                                    const bool last_of_tile = nt == NT - 1 && u == 1 && half == 1 && e == 3;
-                                    if (!last_of_tile) {
-                                        const int out_from = e == 3 ? 27 : 31;     // lanes whose value leaves the half
-                                        if (lr >= out_from) { atomicAdd(&hist_rel[x], diag); diag = 0.f; }
+                            asm volatile("" ::: "memory");     // (LDS accesses of a wavefront keep their order)
+                            float c0 = 0.f, c1s = 0.f, c2 = 0.f, c3 = 0.f;
 #pragma unroll
-                                        for (int sh = 0; sh < (e == 3 ? 5 : 1); ++sh)
-                                            diag = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(diag), 0x138, 0xf, 0xf, true));
-                                    }
-                                }
+                            for (int q = 0; q < R; q += 4) {
+                                c0 += skew[q * 64 + lane]; c1s += skew[(q + 1) * 64 + lane];
+                                c2 += skew[(q + 2) * 64 + lane]; c3 += skew[(q + 3) * 64 + lane];
                             }
+                            asm volatile("" ::: "memory");
+                            const int rel = s0 - (w_lo + P) - R * round + lane - (R - 1);
+                            if (lane < 31 + R) atomicAdd(&hist_rel[min(max(rel, -sat), sat) + sat], (c0 + c1s) + (c2 + c3));
                         }
                     }
-                    const v8 dsb = __builtin_convertvector(ds8, v8);
-#pragma unroll
-                    for (int dt = 0; dt < DT; ++dt)
-                        acc_a[dt] = H16::mfma(tr_frag(ta, 2 * nt + u, dt), dsb, acc_a[dt]);
-                    if constexpr (KV) {
-                        const v8 pb = __builtin_convertvector(pv8, v8);
-#pragma unroll
-                        for (int dt = 0; dt < DT; ++dt)
-                            acc_b[dt] = H16::mfma(tr_frag(tb, 2 * nt + u, dt), pb, acc_b[dt]);
-                    }
                 }
-            if constexpr (!KV && LUT) atomicAdd(&hist_rel[x_last], diag);
-        };
-        const bool use_lut = has_bias && side == 0;
-        if (all_visible && !use_lut) second_stage(std::false_type{}, std::false_type{});
-        else if (all_visible) second_stage(std::false_type{}, std::true_type{});
-        else if (!use_lut) second_stage(std::true_type{}, std::false_type{});
-        else second_stage(std::true_type{}, std::true_type{});
-        if (side == 1) sum_lo += tile_sum; else if (side == 2) sum_hi += tile_sum;
-        if (t + 1 < t_hi) stage_stat(buf ^ 1);
+            }
+        }
     }
 
-    const float scale = p.c1 * 0.6931471805599453f;
-    if (own_ok) {
-        T* oa = KV ? reinterpret_cast<T*>(p.dk) + (int64_t)b * p.dk_sb + (int64_t)h * p.dk_sh + (k_first + own_row) * p.dk_sr
-                   : reinterpret_cast<T*>(p.dq) + (int64_t)b * p.dq_sb + (int64_t)h * p.dq_sh + (q_first + own_row) * p.dq_sr;
-        T* ob = KV ? reinterpret_cast<T*>(p.dv) + (int64_t)b * p.dv_sb + (int64_t)h * p.dv_sh + (k_first + own_row) * p.dv_sr : nullptr;
+    if constexpr (SPLIT > 1) {
+        // the partial gradients of the second half's wavefronts, in lane order through the tile buffers
+        float* const red = reinterpret_cast<float*>(bwd_smem) + ow * (((DA ? 1 : 0) + (DV ? 1 : 0)) * DT * 16 * 64) + lane;
+        constexpr int AT_B = DA ? DT * 16 : 0;
+        __syncthreads();
+        if (sub0 != 0) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    if constexpr (DA) red[(dt * 16 + r) * 64] = acc_a[dt][r];
+                    if constexpr (DV) red[(AT_B + dt * 16 + r) * 64] = acc_b[dt][r];
+                }
+        }
+        __syncthreads();
+        if (sub0 == 0) {
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    if constexpr (DA) acc_a[dt][r] += red[(dt * 16 + r) * 64];
+                    if constexpr (DV) acc_b[dt][r] += red[(AT_B + dt * 16 + r) * 64];
+                }
+        }
+    }
+    const float scale = p.c1 * 0.6931471805599453f;     // d score / d (q . k), natural units; dv has none
+    if (own_ok && sub0 == 0) {
+        T* oa = !KV ? reinterpret_cast<T*>(p.dq) + (int64_t)b * p.dq_sb + (int64_t)h * p.dq_sh + (q_first + own_row) * p.dq_sr
+                    : reinterpret_cast<T*>(p.dk) + (int64_t)b * p.dk_sb + (int64_t)h * p.dk_sh + (k_first + own_row) * p.dk_sr;
+        T* ob = DV ? reinterpret_cast<T*>(p.dv) + (int64_t)b * p.dv_sb + (int64_t)h * p.dv_sh + (k_first + own_row) * p.dv_sr : nullptr;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int d0 = 32 * dt + 8 * g + 4 * hh;
-                store4(oa + d0, f32x4{acc_a[dt][4 * g] * scale, acc_a[dt][4 * g + 1] * scale,
-                                      acc_a[dt][4 * g + 2] * scale, acc_a[dt][4 * g + 3] * scale});
-                if constexpr (KV)
+                if constexpr (DA)
+                    store4(oa + d0, f32x4{acc_a[dt][4 * g] * scale, acc_a[dt][4 * g + 1] * scale,
+                                          acc_a[dt][4 * g + 2] * scale, acc_a[dt][4 * g + 3] * scale});
+                if constexpr (DV)
                     store4(ob + d0, f32x4{acc_b[dt][4 * g], acc_b[dt][4 * g + 1], acc_b[dt][4 * g + 2], acc_b[dt][4 * g + 3]});
             }
     }
@@ -694,340 +777,16 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd16_kernel(const BwdParams p
                 sum_lo += __shfl_xor(sum_lo, off, 64);
                 sum_hi += __shfl_xor(sum_hi, off, 64);
             }
-            if (lane == 0) {
-                if (sum_lo != 0.f) atomicAdd(&hist[lut_bucket[0]], sum_lo);
-                if (sum_hi != 0.f) atomicAdd(&hist[lut_bucket[2 * sat]], sum_hi);
-            }
+            float* const hist = reinterpret_cast<float*>(bwd_smem);     // (the tiles are done with)
             __syncthreads();
-            for (int x = tid; x <= 2 * sat; x += kBwdThreads)     // distances -> buckets
-                if (hist_rel[x] != 0.f) atomicAdd(&hist[lut_bucket[x]], hist_rel[x]);
-            __syncthreads();
-            for (int x = tid; x < p.n_buckets; x += kBwdThreads)
-                if (hist[x] != 0.f) atomicAdd(&p.dtable[(int64_t)x * p.H + h], hist[x]);
-        }
-    }
-}
-
-// head_dim 128 (the T5-3B / 11B head shape), 16-bit tensors: the same scheme with rows of 256 bytes.  A row's head_dim
-// and two gradients of it no longer fit a wavefront's registers next to the scores, so there are three passes instead
-// of two -- PASS 0: dq (and the table gradient), 2: dk, 3: dv (which needs no dP) -- each with one output accumulator;
-// the tiles are single-buffered in LDS (two of 16 KB) and staged without a register prefetch.
-__device__ __forceinline__ int tile_swz128(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
-
-template <typename T, bool CAUSAL, int PASS>
-__global__ __launch_bounds__(kBwdThreads, 2) void bwd16_d128_kernel(const BwdParams p) {
-    constexpr bool KV = PASS != 0;
-    constexpr bool WANT_DS = PASS != 3;     // dS and the products with it (dq, dk)
-    constexpr bool WANT_DV = PASS == 3;
-    constexpr int D = 128, DT = 4, KS = 8, NT = kBwdOther / 32;
-    using H16 = Half16<T>;
-    using v8 = typename H16::v8;
-    __shared__ __attribute__((aligned(16))) T ta2[1][kBwdOther * D];   // K (dq) / Q (dk, dv) tile
-    __shared__ __attribute__((aligned(16))) T tb2[1][kBwdOther * D];   // V (dq) / dO (dk, dv) tile
-    __shared__ __attribute__((aligned(16))) float rowstat2[1][2 * kBwdOther];   // KV: lse2 and delta of the tile's queries
-    __shared__ float lut_bias[2 * kMaxSaturation + 1];
-    __shared__ int lut_bucket[KV ? 1 : 2 * kMaxSaturation + 1];
-    __shared__ float hist[KV ? 1 : kMaxBuckets];
-    __shared__ float hist_rel[KV ? 1 : 2 * kMaxSaturation + 1];   // dS summed per clamped distance (tiles around the diagonal)
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, hh = lane >> 5;
-    // Grid: (own blocks, heads, batch).  With a causal mask the own blocks differ in length (a query block sees the
-    // keys up to its own end, a key block the queries from its own start on), and whatever is dispatched last should
-    // be short: the launch is then (heads, batch, own blocks), the slowest index walking the blocks longest first.
-    const int h = CAUSAL ? blockIdx.x : blockIdx.y, b = CAUSAL ? blockIdx.y : blockIdx.z;
-    const int own_block = !CAUSAL ? blockIdx.x : (KV ? blockIdx.z : gridDim.z - 1 - blockIdx.z);
-    const int own_base = own_block * kBwdOwn;
-    const int own_row = own_base + wave * 32 + lr;
-    int M = p.M, N = p.N;
-    int64_t q_first = 0, k_first = 0;
-    if (p.cu_q != nullptr) {
-        q_first = p.cu_q[b]; k_first = p.cu_k[b];
-        M = p.len_q != nullptr ? p.len_q[b] : p.cu_q[b + 1] - (int)q_first;
-        N = p.len_k != nullptr ? p.len_k[b] : p.cu_k[b + 1] - (int)k_first;
-        if (own_base >= (KV ? N : M)) return;     // (the grid is sized for the longest sequence)
-    }
-    const int n_own = KV ? N : M, n_other = KV ? M : N;
-    const int P = N - M;
-    const bool has_bias = p.table != nullptr;
-    const int sat = has_bias ? p.bs.sat : 0;
-
-    const T* qp = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + q_first * p.q_sr;
-    const T* kp = reinterpret_cast<const T*>(p.k) + (int64_t)b * p.k_sb + (int64_t)h * p.k_sh + k_first * p.k_sr;
-    const T* vp = reinterpret_cast<const T*>(p.v) + (int64_t)b * p.v_sb + (int64_t)h * p.v_sh + k_first * p.v_sr;
-    const T* gp = reinterpret_cast<const T*>(p.dout) + (int64_t)b * p.do_sb + (int64_t)h * p.do_sh + q_first * p.do_sr;
-    const int64_t stat_sr = p.cu_q != nullptr ? p.H : 1;
-    const int64_t stat_base = p.cu_q != nullptr ? q_first * p.H + h : ((int64_t)b * p.H + h) * p.M;
-
-    if (has_bias) {
-        for (int x = tid; x <= 2 * sat; x += kBwdThreads) {
-            const int bk = bucket_of(p.bs, x - sat);
-            lut_bias[x] = load_table(p.table, p.table_dtype, (int64_t)bk * p.t_sbucket + (int64_t)h * p.t_shead) * 1.4426950408889634f;
-            if constexpr (!KV) { lut_bucket[x] = bk; hist_rel[x] = 0.f; }
-        }
-        if constexpr (!KV)
             for (int x = tid; x < p.n_buckets; x += kBwdThreads) hist[x] = 0.f;
-    }
-
-    // own rows as B operands: lane (lr, hh) holds elements 16 s + 8 hh .. + 7 of its row
-    const bool own_ok = own_row < n_own;
-    v8 fa[KS], fb[KS];
-    {
-        const T* a = (KV ? kp + (int64_t)own_row * p.k_sr : qp + (int64_t)own_row * p.q_sr);
-        const T* c = (KV ? vp + (int64_t)own_row * p.v_sr : gp + (int64_t)own_row * p.do_sr);
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) { fa[s][e] = (T)0.0f; fb[s][e] = (T)0.0f; }
-            if (own_ok) {
-                fa[s] = *reinterpret_cast<const v8*>(a + 16 * s + 8 * hh);
-                if constexpr (WANT_DS) fb[s] = *reinterpret_cast<const v8*>(c + 16 * s + 8 * hh);
-            }
-        }
-    }
-    float lse2_own = INFINITY, delta_own = 0.f;
-    if (!KV && own_ok) { lse2_own = p.lse2[stat_base + own_row * stat_sr]; delta_own = p.delta[stat_base + own_row * stat_sr]; }
-
-    int t_lo = 0, t_hi = (n_other + kBwdOther - 1) / kBwdOther;
-    if (CAUSAL) {
-        if (!KV) t_hi = min(t_hi, max(0, (own_base + kBwdOwn - 1 + P) / kBwdOther + 1));
-        else t_lo = max(0, own_base - P) / kBwdOther;
-    }
-
-    // staging: thread -> four 16-byte chunks of each tile (row = idx / 16, chunk = idx % 16)
-    const T* src_a = KV ? qp : kp;
-    const T* src_b = KV ? gp : vp;
-    const int64_t a_sr = KV ? p.q_sr : p.k_sr, b_sr = KV ? p.do_sr : p.v_sr;
-    u32x4 ra[4], rb[4];
-    float rstat = 0.f;
-    auto fetch = [&](int t) {
-        const int o0 = t * kBwdOther;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int idx = tid + c * kBwdThreads, row = idx >> 4, ch = idx & 15;
-            ra[c] = u32x4{0u, 0u, 0u, 0u}; rb[c] = u32x4{0u, 0u, 0u, 0u};
-            if (o0 + row < n_other) {
-                ra[c] = *reinterpret_cast<const u32x4*>(src_a + (int64_t)(o0 + row) * a_sr + 8 * ch);
-                rb[c] = *reinterpret_cast<const u32x4*>(src_b + (int64_t)(o0 + row) * b_sr + 8 * ch);
-            }
-        }
-        if (KV && tid < 2 * kBwdOther) {
-            const int row = tid & (kBwdOther - 1);
-            rstat = tid < kBwdOther ? INFINITY : 0.f;
-            if (o0 + row < n_other)
-                rstat = tid < kBwdOther ? p.lse2[stat_base + (o0 + row) * stat_sr] : p.delta[stat_base + (o0 + row) * stat_sr];
-        }
-    };
-    auto stage = [&](int buf) {
-        T* ta = ta2[buf]; T* tb = tb2[buf];
-        float* rowstat = rowstat2[buf];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const int idx = tid + c * kBwdThreads, row = idx >> 4, ch = idx & 15;
-            const int at = row * D + ((ch ^ tile_swz128(row)) * 8);
-            *reinterpret_cast<u32x4*>(ta + at) = ra[c];
-            *reinterpret_cast<u32x4*>(tb + at) = rb[c];
-        }
-        if (KV && tid < 2 * kBwdOther) rowstat[tid] = rstat;
-    };
-    // row reads: element offsets of this lane's chunk (2 s + hh) of row 32 nt + lr
-    int row_off[NT][KS];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const int row = 32 * nt + lr;
-            row_off[nt][s] = row * D + (((2 * s + hh) ^ tile_swz128(row)) * 8);
-        }
-    // transposing reads: within a group of 16 lanes, lane 4 j + a supplies the address of elements 4 a' .. of row j
-    // and receives, for column (lane % 16) of the group's 16 columns, the rows j = 0 .. 3.  Group g covers the
-    // columns 32 dt + 16 (g & 1) .. + 15 and the rows 4 (g >> 1) .. + 3 (first read) and 8 more (second read).
-    int tr_lo[DT], tr_hi[DT];
-    {
-        const int g = lane >> 4, r = lane & 15, jj = r >> 2, aa = r & 3;
-        const int row = 4 * (g >> 1) + jj, x = 2 * (g & 1) + (aa >> 1);
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) {
-            tr_lo[dt] = row * D + (((4 * dt + x) ^ tile_swz128(row)) * 8) + (aa & 1) * 4;
-            tr_hi[dt] = (row + 8) * D + (((4 * dt + x) ^ tile_swz128(row + 8)) * 8) + (aa & 1) * 4;
-        }
-    }
-    auto tr_frag = [&](const T* tile, int g16, int dt) {   // columns 32 dt .. + 31 x rows 16 g16 .. + 15 of the tile, as an A operand
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + tr_lo[dt] + 16 * g16 * D));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3)))*)(tile + tr_hi[dt] + 16 * g16 * D));
-        return __builtin_bit_cast(v8, (s16x8)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    };
-
-    f32x16 acc_a[DT];     // dQ^T, dK^T or dV^T
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc_a[dt][r] = 0.f;
-    float sum_lo = 0.f, sum_hi = 0.f;
-
-    for (int t = t_lo; t < t_hi; ++t) {
-        const int o0 = t * kBwdOther;
-        __syncthreads();     // the previous tile's readers are done (and the LUT is written, first time round)
-        fetch(t);
-        stage(0);
-        __syncthreads();
-        const T* ta = ta2[0]; const T* tb = tb2[0];
-        const float* rowstat = rowstat2[0];
-        (void)rowstat;
-
-        f32x16 s[NT], dp[NT];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            // (dP starts at -delta: the matrix core subtracts it for free)
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) {
-                f32x4 d4 = {delta_own, delta_own, delta_own, delta_own};
-                if constexpr (KV) d4 = *reinterpret_cast<const f32x4*>(rowstat + kBwdOther + 32 * nt + 8 * r4 + 4 * hh);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) { s[nt][4 * r4 + e] = 0.f; dp[nt][4 * r4 + e] = WANT_DS ? -d4[e] : 0.f; }
-            }
-#pragma unroll
-            for (int k2 = 0; k2 < KS; ++k2) {
-                s[nt] = H16::mfma(*reinterpret_cast<const v8*>(ta + row_off[nt][k2]), fa[k2], s[nt]);
-                if constexpr (WANT_DS) dp[nt] = H16::mfma(*reinterpret_cast<const v8*>(tb + row_off[nt][k2]), fb[k2], dp[nt]);
-            }
-        }
-
-        // wavefront-uniform tile classes: every pair at a saturated distance on one side (constant bias); every pair
-        // visible (no per-element test)
-        const int w_lo = own_base + wave * 32, w_hi = w_lo + 31;            // this wavefront's own rows
-        // rel = j - (i + P): dq pass j in the tile, i own; dk/dv pass i in the tile, j own
-        const int rel_min = KV ? w_lo - (o0 + kBwdOther - 1 + P) : o0 - (w_hi + P);
-        const int rel_max = KV ? w_hi - (o0 + P) : o0 + kBwdOther - 1 - (w_lo + P);
-        int side = 0;
-        if (rel_max <= -sat) side = 1; else if (rel_min >= sat) side = 2;
-        const bool all_visible = o0 + kBwdOther <= n_other && w_hi < n_own && (!CAUSAL || rel_max <= 0);
-        const float c1 = p.c1;
-        float tile_sum = 0.f;
-        // Second stage, 16 rows of the tile at a time: probabilities and dS of this lane's eight pairs, rounded to
-        // the input type, then the products that contract over those rows --
-        //   dQ^T += K^T dS^T   /   dK^T += Q^T dS, dV^T += dO^T P
-        // -- so that the matrix cores work on one group while the vector units form the next.
-        auto second_stage = [&](auto check_c, auto lut_c) {
-            constexpr bool CHECK = decltype(check_c)::value, LUT = decltype(lut_c)::value;
-            const float bias_c = (has_bias && !LUT) ? lut_bias[side == 1 ? 0 : 2 * sat] : 0.f;
-            // Table gradient around the diagonal (dq pass, LUT variants): dS summed per distance.  Pairs at one
-            // distance lie on a diagonal of the (key, query) tile, and a lane half walks its keys in ascending order:
-            // each lane adds its dS to a running value that then moves one lane up (one query further) with every
-            // key, so a diagonal's sum travels with it.  A lane half holds the keys 8 k + 4 hh .. + 3: five lanes up
-            // between two groups.  What leaves a half at lane 31 is added to the distance's word in LDS first, and
-            // at the end of the tile every lane adds what it holds: some 190 single-lane atomic adds per tile and
-            // wavefront instead of 2 048 (an LDS floating-point atomic handles about one lane per cycle).
-            float diag = 0.f;
-            int x_last = 0;
-            (void)x_last;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                for (int u = 0; u < 2; ++u) {
-                    f32x8 ds8, pv8;
-#pragma unroll
-                    for (int half = 0; half < 2; ++half) {
-                        const int r4 = 2 * u + half;
-                        const int ol0 = 32 * nt + 8 * r4 + 4 * hh;     // first of four consecutive rows of the other kind
-                        f32x4 l4 = {lse2_own, lse2_own, lse2_own, lse2_own};
-                        if constexpr (KV) l4 = *reinterpret_cast<const f32x4*>(rowstat + ol0);
-                        f32x4 bl4;   // constant bias minus log-sum-exp
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) bl4[e] = bias_c - l4[e];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int r = 4 * r4 + e, ol = ol0 + e;
-                            const int i = KV ? o0 + ol : own_row, j = KV ? own_row : o0 + ol;
-                            const int rel = j - (i + P);
-                            int x = 0;
-                            float bias2 = bias_c;
-                            if constexpr (LUT) {
-                                x = min(max(rel, -sat), sat) + sat;
-                                bias2 = lut_bias[x];
-                            }
-                            float pv = LUT ? __builtin_amdgcn_exp2f(__builtin_fmaf(c1, s[nt][r], bias2) - l4[e])
-                                           : __builtin_amdgcn_exp2f(__builtin_fmaf(c1, s[nt][r], bl4[e]));
-                            if constexpr (CHECK) {
-                                const bool valid = i < M && j < N && (!CAUSAL || rel <= 0);
-                                pv = valid ? pv : 0.f;
-                            }
-                            const float ds = pv * dp[nt][r];
-                            pv8[4 * half + e] = pv;
-                            ds8[4 * half + e] = ds;
-                            if constexpr (!KV) {
-                                // table gradient (no test for a table here: a branch per element would cut the
-                                // loop into pieces; without one the sum is simply not used, and the LUT variants
-                                // run only with one).  Per clamped distance: neighbouring lanes hold neighbouring
-                                // distances, so the adds of one instruction go to different words; a pair that
-                                // is not visible adds 0.
-                                if constexpr (!LUT) {
-                                    tile_sum += ds;
-                                } else {
-                                    diag += ds;      // (a pair that is not visible adds 0)
-                                    x_last = x;
-                                    const bool last_of_tile = nt == NT - 1 && u == 1 && half == 1 && e == 3;
-                                    if (!last_of_tile) {
-                                        const int out_from = e == 3 ? 27 : 31;     // lanes whose value leaves the half
-                                        if (lr >= out_from) { atomicAdd(&hist_rel[x], diag); diag = 0.f; }
-#pragma unroll
-                                        for (int sh = 0; sh < (e == 3 ? 5 : 1); ++sh)
-                                            diag = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(diag), 0x138, 0xf, 0xf, true));
-                                    }
-                                }
-                            }
-                        }
-                    }
-                    if constexpr (WANT_DS) {
-                        const v8 dsb = __builtin_convertvector(ds8, v8);
-#pragma unroll
-                        for (int dt = 0; dt < DT; ++dt)
-                            acc_a[dt] = H16::mfma(tr_frag(ta, 2 * nt + u, dt), dsb, acc_a[dt]);
-                    }
-                    if constexpr (WANT_DV) {
-                        const v8 pb = __builtin_convertvector(pv8, v8);
-#pragma unroll
-                        for (int dt = 0; dt < DT; ++dt)
-                            acc_a[dt] = H16::mfma(tr_frag(tb, 2 * nt + u, dt), pb, acc_a[dt]);
-                    }
-                }
-            if constexpr (!KV && LUT) atomicAdd(&hist_rel[x_last], diag);
-        };
-        const bool use_lut = has_bias && side == 0;
-        if (all_visible && !use_lut) second_stage(std::false_type{}, std::false_type{});
-        else if (all_visible) second_stage(std::false_type{}, std::true_type{});
-        else if (!use_lut) second_stage(std::true_type{}, std::false_type{});
-        else second_stage(std::true_type{}, std::true_type{});
-        if (side == 1) sum_lo += tile_sum; else if (side == 2) sum_hi += tile_sum;
-    }
-
-    const float scale = WANT_DV ? 1.0f : p.c1 * 0.6931471805599453f;     // d score / d (q . k), natural units; dv has none
-    if (own_ok) {
-        T* oa = PASS == 0 ? reinterpret_cast<T*>(p.dq) + (int64_t)b * p.dq_sb + (int64_t)h * p.dq_sh + (q_first + own_row) * p.dq_sr
-              : PASS == 2 ? reinterpret_cast<T*>(p.dk) + (int64_t)b * p.dk_sb + (int64_t)h * p.dk_sh + (k_first + own_row) * p.dk_sr
-                          : reinterpret_cast<T*>(p.dv) + (int64_t)b * p.dv_sb + (int64_t)h * p.dv_sh + (k_first + own_row) * p.dv_sr;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d0 = 32 * dt + 8 * g + 4 * hh;
-                store4(oa + d0, f32x4{acc_a[dt][4 * g] * scale, acc_a[dt][4 * g + 1] * scale,
-                                      acc_a[dt][4 * g + 2] * scale, acc_a[dt][4 * g + 3] * scale});
-            }
-    }
-    if constexpr (!KV) {
-        if (has_bias && p.dtable != nullptr) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                sum_lo += __shfl_xor(sum_lo, off, 64);
-                sum_hi += __shfl_xor(sum_hi, off, 64);
-            }
-            if (lane == 0) {
-                if (sum_lo != 0.f) atomicAdd(&hist[lut_bucket[0]], sum_lo);
-                if (sum_hi != 0.f) atomicAdd(&hist[lut_bucket[2 * sat]], sum_hi);
-            }
             __syncthreads();
+            if (lane == 0) {
+                if (sum_lo != 0.f) atomicAdd(&hist[bucket_of(p.bs, -sat)], sum_lo);
+                if (sum_hi != 0.f) atomicAdd(&hist[bucket_of(p.bs, sat)], sum_hi);
+            }
             for (int x = tid; x <= 2 * sat; x += kBwdThreads)     // distances -> buckets
-                if (hist_rel[x] != 0.f) atomicAdd(&hist[lut_bucket[x]], hist_rel[x]);
+                if (hist_rel[x] != 0.f) atomicAdd(&hist[bucket_of(p.bs, x - sat)], hist_rel[x]);
             __syncthreads();
             for (int x = tid; x < p.n_buckets; x += kBwdThreads)
                 if (hist[x] != 0.f) atomicAdd(&p.dtable[(int64_t)x * p.H + h], hist[x]);
@@ -1035,6 +794,48 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd16_d128_kernel(const BwdPar
     }
 }
 
+// Whether a pass runs with SPLIT 2: own blocks of 64 instead of 128 rows, each block of scores walked by two wavefronts.
+// It halves the longest chain and doubles the workgroups, at twice the fetches per product, so it pays where 128-row
+// blocks leave the chip idle (256 compute units with room for three workgroups at head_dim 64, two at 128).  Both
+// sides, us, three kernels, bf16: head_dim 64 full attention, 256 workgroups 245 / 190 (SPLIT 1 / 2), 384 294 / 276, 512
+// 302 / 333; causal, where the longest block counts, 512 233 / 182, 1536 181 / 228; head_dim 128 256 440 / 325, 384
+// 504 / 586, causal 256 208 / 140, 512 259 / 221, 1024 390 / 441.  Packed, head_dim 64 (workgroups counted from the
+// tokens): 424 67 / 73, causal 58 / 58, 564 186 / 183, 1464 212 / 222.
+bool bwd16_split(const BwdParams& p, int D, bool causal, int rows) {
+    const int64_t blocks = p.cu_q != nullptr ? ((int64_t)p.total_q / 128 + p.B) * p.H : (int64_t)((rows + 127) / 128) * p.H * p.B;
+    return blocks < (p.cu_q != nullptr ? 320 : causal ? 768 : D == 64 ? 512 : 320);
+}
+
+template <typename T, int D, bool CAUSAL, int PASS, int SPLIT>
+hipError_t launch_bwd16_pass(const BwdParams& p, hipStream_t stream) {
+    using G = Bwd16Geom<D, PASS, SPLIT>;
+    const int rows = PASS != 0 ? p.N : p.M;
+    if (rows <= 0) return hipSuccess;
+    const int nblk = (rows + G::OWN - 1) / G::OWN;
+    const int64_t blocks = (int64_t)nblk * p.H * p.B;
+    if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
+    const bool bias = p.table != nullptr;
+    hipLaunchKernelGGL((bwd16_kernel<T, D, CAUSAL, PASS, SPLIT>), dim3((unsigned)blocks), dim3(kBwdThreads),
+                       G::bytes(bias ? p.bs.sat : 0, bias), stream, p, nblk);
+    return hipGetLastError();
+}
+
+template <typename T, int D, bool CAUSAL, int PASS>
+hipError_t launch_bwd16_rows(const BwdParams& p, hipStream_t stream) {
+    return bwd16_split(p, D, CAUSAL, PASS != 0 ? p.N : p.M) ? launch_bwd16_pass<T, D, CAUSAL, PASS, 2>(p, stream)
+                                                            : launch_bwd16_pass<T, D, CAUSAL, PASS, 1>(p, stream);
+}
+
+template <typename T, int D, bool CAUSAL>
+hipError_t launch_bwd16(const BwdParams& p, hipStream_t stream) {
+    hipError_t e = launch_bwd16_rows<T, D, CAUSAL, 0>(p, stream);
+    if (e != hipSuccess) return e;
+    if constexpr (D == 64) return launch_bwd16_rows<T, D, CAUSAL, 1>(p, stream);
+    // head_dim 128: a row's head_dim twice and two gradients of it do not fit 256 registers next to the scores
+    // (the joint pass spills and takes 721 us where the two take 592: B4 H6 L4096)
+    if ((e = launch_bwd16_rows<T, D, CAUSAL, 2>(p, stream)) != hipSuccess) return e;
+    return launch_bwd16_rows<T, D, CAUSAL, 3>(p, stream);
+}
 
 template <typename T, int D>
 hipError_t launch_bwd_d(const BwdParams& p, bool causal, hipStream_t stream) {
@@ -1042,56 +843,19 @@ hipError_t launch_bwd_d(const BwdParams& p, bool causal, hipStream_t stream) {
     hipLaunchKernelGGL((bwd_rows_kernel<T, D>), dim3((unsigned)((rows + RowsGeom<T, D>::ROWS - 1) / RowsGeom<T, D>::ROWS)), dim3(256), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const dim3 gq((p.M + kBwdOwn - 1) / kBwdOwn, p.H, p.B), gk((p.N + kBwdOwn - 1) / kBwdOwn, p.H, p.B);
-    if constexpr (sizeof(T) == 2 && D == 64) {
-        if (p.fp32_math == 0) {
-            if (causal) {
-                const dim3 cq(p.H, p.B, gq.x), ck(p.H, p.B, gk.x);
-                hipLaunchKernelGGL((bwd16_kernel<T, true, false>), cq, dim3(kBwdThreads), 0, stream, p);
-                if (p.N > 0) hipLaunchKernelGGL((bwd16_kernel<T, true, true>), ck, dim3(kBwdThreads), 0, stream, p);
-            } else {
-                hipLaunchKernelGGL((bwd16_kernel<T, false, false>), gq, dim3(kBwdThreads), 0, stream, p);
-                if (p.N > 0) hipLaunchKernelGGL((bwd16_kernel<T, false, true>), gk, dim3(kBwdThreads), 0, stream, p);
-            }
-            return hipGetLastError();
-        }
+    if constexpr (sizeof(T) == 2 && (D == 64 || D == 128)) {
+        if (p.fp32_math == 0) return causal ? launch_bwd16<T, D, true>(p, stream) : launch_bwd16<T, D, false>(p, stream);
     }
-    if (causal) {
-        hipLaunchKernelGGL((bwd_kernel<T, D, true, false>), gq, dim3(kBwdThreads), 0, stream, p);
-        if (p.N > 0) hipLaunchKernelGGL((bwd_kernel<T, D, true, true>), gk, dim3(kBwdThreads), 0, stream, p);
+    if constexpr (D == 128) {
+        return hipErrorInvalidValue;     // (the fp32 kernels hold a row's head_dim in registers: up to 64)
     } else {
-        hipLaunchKernelGGL((bwd_kernel<T, D, false, false>), gq, dim3(kBwdThreads), 0, stream, p);
-        if (p.N > 0) hipLaunchKernelGGL((bwd_kernel<T, D, false, true>), gk, dim3(kBwdThreads), 0, stream, p);
-    }
-    return hipGetLastError();
-}
-
-// head_dim 128, 16-bit tensors: row statistics, then one pass per gradient
-template <typename T>
-hipError_t launch_bwd_d128(const BwdParams& p, bool causal, hipStream_t stream) {
-    if constexpr (sizeof(T) != 2) {
-        return hipErrorInvalidValue;
-    } else {
-        if (p.fp32_math != 0) return hipErrorInvalidValue;     // (the fp32 kernels hold a row's head_dim in registers: up to 64)
-        const int64_t rows = p.cu_q != nullptr ? (int64_t)p.total_q * p.H : (int64_t)p.B * p.H * p.M;
-        hipLaunchKernelGGL((bwd_rows_kernel<T, 128>), dim3((unsigned)((rows + RowsGeom<T, 128>::ROWS - 1) / RowsGeom<T, 128>::ROWS)), dim3(256), 0, stream, p);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        const unsigned nq = (p.M + kBwdOwn - 1) / kBwdOwn, nk = (p.N + kBwdOwn - 1) / kBwdOwn;
+        const dim3 gq((p.M + kBwdOwn - 1) / kBwdOwn, p.H, p.B), gk((p.N + kBwdOwn - 1) / kBwdOwn, p.H, p.B);
         if (causal) {
-            const dim3 cq(p.H, p.B, nq), ck(p.H, p.B, nk);
-            hipLaunchKernelGGL((bwd16_d128_kernel<T, true, 0>), cq, dim3(kBwdThreads), 0, stream, p);
-            if (p.N > 0) {
-                hipLaunchKernelGGL((bwd16_d128_kernel<T, true, 2>), ck, dim3(kBwdThreads), 0, stream, p);
-                hipLaunchKernelGGL((bwd16_d128_kernel<T, true, 3>), ck, dim3(kBwdThreads), 0, stream, p);
-            }
+            hipLaunchKernelGGL((bwd_kernel<T, D, true, false>), gq, dim3(kBwdThreads), 0, stream, p);
+            if (p.N > 0) hipLaunchKernelGGL((bwd_kernel<T, D, true, true>), gk, dim3(kBwdThreads), 0, stream, p);
         } else {
-            const dim3 gq(nq, p.H, p.B), gk(nk, p.H, p.B);
-            hipLaunchKernelGGL((bwd16_d128_kernel<T, false, 0>), gq, dim3(kBwdThreads), 0, stream, p);
-            if (p.N > 0) {
-                hipLaunchKernelGGL((bwd16_d128_kernel<T, false, 2>), gk, dim3(kBwdThreads), 0, stream, p);
-                hipLaunchKernelGGL((bwd16_d128_kernel<T, false, 3>), gk, dim3(kBwdThreads), 0, stream, p);
-            }
+            hipLaunchKernelGGL((bwd_kernel<T, D, false, false>), gq, dim3(kBwdThreads), 0, stream, p);
+            if (p.N > 0) hipLaunchKernelGGL((bwd_kernel<T, D, false, true>), gk, dim3(kBwdThreads), 0, stream, p);
         }
         return hipGetLastError();
     }
@@ -1100,7 +864,9 @@ hipError_t launch_bwd_d128(const BwdParams& p, bool causal, hipStream_t stream) 
 template <typename T>
 hipError_t launch_bwd_t(const BwdParams& p, int D, bool causal, hipStream_t s) {
     switch (D) {
-        case 128: return launch_bwd_d128<T>(p, causal, s);
+        case 128:
+            if constexpr (sizeof(T) == 2) return launch_bwd_d<T, 128>(p, causal, s);
+            break;
         case 16: return launch_bwd_d<T, 16>(p, causal, s);
         case 32: return launch_bwd_d<T, 32>(p, causal, s);
         case 64: return launch_bwd_d<T, 64>(p, causal, s);

@@ -116,6 +116,24 @@ def test_16_bit_gradients_at_head_dim_128(gpu_device, dtype, causal, B, H, M, N)
         check(name, g, w, TOL[dtype])
 
 
+@pytest.mark.parametrize("D", [16, 32, 64])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("M,N", [(450, 513), (63, 33), (257, 64)])
+def test_fp32_gradients_over_blocks_of_64_rows(gpu_device, causal, M, N, D):
+    """The fp32 kernels own 64 rows per workgroup and share a tile of 64 between two wavefronts: sizes around a block, rows
+    with distances saturated on both sides of the diagonal."""
+    from turbot5_amd import ops
+    B, H = 1, 3
+    q, k, v = (rnd(B, H, n, D, seed=101 + i) for i, n in enumerate((M, N, N)))
+    table = rnd(32, H, seed=104, scale=1.0)
+    dout = rnd(B, H, M, D, seed=105, scale=1.0)
+    _, wq, wk, wv, wt = oracle_grads(q, k, v, table, dout, causal, 1.0)
+    dq, dk, dv, dt = (t.to(gpu_device).requires_grad_(True) for t in (q, k, v, table))
+    ops.flash_attention_with_fusing_bias(dq, dk, dv, dt, causal=causal, sm_scale=1.0).backward(dout.to(gpu_device))
+    for name, g, w in (("dq", dq.grad, wq), ("dk", dk.grad, wk), ("dv", dv.grad, wv), ("dtable", dt.grad, wt)):
+        check(name, g, w, TOL[torch.float32])
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("B,H,M,N", [(48, 16, 33, 65), (53, 15, 130, 97), (24, 16, 290, 257)])

@@ -10,14 +10,14 @@
 //
 //   bwd_rows_kernel   delta_i = sum_d o_id do_id and the log-sum-exp in base-2 units, per query row, both negated; also
 //                     clears the table gradient
-//   bwd_kernel<KV=0>  a workgroup owns 128 query rows (32 per wavefront) and walks the key tiles of 64:
-//                     S^T = K Q^T, dP^T = V dO^T (key rows from LDS as the A operand, so a lane owns one query and
-//                     its log-sum-exp and delta are lane scalars), P^T = exp2(c1 S^T + bias - lse),
-//                     dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T.  The table gradient is collected here: tiles whose
-//                     distances are all saturated add their dS to one of two lane sums, the tiles around the
-//                     diagonal add element by element into a per-bucket histogram in LDS; one global atomic per
-//                     bucket and workgroup at the end.
-//   bwd_kernel<KV=1>  a workgroup owns 128 keys and walks the query tiles of 64, the same products with the roles
+//   bwd_kernel<KV=0>  a workgroup owns 64 query rows (32 per wavefront) and walks the key tiles of 64 (32 of the 64 per
+//                     wavefront): S^T = K Q^T, dP^T = V dO^T (key rows from LDS as the A operand, so a lane owns one
+//                     query and its log-sum-exp and delta are lane scalars), P^T = exp2(c1 S^T + bias - lse),
+//                     dS^T = P^T (dP^T - delta), dQ^T += K^T dS^T.  The table gradient is collected here: blocks whose
+//                     distances are all saturated add their dS to one of two lane sums, the blocks around the
+//                     diagonal are summed per distance through LDS; distances go to buckets at the end, and one
+//                     global atomic per bucket and workgroup to the table.
+//   bwd_kernel<KV=1>  a workgroup owns 64 keys and walks the query tiles of 64, the same products with the roles
 //                     swapped (query rows from LDS; log-sum-exp and delta of the 64 queries staged in LDS):
 //                     dV^T += dO^T P, dK^T += Q^T dS.
 //
@@ -37,7 +37,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kBwdThreads = 256;
-constexpr int kBwdOwn = 128;     // own rows per workgroup (queries for dq, keys for dk / dv)
+constexpr int kBwdOwn = 64;      // own rows per workgroup of the fp32 kernels (queries for dq, keys for dk / dv)
 constexpr int kBwdOther = 64;    // rows of the other kind per tile
 constexpr int kMaxBuckets = 2 * 2 * kMaxThresholds;
 
@@ -121,23 +121,35 @@ __global__ __launch_bounds__(256) void bwd_rows_kernel(const BwdParams p) {
     p.lse2[row] = l == -INFINITY ? -INFINITY : l * -1.4426950408889634f;
 }
 
+// A workgroup owns 64 rows and walks tiles of 64, whose halves go to different wavefronts; their partial gradients are
+// added through LDS at the end.  One 32 x 32 block of scores per wavefront leaves registers to fetch the next tile's rows
+// under the current tile's products.  The fp32 matrix cores (64 cycles per product) bound it.  128 own rows and no
+// prefetch took, with every table-gradient pair added to LDS by an atomic, 259 us where this takes 135 (B4 H8 L512 D64, the
+// three kernels: 64-row blocks fill 256 compute units, 128-row blocks half of them), 674 / 515 at B4 H12 L1024 and
+// 1210 / 925 at B8 H12 L1024; without the atomics 219, 615 and 1004, so the small blocks are the better at every size.
 template <typename T, int D, bool CAUSAL, bool KV>
 __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) {
     constexpr int STR = D + 1;              // fp32 tile rows padded by one float
     constexpr int DT = (D + 31) / 32;       // 32-row blocks of the transposed gradients
     constexpr int KS = D / 2;               // k-steps of a product over head_dim
-    constexpr int NT = kBwdOther / 32;
-    __shared__ float ta[kBwdOther * STR + 32];     // K (dq) / Q (dk, dv) tile
-    __shared__ float tb[kBwdOther * STR + 32];     // V (dq) / dO (dk, dv) tile
+    constexpr int OWNW = kBwdOwn / 32;
+    constexpr int TILE = kBwdOther * STR + 32;
+    constexpr int RED = OWNW * (KV ? 2 : 1) * DT * 16 * 64;
+    constexpr int SKEW_ROWS = 8;
+    __shared__ float tiles[2 * TILE > RED ? 2 * TILE : RED];
+    float* const ta = tiles;               // K (dq) / Q (dk, dv) tile
+    float* const tb = tiles + TILE;        // V (dq) / dO (dk, dv) tile
     __shared__ float rowstat[2 * kBwdOther];       // KV: lse2 and delta of the tile's queries
     __shared__ float lut_bias[2 * kMaxSaturation + 1];   // bias * log2(e) per clamped distance
-    __shared__ int lut_bucket[KV ? 1 : 2 * kMaxSaturation + 1];
-    __shared__ float hist[KV ? 1 : kMaxBuckets];
+    __shared__ float hist_rel[KV ? 1 : 2 * kMaxSaturation + 1];   // dS summed per clamped distance
+    __shared__ float skew_all[KV ? 1 : 4 * SKEW_ROWS * 64];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, lr = lane & 31, hh = lane >> 5;
     const int h = blockIdx.y, b = blockIdx.z;
     const int own_base = blockIdx.x * kBwdOwn;
-    const int own_row = own_base + wave * 32 + lr;
+    const int w_lo = own_base + (wave % OWNW) * 32, own_row = w_lo + lr;
+    const int sub0 = (wave / OWNW) * 32;      // first tile row of this wavefront's block
+    float* const skew = skew_all + (KV ? 0 : wave * SKEW_ROWS * 64);
     // packed batch: sequence b is the rows [cu[b], cu[b] + len) of the (total, H, D) tensors (len from seq_lens when
     // given, else up to cu[b + 1]); the batch strides are 0 and everything below works on that sequence
     int M = p.M, N = p.N;
@@ -166,10 +178,10 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
         for (int x = tid; x <= 2 * sat; x += kBwdThreads) {
             const int bk = bucket_of(p.bs, x - sat);
             lut_bias[x] = load_table(p.table, p.table_dtype, (int64_t)bk * p.t_sbucket + (int64_t)h * p.t_shead) * 1.4426950408889634f;
-            if constexpr (!KV) lut_bucket[x] = bk;
+            if constexpr (!KV) hist_rel[x] = 0.f;
         }
         if constexpr (!KV)
-            for (int x = tid; x < p.n_buckets; x += kBwdThreads) hist[x] = 0.f;
+            for (int x = lane; x < SKEW_ROWS * 64; x += 64) skew[x] = 0.f;
     }
 
     // own rows as B operands of the 32x32x2 products: lane (lr, hh) holds elements 2s + hh of its row
@@ -203,97 +215,140 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
         for (int r = 0; r < 16; ++r) { acc_a[dt][r] = 0.f; acc_b[dt][r] = 0.f; }
     float sum_lo = 0.f, sum_hi = 0.f;   // dS of the tiles saturated on the left / on the right of the diagonal
 
+    // staging: thread -> 16-byte (of fp32) chunks of both tiles' rows, and with KV one row statistic
+    constexpr int CHUNKS = kBwdOther * (D / 4) / kBwdThreads;
+    f32x4 xa[CHUNKS], xb[CHUNKS];
+    float stat = 0.f;
+    auto fetch = [&](int o0) {
+        const T* a = KV ? qp : kp;
+        const T* c = KV ? gp : vp;
+        const int64_t a_sr = KV ? p.q_sr : p.k_sr, c_sr = KV ? p.do_sr : p.v_sr;
+#pragma unroll
+        for (int n = 0; n < CHUNKS; ++n) {
+            const int idx = tid + n * kBwdThreads, row = idx / (D / 4), c4 = idx % (D / 4);
+            xa[n] = f32x4{0.f, 0.f, 0.f, 0.f}; xb[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (o0 + row < n_other) {
+                xa[n] = load4(a + (int64_t)(o0 + row) * a_sr + 4 * c4);
+                xb[n] = load4(c + (int64_t)(o0 + row) * c_sr + 4 * c4);
+            }
+        }
+        if (KV && tid < 2 * kBwdOther) {
+            const int row = tid & (kBwdOther - 1);
+            stat = tid < kBwdOther ? -INFINITY : 0.f;
+            if (o0 + row < n_other)
+                stat = tid < kBwdOther ? p.lse2[stat_base + (o0 + row) * stat_sr] : p.delta[stat_base + (o0 + row) * stat_sr];
+        }
+    };
+    if (t_lo < t_hi) fetch(t_lo * kBwdOther);
+
     for (int t = t_lo; t < t_hi; ++t) {
         const int o0 = t * kBwdOther;
         __syncthreads();     // the previous tile's readers are done (and the LUT is written, first time round)
-        {
-            const T* a = KV ? qp : kp;
-            const T* c = KV ? gp : vp;
-            const int64_t a_sr = KV ? p.q_sr : p.k_sr, c_sr = KV ? p.do_sr : p.v_sr;
-            for (int idx = tid; idx < kBwdOther * (D / 4); idx += kBwdThreads) {
-                const int row = idx / (D / 4), c4 = idx % (D / 4);
-                f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = {0.f, 0.f, 0.f, 0.f};
-                if (o0 + row < n_other) {
-                    x = load4(a + (int64_t)(o0 + row) * a_sr + 4 * c4);
-                    y = load4(c + (int64_t)(o0 + row) * c_sr + 4 * c4);
-                }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) { ta[row * STR + 4 * c4 + e] = x[e]; tb[row * STR + 4 * c4 + e] = y[e]; }
-            }
-            if (KV && tid < 2 * kBwdOther) {
-                const int row = tid & (kBwdOther - 1);
-                float val = tid < kBwdOther ? -INFINITY : 0.f;
-                if (o0 + row < n_other)
-                    val = tid < kBwdOther ? p.lse2[stat_base + (o0 + row) * stat_sr] : p.delta[stat_base + (o0 + row) * stat_sr];
-                rowstat[tid] = val;
-            }
+        for (int n = 0; n < CHUNKS; ++n) {
+            const int idx = tid + n * kBwdThreads, row = idx / (D / 4), c4 = idx % (D / 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { ta[row * STR + 4 * c4 + e] = xa[n][e]; tb[row * STR + 4 * c4 + e] = xb[n][e]; }
         }
+        if (KV && tid < 2 * kBwdOther) rowstat[tid] = stat;
         __syncthreads();
+        if (t + 1 < t_hi) fetch(o0 + kBwdOther);
 
-        f32x16 s[NT], dp[NT];
+        f32x16 s, dp;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
+        for (int r = 0; r < 16; ++r) { s[r] = 0.f; dp[r] = 0.f; }
+        const float* const row_a = ta + (sub0 + lr) * STR + hh;
+        const float* const row_b = tb + (sub0 + lr) * STR + hh;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) { s[nt][r] = 0.f; dp[nt][r] = 0.f; }
-            const int row = 32 * nt + lr;
-#pragma unroll
-            for (int k2 = 0; k2 < KS; ++k2) {
-                s[nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ta[row * STR + 2 * k2 + hh], fa[k2], s[nt], 0, 0, 0);
-                dp[nt] = __builtin_amdgcn_mfma_f32_32x32x2f32(tb[row * STR + 2 * k2 + hh], fb[k2], dp[nt], 0, 0, 0);
-            }
+        for (int k2 = 0; k2 < KS; ++k2) {
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(row_a[2 * k2], fa[k2], s, 0, 0, 0);
+            dp = __builtin_amdgcn_mfma_f32_32x32x2f32(row_b[2 * k2], fb[k2], dp, 0, 0, 0);
         }
 
-        // wavefront-uniform: every pair of this wavefront's tile lies at a saturated distance on one side
-        int side = 0;
-        if constexpr (!KV) {
-            const int i_lo = own_base + wave * 32 + P, i_hi = i_lo + 31;    // query positions
-            if (o0 + kBwdOther - 1 - i_lo <= -sat) side = 1;
-            else if (o0 - i_hi >= sat) side = 2;
-        }
         float tile_sum = 0.f;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+        for (int r = 0; r < 16; ++r) {
+            const int ol = sub0 + 8 * (r >> 2) + 4 * hh + (r & 3);   // row of the other kind inside the tile
+            const int i = KV ? o0 + ol : own_row, j = KV ? own_row : o0 + ol;
+            const int rel = j - (i + P);
+            const bool valid = i < M && j < N && (!CAUSAL || rel <= 0);
+            const float bias2 = has_bias ? lut_bias[min(max(rel, -sat), sat) + sat] : 0.f;
+            const float l2 = KV ? rowstat[ol] : lse2_own;
+            const float dl = KV ? rowstat[kBwdOther + ol] : delta_own;
+            const float pv = valid ? __builtin_amdgcn_exp2f(__builtin_fmaf(p.c1, s[r], bias2) + l2) : 0.f;
+            const float ds = pv * (dp[r] + dl);
+            s[r] = pv;
+            dp[r] = ds;
+            tile_sum += ds;
+        }
+        if constexpr (!KV) {
+            // (wavefront-uniform) every pair of the block at a saturated distance on one side, or dS summed per
+            // distance by way of LDS, as in bwd16_kernel: the pair of key kk and query lr at row lr, column
+            // kk - lr + R - 1.  (One LDS atomic per pair took two thirds of the pass.)
+            const int rel_min = o0 + sub0 - (w_lo + 31 + P), rel_max = rel_min + 62;
+            if (has_bias) {
+                if (rel_max <= -sat) sum_lo += tile_sum;
+                else if (rel_min >= sat) sum_hi += tile_sum;
+                else {
+                    constexpr int R = SKEW_ROWS;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int ol = 32 * nt + 8 * (r >> 2) + 4 * hh + (r & 3);   // row of the other kind inside the tile
-                const int i = KV ? o0 + ol : own_row, j = KV ? own_row : o0 + ol;
-                const int rel = j - (i + P);
-                const bool valid = i < M && j < N && (!CAUSAL || rel <= 0);
-                const int x = min(max(rel, -sat), sat) + sat;
-                const float bias2 = has_bias ? lut_bias[x] : 0.f;
-                const float l2 = KV ? rowstat[ol] : lse2_own;
-                const float dl = KV ? rowstat[kBwdOther + ol] : delta_own;
-                const float pv = valid ? __builtin_amdgcn_exp2f(__builtin_fmaf(p.c1, s[nt][r], bias2) + l2) : 0.f;
-                const float ds = pv * (dp[nt][r] + dl);
-                s[nt][r] = pv;
-                dp[nt][r] = ds;
-                if constexpr (!KV) {
-                    if (has_bias) {
-                        if (side != 0) tile_sum += ds;
-                        else if (valid) atomicAdd(&hist[lut_bucket[x]], ds);
+                    for (int round = 0; round < 32 / R; ++round) {
+                        if (lr / R == round) {
+                            float* w = skew + (lr % R) * 63 + (R - 1) + 4 * hh;
+#pragma unroll
+                            for (int r = 0; r < 16; ++r) w[8 * (r >> 2) + (r & 3)] = dp[r];
+                        }
+                        asm volatile("" ::: "memory");     // (LDS accesses of a wavefront keep their order)
+                        float sum = 0.f;
+#pragma unroll
+                        for (int q = 0; q < R; ++q) sum += skew[q * 64 + lane];
+                        asm volatile("" ::: "memory");
+                        const int rel = rel_min + 31 - R * round + lane - (R - 1);
+                        if (lane < 31 + R) atomicAdd(&hist_rel[min(max(rel, -sat), sat) + sat], sum);
                     }
                 }
             }
-        if (side == 1) sum_lo += tile_sum; else if (side == 2) sum_hi += tile_sum;
+        }
 
-        // dQ^T += K^T dS^T   /   dK^T += Q^T dS, dV^T += dO^T P   (contraction over the tile's 64 rows, two per product)
+        // dQ^T += K^T dS^T   /   dK^T += Q^T dS, dV^T += dO^T P   (contraction over the block's 32 rows, two per product)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
+        for (int r = 0; r < 16; ++r) {
+            const int ol = sub0 + 8 * (r >> 2) + 4 * hh + (r & 3);
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) {
+                acc_a[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ta[ol * STR + 32 * dt + lr], dp[r], acc_a[dt], 0, 0, 0);
+                if constexpr (KV)
+                    acc_b[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(tb[ol * STR + 32 * dt + lr], s[r], acc_b[dt], 0, 0, 0);
+            }
+        }
+    }
+
+    // the partial gradients of the other half's wavefronts, in lane order
+    float* const red = tiles + (wave % OWNW) * ((KV ? 2 : 1) * DT * 16 * 64) + lane;
+    __syncthreads();
+    if (sub0 != 0) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int ol = 32 * nt + 8 * (r >> 2) + 4 * hh + (r & 3);
+                red[(dt * 16 + r) * 64] = acc_a[dt][r];
+                if constexpr (KV) red[((DT + dt) * 16 + r) * 64] = acc_b[dt][r];
+            }
+    }
+    __syncthreads();
+    if (sub0 == 0) {
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) {
-                    acc_a[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(ta[ol * STR + 32 * dt + lr], dp[nt][r], acc_a[dt], 0, 0, 0);
-                    if constexpr (KV)
-                        acc_b[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(tb[ol * STR + 32 * dt + lr], s[nt][r], acc_b[dt], 0, 0, 0);
-                }
+        for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                acc_a[dt][r] += red[(dt * 16 + r) * 64];
+                if constexpr (KV) acc_b[dt][r] += red[((DT + dt) * 16 + r) * 64];
             }
     }
 
     // rows: lane (lr, hh) holds, for its own row, elements 32 dt + 8 g + 4 hh .. + 3 of the transposed gradients
     const float scale = p.c1 * 0.6931471805599453f;     // d score / d (q . k), natural units
-    if (own_ok) {
+    if (own_ok && sub0 == 0) {
         T* oa = KV ? reinterpret_cast<T*>(p.dk) + (int64_t)b * p.dk_sb + (int64_t)h * p.dk_sh + (k_first + own_row) * p.dk_sr
                    : reinterpret_cast<T*>(p.dq) + (int64_t)b * p.dq_sb + (int64_t)h * p.dq_sh + (q_first + own_row) * p.dq_sr;
         T* ob = KV ? reinterpret_cast<T*>(p.dv) + (int64_t)b * p.dv_sb + (int64_t)h * p.dv_sh + (k_first + own_row) * p.dv_sr : nullptr;
@@ -318,10 +373,16 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
                 sum_lo += __shfl_xor(sum_lo, off, 64);
                 sum_hi += __shfl_xor(sum_hi, off, 64);
             }
+            float* const hist = tiles;     // (the tiles are done with)
+            __syncthreads();
+            for (int x = tid; x < p.n_buckets; x += kBwdThreads) hist[x] = 0.f;
+            __syncthreads();
             if (lane == 0) {
-                if (sum_lo != 0.f) atomicAdd(&hist[lut_bucket[0]], sum_lo);
-                if (sum_hi != 0.f) atomicAdd(&hist[lut_bucket[2 * sat]], sum_hi);
+                if (sum_lo != 0.f) atomicAdd(&hist[bucket_of(p.bs, -sat)], sum_lo);
+                if (sum_hi != 0.f) atomicAdd(&hist[bucket_of(p.bs, sat)], sum_hi);
             }
+            for (int x = tid; x <= 2 * sat; x += kBwdThreads)     // distances -> buckets
+                if (hist_rel[x] != 0.f) atomicAdd(&hist[bucket_of(p.bs, x - sat)], hist_rel[x]);
             __syncthreads();
             for (int x = tid; x < p.n_buckets; x += kBwdThreads)
                 if (hist[x] != 0.f) atomicAdd(&p.dtable[(int64_t)x * p.H + h], hist[x]);

@@ -409,6 +409,24 @@ typedef struct t5a_rmsnorm_args {
 } t5a_rmsnorm_args;
 int t5a_rmsnorm(const t5a_rmsnorm_args* args, t5a_stream_t stream);
 
+/*
+ * The norm of a training step: x (rows, dim) contiguous, rstd (rows) fp32 1 / sqrt(mean square + eps) of each row.
+ * y set: y = weight * (x * rstd) with t5a_rmsnorm's types and roundings.
+ * y NULL: the backward.  dy is the gradient of y in y's type, dsum (optional, x's type) is added to dx; dx has x's type,
+ * dweight the weight's, summed in a fixed order.  dim: a multiple of 8, at most 2048.
+ */
+typedef struct t5a_rmsnorm_train_args {
+    const void* x; const void* weight; const float* rstd;
+    void* y;
+    const void* dy; const void* dsum;
+    void* dx; void* dweight;
+    void* workspace; int64_t workspace_bytes;   /* backward: t5a_rmsnorm_bwd_workspace_bytes(rows, dim), 16-byte aligned */
+    int64_t rows; int32_t dim;
+    int32_t x_dtype; int32_t weight_dtype; int32_t reserved;
+} t5a_rmsnorm_train_args;
+int64_t t5a_rmsnorm_bwd_workspace_bytes(int64_t rows, int32_t dim);
+int t5a_rmsnorm_train(const t5a_rmsnorm_train_args* args, t5a_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -182,3 +182,76 @@ def test_side_token_producer_with_masks_of_any_shape(gpu_device, dtype, L, gbs):
         assert (got[b, counts[b].item():] == 0).all()
     with pytest.raises(ValueError):
         rms_norm(hidden.to(gpu_device), w.to(gpu_device), 1e-6, group=gbs, key_bits=pack_key_bits(dmask, gbs))
+
+
+def _formula(x, w, eps):
+    n = x * torch.rsqrt(x.pow(2).mean(-1, keepdim=True) + eps)
+    return w * n
+
+
+@pytest.mark.parametrize("xdt,wdt", [("f32", "f32"), ("bf16", "bf16"), ("f32", "f16"), ("f16", "f32")])
+@pytest.mark.parametrize("rows,d", [(1, 8), (3, 256), (5, 264), (2050, 512), (9000, 768), (130, 1024), (33, 2048)])
+@pytest.mark.parametrize("with_residual", [False, True])
+def test_norm_gradients_match_the_formula_in_64_bits(gpu_device, xdt, wdt, rows, d, with_residual):
+    """Module in training mode: dx (with the residual stream's gradient added) and dweight.  Rows from one wavefront's
+    to several per wavefront, columns around the register chunks of 256.  Bounds: fp32 sums of up to 9000 terms, 2e-6
+    of the largest times their root; 16-bit weights round n and g (2^-9 each) and the results once more."""
+    from turbot5_amd.attentions import T5LayerNorm
+    g = torch.Generator().manual_seed(rows * 7 + d)
+    x = torch.randn(rows, d, generator=g).to(DT[xdt])
+    r = torch.randn(rows, d, generator=g).to(DT[xdt])
+    w = (1.0 + 0.2 * torch.randn(d, generator=g)).to(DT[wdt])
+    norm = T5LayerNorm(d).to(gpu_device).train()
+    norm.weight = torch.nn.Parameter(w.to(gpu_device))
+    xg, rg = (t.to(gpu_device).requires_grad_() for t in (x, r))
+    total, y = norm.add_norm(xg, rg if with_residual else None)
+    with torch.no_grad():     # bit for bit the formula in torch's operations
+        tt = xg + rg if with_residual else xg
+        n = tt * torch.rsqrt(tt.float().pow(2).mean(-1, keepdim=True) + norm.eps)
+        assert torch.equal(total, tt) and torch.equal(y, norm.weight * (n.to(w.dtype) if w.dtype != torch.float32 else n))
+    dy, ds = torch.randn(rows, d, generator=g).to(y.dtype), torch.randn(rows, d, generator=g).to(total.dtype)
+    outs, grads = ([total, y], [ds, dy]) if with_residual else ([y], [dy])
+    torch.autograd.backward(outs, [t.to(gpu_device) for t in grads])
+    x64 = ((x + r) if with_residual else x).double().requires_grad_()
+    w64 = w.double().requires_grad_()
+    (_formula(x64, w64, 1e-6) * dy.double()).sum().backward()
+    want = x64.grad + (ds.double() if with_residual else 0)
+    tol = 2e-5 if xdt == wdt == "f32" else 2e-2 if "bf16" in (xdt, wdt) else 4e-3
+    scale = want.abs().max().item()
+    assert (xg.grad.double().cpu() - want).abs().max().item() <= tol * scale
+    if with_residual:
+        assert torch.equal(xg.grad, rg.grad)
+    assert xg.grad.dtype == x.dtype and norm.weight.grad.dtype == w.dtype
+    assert (norm.weight.grad.double().cpu() - w64.grad).abs().max().item() <= tol * w64.grad.abs().max().item()
+
+
+def test_norm_gradients_where_the_kernel_is_passed_by(gpu_device):
+    """Differentiating the gradient, function transforms, forward mode, widths past the kernel's and empty batches take the
+    formula in torch's operations; a saved-tensor hook sees what is saved."""
+    from turbot5_amd.attentions import T5LayerNorm
+    norm = T5LayerNorm(64).to(gpu_device).train()
+    with torch.no_grad():
+        norm.weight.copy_(torch.linspace(0.5, 1.5, 64))
+    x = torch.randn(6, 64, generator=torch.Generator().manual_seed(1)).to(gpu_device).requires_grad_()
+
+    def second(f):
+        gx, = torch.autograd.grad(f(x).pow(3).sum(), x, create_graph=True)
+        return torch.autograd.grad(gx.pow(2).sum(), (x, norm.weight))
+    for got, want in zip(second(norm), second(lambda t: _formula(t, norm.weight, 1e-6))):
+        assert torch.allclose(got, want, rtol=1e-3, atol=1e-3)
+    total, y = norm.add_norm(x, 2 * x)
+    gx, = torch.autograd.grad(y.pow(2).sum() + total.sum(), x, create_graph=True)
+    assert gx.requires_grad
+    t = torch.randn_like(x)
+    got = torch.func.jvp(norm, (x.detach(),), (t,))[1]
+    want = torch.func.jvp(lambda v: _formula(v, norm.weight, 1e-6), (x.detach(),), (t,))[1]
+    assert torch.allclose(got, want, atol=1e-5)
+    assert torch.allclose(torch.vmap(norm)(x), norm(x), atol=1e-6)
+    seen = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda s: seen.append(s) or s, lambda s: s):
+        norm(x).sum().backward()
+    assert seen and x.grad is not None
+    wide = T5LayerNorm(4096).to(gpu_device).train()
+    wide(torch.randn(2, 4096, device=gpu_device)).sum().backward()
+    assert wide.weight.grad is not None
+    norm(torch.empty(0, 64, device=gpu_device)).sum().backward()

@@ -22,7 +22,7 @@ EXPORTS = (
     "t5a_version", "t5a_last_error", "t5a_bucket_lut", "t5a_fwd_dense", "t5a_bwd_dense", "t5a_bwd_workspace_bytes", "t5a_bwd_varlen", "t5a_bwd_varlen_workspace_bytes", "t5a_fwd_varlen",
     "t5a_varlen_workspace_bytes", "t5a_bias_lut_bytes", "t5a_bias_lut_bytes_windowed",
     "t5a_fwd_sparse", "t5a_sparse_launch_plan", "t5a_sparse_workspace_bytes", "t5a_sparse_key_bits_words", "t5a_splitk_workspace_bytes", "t5a_fwd_splitk", "t5a_fwd_splitk_static",
-    "t5a_rmsnorm",
+    "t5a_rmsnorm", "t5a_rmsnorm_train", "t5a_rmsnorm_bwd_workspace_bytes",
 )
 
 
@@ -122,6 +122,16 @@ class T5ARmsNormArgs(C.Structure):
                 ("key_bits", C.c_void_p), ("key_bits_stride", C.c_int64), ("group_counts", C.c_void_p)]
 
 
+class T5ARmsNormTrainArgs(C.Structure):
+    _fields_ = [("x", C.c_void_p), ("weight", C.c_void_p), ("rstd", C.c_void_p), ("y", C.c_void_p),
+                ("dy", C.c_void_p), ("dsum", C.c_void_p), ("dx", C.c_void_p), ("dweight", C.c_void_p),
+                ("workspace", C.c_void_p), ("workspace_bytes", C.c_int64),
+                ("rows", C.c_int64), ("dim", C.c_int32), ("x_dtype", C.c_int32), ("weight_dtype", C.c_int32),
+                ("reserved", C.c_int32)]
+
+
+RMSNORM_TRAIN_MAX_DIM = 2048
+
 _lib = None
 _lock = threading.Lock()
 
@@ -167,6 +177,10 @@ def load() -> C.CDLL:
         lib.t5a_splitk_workspace_bytes.restype = C.c_int64
         lib.t5a_rmsnorm.argtypes = [C.POINTER(T5ARmsNormArgs), C.c_void_p]
         lib.t5a_rmsnorm.restype = C.c_int
+        lib.t5a_rmsnorm_train.argtypes = [C.POINTER(T5ARmsNormTrainArgs), C.c_void_p]
+        lib.t5a_rmsnorm_train.restype = C.c_int
+        lib.t5a_rmsnorm_bwd_workspace_bytes.argtypes = [C.c_int64, C.c_int32]
+        lib.t5a_rmsnorm_bwd_workspace_bytes.restype = C.c_int64
         lib.t5a_bias_lut_bytes.argtypes = [C.c_int32] * 4
         lib.t5a_bias_lut_bytes.restype = C.c_int64
         lib.t5a_bias_lut_bytes_windowed.argtypes = [C.c_int32] * 4

@@ -49,12 +49,17 @@ class T5LayerNorm(nn.Module):
         """On a ROCm device: the fused HIP kernel (the reference switches to its Triton kernel there,
         modules.py:61-66).  Host tensors take the reference's eager formula (modules.py:51-59).
         ``group`` > 1 norms the sums of ``group`` consecutive rows of each sequence (side tokens)."""
-        # (the kernel has no backward: a module in training mode that is being differentiated takes the eager formula)
+        # (a module in training mode that is being differentiated: the kernel with its backward where that takes the
+        # call, else the eager formula)
         differentiated = self.training and torch.is_grad_enabled() and (x.requires_grad or self.weight.requires_grad)
         if x.is_cuda and not (differentiated and seq_lens is None and key_bits is None):
             from .ops import rms_norm
             return rms_norm(x, self.weight, self.eps, group, seq_lens=seq_lens, seq_starts=seq_starts,
                             key_bits=key_bits, group_counts=group_counts)
+        if group == 1 and differentiated and seq_lens is None and key_bits is None:
+            from .ops import RmsNorm, rms_norm_differentiable
+            if rms_norm_differentiable(x, self.weight):
+                return RmsNorm.apply(x, self.weight, self.eps, None)[1]
         if group > 1:
             B, L, d = x.shape
             n = L // group
@@ -79,6 +84,10 @@ class T5LayerNorm(nn.Module):
         if x.is_cuda and residual.dtype == x.dtype and not differentiated:
             from .ops import rms_norm
             return rms_norm(x, self.weight, self.eps, 1, residual)
+        if self.training and differentiated:
+            from .ops import RmsNorm, rms_norm_differentiable
+            if rms_norm_differentiable(x, self.weight, residual):
+                return RmsNorm.apply(x, self.weight, self.eps, residual)
         total = x + residual
         return total, self.forward(total)
 

@@ -973,4 +973,34 @@ int t5a_rmsnorm(const t5a_rmsnorm_args* a, t5a_stream_t stream) {
     return finish(launch_rmsnorm(p, a->x_dtype, a->weight_dtype, (hipStream_t)stream), "t5a_rmsnorm");
 }
 
+int64_t t5a_rmsnorm_bwd_workspace_bytes(int64_t rows, int32_t dim) {
+    if (rows < 0 || dim <= 0) return -1;
+    return (int64_t)rmsnorm_bwd_blocks(rows) * dim * (int64_t)sizeof(float);
+}
+
+int t5a_rmsnorm_train(const t5a_rmsnorm_train_args* a, t5a_stream_t stream) {
+    if (a == nullptr) return fail(T5A_ERR_NULL, "args is NULL");
+    for (int dt : {a->x_dtype, a->weight_dtype})
+        if (dt != T5A_BF16 && dt != T5A_F16 && dt != T5A_F32) return fail(T5A_ERR_DTYPE, "unsupported dtype %d", dt);
+    if (a->rows <= 0 || a->rows > (int64_t)4 * 0x7fffffff || a->dim <= 0 || a->dim % 8 != 0 || a->dim > kRmsBwdMaxDim)
+        return fail(T5A_ERR_SHAPE, "bad sizes rows=%lld dim=%d (rows > 0; dim a multiple of 8, at most %d)", (long long)a->rows, a->dim, kRmsBwdMaxDim);
+    if (a->x == nullptr || a->weight == nullptr || a->rstd == nullptr) return fail(T5A_ERR_NULL, "x, weight or rstd is NULL");
+    for (const void* t : {a->x, (const void*)a->y, a->dy, a->dsum, (const void*)a->dx, (const void*)a->workspace})
+        if (!aligned16(t)) return fail(T5A_ERR_STRIDE, "x, y, dy, dsum, dx and workspace must be 16-byte aligned");
+    if (a->y == nullptr) {
+        for (const void* t : {a->dy, (const void*)a->dx, (const void*)a->dweight, (const void*)a->workspace})
+            if (t == nullptr) return fail(T5A_ERR_NULL, "backward: dy, dx, dweight or workspace is NULL");
+        const int64_t need = t5a_rmsnorm_bwd_workspace_bytes(a->rows, a->dim);
+        if (a->workspace_bytes < need)
+            return fail(T5A_ERR_WORKSPACE, "t5a_rmsnorm_train: workspace of %lld bytes needed, %lld given", (long long)need, (long long)a->workspace_bytes);
+    }
+    RmsBwdParams p;
+    memset(&p, 0, sizeof(p));
+    p.x = a->x; p.weight = a->weight; p.rstd = a->rstd; p.y = a->y;
+    p.dy = a->dy; p.dsum = a->dsum; p.dx = a->dx; p.dweight = a->dweight;
+    p.partial = reinterpret_cast<float*>(a->workspace);
+    p.rows = a->rows; p.dim = a->dim; p.n_partial = rmsnorm_bwd_blocks(a->rows);
+    return finish(launch_rmsnorm_train(p, a->x_dtype, a->weight_dtype, (hipStream_t)stream), "t5a_rmsnorm_train");
+}
+
 }  // extern "C"

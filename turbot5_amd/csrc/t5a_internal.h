@@ -162,4 +162,15 @@ struct RmsParams {
 };
 hipError_t launch_rmsnorm(const RmsParams& p, int x_dtype, int w_dtype, hipStream_t stream);
 
+// The norm of a training step over contiguous rows whose factors 1 / sqrt(mean square + eps) are given: y set: the scaled rows; else the
+// backward, with partial holding rmsnorm_bwd_blocks(rows) x dim floats
+constexpr int kRmsBwdMaxDim = 2048;   // a row and its sums stay in registers
+struct RmsBwdParams {
+    const void* x; const void* weight; const float* rstd; const void* dy; const void* dsum;
+    void* y; void* dx; void* dweight; float* partial;
+    int64_t rows; int dim, n_partial;
+};
+int rmsnorm_bwd_blocks(int64_t rows);
+hipError_t launch_rmsnorm_train(const RmsBwdParams& p, int x_dtype, int w_dtype, hipStream_t stream);
+
 }  // namespace t5a

@@ -748,6 +748,88 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, group: in
     return y if total is None else (total, y)
 
 
+def _rms_norm_eager(x, weight, eps):
+    """The reference's formula (src/turbot5/model/modules.py:51-59)."""
+    n = x * torch.rsqrt(x.to(torch.float32).pow(2).mean(-1, keepdim=True) + eps)
+    return weight * (n.to(weight.dtype) if weight.dtype in (torch.float16, torch.bfloat16) else n)
+
+
+def _rms_norm_train(x, weight, rstd, dy=None, dsum=None):
+    """t5a_rmsnorm_train over contiguous rows: y, or with ``dy`` (dx, dweight)."""
+    d = x.shape[-1]
+    lib = L.load()
+    a = L.T5ARmsNormTrainArgs()
+    a.x, a.weight, a.rstd = x.data_ptr(), weight.data_ptr(), rstd.data_ptr()
+    a.rows, a.dim = x.numel() // d, d
+    a.x_dtype, a.weight_dtype = _dtype_code(x), _dtype_code(weight)
+    if dy is None:
+        out = torch.empty(x.shape, device=x.device, dtype=weight.dtype if weight.dtype in (torch.float16, torch.bfloat16) else torch.float32)
+        a.y = out.data_ptr()
+    else:
+        out = torch.empty_like(x), torch.empty_like(weight)
+        ws = torch.empty(int(lib.t5a_rmsnorm_bwd_workspace_bytes(a.rows, d)), device=x.device, dtype=torch.uint8)
+        a.dy, a.dx, a.dweight = dy.data_ptr(), out[0].data_ptr(), out[1].data_ptr()
+        a.dsum = dsum.data_ptr() if dsum is not None else None
+        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
+    with _on_device(x):
+        L.check(lib.t5a_rmsnorm_train(C.byref(a), _stream(x)))
+    return out
+
+
+def _rows16(t: torch.Tensor) -> torch.Tensor:
+    t = t.detach().contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+class RmsNorm(torch.autograd.Function):
+    """The norm of x, or of x + residual, with its backward: (x + residual, norm), or (None, norm)."""
+
+    @staticmethod
+    def forward(ctx, x, weight, eps, residual):
+        total = x if residual is None else x + residual
+        rstd = torch.rsqrt(total.to(torch.float32).pow(2).mean(-1, keepdim=True) + eps).contiguous()
+        y = _rms_norm_train(_rows16(total), weight.detach().contiguous(), rstd)
+        ctx.save_for_backward(total, weight, rstd)
+        ctx.eps = eps
+        ctx.set_materialize_grads(False)
+        return None if residual is None else total, y
+
+    @staticmethod
+    def backward(ctx, dsum, dy):
+        x, weight, rstd = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        if dy is None:
+            dx, dw = dsum, None
+        elif torch.is_grad_enabled():
+            # the gradient itself is to be differentiated: through the formula
+            y = _rms_norm_eager(x, weight, ctx.eps)
+            ins = [t for t in (x, weight) if t.requires_grad]
+            got = dict(zip(map(id, ins), torch.autograd.grad(y, ins, dy, create_graph=True)))
+            dx, dw = got.get(id(x)), got.get(id(weight))
+            if dx is not None and dsum is not None:
+                dx = dx + dsum
+        else:
+            dx, dw = _rms_norm_train(_rows16(x), weight.detach().contiguous(), rstd, _rows16(dy),
+                                     _rows16(dsum) if dsum is not None else None)
+            dw = dw.view_as(weight)
+        return dx if need[0] else None, dw if need[1] else None, None, dx if need[3] else None
+
+
+def rms_norm_differentiable(x, weight, residual=None) -> bool:
+    """Whether ``RmsNorm`` takes this call: plain tensors of the kernels' types on one ROCm device, rows that stay in
+    registers, and plain reverse-mode autograd (no tracing, function transform, forward-mode level or dispatch mode, for
+    which the formula in torch's own operations is the one that works)."""
+    f = torch._C._functorch
+    return (x.is_cuda and weight.device == x.device and x.dtype in _DTYPES and weight.dtype in _DTYPES and x.numel() > 0
+            and weight.shape == x.shape[-1:] and x.shape[-1] % 8 == 0 and x.shape[-1] <= L.RMSNORM_TRAIN_MAX_DIM
+            and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in (x, weight))
+            and (residual is None or (type(residual) is torch.Tensor and residual.shape == x.shape
+                                      and residual.dtype == x.dtype and residual.device == x.device))
+            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
+            and torch.autograd.forward_ad._current_level < 0 and f.peek_interpreter_stack() is None
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
 _CU_COUNT = {}
 
 

@@ -87,14 +87,13 @@ def _forward_only(what: str, *tensors):
                                   "use attention_type='flash', whose kernels have one")
 
 
-def _unit(t: torch.Tensor) -> int:
-    return 4 if t.dtype == torch.float32 else 8
-
-
 def _kernel_ready(t: torch.Tensor) -> torch.Tensor:
     """The kernels need head_dim contiguous, 16-byte aligned rows; copy only when that fails."""
-    u = _unit(t)
-    ok = t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and all(s % u == 0 for s in t.stride()[:-1])
+    st = t.stride()
+    bits = 0
+    for s in st[:-1]:
+        bits |= s
+    ok = st[-1] == 1 and not t.data_ptr() & 15 and not bits & (3 if t.dtype == torch.float32 else 7)
     return t if ok else t.contiguous()
 
 
@@ -151,10 +150,8 @@ def clear_bias_luts():
 
 def _bias_struct(bias: Optional[torch.Tensor], H: int, num_buckets: int, max_distance: int, ref: torch.Tensor,
                  causal: bool = False, window: int = 0):
-    b = L.T5ABias()
     if bias is None:
-        b.table = None
-        return b, None
+        return L.T5ABias(), None
     if bias.dim() != 2 or bias.shape[0] != num_buckets or bias.shape[1] != H:
         raise ValueError(f"bias table must be (NUM_BUCKETS={num_buckets}, H={H}), got {tuple(bias.shape)}")
     if bias.device != ref.device:
@@ -162,12 +159,7 @@ def _bias_struct(bias: Optional[torch.Tensor], H: int, num_buckets: int, max_dis
     table = bias.detach()
     if table.dtype not in _DTYPES:
         table = table.float()
-    b.table = table.data_ptr()
-    b.table_dtype = _DTYPES[table.dtype]
-    b.num_buckets = num_buckets
-    b.max_distance = max_distance
-    b.stride_bucket = table.stride(0)
-    b.stride_head = table.stride(1)
+    b = L.T5ABias(table.data_ptr(), _DTYPES[table.dtype], num_buckets, max_distance, 0, *table.stride())
     lut, pending = (_bias_lut(b, bias, H, num_buckets, max_distance, causal, ref, window)
                     if table.data_ptr() == bias.data_ptr() else (None, None))
     return b, (table, lut, pending, bias)   # alive until the launch has been queued; see _commit_lut
@@ -183,12 +175,15 @@ def _stream(t: torch.Tensor) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
+
+
 class _on_device:
     """Makes t's device current for the launch; a no-op (no context switch) when it already is."""
 
     def __init__(self, t: torch.Tensor):
         idx = t.device.index
-        self.ctx = None if idx is None or idx == torch.cuda.current_device() else torch.cuda.device(idx)
+        self.ctx = None if idx is None or idx == _current_device() else torch.cuda.device(idx)
 
     def __enter__(self):
         if self.ctx is not None:
@@ -200,7 +195,11 @@ class _on_device:
 
 
 def _strides3(t):
-    return (C.c_int64 * 3)(t.stride(0), t.stride(1), t.stride(2))
+    return t.stride()[:3]
+
+
+def _strides2(t):
+    return t.stride()[:2]
 
 
 def _dense_forward(q, k, v, bias, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, return_lse, exact_scores):
@@ -214,18 +213,25 @@ def _dense_forward(q, k, v, bias, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, r
     q_, k_, v_ = (_kernel_ready(t) for t in (q, k, v))
     o = torch.empty_like(q_)
     lse = torch.empty((B, H, M), device=q.device, dtype=torch.float32) if return_lse else None
-    a = L.T5ADenseArgs()
-    a.q, a.k, a.v, a.o = q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o.data_ptr()
-    a.lse = lse.data_ptr() if lse is not None else None
-    a.q_strides, a.k_strides, a.v_strides, a.o_strides = _strides3(q_), _strides3(k_), _strides3(v_), _strides3(o)
-    a.dtype, a.B, a.H, a.M, a.N, a.D = _dtype_code(q), B, H, M, N, D
-    a.causal, a.sm_scale = int(bool(causal)), float(sm_scale)
-    a.exact_scores = _exact(exact_scores)
-    a.bias, keep = _bias_struct(bias, H, NUM_BUCKETS, MAX_DISTANCE, q, causal)
+    bias_args, keep = _bias_struct(bias, H, NUM_BUCKETS, MAX_DISTANCE, q, causal)
+    # (all fields in one call, in the struct's order: filled one by one they cost as much as the launch)
+    a = L.T5ADenseArgs(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o.data_ptr(), lse.data_ptr() if lse is not None else None,
+                       _strides3(q_), _strides3(k_), _strides3(v_), _strides3(o),
+                       _dtype_code(q), B, H, M, N, D, int(bool(causal)), float(sm_scale), _exact(exact_scores), 0, bias_args)
     with _on_device(q):
         L.check(L.load().t5a_fwd_dense(C.byref(a), _stream(q)))
     _commit_lut(keep, B > 0 and M > 0)
     return (o, lse) if return_lse else o
+
+
+def _backward_bias_struct(bias, NUM_BUCKETS, MAX_DISTANCE):
+    """-> (struct, table to keep alive until the launch has been queued)"""
+    if bias is None:
+        return L.T5ABias(), None
+    table = bias.detach()
+    if table.dtype not in _DTYPES:
+        table = table.float()
+    return L.T5ABias(table.data_ptr(), _DTYPES[table.dtype], NUM_BUCKETS, MAX_DISTANCE, 0, *table.stride()), table
 
 
 def _dense_backward(q, k, v, bias, o, lse, dout, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, exact_scores):
@@ -241,29 +247,12 @@ def _dense_backward(q, k, v, bias, o, lse, dout, causal, sm_scale, NUM_BUCKETS, 
     dtable = torch.empty((NUM_BUCKETS, H), device=q.device, dtype=torch.float32) if bias is not None else None
     lib = L.load()
     ws = torch.empty(max(int(lib.t5a_bwd_workspace_bytes(B, H, M)), 16), device=q.device, dtype=torch.uint8)
-    a = L.T5ADenseBwdArgs()
-    a.q, a.k, a.v, a.o, a.dout, a.lse = (t.data_ptr() for t in (q_, k_, v_, o_, g_, lse))
-    a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
-    a.dtable = dtable.data_ptr() if dtable is not None else None
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    for name, t in (("q_strides", q_), ("k_strides", k_), ("v_strides", v_), ("o_strides", o_), ("dout_strides", g_),
-                    ("dq_strides", dq), ("dk_strides", dk), ("dv_strides", dv)):
-        setattr(a, name, _strides3(t))
-    a.dtype, a.B, a.H, a.M, a.N, a.D = _dtype_code(q), B, H, M, N, D
-    a.causal, a.sm_scale = int(bool(causal)), float(sm_scale)
-    a.exact_scores = _exact(exact_scores)
-    a.fp32_math = int(bool(BACKWARD_FP32_MATH))
-    b = L.T5ABias()
-    keep = None
-    if bias is not None:
-        table = bias.detach()
-        if table.dtype not in _DTYPES:
-            table = table.float()
-        b.table, b.table_dtype = table.data_ptr(), _DTYPES[table.dtype]
-        b.num_buckets, b.max_distance = NUM_BUCKETS, MAX_DISTANCE
-        b.stride_bucket, b.stride_head = table.stride(0), table.stride(1)
-        keep = table
-    a.bias = b
+    bias_args, keep = _backward_bias_struct(bias, NUM_BUCKETS, MAX_DISTANCE)
+    a = L.T5ADenseBwdArgs(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(), g_.data_ptr(), lse.data_ptr(),
+                          dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dtable.data_ptr() if dtable is not None else None,
+                          ws.data_ptr(), ws.numel(), _strides3(q_), _strides3(k_), _strides3(v_), _strides3(o_), _strides3(g_),
+                          _strides3(dq), _strides3(dk), _strides3(dv), _dtype_code(q), B, H, M, N, D, int(bool(causal)),
+                          float(sm_scale), _exact(exact_scores), int(bool(BACKWARD_FP32_MATH)), bias_args)
     with _on_device(q):
         L.check(lib.t5a_bwd_dense(C.byref(a), _stream(q)))
     del keep
@@ -304,7 +293,8 @@ def flash_attention_with_fusing_bias(q, k, v, bias, causal=False, sm_scale=None,
     log-sum-exp when ``return_lse``.  Differentiable in q, k, v and the table (fp32 tensors: head_dim up to 64), as the
     reference's autograd function is (fused_bias_attention.py:821-873).
     """
-    needs_grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (q, k, v, bias))
+    needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
+                                              or (bias is not None and bias.requires_grad))
     if needs_grad:
         o, lse = FlashAttentionBias.apply(q, k, v, bias, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, exact_scores)
         return (o, lse) if return_lse else o
@@ -375,8 +365,7 @@ def _varlen_forward(q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max
     a = L.T5AVarlenArgs()
     a.q, a.k, a.v, a.o = q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o.data_ptr()
     a.lse = lse.data_ptr() if lse is not None else None
-    for name, t in (("q_strides", q_), ("k_strides", k_), ("v_strides", v_), ("o_strides", o)):
-        setattr(a, name, (C.c_int64 * 2)(t.stride(0), t.stride(1)))
+    a.q_strides, a.k_strides, a.v_strides, a.o_strides = _strides2(q_), _strides2(k_), _strides2(v_), _strides2(o)
     a.cu_seqlens_q, a.cu_seqlens_k = cq.data_ptr(), ck.data_ptr()
     a.seq_lens_q = lens[0].data_ptr() if lens[0] is not None else None
     a.seq_lens_k = lens[1].data_ptr() if lens[1] is not None else None
@@ -435,36 +424,17 @@ def _varlen_backward(q, k, v, bias, o, lse, dout, cu_seqlens_q, cu_seqlens_k, ma
     dtable = torch.empty((NUM_BUCKETS, H), device=q.device, dtype=torch.float32) if bias is not None else None
     lib = L.load()
     ws = torch.empty(max(int(lib.t5a_bwd_varlen_workspace_bytes(total_q, H)), 16), device=q.device, dtype=torch.uint8)
-    a = L.T5AVarlenBwdArgs()
-    a.q, a.k, a.v, a.o, a.dout, a.lse = (t.data_ptr() for t in (q_, k_, v_, o_, g_, lse))
-    a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
-    a.dtable = dtable.data_ptr() if dtable is not None else None
-    a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    for name, t in (("q_strides", q_), ("k_strides", k_), ("v_strides", v_), ("o_strides", o_), ("dout_strides", g_),
-                    ("dq_strides", dq), ("dk_strides", dk), ("dv_strides", dv)):
-        setattr(a, name, (C.c_int64 * 2)(t.stride(0), t.stride(1)))
-    a.cu_seqlens_q, a.cu_seqlens_k = cq.data_ptr(), ck.data_ptr()
-    a.seq_lens_q = lens[0].data_ptr() if lens[0] is not None else None
-    a.seq_lens_k = lens[1].data_ptr() if lens[1] is not None else None
-    a.dtype, a.B, a.H, a.D = _dtype_code(q), B, H, D
-    a.total_q, a.total_k = total_q, k.shape[0]
-    a.max_seqlen_q, a.max_seqlen_k = int(max_seqlen_q), int(max_seqlen_k)
-    a.causal, a.sm_scale = int(bool(causal)), float(sm_scale)
-    a.exact_scores = _exact(exact_scores)
-    a.fp32_math = int(bool(BACKWARD_FP32_MATH))
-    b = L.T5ABias()
-    table = None
-    if bias is not None:
-        table = bias.detach()
-        if table.dtype not in _DTYPES:
-            table = table.float()
-        b.table, b.table_dtype = table.data_ptr(), _DTYPES[table.dtype]
-        b.num_buckets, b.max_distance = NUM_BUCKETS, MAX_DISTANCE
-        b.stride_bucket, b.stride_head = table.stride(0), table.stride(1)
-    a.bias = b
+    bias_args, keep = _backward_bias_struct(bias, NUM_BUCKETS, MAX_DISTANCE)
+    a = L.T5AVarlenBwdArgs(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(), g_.data_ptr(), lse.data_ptr(),
+                           dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dtable.data_ptr() if dtable is not None else None,
+                           ws.data_ptr(), ws.numel(), _strides2(q_), _strides2(k_), _strides2(v_), _strides2(o_), _strides2(g_),
+                           _strides2(dq), _strides2(dk), _strides2(dv), cq.data_ptr(), ck.data_ptr(),
+                           *(t.data_ptr() if t is not None else None for t in lens), _dtype_code(q), B, H, D, total_q,
+                           k.shape[0], int(max_seqlen_q), int(max_seqlen_k), int(bool(causal)), float(sm_scale),
+                           _exact(exact_scores), int(bool(BACKWARD_FP32_MATH)), bias_args)
     with _on_device(q):
         L.check(lib.t5a_bwd_varlen(C.byref(a), _stream(q)))
-    del table
+    del keep
     return dq, dk, dv, dtable
 
 
@@ -512,7 +482,8 @@ def flash_attention_with_fusing_bias_varlen(q, k, v, bias, cu_seqlens_q, cu_seql
     False never does, ``"always"`` does whatever the size.  A ``LaunchPlan`` object keeps the plan
     for later calls over the same batch.  The results do not depend on any of this.
     """
-    needs_grad = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (q, k, v, bias))
+    needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
+                                              or (bias is not None and bias.requires_grad))
     if needs_grad:
         o, lse = FlashAttentionBiasVarlen.apply(q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal,
                                                 sm_scale, NUM_BUCKETS, MAX_DISTANCE, seq_lens_q, seq_lens_k, launch_plan,

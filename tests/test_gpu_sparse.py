@@ -504,3 +504,38 @@ def test_tglobal_with_masks_of_any_shape(gpu_device, dtype, L, Bl, gbs):
     with pytest.raises(ValueError):   # the counts are not optional
         ops.transient_global_attention_with_fusing_bias(
             *(t.to(gpu_device) for t in (q, k, v, sk, sv)), table.to(gpu_device), Bl, gbs, key_bits=bits)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("with_side", [False, True])
+@pytest.mark.parametrize("L,Bl,gbs", [(1, 128, 16), (31, 1, 8), (33, 33, 32), (129, 64, 5), (160, 256, 7), (700, 128, 16), (1025, 100, 33)])
+def test_window_kernel_agrees_with_the_general_kernel(gpu_device, monkeypatch, dtype, with_side, L, Bl, gbs):
+    """16-bit tensors at head_dim 64 with a window of up to 256 take the kernel of 32 x 32 blocks; a pinned run length takes
+    the general one.  Over the forms both accept: contiguous heads and (B, L, H, D) views, with and without a table,
+    the three score modes, no padding, right padding, padding on both sides, an empty sequence.  Both round the
+    probabilities to the type (2^-9 / 2^-12) and the result once more, and sum in other orders."""
+    from turbot5_amd import ops
+    B, H, D = 3, 4, 64
+    side = L // gbs if with_side else 0
+    q, k, v = (rnd(B, L, H, D, seed=301 + i, dtype=dtype).to(gpu_device).transpose(1, 2) for i in range(3))
+    sk, sv = (rnd(B, H, side, D, seed=304 + i, dtype=dtype).to(gpu_device) for i in range(2))
+    table = rnd(32, H, seed=306, scale=1.0).to(gpu_device)
+    lens = torch.tensor([L, (2 * L) // 3, 0], dtype=torch.int32, device=gpu_device)
+    starts = torch.tensor([0, L // 4, 0], dtype=torch.int32, device=gpu_device)
+    tol = 2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -9
+    for contiguous, tab, exact, kw in ((False, table, None, {}), (True, None, True, {}), (False, table, "prescaled", {}),
+                                       (False, table, None, dict(seq_lens=lens)),
+                                       (True, table, None, dict(seq_lens=lens, seq_starts=starts))):
+        a, b, c = (t.contiguous() if contiguous else t for t in (q, k, v))
+        got = []
+        for run_len in (0, 1):
+            monkeypatch.setattr(ops, "RUN_LEN", run_len)
+            got.append(ops.transient_global_attention_with_fusing_bias(a, b, c, sk, sv, tab, Bl, gbs, exact_scores=exact, **kw) if with_side
+                       else ops.local_attention_with_fusing_bias(a, b, c, tab, Bl, exact_scores=exact, **kw))
+        new, old = (t.float().cpu() for t in got)
+        for s in range(B):
+            lo, hi = (0, L) if not kw else (int(starts[s]) if "seq_starts" in kw else 0, 0)
+            if kw:
+                hi = lo + int(lens[s])
+            assert torch.isfinite(new[s]).all()
+            assert (new[s, :, lo:hi] - old[s, :, lo:hi]).abs().max().item() <= tol if hi > lo else True, (contiguous, exact, list(kw), s)

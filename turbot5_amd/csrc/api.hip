@@ -823,6 +823,8 @@ int t5a_fwd_sparse(const t5a_sparse_args* a, t5a_stream_t stream) {
         }
         return finish(launch_fwd(g, a->dtype, a->D, kDense, false, s), "t5a_fwd_sparse(block, global rows)");
     }
+    if (a->D == 64 && a->dtype != T5A_F32 && a->block_len <= kMaxLutWindow && a->run_len == 0 && a->key_bits == nullptr)
+        return finish(launch_window(p, a->dtype, a->pattern == T5A_PATTERN_TGLOBAL && a->n_side > 0, s), "t5a_fwd_sparse(window)");
     p.tiles_per_seq = (a->L + 127) / 128;
     // (validity bit sets go with the instantiation that masks per element)
     const int mode = a->pattern == T5A_PATTERN_TGLOBAL ? (a->key_bits != nullptr ? kTGlobalBits : kTGlobal)

@@ -26,15 +26,13 @@
 // Scores use the key position j and the query position i + N - M, as the forward does; rows whose log-sum-exp is
 // -inf (no visible key) have no gradient.  Rows and keys past the end of a tensor are read as zeros and masked.
 #include "lut_device.h"
+#include "mfma16_device.h"
 #include "t5a_internal.h"
 
 namespace t5a {
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kBwdThreads = 256;
 constexpr int kBwdOwn = 64;      // own rows per workgroup of the fp32 kernels (queries for dq, keys for dk / dv)
@@ -414,53 +412,6 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
 // takes costs more than the wait it saves.  Before / after, us, the passes with bwd_rows_kernel, bf16: B16 H12
 // L1024 D64 299 / 248, the same causal 205 / 180, B4 H12 L4096 D64 840 / 762, B4 H6 L4096 D128 1274 / 835, B2 H8
 // L1999 D128 causal 280 / 135.
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-
-template <typename T> struct Half16;
-template <> struct Half16<__bf16> {
-    typedef __bf16 v8 __attribute__((ext_vector_type(8)));
-    static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
-};
-template <> struct Half16<_Float16> {
-    typedef _Float16 v8 __attribute__((ext_vector_type(8)));
-    static __device__ __forceinline__ f32x16 mfma(v8 a, v8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
-};
-
-// chunk swizzle of a tile row: 16 consecutive rows put a chunk into 16 different 16-byte slots of a 256-byte bank
-// line (row reads), and rows 2, 3 (mod 4) swap their 64-byte halves (the transposing read touches four consecutive
-// rows x 64 bytes at a time)
-__device__ __forceinline__ int tile_swz(int row) { return ((row >> 1) & 7) ^ (((row >> 1) & 1) << 2); }
-
-// LDS-DMA: a wavefront instruction fetches 64 x 16 bytes at per-lane byte offsets of a buffer (zeros past its end) and
-// writes them to 1 KB of consecutive LDS addresses in lane order, without passing through registers.  Issued from
-// assembly, so the wait for it (vmcnt) is the kernel's own.
-__device__ __forceinline__ u32x4 dma_rsrc(const void* base, unsigned bytes) {
-    const unsigned long long a = reinterpret_cast<unsigned long long>(base);
-    return u32x4{(unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)a),
-                 (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)(a >> 32) & 0xffffu)),
-                 (unsigned)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-__device__ __forceinline__ void dma_16(u32x4 rs, unsigned lds_addr, int voffset) {
-    const u32x4 rsrc = {(unsigned)__builtin_amdgcn_readfirstlane((int)rs[0]), (unsigned)__builtin_amdgcn_readfirstlane((int)rs[1]),
-                        (unsigned)__builtin_amdgcn_readfirstlane((int)rs[2]), (unsigned)__builtin_amdgcn_readfirstlane((int)rs[3])};
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-                 :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voffset), "s"(rsrc) : "memory", "m0");
-}
-// the same with 4 bytes per lane (256 consecutive bytes of LDS)
-__device__ __forceinline__ void dma_4(u32x4 rs, unsigned lds_addr, int voffset) {
-    const u32x4 rsrc = {(unsigned)__builtin_amdgcn_readfirstlane((int)rs[0]), (unsigned)__builtin_amdgcn_readfirstlane((int)rs[1]),
-                        (unsigned)__builtin_amdgcn_readfirstlane((int)rs[2]), (unsigned)__builtin_amdgcn_readfirstlane((int)rs[3])};
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds"
-                 :: "s"(__builtin_amdgcn_readfirstlane(lds_addr)), "v"(voffset), "s"(rsrc) : "memory", "m0");
-}
-// waits until at most N of this wavefront's memory requests are outstanding (they complete in order)
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N < 64, "");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
-
 // head_dim 128 (the T5-3B / 11B head shape): rows of 256 bytes, sixteen chunks
 __device__ __forceinline__ int tile_swz128(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 
@@ -486,34 +437,6 @@ struct Bwd16Geom {
     static __host__ __device__ int skew(int sat) { return hist(sat) + (KV ? 0 : 4 * ((2 * sat + 4) & ~3)); }
     static __host__ __device__ int bytes(int sat, bool bias) { return skew(sat) + (KV || !bias ? 0 : 4 * SKEW_ROWS * 64 * 4); }
 };
-
-// Workgroup -> (own block, head, sequence).  Workgroups go to the eight XCDs in turn; all own blocks of a (head,
-// sequence) pair go to one XCD, whose L2 then holds the pair's rows of the other kind for all of them.  Where the
-// pairs do not divide by eight they are dealt out in turn instead.  With a causal mask the own blocks differ in length
-// (a query block sees the keys up to its own end, a key block the queries from its own start on), and whatever is
-// dispatched last should be short: the blocks are then the slowest index, longest first.
-template <bool CAUSAL, bool KV>
-__device__ __forceinline__ void bwd_place(int H, int B, int nblk, int& blk, int& h, int& b) {
-    const int pairs = H * B, id = blockIdx.x;
-    int pair, level;
-    if ((pairs & 7) == 0) {
-        const int pp = pairs >> 3, slot = id >> 3;
-        if (CAUSAL) { level = slot / pp; pair = (id & 7) * pp + (slot - level * pp); }
-        else { const int q = slot / nblk; level = slot - q * nblk; pair = (id & 7) * pp + q; }
-    } else {
-        level = id / pairs; pair = id - level * pairs;
-    }
-    blk = (CAUSAL && !KV) ? nblk - 1 - level : level;
-    h = pair / B; b = pair - h * B;
-}
-
-// rows 16 u .. + 15 of a 32-row accumulator as a B operand
-template <typename v8> __device__ __forceinline__ v8 to_frag(const f32x16& x, int u) {
-    f32x8 y;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = x[8 * u + e];
-    return __builtin_convertvector(y, v8);
-}
 
 template <int D> __device__ __forceinline__ int row_swz(int row) { return D == 64 ? tile_swz(row) : tile_swz128(row); }
 

@@ -94,6 +94,10 @@ hipError_t launch_fwd_bf16(const FwdParams& p, int D, int mode, bool causal, hip
 hipError_t launch_fwd_f16(const FwdParams& p, int D, int mode, bool causal, hipStream_t stream);
 hipError_t launch_fwd_f32(const FwdParams& p, int D, int mode, bool causal, hipStream_t stream);
 
+// local (side: transient-global) pattern, 16-bit tensors at head_dim 64, block_len <= kMaxLutWindow
+// (attn_window.hip)
+hipError_t launch_window(const FwdParams& p, int dtype, bool side, hipStream_t stream);
+
 struct SplitKParams {
     const void* q; const void* k; const void* v; void* o;
     const float* bias;

@@ -509,6 +509,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
         }
         if constexpr (KV) dma_4(rs_s, lds0 + G::STAT + buf * 512 + (wave & 1) * 256, (t * OTHER + lane) * (int)stat_sr * 4);
     };
+    const BiasColumn bias(p, h, lane);
     // Tile t + STAGES - 1 is requested when the barrier at the top of tile t has shown that every wavefront is done with
     // the buffer it goes into (tile t - 1's): it has STAGES - 1 tiles' work to arrive in.
 #pragma unroll
@@ -539,13 +540,14 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
     // rows are consecutive words; padded by 64 on both sides, more than the distances of a lane's rows span
     float bias_lo = 0.f, bias_hi = 0.f;     // ... and of the two saturated sides
     {
-        auto bias_at = [&](int rel) {
-            return load_table(p.table, p.table_dtype, (int64_t)bucket_of(p.bs, rel) * p.t_sbucket + (int64_t)h * p.t_shead) * 1.4426950408889634f;
-        };
         const int mid = sat + G::LUT_PAD16;
-        for (int x = tid; x <= 2 * mid; x += kBwdThreads) lut[x] = has_bias ? bias_at(KV ? mid - x : x - mid) : 0.f;
+        for (int x0 = 0; x0 <= 2 * mid; x0 += kBwdThreads) {
+            const int x = x0 + tid;
+            const float v = bias.at(KV ? mid - x : x - mid);
+            if (x <= 2 * mid) lut[x] = v;
+        }
         if (has_bias) {
-            bias_lo = bias_at(-sat); bias_hi = bias_at(sat);
+            bias_lo = bias.at(-sat); bias_hi = bias.at(sat);
             if constexpr (!KV) {
                 for (int x = tid; x <= 2 * sat; x += kBwdThreads) hist_rel[x] = 0.f;
                 for (int x = lane; x < G::SKEW_ROWS * 64; x += 64) skew[x] = 0.f;

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "lut_device.h"
+
 namespace t5a {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -91,5 +93,26 @@ __device__ __forceinline__ void bwd_place(int H, int B, int nblk, int& blk, int&
     blk = (CAUSAL && !KV) ? nblk - 1 - level : level;
     h = pair / B; b = pair - h * B;
 }
+
+// The bias of one head by distance, times log2(e).  With up to 64 buckets lane b of every wavefront holds bucket b: one
+// load, and a look-up is an exchange between lanes instead of a round trip to memory.  `at` is for all lanes at once.
+struct BiasColumn {
+    const BucketSpec& bs;
+    const void* table; int dtype; int64_t first, step;
+    bool in_lanes;
+    float mine;
+    template <typename P> __device__ __forceinline__ BiasColumn(const P& p, int h, int lane)
+        : bs(p.bs), table(p.table), dtype(p.table_dtype), first((int64_t)h * p.t_shead), step(p.t_sbucket), mine(0.f) {
+        const int n = p.bs.bidirectional ? 2 * p.bs.nb : p.bs.nb;
+        in_lanes = n <= 64;
+        if (table != nullptr && in_lanes && lane < n) mine = load_table(table, dtype, first + lane * step) * 1.4426950408889634f;
+    }
+    __device__ __forceinline__ float at(int rel) const {
+        if (table == nullptr) return 0.f;
+        const int b = bucket_of(bs, rel);
+        if (in_lanes) return __int_as_float(__builtin_amdgcn_ds_bpermute(b << 2, __float_as_int(mine)));
+        return load_table(table, dtype, first + b * step) * 1.4426950408889634f;
+    }
+};
 
 }  // namespace t5a

@@ -34,7 +34,7 @@ LOG2E = 1.4426950408889634
 # depend on it; tests pin every path of the run logic with it.
 RUN_LEN = 0
 
-# Backward of 16-bit tensors at head_dim 64.  False: the 16-bit matrix cores, probabilities and dS rounded to the
+# Backward of 16-bit tensors at head_dim 64 (and 128, which has no fp32 path).  False: the 16-bit matrix cores, probabilities and dS rounded to the
 # tensors' type before the products that form dq, dk and dv, as the reference's kernels round them
 # (fused_bias_attention.py:575-590).  True: every product on the fp32 matrix cores (about five times slower).
 BACKWARD_FP32_MATH = False
@@ -80,7 +80,7 @@ def _check_inputs(q, k, v):
 
 
 def _forward_only(what: str, *tensors):
-    """The sparse patterns, split-K decoding and the RMS norm kernel have no backward: say so instead of returning
+    """The sparse patterns and split-K decoding have no backward: say so instead of returning
     a result that silently carries no graph."""
     if torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in tensors):
         raise NotImplementedError(f"{what} is forward only (no backward kernel); run it under torch.no_grad() or "

@@ -539,3 +539,31 @@ def test_window_kernel_agrees_with_the_general_kernel(gpu_device, monkeypatch, d
                 hi = lo + int(lens[s])
             assert torch.isfinite(new[s]).all()
             assert (new[s, :, lo:hi] - old[s, :, lo:hi]).abs().max().item() <= tol if hi > lo else True, (contiguous, exact, list(kw), s)
+
+
+def _window_launch_batch(gpu_device, H, L):
+    """a batch whose 128-row blocks outnumber two per compute unit"""
+    cus = torch.cuda.get_device_properties(gpu_device).multi_processor_count
+    return 2 * cus // (H * ((L + 127) // 128)) + 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("L,Bl,gbs,at", [(700, 128, 16, 300), (333, 33, 5, 0), (600, 256, 32, 599), (400, 1, 8, 77)])
+def test_transient_global_keeps_a_non_finite_key_to_the_rows_that_see_it(gpu_device, dtype, bad, L, Bl, gbs, at):
+    """A key row of infinities or NaN reaches the rows whose window holds it and no other: those agree bit for bit with
+    the call without it."""
+    from turbot5_amd import ops
+    H, D = 12, 64
+    B = _window_launch_batch(gpu_device, H, L)
+    q, k, v = (rnd(B, H, L, D, seed=501 + i, dtype=dtype).to(gpu_device) for i in range(3))
+    sk, sv = (rnd(B, H, L // gbs, D, seed=504 + i, dtype=dtype).to(gpu_device) for i in range(2))
+    table = rnd(32, H, seed=506, scale=1.0).to(gpu_device)
+    clean = ops.transient_global_attention_with_fusing_bias(q, k, v, sk, sv, table, Bl, gbs)
+    k[:, :, at] = bad
+    out = ops.transient_global_attention_with_fusing_bias(q, k, v, sk, sv, table, Bl, gbs)
+    rows = torch.arange(L, device=gpu_device)
+    apart = (rows - at).abs() >= Bl
+    assert torch.isfinite(out[:, :, apart]).all() and torch.equal(out[:, :, apart], clean[:, :, apart])
+    if bad != bad:
+        assert torch.isnan(out[:, :, ~apart]).all()

@@ -48,6 +48,7 @@ __global__ __launch_bounds__(kWinThreads, 4) void window16_kernel(const FwdParam
     using H16 = Half16<T>;
     using v8 = typename H16::v8;
     extern __shared__ __attribute__((aligned(16))) unsigned char win_smem[];
+    __shared__ int again;
 
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, hh = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -108,6 +109,7 @@ __global__ __launch_bounds__(kWinThreads, 4) void window16_kernel(const FwdParam
         }
     };
     if (n_tiles > 0) request(0, 0);
+    if (SIDE && tid == 0) again = 0;
 
     // the query row as B operands: lane (lr, hh) holds elements 16 s + 8 hh .. + 7; multiplied by the score factor and
     // rounded back unless the factor is to be applied to the product
@@ -167,12 +169,20 @@ __global__ __launch_bounds__(kWinThreads, 4) void window16_kernel(const FwdParam
     };
 
     f32x16 acc[DT];
+    float m, sums[2];      // what is subtracted from the row's scores; this lane half's sum, in two parts
+    float limit;            // a shifted score above it raises m (any, until the row's first visible key)
+    // A key row of NaN or infinity is not outweighed by the folded -inf.  With side tokens it has to stay with the rows that see
+    // it (the general kernel masks that pattern per element, and folds the local one as this does): a workgroup with a NaN
+    // among its sums goes over its tiles once more with every window block masked per element.  (The mask in every block at
+    // a window's edge, or asked for by the block's own sums, took 2 us of launches of 25 to 75.)
+    bool masked = false;
+again_masked:
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
-    float m = 0.f, sums[2] = {0.f, 0.f};      // what is subtracted from the row's scores; this lane half's sum, in two parts
-    float limit = -INFINITY;        // a shifted score above it raises m (any, until the row's first visible key)
+    m = 0.f; sums[0] = 0.f; sums[1] = 0.f;
+    limit = -INFINITY;
 
     // (kept a loop: unrolled by two it takes 128 registers and 39.9 us where this takes 110 and 35.8)
 #pragma unroll 1
@@ -206,9 +216,12 @@ __global__ __launch_bounds__(kWinThreads, 4) void window16_kernel(const FwdParam
 #pragma unroll
                     for (int r = 0; r < 16; ++r) s[r] = __builtin_fmaf(c1, s[r], lp[8 * (r >> 2) + (r & 3)]) - m;
                 }
-                if (s0 + 32 > rows) {
+                if (masked || s0 + 32 > rows) {
+                    const int ends = rows - s0 - 4 * hh;
+                    const int first = SIDE && !side ? own_row - w + 1 - s0 - 4 * hh : 0;
+                    const int last = SIDE && !side ? min(ends, own_row + w - s0 - 4 * hh) : ends;
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) s[r] = 8 * (r >> 2) + (r & 3) < rows - s0 - 4 * hh ? s[r] : -INFINITY;
+                    for (int r = 0; r < 16; ++r) s[r] = (!SIDE || 8 * (r >> 2) + (r & 3) >= first) && 8 * (r >> 2) + (r & 3) < last ? s[r] : -INFINITY;
                 }
                 float top = fmaxf(fmaxf(s[0], s[1]), s[2]);
 #pragma unroll
@@ -246,6 +259,15 @@ __global__ __launch_bounds__(kWinThreads, 4) void window16_kernel(const FwdParam
 
     float sum = sums[0] + sums[1];
     sum += __shfl_xor(sum, 32, 64);
+    if (SIDE && !masked && n_tiles > 0) {
+        if (__builtin_amdgcn_ballot_w64(sum != sum) != 0) again = 1;
+        __syncthreads();      // (and every wavefront is done with the tile buffers)
+        if (again != 0) {
+            masked = true;
+            request(0, 0);
+            goto again_masked;
+        }
+    }
     const float inv = sum > 0.f || sum != sum ? 1.0f / sum : 0.f;      // (a row without a visible key: zeros)
     // A lane holds elements 8 g + 4 hh .. + 3 of its row, the lane 32 further on the other halves: they exchange, and each
     // writes 16 bytes of every second group of eight.

@@ -134,6 +134,24 @@ def test_fp32_gradients_over_blocks_of_64_rows(gpu_device, causal, M, N, D):
         check(name, g, w, TOL[torch.float32])
 
 
+@pytest.mark.parametrize("D", [32, 64])
+@pytest.mark.parametrize("B,H,M,N,row", [(1, 3, 290, 257, 201), (1, 2, 100, 70, 99)])
+def test_fp32_table_gradient_leaves_out_keys_past_the_end(gpu_device, D, B, H, M, N, row):
+    """A query row whose gradient is NaN spoils the buckets of its own distances and no others: the rows past the last key
+    that fill up a tile are no pairs."""
+    from oracle import t5_basic as O
+    from turbot5_amd import ops
+    q, k, v = (rnd(B, H, n, D, seed=111 + i).to(gpu_device).requires_grad_() for i, n in enumerate((M, N, N)))
+    table = rnd(32, H, seed=114, scale=1.0).to(gpu_device).requires_grad_()
+    dout = rnd(B, H, M, D, seed=115, scale=1.0).to(gpu_device)
+    dout[:, :, row] = float("nan")
+    ops.flash_attention_with_fusing_bias(q, k, v, table, sm_scale=1.0).backward(dout)
+    met = torch.zeros(32, dtype=torch.bool)
+    met[O.relative_position_bucket(torch.arange(N) - (row + N - M), True, 32, 128)] = True
+    assert not met.all()
+    assert torch.equal(torch.isfinite(table.grad).cpu(), ~met[:, None].expand(32, H))
+
+
 @pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("B,H,M,N", [(48, 16, 33, 65), (53, 15, 130, 97), (24, 16, 290, 257)])

@@ -274,7 +274,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
             const float l2 = KV ? rowstat[ol] : lse2_own;
             const float dl = KV ? rowstat[kBwdOther + ol] : delta_own;
             const float pv = valid ? __builtin_amdgcn_exp2f(__builtin_fmaf(p.c1, s[r], bias2) + l2) : 0.f;
-            const float ds = pv * (dp[r] + dl);
+            const float ds = valid ? pv * (dp[r] + dl) : 0.f;     // (a NaN of dP stays out of the sums over pairs that exist)
             s[r] = pv;
             dp[r] = ds;
             tile_sum += ds;

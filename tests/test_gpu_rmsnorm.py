@@ -255,3 +255,35 @@ def test_norm_gradients_where_the_kernel_is_passed_by(gpu_device):
     wide(torch.randn(2, 4096, device=gpu_device)).sum().backward()
     assert wide.weight.grad is not None
     norm(torch.empty(0, 64, device=gpu_device)).sum().backward()
+
+
+def test_norm_gradients_in_batches_and_with_tangents(gpu_device):
+    """Several gradients at once (batched reverse mode, a vmap around it, a vectorised jacobian) and a gradient that carries
+    a tangent: a module in training mode takes them, row for row what they are one at a time."""
+    import torch.autograd.forward_ad as fwd
+    from turbot5_amd.attentions import T5LayerNorm
+    norm = T5LayerNorm(64).to(gpu_device).train()
+    with torch.no_grad():
+        norm.weight.copy_(torch.linspace(0.5, 1.5, 64))
+    g = torch.Generator().manual_seed(2)
+    x, r = (torch.randn(3, 64, generator=g).to(gpu_device).requires_grad_() for _ in range(2))
+    dy, ds = (torch.randn(5, 3, 64, generator=g).to(gpu_device) for _ in range(2))
+    total, y = norm.add_norm(x, r)
+    ins = (x, r, norm.weight)
+    want = [torch.autograd.grad((total, y), ins, (a, b), retain_graph=True) for a, b in zip(ds, dy)]
+    for got in (torch.autograd.grad((total, y), ins, (ds, dy), retain_graph=True, is_grads_batched=True),
+                torch.vmap(lambda a, b: torch.autograd.grad((total, y), ins, (a, b), retain_graph=True))(ds, dy),
+                torch.autograd.grad((total, y), ins, (ds, dy), retain_graph=True, is_grads_batched=True, create_graph=True)):
+        for i in range(3):
+            assert torch.allclose(got[i], torch.stack([w[i] for w in want]), rtol=1e-5, atol=1e-5)
+    eye = torch.eye(3 * 64, device=gpu_device).view(-1, 3, 64)
+    z = norm(x)
+    rows = torch.stack([torch.autograd.grad(z, x, e, retain_graph=True)[0] for e in eye]).view(3, 64, 3, 64)
+    jac = torch.autograd.functional.jacobian(norm, x.detach(), vectorize=True)
+    assert torch.allclose(jac, rows, rtol=1e-5, atol=1e-5)
+    with fwd.dual_level():     # the backward is linear in dy: its tangent is the gradient of the tangent
+        gx, = torch.autograd.grad(z, x, fwd.make_dual(dy[0], dy[1]), retain_graph=True)
+        value, tangent = fwd.unpack_dual(gx)
+    assert tangent is not None
+    for got, seed in ((value, dy[0]), (tangent, dy[1])):
+        assert torch.allclose(got, torch.autograd.grad(z, x, seed, retain_graph=True)[0], rtol=1e-5, atol=1e-5)

@@ -719,10 +719,20 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, group: in
     return y if total is None else (total, y)
 
 
-def _rms_norm_eager(x, weight, eps):
-    """The reference's formula (src/turbot5/model/modules.py:51-59)."""
-    n = x * torch.rsqrt(x.to(torch.float32).pow(2).mean(-1, keepdim=True) + eps)
-    return weight * (n.to(weight.dtype) if weight.dtype in (torch.float16, torch.bfloat16) else n)
+def _rms_norm_backward_ops(x, weight, eps, dy, dsum):
+    """The kernel's backward in torch's operations, for whatever needs those: gradients that are differentiated in their
+    turn, batches of gradients, forward-mode levels, tracing."""
+    x32 = x.to(torch.float32)
+    rstd = torch.rsqrt(x32.pow(2).mean(-1, keepdim=True) + eps)
+    n = x32 * rstd
+    if weight.dtype in (torch.float16, torch.bfloat16):
+        n = n.to(weight.dtype)
+    g = (dy * weight).to(torch.float32)
+    dx = rstd * g - x32 * (rstd.pow(3) * (g * x32).mean(-1, keepdim=True))
+    if dsum is not None:
+        dx = dx + dsum
+    dw = (dy.to(torch.float32) * n).sum(tuple(range(dy.dim() - 1)))
+    return dx.to(x.dtype), dw.to(weight.dtype)
 
 
 def _rms_norm_train(x, weight, rstd, dy=None, dsum=None):
@@ -771,14 +781,8 @@ class RmsNorm(torch.autograd.Function):
         need = ctx.needs_input_grad
         if dy is None:
             dx, dw = dsum, None
-        elif torch.is_grad_enabled():
-            # the gradient itself is to be differentiated: through the formula
-            y = _rms_norm_eager(x, weight, ctx.eps)
-            ins = [t for t in (x, weight) if t.requires_grad]
-            got = dict(zip(map(id, ins), torch.autograd.grad(y, ins, dy, create_graph=True)))
-            dx, dw = got.get(id(x)), got.get(id(weight))
-            if dx is not None and dsum is not None:
-                dx = dx + dsum
+        elif torch.is_grad_enabled() or not _plain(x, weight, dy, dsum):
+            dx, dw = _rms_norm_backward_ops(x, weight, ctx.eps, dy, dsum)
         else:
             dx, dw = _rms_norm_train(_rows16(x), weight.detach().contiguous(), rstd, _rows16(dy),
                                      _rows16(dsum) if dsum is not None else None)
@@ -786,19 +790,25 @@ class RmsNorm(torch.autograd.Function):
         return dx if need[0] else None, dw if need[1] else None, None, dx if need[3] else None
 
 
-def rms_norm_differentiable(x, weight, residual=None) -> bool:
-    """Whether ``RmsNorm`` takes this call: plain tensors of the kernels' types on one ROCm device, rows that stay in
-    registers, and plain reverse-mode autograd (no tracing, function transform, forward-mode level or dispatch mode, for
-    which the formula in torch's own operations is the one that works)."""
+def _plain(*tensors) -> bool:
+    """Plain tensors and plain reverse-mode autograd: no batch of gradients, no tracing, function transform, forward-mode level
+    or dispatch mode, for which a formula in torch's own operations is the one that works."""
     f = torch._C._functorch
-    return (x.is_cuda and weight.device == x.device and x.dtype in _DTYPES and weight.dtype in _DTYPES and x.numel() > 0
-            and weight.shape == x.shape[-1:] and x.shape[-1] % 8 == 0 and x.shape[-1] <= L.RMSNORM_TRAIN_MAX_DIM
-            and all(type(t) in (torch.Tensor, torch.nn.Parameter) for t in (x, weight))
-            and (residual is None or (type(residual) is torch.Tensor and residual.shape == x.shape
-                                      and residual.dtype == x.dtype and residual.device == x.device))
+    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and not f.is_batchedtensor(t) and not f.is_legacy_batchedtensor(t)
+                for t in tensors if t is not None)
             and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
             and torch.autograd.forward_ad._current_level < 0 and f.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def rms_norm_differentiable(x, weight, residual=None) -> bool:
+    """Whether ``RmsNorm`` takes this call: plain tensors of the kernels' types on one ROCm device, rows that stay in
+    registers, and plain reverse-mode autograd."""
+    return (x.is_cuda and weight.device == x.device and x.dtype in _DTYPES and weight.dtype in _DTYPES and x.numel() > 0
+            and weight.shape == x.shape[-1:] and x.shape[-1] % 8 == 0 and x.shape[-1] <= L.RMSNORM_TRAIN_MAX_DIM
+            and (residual is None or (type(residual) is torch.Tensor and residual.shape == x.shape
+                                      and residual.dtype == x.dtype and residual.device == x.device))
+            and _plain(x, weight, residual))
 
 
 _CU_COUNT = {}

@@ -287,3 +287,15 @@ def test_norm_gradients_in_batches_and_with_tangents(gpu_device):
     assert tangent is not None
     for got, seed in ((value, dy[0]), (tangent, dy[1])):
         assert torch.allclose(got, torch.autograd.grad(z, x, seed, retain_graph=True)[0], rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("x_grad,r_grad", [(False, False), (True, False), (False, True)])
+def test_residual_stream_carries_a_graph_only_where_it_has_one(gpu_device, x_grad, r_grad):
+    """Training the norm's weight alone does not make the residual stream part of the graph."""
+    from turbot5_amd.attentions import T5LayerNorm
+    norm = T5LayerNorm(64).to(gpu_device).train()
+    x, r = torch.randn(3, 64, device=gpu_device, requires_grad=x_grad), torch.randn(3, 64, device=gpu_device, requires_grad=r_grad)
+    total, y = norm.add_norm(x, r)
+    assert total.requires_grad == (x_grad or r_grad) and y.requires_grad
+    y.sum().backward()
+    assert norm.weight.grad is not None and (x.grad is not None) == x_grad and (r.grad is not None) == r_grad

@@ -773,6 +773,8 @@ class RmsNorm(torch.autograd.Function):
         ctx.save_for_backward(total, weight, rstd)
         ctx.eps = eps
         ctx.set_materialize_grads(False)
+        if residual is not None and not (ctx.needs_input_grad[0] or ctx.needs_input_grad[3]):
+            ctx.mark_non_differentiable(total)      # (only the weight is trained: the residual stream carries no graph)
         return None if residual is None else total, y
 
     @staticmethod

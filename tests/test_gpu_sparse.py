@@ -506,45 +506,75 @@ def test_tglobal_with_masks_of_any_shape(gpu_device, dtype, L, Bl, gbs):
             *(t.to(gpu_device) for t in (q, k, v, sk, sv)), table.to(gpu_device), Bl, gbs, key_bits=bits)
 
 
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("with_side", [False, True])
-@pytest.mark.parametrize("L,Bl,gbs", [(1, 128, 16), (31, 1, 8), (33, 33, 32), (129, 64, 5), (160, 256, 7), (700, 128, 16), (1025, 100, 33)])
-def test_window_kernel_agrees_with_the_general_kernel(gpu_device, monkeypatch, dtype, with_side, L, Bl, gbs):
-    """16-bit tensors at head_dim 64 with a window of up to 256 take the kernel of 32 x 32 blocks; a pinned run length takes
-    the general one.  Over the forms both accept: contiguous heads and (B, L, H, D) views, with and without a table,
-    the three score modes, no padding, right padding, padding on both sides, an empty sequence.  Both round the
-    probabilities to the type (2^-9 / 2^-12) and the result once more, and sum in other orders."""
-    from turbot5_amd import ops
-    B, H, D = 3, 4, 64
-    side = L // gbs if with_side else 0
-    q, k, v = (rnd(B, L, H, D, seed=301 + i, dtype=dtype).to(gpu_device).transpose(1, 2) for i in range(3))
-    sk, sv = (rnd(B, H, side, D, seed=304 + i, dtype=dtype).to(gpu_device) for i in range(2))
-    table = rnd(32, H, seed=306, scale=1.0).to(gpu_device)
-    lens = torch.tensor([L, (2 * L) // 3, 0], dtype=torch.int32, device=gpu_device)
-    starts = torch.tensor([0, L // 4, 0], dtype=torch.int32, device=gpu_device)
-    tol = 2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -9
-    for contiguous, tab, exact, kw in ((False, table, None, {}), (True, None, True, {}), (False, table, "prescaled", {}),
-                                       (False, table, None, dict(seq_lens=lens)),
-                                       (True, table, None, dict(seq_lens=lens, seq_starts=starts))):
-        a, b, c = (t.contiguous() if contiguous else t for t in (q, k, v))
-        got = []
-        for run_len in (0, 1):
-            monkeypatch.setattr(ops, "RUN_LEN", run_len)
-            got.append(ops.transient_global_attention_with_fusing_bias(a, b, c, sk, sv, tab, Bl, gbs, exact_scores=exact, **kw) if with_side
-                       else ops.local_attention_with_fusing_bias(a, b, c, tab, Bl, exact_scores=exact, **kw))
-        new, old = (t.float().cpu() for t in got)
-        for s in range(B):
-            lo, hi = (0, L) if not kw else (int(starts[s]) if "seq_starts" in kw else 0, 0)
-            if kw:
-                hi = lo + int(lens[s])
-            assert torch.isfinite(new[s]).all()
-            assert (new[s, :, lo:hi] - old[s, :, lo:hi]).abs().max().item() <= tol if hi > lo else True, (contiguous, exact, list(kw), s)
-
-
 def _window_launch_batch(gpu_device, H, L):
     """a batch whose 128-row blocks outnumber two per compute unit"""
     cus = torch.cuda.get_device_properties(gpu_device).multi_processor_count
     return 2 * cus // (H * ((L + 127) // 128)) + 1
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("with_side", [False, True])
+@pytest.mark.parametrize("L,Bl,gbs", [(1, 128, 16), (31, 1, 8), (33, 33, 32), (129, 64, 5), (160, 256, 7), (700, 128, 16), (1025, 100, 33)])
+def test_window_kernel_agrees_with_the_general_kernel(gpu_device, dtype, with_side, L, Bl, gbs):
+    """16-bit tensors at head_dim 64 with a window of up to 256 take the kernel of 32 x 32 blocks, with side tokens if there are
+    more than two blocks of 128 rows per compute unit; validity bits take the general one.  Over the forms both accept:
+    contiguous heads and (B, L, H, D) views, with and without a table, the three score modes, no padding, right padding,
+    padding on both sides, an empty sequence.  Both round the probabilities to the type (2^-9 / 2^-12) and the result once
+    more, and sum in other orders."""
+    from turbot5_amd import ops
+    S, H, D = 3, 4, 64
+    B = S * (_window_launch_batch(gpu_device, H, L) // S + 1)      # three sequences, over and over
+    side = L // gbs if with_side else 0
+    q, k, v = (rnd(S, L, H, D, seed=301 + i, dtype=dtype).to(gpu_device).transpose(1, 2) for i in range(3))
+    sk, sv = (rnd(S, H, side, D, seed=304 + i, dtype=dtype).to(gpu_device) for i in range(2))
+    table = rnd(32, H, seed=306, scale=1.0).to(gpu_device)
+    lens = torch.tensor([L, (2 * L) // 3, 0], dtype=torch.int32, device=gpu_device)
+    starts = torch.tensor([0, L // 4, 0], dtype=torch.int32, device=gpu_device)
+    tol = 2.0 ** -6 if dtype == torch.bfloat16 else 2.0 ** -9
+    pos = torch.arange(L, device=gpu_device)[None, :]
+
+    def run(a, b, c, d, e, tab, exact, **kw):
+        if with_side:
+            return ops.transient_global_attention_with_fusing_bias(a, b, c, d, e, tab, Bl, gbs, exact_scores=exact, **kw)
+        return ops.local_attention_with_fusing_bias(a, b, c, tab, Bl, exact_scores=exact, **kw)
+    for contiguous, tab, exact, ln, st in ((False, table, None, None, None), (True, None, True, None, None),
+                                           (False, table, "prescaled", None, None), (False, table, None, lens, None),
+                                           (True, table, None, lens, starts)):
+        lo = torch.zeros_like(lens) if st is None else st
+        mask = (pos >= lo[:, None]) & (pos < (lo + (torch.full_like(lens, L) if ln is None else ln))[:, None])
+        bits = dict(key_bits=ops.pack_key_bits(mask, Bl, gbs if with_side else 0))
+        if with_side:
+            bits["side_counts"] = ops.side_token_counts(mask, gbs)
+        few = [t.contiguous() if contiguous else t for t in (q, k, v)]
+        many = [t.transpose(1, 2).repeat(B // S, 1, 1, 1).transpose(1, 2) for t in (q, k, v)]
+        many = [t.contiguous() if contiguous else t for t in many] + [t.repeat(B // S, 1, 1, 1) for t in (sk, sv)]
+        kw = {name: t.repeat(B // S) for name, t in (("seq_lens", ln), ("seq_starts", st)) if t is not None}
+        new = run(*many, tab, exact, **kw)
+        assert torch.isfinite(new).all()
+        assert torch.equal(new[:S], new[-S:])          # (a sequence's result does not depend on where it stands)
+        old = run(*few, sk, sv, tab, exact, **bits)
+        rows = mask[:, None, :, None].expand_as(old)
+        assert not rows.any() or (new[:S].float() - old.float())[rows].abs().max().item() <= tol, (contiguous, exact, ln is None, st is None)
+
+
+def test_transient_global_launches_that_fit_the_chip_at_once_take_the_general_kernel(gpu_device):
+    """Up to two blocks of 128 rows per compute unit: bit for bit what validity bits, which only the general kernel takes,
+    give; one block more: the window kernel, the same up to rounding."""
+    from turbot5_amd import ops
+    cus = torch.cuda.get_device_properties(gpu_device).multi_processor_count
+    H, L, D, Bl, gbs = 8, 500, 64, 128, 16
+    most = 2 * cus // (H * 4)
+    q, k, v = (rnd(most + 1, H, L, D, seed=601 + i, dtype=torch.bfloat16).to(gpu_device) for i in range(3))
+    sk, sv = (rnd(most + 1, H, L // gbs, D, seed=604 + i, dtype=torch.bfloat16).to(gpu_device) for i in range(2))
+    table = rnd(32, H, seed=606, scale=1.0).to(gpu_device)
+    mask = torch.ones(most + 1, L, device=gpu_device)
+    bits, counts = ops.pack_key_bits(mask, Bl, gbs), ops.side_token_counts(mask, gbs)
+    f = ops.transient_global_attention_with_fusing_bias
+    general = f(q, k, v, sk, sv, table, Bl, gbs, key_bits=bits, side_counts=counts)
+    fits = f(q[:most], k[:most], v[:most], sk[:most], sv[:most], table, Bl, gbs)
+    assert torch.equal(fits, general[:most])
+    more = f(q, k, v, sk, sv, table, Bl, gbs)
+    assert not torch.equal(more, general) and (more.float() - general.float()).abs().max().item() <= 2.0 ** -6
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

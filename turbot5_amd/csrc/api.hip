@@ -549,6 +549,20 @@ static void choose_runs(FwdParams* p, int mode, int dtype, int D, int cus, int f
     p->total_items = (int)((entries + p->run_len - 1) / p->run_len);
 }
 
+// Whether a local or transient-global call goes to window16_kernel.  With side tokens only launches of more than two
+// 128-row blocks per compute unit do: up to there the general kernel's blocks all run at once and are the shorter ones,
+// beyond it needs a second round where the window kernel, with four blocks per compute unit, does not.  us, general / window,
+// window 128, side tokens every 16, bf16: 8 heads x 2048 14.7 / 18.5, 12 x 4096 (384 blocks) 21.6 / 26.0, 8 x 8000 (504)
+// 27.6 / 32.2, 12 x 5504 (516) 37.5 / 33.3, 8 x 12 x 1024 30.8 / 26.7, 12 x 8192 41.6 / 39.4, 3 x 12 x 10000 147 / 131,
+// 2 x 12 x 16384 186 / 177; single documents of 12 heads from 11000 on are even (12288 71.8 / 73.4, 16384 103 / 100, 24576
+// 178 / 180), with side tokens every 32 16384 71.1 / 68.2.  Without side tokens: 12 x 1024 12.6 / 13.2, window 256 17.1 /
+// 18.4 (256 blocks, both with a ready LUT image; a captured graph has none), 8 x 4500 15.6 / 14.9, 8 x 12 x 1024 27 / 21, 12 x
+// 16384 45 / 40, 32768 75 / 63, window 64 and 96 faster at every size.
+static bool takes_window_kernel(int dtype, int D, int block_len, bool with_side, int B, int H, int L, int cus) {
+    if (dtype == T5A_F32 || D != 64 || block_len > kMaxLutWindow) return false;
+    return !with_side || (int64_t)((L + 127) / 128) * H * B > 2 * (int64_t)cus;
+}
+
 // Key splits for the global rows of the block pattern: enough (batch, head, split) items to fill the
 // device about twice, at least four key tiles of 64 per split.
 static void global_row_splits(int B, int H, int L, int* nsplit, int* split_rows) {
@@ -823,8 +837,9 @@ int t5a_fwd_sparse(const t5a_sparse_args* a, t5a_stream_t stream) {
         }
         return finish(launch_fwd(g, a->dtype, a->D, kDense, false, s), "t5a_fwd_sparse(block, global rows)");
     }
-    if (a->D == 64 && a->dtype != T5A_F32 && a->block_len <= kMaxLutWindow && a->run_len == 0 && a->key_bits == nullptr)
-        return finish(launch_window(p, a->dtype, a->pattern == T5A_PATTERN_TGLOBAL && a->n_side > 0, s), "t5a_fwd_sparse(window)");
+    const bool with_side = a->pattern == T5A_PATTERN_TGLOBAL && a->n_side > 0;
+    if (a->run_len == 0 && a->key_bits == nullptr && takes_window_kernel(a->dtype, a->D, a->block_len, with_side, a->B, a->H, a->L, cus))
+        return finish(launch_window(p, a->dtype, with_side, s), "t5a_fwd_sparse(window)");
     p.tiles_per_seq = (a->L + 127) / 128;
     // (validity bit sets go with the instantiation that masks per element)
     const int mode = a->pattern == T5A_PATTERN_TGLOBAL ? (a->key_bits != nullptr ? kTGlobalBits : kTGlobal)

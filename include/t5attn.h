@@ -306,7 +306,8 @@ typedef struct t5a_sparse_args {
     const int32_t* side_counts;   /* TGLOBAL with key_bits: (B) int32, side tokens of each sequence */
     /* LOCAL (windows up to 256) and BLOCK with 16-bit inputs at head_dim 64 / 128: a work item takes run_len
      * consecutive q tiles of one (batch, head).  0: the library chooses from the shape and the device's size;
-     * 1..16: this many (tests pin every path with it; results do not depend on it). */
+     * 1..16: this many (tests pin every path with it; results do not depend on it).  Calls whose work items are no
+     * runs (the other patterns and types, and LOCAL at head_dim 64 without key_bits) ignore it. */
     int32_t run_len; int32_t reserved;
 } t5a_sparse_args;
 /* words per sequence that key_bits needs (front padding, ceil(L / 32), back padding) */

@@ -219,18 +219,20 @@ def test_splitk_over_padded_memories(gpu_device, dtype, M, N, S):
         flash_decoding_attention(dq, dk, dv, None, 1.0, key_starts=ts)
 
 
+@pytest.mark.parametrize("D", [64, 128])
 @pytest.mark.parametrize("run_len", [1, 2, 3, 5, 16])
 @pytest.mark.parametrize("L,Bl", [(640, 128), (333, 100), (1000, 16), (896, 256), (700, 300)])
-def test_local_with_runs_of_q_tiles(gpu_device, monkeypatch, run_len, L, Bl):
+def test_local_with_runs_of_q_tiles(gpu_device, monkeypatch, run_len, L, Bl, D):
     """The local pattern's work items are runs of consecutive q tiles (one stream of key tiles through the LDS
     rings, the distance LUT built once per run); a run may end inside a (batch, head) or cross into the next
     one.  Every run length must give what the window definition gives, for sequence lengths that are no
-    multiple of anything, with per-sequence lengths, and for windows too wide for the LUT (masked path)."""
+    multiple of anything, with per-sequence lengths, and for windows too wide for the LUT (masked path).  (head_dim 64
+    with a window that fits the LUT has a kernel without runs: the same whatever the run length.)"""
     from turbot5_amd import ops
     from turbot5_amd.ops import local_attention_with_fusing_bias
     monkeypatch.setattr(ops, "RUN_LEN", run_len)
-    B, H, D = 2, 3, 64
-    q, k, v = (rnd(B, H, L, D, seed=300 + i, dtype=torch.bfloat16) for i in range(3))
+    B, H = 2, 3
+    q, k, v = (rnd(B, H, L, D, seed=300 + i, scale=0.5 if D == 64 else 0.42, dtype=torch.bfloat16) for i in range(3))
     table = rnd(32, H, seed=303, scale=1.0)
     lens = torch.tensor([L, max(1, L - 217)], dtype=torch.int32)
     dev = [t.to(gpu_device) for t in (q, k, v, table)]
@@ -247,6 +249,27 @@ def test_local_with_runs_of_q_tiles(gpu_device, monkeypatch, run_len, L, Bl):
         wb = O.basic_attention(q[b:b + 1, :, :n].float(), k[b:b + 1, :, :n].float(), v[b:b + 1, :, :n].float(),
                                bias[:, :, :n, :n])
         assert (out_l[b:b + 1, :, :n] - wb).abs().max().item() <= 2e-2, b
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("pattern", ["local", "tglobal", "block"])
+def test_results_do_not_depend_on_the_run_length(gpu_device, monkeypatch, pattern, D, dtype):
+    """Bit for bit; the block pattern's global rows are spread over key splits whose number goes with the run length, so
+    they are left out."""
+    from turbot5_amd import ops
+    B, H, L, Bl = 2, 3, 700, 128
+    q, k, v = (rnd(B, H, L, D, seed=340 + i, dtype=dtype).to(gpu_device) for i in range(3))
+    sk, sv = (rnd(B, H, L // 16, D, seed=343 + i, dtype=dtype).to(gpu_device) for i in range(2))
+    table = rnd(32, H, seed=345, scale=1.0).to(gpu_device)
+    call = {"local": lambda: ops.local_attention_with_fusing_bias(q, k, v, table, Bl),
+            "tglobal": lambda: ops.transient_global_attention_with_fusing_bias(q, k, v, sk, sv, table, Bl, 16),
+            "block": lambda: ops.block_attention_with_fusing_bias(q, k, v, table, Bl, 64)[:, :, 64:]}[pattern]
+    out = []
+    for run_len in (0, 1, 3, 16):
+        monkeypatch.setattr(ops, "RUN_LEN", run_len)
+        out.append(call())
+    assert all(torch.equal(out[0], o) for o in out[1:])
 
 
 @pytest.mark.parametrize("run_len", [1, 2, 3, 7, 16])

@@ -838,7 +838,7 @@ int t5a_fwd_sparse(const t5a_sparse_args* a, t5a_stream_t stream) {
         return finish(launch_fwd(g, a->dtype, a->D, kDense, false, s), "t5a_fwd_sparse(block, global rows)");
     }
     const bool with_side = a->pattern == T5A_PATTERN_TGLOBAL && a->n_side > 0;
-    if (a->run_len == 0 && a->key_bits == nullptr && takes_window_kernel(a->dtype, a->D, a->block_len, with_side, a->B, a->H, a->L, cus))
+    if (a->key_bits == nullptr && takes_window_kernel(a->dtype, a->D, a->block_len, with_side, a->B, a->H, a->L, cus))
         return finish(launch_window(p, a->dtype, with_side, s), "t5a_fwd_sparse(window)");
     p.tiles_per_seq = (a->L + 127) / 128;
     // (validity bit sets go with the instantiation that masks per element)

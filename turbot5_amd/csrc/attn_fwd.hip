@@ -2158,7 +2158,9 @@ static hipError_t launch_mode(const FwdParams& p, int mode, bool causal, hipStre
     switch (mode) {
         case kDense: return causal ? launch_one<T, D, kDense, true>(p, s) : launch_one<T, D, kDense, false>(p, s);
         case kPacked: return causal ? launch_one<T, D, kPacked, true>(p, s) : launch_one<T, D, kPacked, false>(p, s);
-        case kLocal: return launch_one<T, D, kLocal, false>(p, s);
+        case kLocal:
+            if constexpr (sizeof(T) == 2 && D == 64) return hipErrorInvalidValue;     // (launch_window's)
+            else return launch_one<T, D, kLocal, false>(p, s);
         case kLocalWide: return launch_one<T, D, kLocalWide, false>(p, s);
         case kBlock: return launch_one<T, D, kBlock, false>(p, s);
         case kBlockBits: return launch_one<T, D, kBlockBits, false>(p, s);

@@ -355,10 +355,17 @@ def test_sparse_launch_plans_cover_every_item(lib, cus):
                             assert nsplit == 0
     assert seen_single_split or cus > 256
     # the local pattern: runs only; fp32 and other head dims: one q tile per item
-    for dtype, D, want_runs in ((lib.T5A_BF16, 64, True), (lib.T5A_F32, 64, False), (lib.T5A_BF16, 32, False)):
-        assert L_.t5a_sparse_launch_plan(lib.PATTERN_LOCAL, dtype, 1, 12, 16384, D, 128, 0, 0, cus, 0, out) == 0
-        rl, items, block_items, nsplit, split_rows, tps = list(out)
-        assert tps == 128 and block_items == 0 and items * rl >= 128 * 12 > (items - 1) * rl
-        assert (rl > 1) == (want_runs and 2 * cus < 128 * 12)
+    # (the 16-bit kernel for windows up to 256 at head_dim 64 has no runs either, pinned or not)
+    for dtype, D, window, want_runs in ((lib.T5A_BF16, 128, 128, True), (lib.T5A_F32, 64, 128, False), (lib.T5A_BF16, 32, 128, False),
+                                        (lib.T5A_BF16, 64, 128, False), (lib.T5A_F16, 64, 256, False)):
+        for run_len in (0, 3):
+            assert L_.t5a_sparse_launch_plan(lib.PATTERN_LOCAL, dtype, 1, 12, 16384, D, window, 0, 0, cus, run_len, out) == 0
+            rl, items, block_items, nsplit, split_rows, tps = list(out)
+            assert tps == 128 and block_items == 0 and items * rl >= 128 * 12 > (items - 1) * rl
+            assert (rl > 1) == (want_runs and (run_len > 1 or 2 * cus < 128 * 12))
+    for pattern, aux in ((lib.PATTERN_LOCAL, 0), (lib.PATTERN_TGLOBAL, 16)):
+        for B, L in ((1, 1), (1, 129), (3, 5000), (8, 16384)):
+            assert L_.t5a_sparse_launch_plan(pattern, lib.T5A_BF16, B, 12, L, 64, 128, aux, 0, cus, 0, out) == 0
+            assert list(out) == [1, B * 12 * ((L + 127) // 128), 0, 0, 0, (L + 127) // 128]
     assert L_.t5a_sparse_launch_plan(lib.PATTERN_BLOCK, lib.T5A_BF16, 1, 1, 128, 64, 128, 64, 1, cus, 17, out) < 0
     assert L_.t5a_sparse_launch_plan(9, lib.T5A_BF16, 1, 1, 128, 64, 128, 64, 1, cus, 0, out) < 0

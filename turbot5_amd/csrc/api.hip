@@ -682,7 +682,8 @@ int t5a_sparse_launch_plan(int32_t pattern, int32_t dtype, int32_t B, int32_t H,
         p.tiles_per_seq = (L + 127) / 128;
         const int mode = pattern == T5A_PATTERN_BLOCK ? kDense : pattern == T5A_PATTERN_TGLOBAL ? kTGlobal
                          : (block_len <= kMaxLutWindow ? kLocal : kLocalWide);
-        choose_runs(&p, mode, dtype, D, cus, run_len);
+        const bool window = pattern != T5A_PATTERN_BLOCK && takes_window_kernel(dtype, D, block_len, pattern == T5A_PATTERN_TGLOBAL, B, H, L, cus);
+        choose_runs(&p, window ? kTGlobal : mode, dtype, D, cus, run_len);     // (the window kernel: one block of 128 rows per item)
     } else {
         return fail(T5A_ERR_PATTERN, "unknown pattern %d", pattern);
     }

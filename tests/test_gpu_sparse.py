@@ -370,8 +370,8 @@ def test_local_windowed_lut_buffer_gives_identical_results(gpu_device, L, Bl):
     buffer, on the launch that builds it and on those that find it ready; buffers for different windows and the plain
     one of the same table are separate entries."""
     from turbot5_amd import ops
-    B, H, D = 2, 3, 64
-    q, k, v = (rnd(B, H, L, D, seed=140 + i, dtype=torch.bfloat16).to(gpu_device) for i in range(3))
+    B, H, D = 2, 3, 128      # (head_dim 64 has a kernel that reads no images)
+    q, k, v = (rnd(B, H, L, D, seed=140 + i, scale=0.42, dtype=torch.bfloat16).to(gpu_device) for i in range(3))
     table = rnd(32, H, seed=143, scale=1.0).to(gpu_device)
     run = lambda bl=Bl: ops.local_attention_with_fusing_bias(q, k, v, table, bl).cpu()  # noqa: E731
     ops.clear_bias_luts()
@@ -407,7 +407,7 @@ def test_windowed_lut_buffer_is_only_for_its_window(gpu_device):
     import ctypes as C
     from turbot5_amd import _lib as lib_mod, ops
     lib = lib_mod.load()
-    B, H, L, D, Bl = 1, 2, 256, 64, 64
+    B, H, L, D, Bl = 1, 2, 256, 128, 64
     q, k, v = (rnd(B, H, L, D, seed=150 + i, dtype=torch.bfloat16).to(gpu_device) for i in range(3))
     table = rnd(32, H, seed=153, scale=1.0).to(gpu_device)
     o = torch.empty_like(q)
@@ -620,3 +620,28 @@ def test_transient_global_keeps_a_non_finite_key_to_the_rows_that_see_it(gpu_dev
     assert torch.isfinite(out[:, :, apart]).all() and torch.equal(out[:, :, apart], clean[:, :, apart])
     if bad != bad:
         assert torch.isnan(out[:, :, ~apart]).all()
+
+
+def test_lut_images_are_built_for_the_calls_that_read_them(gpu_device):
+    """Sliding windows of 16-bit tensors at head_dim 64 fill their table per workgroup: no image is built or kept for them;
+    the other kernels' calls keep one."""
+    from turbot5_amd import ops
+    H, L = 4, 300
+    table = rnd(32, H, seed=703, scale=1.0).to(gpu_device)
+
+    def entries(B, D, dtype, Bl, gbs=0, side=True):
+        q, k, v = (rnd(B, H, L, D, seed=700 + i, dtype=dtype).to(gpu_device) for i in range(3))
+        ops.clear_bias_luts()
+        if gbs:
+            sk, sv = (rnd(B, H, L // gbs if side else 0, D, seed=704 + i, dtype=dtype).to(gpu_device) for i in range(2))
+            ops.transient_global_attention_with_fusing_bias(q, k, v, sk, sv, table, Bl, gbs)
+        else:
+            ops.local_attention_with_fusing_bias(q, k, v, table, Bl)
+        return len(ops._BIAS_LUTS)
+    many = _window_launch_batch(gpu_device, H, L)
+    bf16 = torch.bfloat16
+    assert entries(1, 64, bf16, 128) == entries(1, 64, torch.float16, 64) == entries(many, 64, bf16, 128, 16) == 0
+    assert entries(1, 64, bf16, 128, 16, side=False) == 0
+    assert entries(1, 128, bf16, 128) == entries(1, 64, torch.float32, 128) == entries(1, 64, bf16, 300) == 1
+    assert entries(1, 64, bf16, 128, 16) == entries(many - 1, 64, bf16, 128, 16) == entries(many, 128, bf16, 128, 16) == 1
+    ops.clear_bias_luts()

@@ -149,7 +149,8 @@ def clear_bias_luts():
 
 
 def _bias_struct(bias: Optional[torch.Tensor], H: int, num_buckets: int, max_distance: int, ref: torch.Tensor,
-                 causal: bool = False, window: int = 0):
+                 causal: bool = False, window: Optional[int] = 0):
+    """``window`` None: a call whose kernel reads no distance LUT from memory."""
     if bias is None:
         return L.T5ABias(), None
     if bias.dim() != 2 or bias.shape[0] != num_buckets or bias.shape[1] != H:
@@ -161,7 +162,7 @@ def _bias_struct(bias: Optional[torch.Tensor], H: int, num_buckets: int, max_dis
         table = table.float()
     b = L.T5ABias(table.data_ptr(), _DTYPES[table.dtype], num_buckets, max_distance, 0, *table.stride())
     lut, pending = (_bias_lut(b, bias, H, num_buckets, max_distance, causal, ref, window)
-                    if table.data_ptr() == bias.data_ptr() else (None, None))
+                    if window is not None and table.data_ptr() == bias.data_ptr() else (None, None))
     return b, (table, lut, pending, bias)   # alive until the launch has been queued; see _commit_lut
 
 
@@ -576,8 +577,13 @@ def _sparse(pattern, q, k, v, bias, block_len, aux, side_k=None, side_v=None, sm
         a.key_bits, a.key_bits_stride = key_bits.data_ptr(), key_bits.shape[1]
         if side_counts is not None:
             a.side_counts = side_counts.data_ptr()
-    # the local pattern's work items fetch LUT images that have the window folded in (windows up to 256)
+    # The local pattern's work items fetch LUT images that have the window folded in (windows up to 256); the kernel for
+    # sliding windows of 16-bit tensors at head_dim 64 fetches none (takes_window_kernel of the library: if the two rules
+    # ever differ, a call fills its LUTs itself, or builds a buffer that it does not read)
     window = int(block_len) if pattern == L.PATTERN_LOCAL and int(block_len) <= 256 and key_bits is None else 0
+    if (pattern != L.PATTERN_BLOCK and D == 64 and q.dtype != torch.float32 and int(block_len) <= 256 and key_bits is None
+            and (pattern == L.PATTERN_LOCAL or a.n_side == 0 or (Lq + 127) // 128 * H * B > 2 * _cu_count(q.device))):
+        window = None
     a.bias, keep = _bias_struct(bias, H, NUM_BUCKETS, MAX_DISTANCE, q, window=window)
     lib = L.load()
     ws_bytes = lib.t5a_sparse_workspace_bytes(pattern, B, H, Lq, D, int(block_len), int(aux))

@@ -801,8 +801,12 @@ hipError_t launch_bwd16_pass(const BwdParams& p, hipStream_t stream) {
     const int64_t blocks = (int64_t)nblk * p.H * p.B;
     if (blocks > 0x7fffffff) return hipErrorInvalidConfiguration;
     const bool bias = p.table != nullptr;
-    hipLaunchKernelGGL((bwd16_kernel<T, D, CAUSAL, PASS, SPLIT>), dim3((unsigned)blocks), dim3(kBwdThreads),
-                       G::bytes(bias ? p.bs.sat : 0, bias), stream, p, nblk);
+    const int lds = G::bytes(bias ? p.bs.sat : 0, bias);
+    auto kern = bwd16_kernel<T, D, CAUSAL, PASS, SPLIT>;
+    static LdsLimit limit;     // (per instantiation; 67 KB and more at head_dim 128 with SPLIT 2, 90.6 with the widest bucketing)
+    const hipError_t e = limit.allow(reinterpret_cast<const void*>(kern), lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBwdThreads), lds, stream, p, nblk);
     return hipGetLastError();
 }
 

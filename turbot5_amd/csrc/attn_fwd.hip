@@ -46,7 +46,6 @@
 //
 // Sparsity patterns are tile skipping: the key segments of a work item are
 // computed from integer positions; nothing outside them is loaded.
-#include <atomic>
 #include <type_traits>
 
 #include "t5a_internal.h"
@@ -2114,22 +2113,9 @@ static hipError_t launch_exact(const FwdParams& p, hipStream_t stream) {
     const size_t lut_bytes = (((size_t)16 * lut_quads(sat, CAUSAL) * sizeof(float) + 1023) & ~(size_t)1023) + 1024;
     const size_t smem = Geometry<T, D>::kTileBytes + lut_bytes;
     auto kern = fwd_kernel<T, D, MODE, CAUSAL, EXACT>;
-    // per instantiation and device: largest dynamic LDS size already allowed (the attribute belongs to the
-    // function as loaded on one device)
-    constexpr int kMaxDevices = 64;
-    static std::atomic<size_t> granted[kMaxDevices] = {};
-    int dev = 0;
-    if (smem > 48 * 1024) {
-        hipError_t e = hipGetDevice(&dev);
-        if (e != hipSuccess) return e;
-        const bool known = dev >= 0 && dev < kMaxDevices;
-        if (!known || smem > granted[dev].load(std::memory_order_relaxed)) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
-            if (e != hipSuccess) return e;
-            if (known) granted[dev].store(smem, std::memory_order_relaxed);
-        }
-    }
+    static LdsLimit limit;     // (per instantiation)
+    const hipError_t e = limit.allow(reinterpret_cast<const void*>(kern), smem);
+    if (e != hipSuccess) return e;
     unsigned grid = (unsigned)(((p.total_items + 7) / 8) * 8);
     if ((MODE == kBlock || MODE == kBlockBits) && p.block_items > 0)
         grid = (unsigned)(((p.total_items - p.block_items + 7) / 8) * 8 + ((p.block_items + 7) / 8) * 8);

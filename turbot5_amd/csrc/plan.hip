@@ -26,8 +26,6 @@
 // how many entries of list x are in use.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-
 #include "t5a_internal.h"
 
 namespace t5a {
@@ -261,21 +259,9 @@ bool plan_can_stage(int slots, int H, int max_seqlen_q) {
 
 hipError_t launch_varlen_plan(const PlanParams& p, hipStream_t stream) {
     const size_t dyn = p.staged ? (size_t)8 * p.slots * sizeof(int) : 0;
-    // per device: largest dynamic LDS size already allowed (the attribute belongs to the function as loaded on one device)
-    constexpr int kMaxDevices = 64;
-    static std::atomic<size_t> granted[kMaxDevices] = {};
-    if (dyn > 0) {   // static + dynamic LDS beyond 64 KB must be allowed first
-        int dev = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e != hipSuccess) return e;
-        const bool known = dev >= 0 && dev < kMaxDevices;
-        if (!known || dyn > granted[dev].load(std::memory_order_relaxed)) {
-            e = hipFuncSetAttribute(reinterpret_cast<const void*>(varlen_plan_kernel),
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);
-            if (e != hipSuccess) return e;
-            if (known) granted[dev].store(dyn, std::memory_order_relaxed);
-        }
-    }
+    static LdsLimit limit;
+    const hipError_t e = limit.allow(reinterpret_cast<const void*>(varlen_plan_kernel), dyn, 48 * 1024);
+    if (e != hipSuccess) return e;
     hipLaunchKernelGGL(varlen_plan_kernel, dim3(1), dim3(PLAN_THREADS), dyn, stream, p);
     return hipGetLastError();
 }

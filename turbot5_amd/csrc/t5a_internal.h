@@ -3,12 +3,39 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <mutex>
+
 #include "../../include/t5attn.h"
 
 namespace t5a {
 
 constexpr int kMaxThresholds = 128;   // supports num_buckets up to 256
 constexpr int kMaxSaturation = 1024;  // largest distance at which buckets still change
+
+// LDS past 48 KB is allowed before the launch that asks for it (`bytes` of dynamic LDS next to `fixed` ones).  The attribute belongs to the function as loaded on
+// one device: one of these per kernel keeps the largest size allowed on each.
+class LdsLimit {
+public:
+    hipError_t allow(const void* kernel, size_t bytes, size_t fixed = 0) {
+        if (bytes == 0 || bytes + fixed <= 48 * 1024) return hipSuccess;
+        int dev = 0;
+        hipError_t e = hipGetDevice(&dev);
+        if (e != hipSuccess) return e;
+        const bool known = dev >= 0 && dev < kMaxDevices;
+        if (known && bytes <= granted_[dev].load(std::memory_order_acquire)) return hipSuccess;
+        std::lock_guard<std::mutex> g(mu_);      // (a smaller size must not follow a larger one)
+        if (known && bytes <= granted_[dev].load(std::memory_order_relaxed)) return hipSuccess;
+        e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        if (e == hipSuccess && known) granted_[dev].store(bytes, std::memory_order_release);
+        return e;
+    }
+
+private:
+    static constexpr int kMaxDevices = 64;
+    std::atomic<size_t> granted_[kMaxDevices] = {};
+    std::mutex mu_;
+};
 
 // Integer description of the T5 bucket function, derived on the host from the
 // per-distance table so that device code never evaluates a logarithm.

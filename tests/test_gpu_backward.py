@@ -156,8 +156,8 @@ def test_fp32_table_gradient_leaves_out_keys_past_the_end(gpu_device, D, B, H, M
 @pytest.mark.parametrize("causal", [False, True])
 @pytest.mark.parametrize("B,H,M,N", [(48, 16, 33, 65), (53, 15, 130, 97), (24, 16, 290, 257)])
 def test_16_bit_gradients_of_launches_that_fill_the_chip(gpu_device, causal, D, B, H, M, N):
-    """From 512 (causal 768) blocks of 128 own rows on a workgroup owns 128 rows and walks tiles of 32; below, 64 rows
-    and tiles of 64 whose halves go to two wavefronts each.  Both kinds of placement ((head, batch) pairs that divide by
+    """From 512 blocks of 128 own rows on (causal 768; head_dim 128 320, causal 768) a workgroup owns 128 rows and walks tiles of
+    32; below, 64 rows and tiles of 64 whose halves go to two wavefronts each.  Both kinds of placement ((head, batch) pairs that divide by
     eight and that do not), a tile more than a multiple of 32 and one row more than a tile."""
     from turbot5_amd import ops
     dtype = torch.bfloat16
@@ -399,6 +399,48 @@ def test_packed_gradients_at_head_dim_128(gpu_device, causal):
     out.backward(dout.to(gpu_device))
     for name, g, w in (("dq", dq.grad, wq), ("dk", dk.grad, wk), ("dv", dv.grad, wv), ("dtable", dt.grad, wt)):
         check(name, g, w, 2e-2)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float16, 64), (torch.bfloat16, 128), (torch.float16, 128)])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("kind", ["self", "padded", "short queries", "short keys"])
+def test_packed_16_bit_gradients_of_launches_that_fill_the_chip(gpu_device, kind, causal, dtype, D):
+    """From 320 blocks of 128 own rows on (counted from the tokens of the pass's own kind) a packed launch owns 128 rows per
+    workgroup and walks tiles of 32.  Twenty sequences of lengths around a tile, packed and padded in place, and as
+    cross-attention in which only one of the passes fills the chip."""
+    from turbot5_amd import ops
+    lens = [1, 33, 65, 97, 129, 2, 31, 32, 64, 96, 128, 130, 17, 5, 48, 80, 112, 7, 100, 127]
+    B, H, room = len(lens), 16 if "short" not in kind else 2, 131
+    lq, lk = lens, lens
+    if kind == "short queries":      # 2 heads: 2 * (20 + 20 * 1000 / 128) blocks of keys, 2 * 31 of queries
+        lk = [1000 + n for n in lens]
+    elif kind == "short keys":
+        lq = [1000 + n for n in lens]
+    def offsets(ls):
+        return torch.tensor([room * b for b in range(B + 1)] if kind == "padded" else [0] + list(torch.tensor(ls).cumsum(0)), dtype=torch.int32)
+    cq, ck = offsets(lq), offsets(lk)
+    Tq, Tk = int(cq[-1]), int(ck[-1])
+    q, k, v = (rnd(n, H, D, seed=120 + i, scale=0.5 if D == 64 else 0.42, dtype=dtype) for i, n in enumerate((Tq, Tk, Tk)))
+    table = rnd(32, H, seed=123, scale=1.0)
+    dout = rnd(Tq, H, D, seed=124, scale=1.0, dtype=dtype)
+    want = [torch.zeros(n, H, D) for n in (Tq, Tk, Tk)]
+    wt = torch.zeros(32, H)
+    for b in range(B):
+        i, j = slice(int(cq[b]), int(cq[b]) + lq[b]), slice(int(ck[b]), int(ck[b]) + lk[b])
+        _, *gs, gt = oracle_grads(*(t[s].transpose(0, 1)[None] for t, s in ((q, i), (k, j), (v, j))), table,
+                                  dout[i].transpose(0, 1)[None], causal, 1.0)
+        for w, s, g in zip(want, (i, j, j), gs):
+            w[s] = g[0].transpose(0, 1)
+        wt += gt
+    dq, dk, dv, dt = (t.to(gpu_device).requires_grad_(True) for t in (q, k, v, table))
+    kw = {}
+    if kind == "padded":
+        kw = {n: torch.tensor(lens, dtype=torch.int32, device=gpu_device) for n in ("seq_lens_q", "seq_lens_k")}
+    out = ops.flash_attention_with_fusing_bias_varlen(dq, dk, dv, dt, cq.to(gpu_device), ck.to(gpu_device), max(lq), max(lk),
+                                                      causal=causal, sm_scale=1.0, **kw)
+    out.backward(dout.to(gpu_device))
+    for name, g, w in (("dq", dq.grad, want[0]), ("dk", dk.grad, want[1]), ("dv", dv.grad, want[2]), ("dtable", dt.grad, wt)):
+        check(name, g, w, TOL[dtype])
 
 
 def test_packed_gradients_of_a_padded_batch_in_place(gpu_device):

@@ -411,7 +411,7 @@ int t5a_bwd_varlen(const t5a_varlen_bwd_args* a, t5a_stream_t stream) {
     p.dv_sr = a->dv_strides[0]; p.dv_sh = a->dv_strides[1];
     p.B = a->B; p.H = a->H; p.M = a->max_seqlen_q; p.N = a->max_seqlen_k;
     p.cu_q = a->cu_seqlens_q; p.cu_k = a->cu_seqlens_k; p.len_q = a->seq_lens_q; p.len_k = a->seq_lens_k;
-    p.total_q = a->total_q;
+    p.total_q = a->total_q; p.total_k = a->total_k;
     FwdParams f;
     memset(&f, 0, sizeof(f));
     if ((rc = score_mode(a->exact_scores, a->sm_scale, &f))) return rc;

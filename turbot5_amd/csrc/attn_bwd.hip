@@ -786,9 +786,12 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
 // sides, us, three kernels, bf16: head_dim 64 full attention, 256 workgroups 245 / 190 (SPLIT 1 / 2), 384 294 / 276, 512
 // 302 / 333; causal, where the longest block counts, 512 233 / 182, 1536 181 / 228; head_dim 128 256 440 / 325, 384
 // 504 / 586, causal 256 208 / 140, 512 259 / 221, 1024 390 / 441.  Packed, head_dim 64 (workgroups counted from the
-// tokens): 424 67 / 73, causal 58 / 58, 564 186 / 183, 1464 212 / 222.
-bool bwd16_split(const BwdParams& p, int D, bool causal, int rows) {
-    const int64_t blocks = p.cu_q != nullptr ? ((int64_t)p.total_q / 128 + p.B) * p.H : (int64_t)((rows + 127) / 128) * p.H * p.B;
+// tokens of the pass's own kind): 424 67 / 73, causal 58 / 58, 564 186 / 183, 1464 212 / 222; cross-attention of 16 x 32
+// queries over 16 x 2048 keys, 12 heads, where only the key pass fills the chip: 115 us with both passes by the queries'
+// count, 94 each by its own (head_dim 128, 8 heads 175 / 135; 2048 queries over 32 keys 136 / 111).
+bool bwd16_split(const BwdParams& p, int D, bool causal, bool keys) {
+    const int rows = keys ? p.N : p.M;
+    const int64_t blocks = p.cu_q != nullptr ? ((int64_t)(keys ? p.total_k : p.total_q) / 128 + p.B) * p.H : (int64_t)((rows + 127) / 128) * p.H * p.B;
     return blocks < (p.cu_q != nullptr ? 320 : causal ? 768 : D == 64 ? 512 : 320);
 }
 
@@ -812,7 +815,7 @@ hipError_t launch_bwd16_pass(const BwdParams& p, hipStream_t stream) {
 
 template <typename T, int D, bool CAUSAL, int PASS>
 hipError_t launch_bwd16_rows(const BwdParams& p, hipStream_t stream) {
-    return bwd16_split(p, D, CAUSAL, PASS != 0 ? p.N : p.M) ? launch_bwd16_pass<T, D, CAUSAL, PASS, 2>(p, stream)
+    return bwd16_split(p, D, CAUSAL, PASS != 0) ? launch_bwd16_pass<T, D, CAUSAL, PASS, 2>(p, stream)
                                                             : launch_bwd16_pass<T, D, CAUSAL, PASS, 1>(p, stream);
 }
 

@@ -168,7 +168,7 @@ struct BwdParams {
     int B, H, M, N;                   // packed: M, N are the longest sequence's lengths
     // packed batch (optional): (B+1) offsets and optional lengths, as in the forward; tensors are (total, H, D),
     // the statistics (total_q, H)
-    const int32_t* cu_q; const int32_t* cu_k; const int32_t* len_q; const int32_t* len_k; int total_q;
+    const int32_t* cu_q; const int32_t* cu_k; const int32_t* len_q; const int32_t* len_k; int total_q, total_k;
     float c1;                         // base-2 score factor: sm_scale * log2(e), or 1 for pre-scaled query rows
     int fp32_math;                    // nonzero: fp32 matrix cores also for 16-bit inputs at head_dim 64
     int n_buckets;

@@ -443,6 +443,42 @@ def test_packed_16_bit_gradients_of_launches_that_fill_the_chip(gpu_device, kind
         check(name, g, w, TOL[dtype])
 
 
+def bucket_grads(q, k, v, table, dout, causal, num_buckets, max_distance):
+    """oracle_grads for any bucketing"""
+    q, k, v, tb = (t.float().clone().requires_grad_(True) for t in (q, k, v, table))
+    M, N = q.shape[2], k.shape[2]
+    rel = torch.arange(N)[None, :] - (torch.arange(M)[:, None] + N - M)
+    bias = tb[O.relative_position_bucket(rel, not causal, num_buckets, max_distance)].permute(2, 0, 1)[None]
+    if causal:
+        bias = bias.masked_fill(rel > 0, float("-inf"))
+    O.basic_attention(q, k, v, bias).backward(dout.float())
+    return q.grad, k.grad, v.grad, tb.grad
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float16, 128), (torch.float32, 64), (torch.float32, 16)])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("num_buckets,max_distance", [(32, 20), (64, 128), (66, 700), (128, 1024), (512, 1000), (8, 1000)])
+@pytest.mark.parametrize("B,H,M,N", [(1, 2, 700, 777), (36, 16, 33, 131)])
+def test_gradients_with_other_bucketings(gpu_device, B, H, M, N, num_buckets, max_distance, causal, dtype, D):
+    """The tables of the backward passes in LDS are laid out by the distance from which buckets no longer change, and
+    up to 64 buckets are kept in the lanes of a wavefront, more are read from memory: few and many buckets, short
+    and long distances, with blocks of 64 and (36 x 16 heads and more keys than 128) of 128 own rows."""
+    from turbot5_amd import ops
+    if dtype == torch.float32 and B > 1:
+        B, H = 2, 3
+    if causal:
+        num_buckets = min(num_buckets, 256)
+    q, k, v = (rnd(B, H, n, D, seed=131 + i, scale=0.42 if D == 128 else 0.5, dtype=dtype) for i, n in enumerate((M, N, N)))
+    table = rnd(num_buckets, H, seed=134, scale=1.0)
+    dout = rnd(B, H, M, D, seed=135, scale=1.0, dtype=dtype)
+    want = bucket_grads(q, k, v, table, dout, causal, num_buckets, max_distance)
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in (q, k, v, table)]
+    ops.flash_attention_with_fusing_bias(*leaves, causal=causal, sm_scale=1.0, NUM_BUCKETS=num_buckets,
+                                         MAX_DISTANCE=max_distance).backward(dout.to(gpu_device))
+    for name, t, w in zip(("dq", "dk", "dv", "dtable"), leaves, want):
+        check(name, t.grad, w, TOL[dtype])
+
+
 def test_packed_gradients_of_a_padded_batch_in_place(gpu_device):
     """A right-padded (B, L) batch run in place (cu = multiples of L, seq_lens = the lengths), keys longer than the
     queries in one call (cached decoding shape): padding rows get zero gradients, the rest matches the oracle."""

@@ -645,3 +645,29 @@ def test_lut_images_are_built_for_the_calls_that_read_them(gpu_device):
     assert entries(1, 128, bf16, 128) == entries(1, 64, torch.float32, 128) == entries(1, 64, bf16, 300) == 1
     assert entries(1, 64, bf16, 128, 16) == entries(many - 1, 64, bf16, 128, 16) == entries(many, 128, bf16, 128, 16) == 1
     ops.clear_bias_luts()
+
+
+@pytest.mark.parametrize("with_side", [False, True])
+@pytest.mark.parametrize("num_buckets,max_distance", [(32, 16), (66, 700), (128, 1024), (8, 1000)])
+@pytest.mark.parametrize("L,Bl,gbs", [(700, 128, 16), (600, 256, 3), (333, 20, 32)])
+def test_window_kernel_with_other_bucketings(gpu_device, L, Bl, gbs, num_buckets, max_distance, with_side):
+    """Its tables are laid out by the window and, for the side tokens, by the distance from which buckets no longer change."""
+    from turbot5_amd import ops
+    S, H, D = 2, 3, 64
+    q, k, v = (rnd(S, H, L, D, seed=801 + i, dtype=torch.bfloat16) for i in range(3))
+    sk, sv = (rnd(S, H, L // gbs, D, seed=804 + i, dtype=torch.bfloat16) for i in range(2))
+    table = rnd(num_buckets, H, seed=806, scale=1.0)
+    rel = torch.arange(L)[None, :] - torch.arange(L)[:, None]
+    of = lambda r: table[O.relative_position_bucket(r, True, num_buckets, max_distance)].permute(2, 0, 1)[None]  # noqa: E731
+    bias, keys, values = of(rel).masked_fill(rel.abs() >= Bl, float("-inf")), k, v
+    if with_side:
+        n = L // gbs
+        side = torch.arange(n)[None, :] - (torch.arange(L) // gbs).clamp(max=n - 1)[:, None]
+        bias, keys, values = torch.cat([bias, of(side)], -1), torch.cat([k, sk], 2), torch.cat([v, sv], 2)
+    want = O.basic_attention(q.float(), keys.float(), values.float(), bias)
+    reps = _window_launch_batch(gpu_device, H, L) // S + 1
+    dev = [t.repeat(reps, 1, 1, 1).to(gpu_device) for t in (q, k, v, sk, sv)]
+    kw = dict(NUM_BUCKETS=num_buckets, MAX_DISTANCE=max_distance)
+    out = (ops.transient_global_attention_with_fusing_bias(*dev, table.to(gpu_device), Bl, gbs, **kw) if with_side
+           else ops.local_attention_with_fusing_bias(*dev[:3], table.to(gpu_device), Bl, **kw)).float().cpu()
+    assert (out[:S] - want).abs().max().item() <= 2e-2 and (out[-S:] - want).abs().max().item() <= 2e-2

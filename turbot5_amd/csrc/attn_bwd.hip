@@ -37,7 +37,7 @@ namespace {
 constexpr int kBwdThreads = 256;
 constexpr int kBwdOwn = 64;      // own rows per workgroup of the fp32 kernels (queries for dq, keys for dk / dv)
 constexpr int kBwdOther = 64;    // rows of the other kind per tile
-constexpr int kMaxBuckets = 2 * 2 * kMaxThresholds;
+constexpr int kMaxBuckets = 4 * kMaxThresholds;     // of a table; the dq pass sums them in the memory of its tiles
 
 template <typename T> __device__ __forceinline__ float to_f32(T x) { return static_cast<float>(x); }
 
@@ -134,6 +134,7 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
     constexpr int TILE = kBwdOther * STR + 32;
     constexpr int RED = OWNW * (KV ? 2 : 1) * DT * 16 * 64;
     constexpr int SKEW_ROWS = 8;
+    static_assert(2 * TILE >= kMaxBuckets, "");
     __shared__ float tiles[2 * TILE > RED ? 2 * TILE : RED];
     float* const ta = tiles;               // K (dq) / Q (dk, dv) tile
     float* const tb = tiles + TILE;        // V (dq) / dO (dk, dv) tile
@@ -429,6 +430,7 @@ struct Bwd16Geom {
     static constexpr int STAGES = 2;                               // tile buffers
     static constexpr int REQS = 2 * SLABS + (KV ? 1 : 0);         // requests per wavefront and tile
     static constexpr int SKEW_ROWS = (D == 128 && SPLIT == 2) ? 8 : 32;   // queries per round of the table gradient
+    static_assert(STAGES * 2 * TILE >= kMaxBuckets * 4, "");
     static constexpr int LUT_PAD16 = 64;                          // a 32 x 32 block spans 63 distances
     static constexpr int STAT = STAGES * 2 * TILE;                // byte offsets
     static constexpr int LUT = STAT + (KV ? STAGES * 2 * 64 * 4 : 0);

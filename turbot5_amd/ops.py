@@ -580,10 +580,14 @@ def _sparse(pattern, q, k, v, bias, block_len, aux, side_k=None, side_v=None, sm
     # The local pattern's work items fetch LUT images that have the window folded in (windows up to 256); the kernel for
     # sliding windows of 16-bit tensors at head_dim 64 fetches none (takes_window_kernel of the library: if the two rules
     # ever differ, a call fills its LUTs itself, or builds a buffer that it does not read)
-    window = int(block_len) if pattern == L.PATTERN_LOCAL and int(block_len) <= 256 and key_bits is None else 0
-    if (pattern != L.PATTERN_BLOCK and D == 64 and q.dtype != torch.float32 and int(block_len) <= 256 and key_bits is None
-            and (pattern == L.PATTERN_LOCAL or a.n_side == 0 or (Lq + 127) // 128 * H * B > 2 * _cu_count(q.device))):
-        window = None
+    window = 0
+    if pattern != L.PATTERN_BLOCK and key_bits is None and int(block_len) <= 256:
+        if pattern == L.PATTERN_LOCAL:
+            window = int(block_len)
+        if D == 64 and q.dtype != torch.float32 and (
+                keep_side is None or keep_side[0].shape[2] == 0
+                or (Lq + 127) // 128 * H * B > 2 * (_CU_COUNT.get(q.device.index) or _cu_count(q.device))):
+            window = None
     a.bias, keep = _bias_struct(bias, H, NUM_BUCKETS, MAX_DISTANCE, q, window=window)
     lib = L.load()
     ws_bytes = lib.t5a_sparse_workspace_bytes(pattern, B, H, Lq, D, int(block_len), int(aux))

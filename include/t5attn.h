@@ -288,6 +288,9 @@ int t5a_bwd_varlen(const t5a_varlen_bwd_args* args, t5a_stream_t stream);
  * the G global rows, which attend all L keys, are computed as key splits spread over the whole
  * device and merged; without it they run as one workgroup per (batch, head).  Results agree to
  * rounding of the merge.
+ *
+ * Which kernel a LOCAL or TGLOBAL call runs in depends on its types and sizes and on the device's size; results of
+ * 16-bit tensors at head_dim 64 agree across kernels up to the rounding of probabilities and outputs to the type.
  */
 typedef struct t5a_sparse_args {
     const void* q; const void* k; const void* v; void* o;

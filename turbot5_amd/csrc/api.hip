@@ -554,10 +554,10 @@ static void choose_runs(FwdParams* p, int mode, int dtype, int D, int cus, int f
 // beyond it needs a second round where the window kernel, with four blocks per compute unit, does not.  us, general / window,
 // window 128, side tokens every 16, bf16: 8 heads x 2048 14.7 / 18.5, 12 x 4096 (384 blocks) 21.6 / 26.0, 8 x 8000 (504)
 // 27.6 / 32.2, 12 x 5504 (516) 37.5 / 33.3, 8 x 12 x 1024 30.8 / 26.7, 12 x 8192 41.6 / 39.4, 3 x 12 x 10000 147 / 131,
-// 2 x 12 x 16384 186 / 177; single documents of 12 heads from 11000 on are even (12288 71.8 / 73.4, 16384 103 / 100, 24576
-// 178 / 180), with side tokens every 32 16384 71.1 / 68.2.  Without side tokens: 12 x 1024 12.6 / 13.2, window 256 17.1 /
-// 18.4 (256 blocks, both with a ready LUT image; a captured graph has none), 8 x 4500 15.6 / 14.9, 8 x 12 x 1024 27 / 21, 12 x
-// 16384 45 / 40, 32768 75 / 63, window 64 and 96 faster at every size.
+// 2 x 12 x 16384 192 / 186.  Single documents from 11000 on are even, 3 % to either side (12 x 12288 72.8 / 73.8, 12 x 16384
+// 99.0 / 98.7, 8 x 24576 129 / 133, 12 x 32768 304 / 297, with side tokens every 32 194 / 183).  Without side tokens: 12 x
+// 1024 12.6 / 13.2, window 256 on 256 blocks 17.1 / 18.4 (with a ready LUT image, which a captured graph does not have), 8 x
+// 4500 15.6 / 14.9, 8 x 12 x 1024 27 / 21, 12 x 16384 45 / 40, 32768 75 / 63, window 64 and 96 faster at every size.
 static bool takes_window_kernel(int dtype, int D, int block_len, bool with_side, int B, int H, int L, int cus) {
     if (dtype == T5A_F32 || D != 64 || block_len > kMaxLutWindow) return false;
     return !with_side || (int64_t)((L + 127) / 128) * H * B > 2 * (int64_t)cus;

@@ -410,9 +410,9 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
 // block classes), accumulators touched by one piece of code only (a class decides about arguments, never about products:
 // with the products in the classes' branches the compiler kept a copy of every accumulator per branch and spilled), and
 // as few instructions per score as the formulas allow.  Deeper staging (3 or 4 tile buffers) was slower: the LDS it
-// takes costs more than the wait it saves.  Before / after, us, the passes with bwd_rows_kernel, bf16: B16 H12
-// L1024 D64 299 / 248, the same causal 205 / 180, B4 H12 L4096 D64 840 / 762, B4 H6 L4096 D128 1274 / 835, B2 H8
-// L1999 D128 causal 280 / 135.
+// takes costs more than the wait it saves.  Two blocks per wavefront and step / this one, us, the passes with
+// bwd_rows_kernel, bf16: B16 H12 L1024 D64 283 / 238, the same causal 198 / 167, B4 H12 L4096 D64 810 / 764, B4 H6
+// L4096 D128 1248 / 846, B2 H8 L1999 D128 causal 284 / 135.
 // head_dim 128 (the T5-3B / 11B head shape): rows of 256 bytes, sixteen chunks
 __device__ __forceinline__ int tile_swz128(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 
@@ -690,7 +690,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
                         // distance; a lane then sums a column.  What lies outside the skewed band is zero and never
                         // written.  16 words written and R read per lane at constant offsets, without bank conflicts.
                         // (A sum that travels through the lanes and leaves them by LDS atomics took 16 instructions per
-                        // score: the pass at B16 H12 L1024 went from 154 to 131 us, of which 36 are the table's.)
+                        // score.  The pass at B16 H12 L1024 with / without a table, us: 138 / 98 then, 119 / 88 now.)
                         constexpr int R = G::SKEW_ROWS;
 #pragma unroll
                         for (int round = 0; round < 32 / R; ++round) {

@@ -13,13 +13,15 @@
 // the sums are fp32, and dividing by the sum at the end undoes whatever m was), or at a row's first visible key; the wavefront
 // asks that of all its rows with one vote per block and shifts what it has in a block of code that is rarely run.
 //
-// What bounds it: waits.  At B1 H12 L16384 the wavefronts spend half of their cycles at the barrier of a tile, the vector
-// port is busy half of the time and the matrix pipe a quarter; per block and lane it is 16 x (fma, subtract, exp2, half a max3,
-// half a conversion and half a dot product) against eight matrix products.  More wavefronts per SIMD (5) or more tile
-// buffers (4) were slower.  The general kernel (fwd_kernel) walks rings of eight 64-key tiles per 128 rows with a scalar
-// prologue that eight wavefronts per compute unit execute at one instruction a cycle; this one has next to none, and a
-// window of 255 keys costs 9 or 10 blocks of 32 keys.  us, general kernel / this one, bf16, 12 heads: window 128 L16384
-// 40.0 / 35.8, L32768 76 / 64, with side tokens every 16 L16384 98 / 97, 8 x 1024 26.7 / 24.2; 8 heads L2048 20 / 17.
+// What bounds it: waits and the vector port.  At B1 H12 L16384, window 128, the wavefronts wait 51 % of their cycles, for each
+// other at the barrier of a tile; the vector port is busy 54 % of the time, the matrix pipe 20 % (with side tokens every 16:
+// 36, 57 and 30 %); per block and lane it is 16 x (fma, subtract, exp2, half a max3, half a conversion and half a dot
+// product) against eight matrix products.  More wavefronts per SIMD (5) or more tile buffers (4) were slower.  The general
+// kernel (fwd_kernel) walks rings of eight 64-key tiles per 128 rows with a scalar prologue that eight wavefronts per
+// compute unit execute at one instruction a cycle; this one has next to none, and a window of 255 keys costs 9 or 10 blocks
+// of 32 keys.  us, general kernel / this one, bf16, 12 heads, window 128: L16384 37.9 / 34.6, L32768 75 / 62, 8 x 1024 27 /
+// 21; L16384 with window 64 32.0 / 27.4, 256 56.5 / 52.8.  With side tokens and where the line between the two kernels lies:
+// takes_window_kernel.
 #include "lut_device.h"
 #include "mfma16_device.h"
 #include "t5a_internal.h"

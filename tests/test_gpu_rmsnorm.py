@@ -299,3 +299,40 @@ def test_residual_stream_carries_a_graph_only_where_it_has_one(gpu_device, x_gra
     assert total.requires_grad == (x_grad or r_grad) and y.requires_grad
     y.sum().backward()
     assert norm.weight.grad is not None and (x.grad is not None) == x_grad and (r.grad is not None) == r_grad
+
+
+@pytest.mark.parametrize("with_residual", [False, True])
+def test_norm_of_a_training_step_under_compilation_and_tracing(gpu_device, with_residual):
+    """A module in training mode compiles as one graph, traces, and runs under a dispatch mode: all in torch's operations,
+    bit for bit what the kernel's forward gives, with gradients that agree."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from turbot5_amd.attentions import T5LayerNorm
+
+    class Count(TorchDispatchMode):
+        n = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Count.n += 1
+            return func(*args, **(kwargs or {}))
+
+    class Step(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.norm = T5LayerNorm(64)
+
+        def forward(self, a, b):
+            return self.norm.add_norm(a, b)[1] if with_residual else self.norm(a)
+    plain = Step().to(gpu_device).train()
+    norm = plain.norm
+    x, r = (torch.randn(3, 64, device=gpu_device, requires_grad=True) for _ in range(2))
+    compiled = torch.compile(plain, backend="aot_eager", fullgraph=True)
+    want = plain(x, r)
+    dy = torch.randn_like(want)
+    grads = torch.autograd.grad(want, (x, norm.weight), dy)
+    with Count():
+        moded = plain(x, r)
+    assert Count.n > 0
+    for got in (compiled(x, r), moded, torch.jit.trace(plain, (x, r), check_trace=False)(x, r)):
+        assert torch.allclose(got, want, rtol=1e-6, atol=1e-6)
+        for a, b in zip(torch.autograd.grad(got, (x, norm.weight), dy), grads):
+            assert torch.allclose(a, b, rtol=1e-5, atol=1e-5)

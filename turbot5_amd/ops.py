@@ -805,10 +805,12 @@ class RmsNorm(torch.autograd.Function):
 def _plain(*tensors) -> bool:
     """Plain tensors and plain reverse-mode autograd: no batch of gradients, no tracing, function transform, forward-mode level
     or dispatch mode, for which a formula in torch's own operations is the one that works."""
+    # (what is being compiled or traced is not asked further)
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
     f = torch._C._functorch
     return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and not f.is_batchedtensor(t) and not f.is_legacy_batchedtensor(t)
                 for t in tensors if t is not None)
-            and not torch.jit.is_tracing() and not torch.compiler.is_compiling()
             and torch.autograd.forward_ad._current_level < 0 and f.peek_interpreter_stack() is None
             and torch._C._len_torch_dispatch_stack() == 0)
 
@@ -816,11 +818,11 @@ def _plain(*tensors) -> bool:
 def rms_norm_differentiable(x, weight, residual=None) -> bool:
     """Whether ``RmsNorm`` takes this call: plain tensors of the kernels' types on one ROCm device, rows that stay in
     registers, and plain reverse-mode autograd."""
-    return (x.is_cuda and weight.device == x.device and x.dtype in _DTYPES and weight.dtype in _DTYPES and x.numel() > 0
+    return (_plain(x, weight, residual) and x.is_cuda and weight.device == x.device and x.dtype in _DTYPES
+            and weight.dtype in _DTYPES and x.numel() > 0
             and weight.shape == x.shape[-1:] and x.shape[-1] % 8 == 0 and x.shape[-1] <= L.RMSNORM_TRAIN_MAX_DIM
             and (residual is None or (type(residual) is torch.Tensor and residual.shape == x.shape
-                                      and residual.dtype == x.dtype and residual.device == x.device))
-            and _plain(x, weight, residual))
+                                      and residual.dtype == x.dtype and residual.device == x.device)))
 
 
 _CU_COUNT = {}

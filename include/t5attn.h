@@ -106,7 +106,7 @@ int64_t t5a_bias_lut_bytes_windowed(int32_t H, int32_t num_buckets, int32_t max_
 
 /* Layout of the argument structs and set of entry points; a binding compares it with t5a_version() before
  * it passes a struct (a stale library would read pointers from the wrong offsets). */
-#define T5A_ABI_VERSION 117
+#define T5A_ABI_VERSION 118
 int t5a_version(void);
 const char* t5a_last_error(void);
 
@@ -430,6 +430,32 @@ typedef struct t5a_rmsnorm_train_args {
 } t5a_rmsnorm_train_args;
 int64_t t5a_rmsnorm_bwd_workspace_bytes(int64_t rows, int32_t dim);
 int t5a_rmsnorm_train(const t5a_rmsnorm_train_args* args, t5a_stream_t stream);
+
+/*
+ * c = a b of fp32 matrices (a linear layer of a training step and its gradients): fp32 sums of products formed on the bf16
+ * matrix cores from operands split into three bf16 parts, which carry all 24 bits; results are as accurate as fp32 products
+ * added in fp32.  The reference leaves its linear layers to torch (src/turbot5/model/attentions.py:59-62).
+ * Group g multiplies a[g] (M, K) and b[g] (N, K) over K; trans: the matrix lies in memory as (K, M) / (K, N).  Rows lda / ldb /
+ * ldc elements apart, contiguous inside.  sum_groups 0: c[g] = the product of group g; 1: c[0] = the sum over the groups.
+ * alpha: a factor of group 0's product.  relu: negative results become 0.  positive (optional, (M, N) fp32, rows ld_positive
+ * apart): results where it is <= 0 become 0.  c_dtype: any type; the result is rounded to it once.
+ * Types (a, b): fp32 and fp32 in all forms; bf16 (exact in one part) for a in all forms, for b only with both transposed.
+ * Forms: neither transposed, b transposed, both transposed.  N, and the dimension along which an operand is contiguous, are multiples of 8.
+ * a, b, c, positive and workspace 16-byte aligned, leading dimensions multiples of 8.
+ */
+typedef struct t5a_gemm_f32_args {
+    const void* a[3]; const void* b[3]; void* c[3];
+    int64_t lda; int64_t ldb; int64_t ldc;
+    const float* positive; int64_t ld_positive;
+    void* workspace; int64_t workspace_bytes;   /* t5a_gemm_f32_workspace_bytes() of the same arguments; may be NULL if that is 0 */
+    int32_t M; int32_t N; int32_t K;
+    int32_t groups; int32_t sum_groups;
+    int32_t a_dtype; int32_t b_dtype; int32_t c_dtype;
+    int32_t a_trans; int32_t b_trans;
+    int32_t relu; float alpha;
+} t5a_gemm_f32_args;
+int64_t t5a_gemm_f32_workspace_bytes(const t5a_gemm_f32_args* args);
+int t5a_gemm_f32(const t5a_gemm_f32_args* args, t5a_stream_t stream);
 
 #ifdef __cplusplus
 }

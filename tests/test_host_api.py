@@ -40,6 +40,42 @@ def test_struct_sizes_follow_the_header(lib):
     assert C.sizeof(lib.T5ARmsNormArgs) == 3 * 8 + 2 * 8 + 8 + 8 * 4 + 5 * 8 + 3 * 8
 
 
+def test_fp32_products_are_checked_without_gpu(lib):
+    """t5a_gemm_f32: arguments refused before any launch, and the workspace its choice of splits asks for."""
+    handle = lib.load()
+    assert C.sizeof(lib.T5AGemmF32Args) == 9 * 8 + 3 * 8 + 2 * 8 + 2 * 8 + 12 * 4
+
+    def args(M=300, N=512, K=2048, groups=1, **kw):
+        a = lib.T5AGemmF32Args((C.c_void_p * 3)(*[4096] * groups), (C.c_void_p * 3)(*[4096] * groups), (C.c_void_p * 3)(*[4096] * groups))
+        at, bt = kw.get("a_trans", 0), kw.get("b_trans", 0)
+        a.lda, a.ldb, a.ldc = M if at else K, N if bt else K, N
+        a.M, a.N, a.K, a.groups, a.a_dtype, a.b_dtype, a.c_dtype, a.alpha = M, N, K, groups, lib.T5A_F32, lib.T5A_F32, lib.T5A_F32, 1.0
+        for name, value in kw.items():
+            setattr(a, name, value)
+        return a
+
+    one = handle.t5a_gemm_f32_workspace_bytes(C.byref(args()))
+    assert one > 0 and one % (300 * 512 * 4) == 0                                # (a long contraction, few tiles: splits)
+    assert handle.t5a_gemm_f32_workspace_bytes(C.byref(args(M=8192, N=2048, K=512))) == 0
+    assert handle.t5a_gemm_f32(C.byref(args()), None) == -7 or b"workspace" in handle.t5a_last_error()
+    third = (C.c_void_p * 3)(4096, 4096, 0)
+    for bad in (dict(K=2044), dict(N=509), dict(M=0), dict(K=-8), dict(groups=4), dict(groups=0), dict(a_trans=1), dict(a_dtype=lib.T5A_F16),
+                dict(b_dtype=lib.T5A_BF16), dict(c_dtype=7), dict(lda=2040), dict(ldb=2052), dict(ldc=500), dict(groups=3, b=third),
+                dict(a=(C.c_void_p * 3)(4100)), dict(positive=4096, ld_positive=8), dict(positive=4100, ld_positive=512),
+                dict(M=1 << 20, K=1 << 12), dict(a_trans=1, b_trans=1, M=300)):
+        a = args(**bad) if not ("groups" in bad and bad["groups"] not in (1, 2, 3)) else args()
+        for name, value in bad.items():
+            if name not in ("M", "N", "K"):
+                setattr(a, name, value)
+        assert handle.t5a_gemm_f32_workspace_bytes(C.byref(a)) == -1, bad
+        assert handle.t5a_gemm_f32(C.byref(a), None) < 0, bad
+    # every choice over the range asks for whole splits
+    for M in (8, 64, 100, 1000, 4500, 20000):
+        for N, K in ((8, 8), (512, 512), (2048, 512), (512, 2048), (32128, 512)):
+            need = handle.t5a_gemm_f32_workspace_bytes(C.byref(args(M=M, N=N, K=K)))
+            assert need % (M * N * 4) == 0 and 0 <= need // (M * N * 4) <= 16 and need // (M * N * 4) != 1
+
+
 def test_key_bits_layout_and_size(lib):
     """Token j is bit (j & 31) of word 8 + (j >> 5); zero words in front and behind, as many as the kernels' tiles
     may look at; the side-token count is the number of valid block ENDs."""

@@ -13,7 +13,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libt5attn.so")
 
 T5A_BF16, T5A_F32, T5A_F16 = 0, 1, 2
-ABI_VERSION = 117   # T5A_ABI_VERSION of include/t5attn.h
+ABI_VERSION = 118   # T5A_ABI_VERSION of include/t5attn.h
 PATTERN_LOCAL, PATTERN_BLOCK, PATTERN_TGLOBAL = 1, 2, 3
 SCORES_DEFAULT, SCORES_EXACT, SCORES_PRESCALED = 0, 1, 2   # the exact_scores field
 STATIC_SCRATCH_BYTES = 8 * 1024 * 1024   # T5A_STATIC_SCRATCH_BYTES
@@ -23,6 +23,7 @@ EXPORTS = (
     "t5a_varlen_workspace_bytes", "t5a_bias_lut_bytes", "t5a_bias_lut_bytes_windowed",
     "t5a_fwd_sparse", "t5a_sparse_launch_plan", "t5a_sparse_workspace_bytes", "t5a_sparse_key_bits_words", "t5a_splitk_workspace_bytes", "t5a_fwd_splitk", "t5a_fwd_splitk_static",
     "t5a_rmsnorm", "t5a_rmsnorm_train", "t5a_rmsnorm_bwd_workspace_bytes",
+    "t5a_gemm_f32", "t5a_gemm_f32_workspace_bytes",
 )
 
 
@@ -130,6 +131,18 @@ class T5ARmsNormTrainArgs(C.Structure):
                 ("reserved", C.c_int32)]
 
 
+class T5AGemmF32Args(C.Structure):
+    _fields_ = [("a", C.c_void_p * 3), ("b", C.c_void_p * 3), ("c", C.c_void_p * 3),
+                ("lda", C.c_int64), ("ldb", C.c_int64), ("ldc", C.c_int64),
+                ("positive", C.c_void_p), ("ld_positive", C.c_int64),
+                ("workspace", C.c_void_p), ("workspace_bytes", C.c_int64),
+                ("M", C.c_int32), ("N", C.c_int32), ("K", C.c_int32),
+                ("groups", C.c_int32), ("sum_groups", C.c_int32),
+                ("a_dtype", C.c_int32), ("b_dtype", C.c_int32), ("c_dtype", C.c_int32),
+                ("a_trans", C.c_int32), ("b_trans", C.c_int32),
+                ("relu", C.c_int32), ("alpha", C.c_float)]
+
+
 RMSNORM_TRAIN_MAX_DIM = 2048
 
 _lib = None
@@ -181,6 +194,10 @@ def load() -> C.CDLL:
         lib.t5a_rmsnorm_train.restype = C.c_int
         lib.t5a_rmsnorm_bwd_workspace_bytes.argtypes = [C.c_int64, C.c_int32]
         lib.t5a_rmsnorm_bwd_workspace_bytes.restype = C.c_int64
+        lib.t5a_gemm_f32.argtypes = [C.POINTER(T5AGemmF32Args), C.c_void_p]
+        lib.t5a_gemm_f32.restype = C.c_int
+        lib.t5a_gemm_f32_workspace_bytes.argtypes = [C.POINTER(T5AGemmF32Args)]
+        lib.t5a_gemm_f32_workspace_bytes.restype = C.c_int64
         lib.t5a_bias_lut_bytes.argtypes = [C.c_int32] * 4
         lib.t5a_bias_lut_bytes.restype = C.c_int64
         lib.t5a_bias_lut_bytes_windowed.argtypes = [C.c_int32] * 4

@@ -30,7 +30,7 @@ from typing import Optional
 import torch
 from torch import nn
 
-from . import ops
+from . import linear, ops
 from .config import T5Config
 from .padding import _get_unpad_data, _upad_input, index_first_axis, pad_input
 
@@ -208,6 +208,23 @@ class _T5AttentionBase(nn.Module):
             return ops.prescaled_query(hidden_states, self.q.weight, adt, 1.0), "prescaled"
         return self.q(hidden_states).to(adt), choice
 
+    def _qkv_rows(self, hidden_states: torch.Tensor, adt: torch.dtype):
+        """q, k and v rows (..., H*D) of self-attention in the attention dtype and the ``exact_scores`` argument for q
+        (see ``_query``); in a training step with fp32 weights one product for the three."""
+        if hidden_states.dtype == torch.float32 and linear.takes(hidden_states, self.q, self.k, self.v):
+            choice = getattr(self.config, "attention_exact_scores", None)
+            folded = choice is None and adt in (torch.bfloat16, torch.float16)
+            q, k, v = linear.project(hidden_states, adt, ops.LOG2E if folded else 1.0, self.q, self.k, self.v)
+            return q, k, v, "prescaled" if folded else choice
+        q, exact = self._query(hidden_states, adt)
+        return q, self.k(hidden_states).to(adt), self.v(hidden_states).to(adt), exact
+
+    def _output_rows(self, rows: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+        """The output projection of attention rows (..., H*D), in the hidden states' dtype."""
+        if dtype == torch.float32 and linear.takes(rows, self.o):
+            return linear.project(rows, dtype, 1.0, self.o)[0]
+        return self.o(rows.to(dtype))
+
     def _table(self, position_bias):
         if position_bias is None and self.has_relative_attention_bias:
             position_bias = self.relative_attention_bias.weight
@@ -266,10 +283,10 @@ class T5FlashAttention(_T5AttentionBase):
                 memory_layout = layout
                 memory_rows = index_first_axis(key_value_states.reshape(n_rows, -1), layout.indices)
 
-        def project(proj_layer, past):
+        def project(proj_layer, past, rows):
             """keys or values: (B, H, key_length, D) in the attention dtype (attentions.py:444-469)."""
             if key_value_states is None:
-                states = self._shape(proj_layer(hidden_states), batch_size).to(adt)
+                states = self._shape(rows, batch_size)
                 if past is not None:
                     states = torch.cat([past, states], dim=2)
                 return states
@@ -281,12 +298,16 @@ class T5FlashAttention(_T5AttentionBase):
                 return self._shape(proj_layer(key_value_states), batch_size).to(adt)
             return past
 
-        query_rows, exact = self._query(hidden_states, adt)
+        key_rows = value_rows = None
+        if key_value_states is None:
+            query_rows, key_rows, value_rows, exact = self._qkv_rows(hidden_states, adt)
+        else:
+            query_rows, exact = self._query(hidden_states, adt)
         query_states = self._shape(query_rows, batch_size)
         # (the split-K kernel scales the fp32 product: rows that carry log2(e) already get ln 2 as their scale)
         dec_scale = 1.0 / ops.LOG2E if exact == "prescaled" else 1.0
-        key_states = project(self.k, past_key_value[0] if past_key_value is not None else None)
-        value_states = project(self.v, past_key_value[1] if past_key_value is not None else None)
+        key_states = project(self.k, past_key_value[0] if past_key_value is not None else None, key_rows)
+        value_states = project(self.v, past_key_value[1] if past_key_value is not None else None, value_rows)
         table = self._table(position_bias)
         nb, md = self.relative_attention_num_buckets, self.relative_attention_max_distance
         key_length = key_states.shape[2]
@@ -361,7 +382,7 @@ class T5FlashAttention(_T5AttentionBase):
                 else:
                     attn_output = out_p.view(batch_size, seq_length, self.n_heads, -1).transpose(1, 2)
 
-        attn_output = self.o(self._unshape(attn_output, batch_size).to(hidden_states.dtype))
+        attn_output = self._output_rows(self._unshape(attn_output, batch_size), hidden_states.dtype)
         present_key_value_state = (key_states, value_states) if (self.is_decoder and use_cache) else None
         return self._outputs(attn_output, present_key_value_state, table, output_attentions)
 
@@ -371,9 +392,8 @@ class T5FlashAttention(_T5AttentionBase):
         sequence, as in the reference's packed call (varlen_fused_bias_attn.py:254, :303)."""
         total = hidden_states.shape[0]
         adt = self._attn_dtype(hidden_states)
-        q, exact = self._query(hidden_states, adt)
-        q = q.view(total, self.n_heads, self.key_value_proj_dim)
-        k, v = (p(hidden_states).view(total, self.n_heads, self.key_value_proj_dim).to(adt) for p in (self.k, self.v))
+        *rows, exact = self._qkv_rows(hidden_states, adt)
+        q, k, v = (t.view(total, self.n_heads, self.key_value_proj_dim) for t in rows)
         table = self._table(position_bias)
         plan = packed.plans.setdefault((self.causal, self.n_heads, self.key_value_proj_dim, adt,
                                         ops._stream(hidden_states)), ops.LaunchPlan())
@@ -381,7 +401,7 @@ class T5FlashAttention(_T5AttentionBase):
             q, k, v, table, packed.cu_seqlens, packed.cu_seqlens, packed.max_len, packed.max_len,
             causal=self.causal, sm_scale=1.0, exact_scores=exact, NUM_BUCKETS=self.relative_attention_num_buckets,
             MAX_DISTANCE=self.relative_attention_max_distance, launch_plan=plan)
-        return (self.o(out.reshape(total, self.inner_dim).to(hidden_states.dtype)), None, table)
+        return (self._output_rows(out.reshape(total, self.inner_dim), hidden_states.dtype), None, table)
 
 
 class _SparseBase(_T5AttentionBase):

@@ -1021,4 +1021,60 @@ int t5a_rmsnorm_train(const t5a_rmsnorm_train_args* a, t5a_stream_t stream) {
     return finish(launch_rmsnorm_train(p, a->x_dtype, a->weight_dtype, (hipStream_t)stream), "t5a_rmsnorm_train");
 }
 
+static int gemm_f32_params(const t5a_gemm_f32_args* a, GemmParams* out) {
+    if (a == nullptr) return fail(T5A_ERR_NULL, "args is NULL");
+    for (int dt : {a->a_dtype, a->b_dtype})
+        if (dt != T5A_BF16 && dt != T5A_F32) return fail(T5A_ERR_DTYPE, "a and b are fp32 or bf16, got dtype %d", dt);
+    if (a->c_dtype != T5A_BF16 && a->c_dtype != T5A_F16 && a->c_dtype != T5A_F32) return fail(T5A_ERR_DTYPE, "unsupported dtype %d", a->c_dtype);
+    if (a->a_trans && !a->b_trans) return fail(T5A_ERR_SHAPE, "a transposed needs b transposed");
+    if (a->b_dtype == T5A_BF16 && (!a->a_trans || !a->b_trans || a->a_dtype == T5A_BF16))
+        return fail(T5A_ERR_DTYPE, "b in bf16 is for fp32 a with both operands transposed");
+    if (a->groups < 1 || a->groups > 3) return fail(T5A_ERR_SHAPE, "%d groups (1 to 3)", a->groups);
+    if (a->M <= 0 || a->N <= 0 || a->K <= 0 || a->N % 8 != 0 || (a->a_trans ? a->M : a->K) % 8 != 0 || (!a->b_trans && a->K % 8 != 0) ||
+        a->K > 0x7ffffff / 3)
+        return fail(T5A_ERR_SHAPE, "bad sizes M=%d N=%d K=%d (N and contiguous dimensions are multiples of 8)", a->M, a->N, a->K);
+    const int64_t wa = a->a_trans ? a->M : a->K, wb = a->b_trans ? a->N : a->K;
+    if (a->lda < wa || a->ldb < wb || a->ldc < a->N || a->lda % 8 != 0 || a->ldb % 8 != 0 || a->ldc % 8 != 0 ||
+        (a->positive != nullptr && (a->ld_positive < a->N || a->ld_positive % 8 != 0)))
+        return fail(T5A_ERR_STRIDE, "leading dimensions must cover a row and be multiples of 8");
+    // (operands are read with 32-bit byte offsets)
+    if ((int64_t)(a->a_trans ? a->K : a->M) * a->lda * (a->a_dtype == T5A_F32 ? 4 : 2) >= 0x7ff00000 ||
+        (int64_t)(a->b_trans ? a->K : a->N) * a->ldb * (a->b_dtype == T5A_F32 ? 4 : 2) >= 0x7ff00000)
+        return fail(T5A_ERR_SHAPE, "an operand of 2 GiB or more (M=%d N=%d K=%d)", a->M, a->N, a->K);
+    GemmParams p;
+    memset(&p, 0, sizeof(p));
+    for (int g = 0; g < a->groups; ++g) {
+        p.a[g] = a->a[g]; p.b[g] = a->b[g]; p.c[g] = a->sum_groups ? a->c[0] : a->c[g];
+        if (p.a[g] == nullptr || p.b[g] == nullptr || p.c[g] == nullptr) return fail(T5A_ERR_NULL, "a, b or c is NULL (group %d)", g);
+        for (const void* t : {p.a[g], p.b[g], (const void*)p.c[g]})
+            if (!aligned16(t)) return fail(T5A_ERR_STRIDE, "a, b and c must be 16-byte aligned");
+    }
+    if (!aligned16(a->positive)) return fail(T5A_ERR_STRIDE, "positive must be 16-byte aligned");
+    p.lda = a->lda; p.ldb = a->ldb; p.ldc = a->ldc;
+    p.M = a->M; p.N = a->N; p.K = a->K;
+    p.groups_out = a->sum_groups ? 1 : a->groups;
+    p.groups_k = a->sum_groups ? a->groups : 1;
+    p.alpha = a->alpha; p.c_dtype = a->c_dtype; p.relu = a->relu;
+    p.positive = a->positive; p.ldpos = a->ld_positive;
+    *out = p;
+    return T5A_OK;
+}
+
+int64_t t5a_gemm_f32_workspace_bytes(const t5a_gemm_f32_args* a) {
+    GemmParams p;
+    return gemm_f32_params(a, &p) == T5A_OK ? gemm_f32_workspace_bytes(p, a->a_dtype, a->b_dtype) : -1;
+}
+
+int t5a_gemm_f32(const t5a_gemm_f32_args* a, t5a_stream_t stream) {
+    GemmParams p;
+    const int rc = gemm_f32_params(a, &p);
+    if (rc != T5A_OK) return rc;
+    const int64_t need = gemm_f32_workspace_bytes(p, a->a_dtype, a->b_dtype);
+    if (need > 0 && (a->workspace == nullptr || a->workspace_bytes < need))
+        return fail(T5A_ERR_WORKSPACE, "t5a_gemm_f32: workspace of %lld bytes needed, %lld given", (long long)need, (long long)a->workspace_bytes);
+    if (!aligned16(a->workspace)) return fail(T5A_ERR_STRIDE, "workspace must be 16-byte aligned");
+    p.part = reinterpret_cast<float*>(a->workspace);
+    return finish(launch_gemm_f32(p, a->a_dtype, a->b_dtype, a->a_trans != 0, a->b_trans != 0, (hipStream_t)stream), "t5a_gemm_f32");
+}
+
 }  // extern "C"

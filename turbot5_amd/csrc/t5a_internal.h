@@ -204,4 +204,21 @@ struct RmsBwdParams {
 int rmsnorm_bwd_blocks(int64_t rows);
 hipError_t launch_rmsnorm_train(const RmsBwdParams& p, int x_dtype, int w_dtype, hipStream_t stream);
 
+// Products of fp32 (or bf16) matrices with fp32 sums (gemm_f32.hip): up to three groups of one shape, either each into its own
+// output (groups_out) or added (groups_k; the factor belongs to group 0 in both cases)
+struct GemmParams {
+    const void* a[3]; const void* b[3]; void* c[3];
+    int64_t lda, ldb, ldc;
+    int M, N, K;
+    int groups_out, groups_k;
+    float alpha;
+    int c_dtype, relu;
+    const float* positive; int64_t ldpos;     // optional: an element of c is 0 where this one is not positive
+    float* part;                              // with more than one split of the contraction: (nsplit, groups_out, M, N)
+    // filled in by the launch
+    int tiles_m, tiles_n, items, steps, steps_split, nsplit;
+};
+int64_t gemm_f32_workspace_bytes(const GemmParams& p, int a_dtype, int b_dtype);
+hipError_t launch_gemm_f32(const GemmParams& p, int a_dtype, int b_dtype, bool a_trans, bool b_trans, hipStream_t stream);
+
 }  // namespace t5a

@@ -21,6 +21,7 @@ from typing import List, Optional, Tuple
 import torch
 from torch import nn
 
+from . import linear
 from .attentions import T5ATTENTION_TYPES, T5FlashAttention, T5LayerNorm, packed_batch
 from .padding import index_first_axis, pad_input
 from .config import T5Config
@@ -54,6 +55,9 @@ class T5DenseActDense(nn.Module):
             x = hidden_states.reshape(-1, hidden_states.shape[-1])
             mid = torch._addmm_activation(self._zero_bias, x, self.wi.weight.t(), use_gelu=False)
             return self.wo(mid).view(*hidden_states.shape[:-1], -1)
+        if (self._relu and hidden_states.dtype == torch.float32 and linear.takes(hidden_states, self.wi)
+                and linear.widths_chain(self.wi, self.wo)):
+            return linear.feed_forward_relu(hidden_states, self.wi, self.wo)
         return self.wo(self.act(self.wi(hidden_states)))
 
 

@@ -104,6 +104,18 @@ def test_values_that_are_not_finite(gpu_device, form):
     assert ((out.double() - a.double() @ b.double().t())[rest].abs() <= (K + 30) * 2.0 ** -23 * scale).all()
 
 
+@pytest.mark.parametrize("scale", [2.0 ** -90, 2.0 ** -106, 2.0 ** -115, 2.0 ** -124])
+def test_small_magnitudes_keep_their_bits(gpu_device, scale):
+    """A whole operand of numbers whose bf16 parts would be denormal."""
+    from turbot5_amd.linear import _gemm
+    g = torch.Generator(device=gpu_device).manual_seed(3)
+    a, b = _rand(g, 130, 64), _rand(g, 72, 64)
+    out = torch.empty(130, 72, device=gpu_device)
+    _gemm([a * scale], [b], [out])
+    want = (a.double() * scale) @ b.double().t()
+    assert (out.double() - want).norm() <= 1e-6 * want.norm()
+
+
 def _layers(g, dev, n, d_in, d_out):
     out = []
     for _ in range(n):

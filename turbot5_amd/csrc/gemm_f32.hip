@@ -241,9 +241,16 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 3) void gemm_kernel(const
         it += n;
     }
 
-    float odd = 0.f;       // NaN if any sum is not finite: the products again on the fp32 matrix cores, straight from memory
-    each([&](float x) { odd += x * 0.f; return x; });
-    if (__any(odd != 0.f || odd != odd)) {
+    // A sum that is not finite, or is so small that the parts of what it was made from may have lost bits (split_device.h): the
+    // products again on the fp32 matrix cores, straight from memory.
+    float odd = 0.f;                     // NaN if any is not finite
+    unsigned least = 0xffffffffu;        // smallest magnitude but zero: twice the bits, less one
+    each([&](float x) {
+        odd += x * 0.f;
+        least = min(least, (__builtin_bit_cast(unsigned, x) << 1) - 1u);
+        return x;
+    });
+    if (__any(odd != odd || least < 2u * __builtin_bit_cast(unsigned, 0x1p-104f))) {
         each([](float) { return 0.f; });
         for (int it = it0; it < it_end; ++it) {
             const int g = it / p.steps, kk = it - g * p.steps;

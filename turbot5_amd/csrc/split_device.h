@@ -5,6 +5,8 @@
 // left out are at most 2^-24 of the product.  v_mfma_f32_32x32x16_bf16 does sixteen times the multiply-adds of
 // v_mfma_f32_32x32x2_f32 per cycle, so six of them take 3/8 of the time.
 //
+// (A part holds multiples of 2^-133: values below 2^-110 keep fewer bits, to an absolute error of 2^-134.)
+//
 // An infinity, or a value that rounds to one in bf16, gives infinity minus infinity in m and l: what fp32 arithmetic would
 // leave finite or infinite may come out as NaN.  Every such case leaves a value in the result that is not finite (h takes part
 // in a product of its own), which is what the kernels test before they store, to form the result again in fp32.
@@ -38,24 +40,6 @@ __device__ __forceinline__ void split3(const f32x8 x, bf16x8 (&out)[kPlanes]) {
     }
 #pragma unroll
     for (int q = 0; q < kPlanes; ++q) out[q] = __builtin_bit_cast(bf16x8, w[q]);
-}
-
-// acc += a b for operands of NA and NB planes (1: the values are bf16 as they are), smallest products first
-template <int NA, int NB>
-__device__ __forceinline__ f32x16 mfma_split(const bf16x8 (&a)[NA], const bf16x8 (&b)[NB], f32x16 acc) {
-    using H = Half16<__bf16>;
-    if constexpr (NA == 3 && NB == 3) {
-        acc = H::mfma(a[2], b[0], acc);
-        acc = H::mfma(a[0], b[2], acc);
-        acc = H::mfma(a[1], b[1], acc);
-    } else if constexpr (NA == 3) {
-        acc = H::mfma(a[2], b[0], acc);
-    } else if constexpr (NB == 3) {
-        acc = H::mfma(a[0], b[2], acc);
-    }
-    if constexpr (NA == 3) acc = H::mfma(a[1], b[0], acc);
-    if constexpr (NB == 3) acc = H::mfma(a[0], b[1], acc);
-    return H::mfma(a[0], b[0], acc);
 }
 
 }  // namespace t5a

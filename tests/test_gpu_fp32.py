@@ -1,0 +1,109 @@
+"""fp32 attention at head_dim 64, whose products run on the bf16 matrix cores: both block sizes, edges, and values whose bf16
+parts are no numbers.  Oracle: the formulas in 64 bits."""
+import math
+
+import pytest
+import torch
+
+from oracle import t5_basic as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _exact(q, k, v, table, causal, scale, dout=None):
+    """o and the gradients of q, k, v and the table in 64 bits, rows without a key zero."""
+    q, k, v, table = (t.detach().double().cpu().requires_grad_() for t in (q, k, v, table))
+    M, N = q.shape[2], k.shape[2]
+    rel = torch.arange(N)[None, :] - (torch.arange(M)[:, None] + N - M)
+    s = q @ k.transpose(2, 3) * scale + table[O.relative_position_bucket(rel, not causal, table.shape[0], 128)].permute(2, 0, 1)
+    seen = (rel <= 0) if causal else torch.ones_like(rel, dtype=torch.bool)
+    s = s.masked_fill(~seen, -math.inf)
+    p = torch.softmax(torch.where(seen.any(1)[:, None], s, torch.zeros_like(s)), -1) * seen.any(1)[:, None]
+    o = p @ v
+    if dout is None:
+        return o.detach()
+    return [o.detach(), *torch.autograd.grad(o, (q, k, v, table), dout.double().cpu())]
+
+
+# (blocks of 64 rows: up to 256, causal 640; of 128 beyond) x tile edges, one row, rows without keys, more keys than rows
+@pytest.mark.parametrize("B,H,M,N,causal", [(1, 2, 1, 1, False), (1, 2, 63, 65, False), (2, 2, 64, 64, True), (1, 3, 33, 300, True),
+                                            (1, 2, 200, 90, True), (2, 4, 257, 257, False), (65, 4, 65, 40, False),
+                                            (40, 8, 97, 161, True), (33, 8, 130, 31, True)])
+def test_forward_and_gradients_against_64_bits(gpu_device, B, H, M, N, causal):
+    import turbot5_amd as t5
+    g = torch.Generator().manual_seed(B + M + N)
+    q, k, v, d = (0.5 * torch.randn(B, n, H, 64, generator=g) for n in (M, N, N, M))
+    table = torch.randn(32, H, generator=g)
+    ins = [t.to(gpu_device).transpose(1, 2).requires_grad_() for t in (q, k, v)] + [table.to(gpu_device).requires_grad_()]
+    dout = d.to(gpu_device).transpose(1, 2)
+    o = t5.flash_attention_with_fusing_bias(*ins, causal=causal, sm_scale=1.0)
+    got = [o, *torch.autograd.grad(o, ins, dout)]
+    want = _exact(*ins, causal, 1.0, dout)
+    # four times what the sums' roundings were seen to leave over such shapes (5e-7 forward, 1.7e-6 gradients)
+    # (with one key the gradients are differences of equal terms, of norm 1 and more)
+    for t, r, tol in zip(got, want, (2e-6, 7e-6, 7e-6, 7e-6, 7e-6)):
+        assert (t.double().cpu() - r).norm() <= tol * r.norm().clamp(min=1.0)
+
+
+@pytest.mark.parametrize("B", [1, 48])
+def test_values_that_have_no_bf16_parts(gpu_device, B):
+    """A number that rounds to infinity in bf16 (3.4e38) among small ones: results that fp32 holds are finite; infinite keys: scores of
+    minus infinity hide them, the other rows are NaN; a NaN key reaches the rows that see it."""
+    import turbot5_amd as t5
+    H, L = 8, 96
+    g = torch.Generator().manual_seed(3)
+    q, k, v, d = (0.5 * torch.randn(B, H, L, 64, generator=g) for _ in range(4))
+    table = torch.randn(32, H, generator=g)
+    big_q, big_k, big_v = q.clone(), k.clone(), v.clone()
+    tiny = 2e-38 * (1.0 + torch.rand(B, H, L, generator=g)) * (1 - 2 * torch.randint(0, 2, (B, H, L), generator=g))
+    big_q[..., 0] = tiny           # (products of some 7 to 14)
+    big_k[:, :, 5, 0] = 3.4e38
+    big_v[:, :, 7, 3] = 3.4e38
+    d2 = d.clone()
+    d2[..., 3] = tiny.flip(-1)
+    ins = [t.to(gpu_device).requires_grad_() for t in (big_q, big_k, big_v, table)]
+    o = t5.flash_attention_with_fusing_bias(*ins, causal=False, sm_scale=1.0)
+    got = [o, *torch.autograd.grad(o, ins, d2.to(gpu_device))]
+    want = _exact(*ins, False, 1.0, d2)
+    for t, r in zip(got, want):
+        t, fits = t.detach().double().cpu(), r.abs() < 3.39e38
+        assert t[fits].isfinite().all() and t[r.abs() > 3.41e38].isinf().all()
+        # (a column's scale; columns of sums below the smallest normal number aside.  Products on the fp32 matrix cores are up to
+        # 5e-5 from the formulas here: scores reach 25 and one key has most rows' weight)
+        assert ((t - r).abs() <= 2e-4 * r.abs().amax(dim=-2, keepdim=True) + 1e-36)[fits].all()
+    bad_k = k.clone()
+    bad_k[:, :, 40, 0] = math.inf
+    for causal in (False, True):
+        out = t5.flash_attention_with_fusing_bias(q.to(gpu_device), bad_k.to(gpu_device), v.to(gpu_device), table.to(gpu_device),
+                                                  causal=causal, sm_scale=1.0).cpu()
+        clean = t5.flash_attention_with_fusing_bias(q.to(gpu_device), k.to(gpu_device), v.to(gpu_device), table.to(gpu_device),
+                                                    causal=causal, sm_scale=1.0).cpu()
+        sees = torch.arange(L)[None, None, :] >= (40 if causal else 0)
+        hidden = q[..., 0] < 0          # score of minus infinity
+        assert out[(sees & ~hidden).expand(B, H, L)].isnan().all()
+        rest = sees & hidden
+        assert out[rest.expand(B, H, L)].isfinite().all()
+        drop = torch.ones(L, dtype=torch.bool)
+        drop[40] = False
+        rel = torch.arange(L)[None, :] - torch.arange(L)[:, None]
+        s = (q.double() @ k.double().transpose(2, 3)) + table.double()[O.relative_position_bucket(rel, not causal, 32, 128)].permute(2, 0, 1)
+        s = s.masked_fill(~drop[None, :] | ((rel > 0) if causal else torch.zeros_like(rel, dtype=torch.bool)), -math.inf)
+        without = torch.softmax(s, -1) @ v.double()
+        pick = rest.expand(B, H, L)
+        assert (out.double()[pick] - without[pick]).norm() <= 2e-6 * without[pick].norm()
+        if causal:
+            before = (~sees).expand(B, H, L) & (torch.arange(L) < 32)[None, None, :]
+            assert (out[before] - clean[before]).norm() <= 2e-6 * clean[before].norm()
+
+
+def test_lut_of_a_table_is_not_marked_built_by_an_fp32_call(gpu_device):
+    """The fp32 kernel reads no distance image: a 16-bit call with the same table builds its own."""
+    import turbot5_amd as t5
+    g = torch.Generator().manual_seed(6)
+    q, k, v = (0.5 * torch.randn(1, 4, 200, 64, generator=g) for _ in range(3))
+    table = torch.randn(32, 4, generator=g).to(gpu_device)
+    t5.flash_attention_with_fusing_bias(*(t.to(gpu_device) for t in (q, k, v)), table, sm_scale=1.0)
+    b = [t.bfloat16() for t in (q, k, v)]
+    out = t5.flash_attention_with_fusing_bias(*(t.to(gpu_device) for t in b), table, sm_scale=1.0)
+    want = O.dense_attention(*b, table.cpu(), False, 1.0)
+    assert (out.float().cpu() - want).abs().max() <= 2e-2

@@ -28,6 +28,7 @@ UNITS = [
     ("attn_bwd.o", "attn_bwd.hip", []),
     ("attn_window.o", "attn_window.hip", []),
     ("gemm_f32.o", "gemm_f32.hip", []),
+    ("attn_f32.o", "attn_f32.hip", []),
     ("attn_fwd_bf16.o", "attn_fwd.hip", ["-DT5A_UNIT_DTYPE=0"]),
     ("attn_fwd_f32.o", "attn_fwd.hip", ["-DT5A_UNIT_DTYPE=1"]),
     ("attn_fwd_f16.o", "attn_fwd.hip", ["-DT5A_UNIT_DTYPE=2"]),

@@ -286,6 +286,7 @@ int t5a_fwd_dense(const t5a_dense_args* a, t5a_stream_t stream) {
     if ((rc = score_mode(a->exact_scores, a->sm_scale, &p))) return rc;
     if ((rc = fill_bias(a->bias, a->causal == 0, &p))) return rc;
     if ((rc = prepare_lut(a->bias, a->causal != 0, (hipStream_t)stream, &p))) return rc;
+    if (a->dtype == T5A_F32 && a->D == 64) return finish(launch_fwd_f32_64(p, a->causal != 0, (hipStream_t)stream), "t5a_fwd_dense");
     return finish(launch_fwd(p, a->dtype, a->D, kDense, a->causal != 0, (hipStream_t)stream), "t5a_fwd_dense");
 }
 

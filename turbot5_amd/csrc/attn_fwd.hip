@@ -2142,7 +2142,10 @@ static hipError_t launch_one(const FwdParams& p, hipStream_t stream) {
 template <typename T, int D>
 static hipError_t launch_mode(const FwdParams& p, int mode, bool causal, hipStream_t s) {
     switch (mode) {
-        case kDense: return causal ? launch_one<T, D, kDense, true>(p, s) : launch_one<T, D, kDense, false>(p, s);
+        case kDense:
+            // (fp32 at head_dim 64: launch_fwd_f32_64's, but for the key splits of the block pattern's global rows)
+            if constexpr (sizeof(T) == 4 && D == 64) return causal ? hipErrorInvalidValue : launch_one<T, D, kDense, false>(p, s);
+            else return causal ? launch_one<T, D, kDense, true>(p, s) : launch_one<T, D, kDense, false>(p, s);
         case kPacked: return causal ? launch_one<T, D, kPacked, true>(p, s) : launch_one<T, D, kPacked, false>(p, s);
         case kLocal:
             if constexpr (sizeof(T) == 2 && D == 64) return hipErrorInvalidValue;     // (launch_window's)

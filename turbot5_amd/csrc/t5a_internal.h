@@ -177,6 +177,10 @@ struct BwdParams {
 };
 hipError_t launch_bwd_dense(const BwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
 
+// fp32 tensors at head_dim 64 (attn_f32.hip): the dense forward, and the backward's passes behind bwd_rows_kernel
+hipError_t launch_fwd_f32_64(const FwdParams& p, bool causal, hipStream_t stream);
+hipError_t launch_bwd_f32_64(const BwdParams& p, bool causal, hipStream_t stream);
+
 struct RmsParams {
     const void* x; const void* weight; void* y;
     const void* residual; void* sum_out;                  // optional: normalise x + residual, write the sum (input type)

@@ -214,7 +214,9 @@ def _dense_forward(q, k, v, bias, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, r
     q_, k_, v_ = (_kernel_ready(t) for t in (q, k, v))
     o = torch.empty_like(q_)
     lse = torch.empty((B, H, M), device=q.device, dtype=torch.float32) if return_lse else None
-    bias_args, keep = _bias_struct(bias, H, NUM_BUCKETS, MAX_DISTANCE, q, causal)
+    # (fp32 at head_dim 64: a kernel that fills its own distance table)
+    window = None if D == 64 and q.dtype == torch.float32 else 0
+    bias_args, keep = _bias_struct(bias, H, NUM_BUCKETS, MAX_DISTANCE, q, causal, window)
     # (all fields in one call, in the struct's order: filled one by one they cost as much as the launch)
     a = L.T5ADenseArgs(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o.data_ptr(), lse.data_ptr() if lse is not None else None,
                        _strides3(q_), _strides3(k_), _strides3(v_), _strides3(o),

@@ -170,6 +170,10 @@ typedef struct t5a_dense_bwd_args {
     t5a_bias bias;
 } t5a_dense_bwd_args;
 int64_t t5a_bwd_workspace_bytes(int32_t B, int32_t H, int32_t M);
+/* More workspace for t5a_bwd_dense and t5a_bwd_varlen, behind the bytes above rounded up to 16: with it the table gradient
+ * is added in a fixed order instead of by atomics (faster, and the same bits every time).  rows: M or max_seqlen_q.  0: not
+ * offered for these sizes (more than 64 buckets, or more than 64 MiB). */
+int64_t t5a_bwd_table_workspace_bytes(int32_t B, int32_t H, int32_t rows, int32_t num_buckets);
 int t5a_bwd_dense(const t5a_dense_bwd_args* args, t5a_stream_t stream);
 
 /*

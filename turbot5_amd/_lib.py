@@ -19,7 +19,7 @@ SCORES_DEFAULT, SCORES_EXACT, SCORES_PRESCALED = 0, 1, 2   # the exact_scores fi
 STATIC_SCRATCH_BYTES = 8 * 1024 * 1024   # T5A_STATIC_SCRATCH_BYTES
 
 EXPORTS = (
-    "t5a_version", "t5a_last_error", "t5a_bucket_lut", "t5a_fwd_dense", "t5a_bwd_dense", "t5a_bwd_workspace_bytes", "t5a_bwd_varlen", "t5a_bwd_varlen_workspace_bytes", "t5a_fwd_varlen",
+    "t5a_version", "t5a_last_error", "t5a_bucket_lut", "t5a_fwd_dense", "t5a_bwd_dense", "t5a_bwd_workspace_bytes", "t5a_bwd_table_workspace_bytes", "t5a_bwd_varlen", "t5a_bwd_varlen_workspace_bytes", "t5a_fwd_varlen",
     "t5a_varlen_workspace_bytes", "t5a_bias_lut_bytes", "t5a_bias_lut_bytes_windowed",
     "t5a_fwd_sparse", "t5a_sparse_launch_plan", "t5a_sparse_workspace_bytes", "t5a_sparse_key_bits_words", "t5a_splitk_workspace_bytes", "t5a_fwd_splitk", "t5a_fwd_splitk_static",
     "t5a_rmsnorm", "t5a_rmsnorm_train", "t5a_rmsnorm_bwd_workspace_bytes",
@@ -184,6 +184,8 @@ def load() -> C.CDLL:
             fn.restype = C.c_int
         lib.t5a_bwd_workspace_bytes.argtypes = [C.c_int32] * 3
         lib.t5a_bwd_workspace_bytes.restype = C.c_int64
+        lib.t5a_bwd_table_workspace_bytes.argtypes = [C.c_int32] * 4
+        lib.t5a_bwd_table_workspace_bytes.restype = C.c_int64
         lib.t5a_bwd_varlen_workspace_bytes.argtypes = [C.c_int32] * 2
         lib.t5a_bwd_varlen_workspace_bytes.restype = C.c_int64
         lib.t5a_splitk_workspace_bytes.argtypes = [C.c_int32] * 5

@@ -295,6 +295,19 @@ int64_t t5a_bwd_workspace_bytes(int32_t B, int32_t H, int32_t M) {
     return 2 * (int64_t)B * H * M * (int64_t)sizeof(float);
 }
 
+int64_t t5a_bwd_table_workspace_bytes(int32_t B, int32_t H, int32_t rows, int32_t num_buckets) {
+    if (B <= 0 || H <= 0 || rows <= 0 || num_buckets <= 0 || num_buckets > kMaxSlotBuckets) return 0;
+    const int64_t bytes = (int64_t)B * H * ((rows + 63) / 64) * num_buckets * (int64_t)sizeof(float);
+    return bytes <= kMaxSlotBytes ? bytes : 0;
+}
+
+// the slots of the table gradient behind the `need` bytes of a backward's workspace, if it is that large
+static void table_slots(void* workspace, int64_t bytes, int64_t need, BwdParams* p) {
+    need = (need + 15) & ~(int64_t)15;
+    const int64_t more = t5a_bwd_table_workspace_bytes(p->B, p->H, p->M, p->n_buckets);
+    if (p->dtable != nullptr && more > 0 && bytes >= need + more) p->slots = reinterpret_cast<float*>(static_cast<unsigned char*>(workspace) + need);
+}
+
 int t5a_bwd_dense(const t5a_dense_bwd_args* a, t5a_stream_t stream) {
     if (a == nullptr) return fail(T5A_ERR_NULL, "args is NULL");
     int rc = check_common(a->dtype, a->D);
@@ -363,6 +376,7 @@ int t5a_bwd_dense(const t5a_dense_bwd_args* a, t5a_stream_t stream) {
     p.fp32_math = a->fp32_math;
     p.delta = reinterpret_cast<float*>(a->workspace);
     p.lse2 = p.delta + (int64_t)a->B * a->H * a->M;
+    table_slots(a->workspace, a->workspace_bytes, need, &p);
     return finish(launch_bwd_dense(p, a->dtype, a->D, a->causal != 0, (hipStream_t)stream), "t5a_bwd_dense");
 }
 
@@ -427,6 +441,7 @@ int t5a_bwd_varlen(const t5a_varlen_bwd_args* a, t5a_stream_t stream) {
     p.fp32_math = a->fp32_math;
     p.delta = reinterpret_cast<float*>(a->workspace);
     p.lse2 = p.delta + (int64_t)a->total_q * a->H;
+    table_slots(a->workspace, a->workspace_bytes, need, &p);
     return finish(launch_bwd_dense(p, a->dtype, a->D, a->causal != 0, (hipStream_t)stream), "t5a_bwd_varlen");
 }
 

@@ -29,6 +29,7 @@
 #include "lut_device.h"
 #include "mfma16_device.h"
 #include "t5a_internal.h"
+#include "table_grad_device.h"
 
 namespace t5a {
 
@@ -431,13 +432,12 @@ struct Bwd16Geom {
     static constexpr int STAGES = 2;                               // tile buffers
     static constexpr int REQS = 2 * SLABS + (KV ? 1 : 0);         // requests per wavefront and tile
     static constexpr int SKEW_ROWS = (D == 128 && SPLIT == 2) ? 8 : 32;   // queries per round of the table gradient
-    static_assert(STAGES * 2 * TILE >= kMaxBuckets * 4, "");
     static constexpr int LUT_PAD16 = 64;                          // a 32 x 32 block spans 63 distances
     static constexpr int STAT = STAGES * 2 * TILE;                // byte offsets
     static constexpr int LUT = STAT + (KV ? STAGES * 2 * 64 * 4 : 0);
     static __host__ __device__ int lut_floats(int sat) { return (2 * (sat + LUT_PAD16) + 4) & ~3; }
     static __host__ __device__ int hist(int sat) { return LUT + 4 * lut_floats(sat); }
-    static __host__ __device__ int skew(int sat) { return hist(sat) + (KV ? 0 : 4 * ((2 * sat + 4) & ~3)); }
+    static __host__ __device__ int skew(int sat) { return hist(sat) + (KV ? 0 : 4 * kTableGradWaves * table_grad_floats(sat)); }
     static __host__ __device__ int bytes(int sat, bool bias) { return skew(sat) + (KV || !bias ? 0 : 4 * SKEW_ROWS * 64 * 4); }
 };
 
@@ -457,6 +457,11 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
     int own_block, h, b;
     bwd_place<CAUSAL, KV>(p.H, p.B, nblk, own_block, h, b);
     const int own_base = own_block * G::OWN;
+    const int64_t slot = ((int64_t)h * p.B + b) * nblk + own_block;     // (of the table gradient)
+    if constexpr (PASS == 1 || PASS == 2) {
+        // (the last block: the shortest of a causal launch)
+        if (p.slots != nullptr && p.table != nullptr && own_block == nblk - 1 && b == 0) table_grad_reduce(p, h, reinterpret_cast<float*>(bwd_smem));
+    }
     const int w_lo = own_base + ow * 32, own_row = w_lo + lr;     // this wavefront's, this lane's own rows
     int M = p.M, N = p.N;
     int64_t q_first = 0, k_first = 0;
@@ -464,14 +469,17 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
         q_first = p.cu_q[b]; k_first = p.cu_k[b];
         M = p.len_q != nullptr ? p.len_q[b] : p.cu_q[b + 1] - (int)q_first;
         N = p.len_k != nullptr ? p.len_k[b] : p.cu_k[b + 1] - (int)k_first;
-        if (own_base >= (KV ? N : M)) return;     // (the grid is sized for the longest sequence)
+        if (own_base >= (KV ? N : M)) {     // (the grid is sized for the longest sequence)
+            if constexpr (PASS == 0) table_grad_none(p, slot);
+            return;
+        }
     }
     const int n_own = KV ? N : M, n_other = KV ? M : N;
     const int P = N - M;
     const bool has_bias = p.table != nullptr;
     const int sat = has_bias ? p.bs.sat : 0;
     float* const lut = reinterpret_cast<float*>(bwd_smem + G::LUT);
-    float* const hist_rel = reinterpret_cast<float*>(bwd_smem + G::hist(sat));   // dS summed per clamped distance
+    float* const dist = reinterpret_cast<float*>(bwd_smem + G::hist(sat)) + wave * table_grad_floats(sat);   // dS per distance
     float* const skew = reinterpret_cast<float*>(bwd_smem + G::skew(sat)) + wave * G::SKEW_ROWS * 64;
 
     const T* qp = reinterpret_cast<const T*>(p.q) + (int64_t)b * p.q_sb + (int64_t)h * p.q_sh + q_first * p.q_sr;
@@ -552,7 +560,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
         if (has_bias) {
             bias_lo = bias.at(-sat); bias_hi = bias.at(sat);
             if constexpr (!KV) {
-                for (int x = tid; x <= 2 * sat; x += kBwdThreads) hist_rel[x] = 0.f;
+                for (int x = lane; x <= 2 * sat; x += 64) dist[x] = 0.f;
                 for (int x = lane; x < G::SKEW_ROWS * 64; x += 64) skew[x] = 0.f;
             }
         }
@@ -686,31 +694,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
                                           ((dp[8] + dp[9]) + (dp[10] + dp[11])) + ((dp[12] + dp[13]) + (dp[14] + dp[15]));
                         if (sat_lo) sum_lo += sum; else sum_hi += sum;
                     } else {
-                        // Table gradient around the diagonal: dS summed per distance.  The block goes to LDS skewed, the
-                        // pair of key kk and query lr at row lr, column kk - lr + R - 1, so that a column holds one
-                        // distance; a lane then sums a column.  What lies outside the skewed band is zero and never
-                        // written.  16 words written and R read per lane at constant offsets, without bank conflicts.
-                        // (A sum that travels through the lanes and leaves them by LDS atomics took 16 instructions per
-                        // score.  The pass at B16 H12 L1024 with / without a table, us: 138 / 98 then, 119 / 88 now.)
-                        constexpr int R = G::SKEW_ROWS;
-#pragma unroll
-                        for (int round = 0; round < 32 / R; ++round) {
-                            if (R == 32 || lr / R == round) {
-                                float* w = skew + (lr % R) * 63 + (R - 1) + 4 * hh;
-#pragma unroll
-                                for (int r = 0; r < 16; ++r) w[8 * (r >> 2) + (r & 3)] = dp[r];
-                            }
-                            asm volatile("" ::: "memory");     // (LDS accesses of a wavefront keep their order)
-                            float c0 = 0.f, c1s = 0.f, c2 = 0.f, c3 = 0.f;
-#pragma unroll
-                            for (int q = 0; q < R; q += 4) {
-                                c0 += skew[q * 64 + lane]; c1s += skew[(q + 1) * 64 + lane];
-                                c2 += skew[(q + 2) * 64 + lane]; c3 += skew[(q + 3) * 64 + lane];
-                            }
-                            asm volatile("" ::: "memory");
-                            const int rel = s0 - (w_lo + P) - R * round + lane - (R - 1);
-                            if (lane < 31 + R) atomicAdd(&hist_rel[min(max(rel, -sat), sat) + sat], (c0 + c1s) + (c2 + c3));
-                        }
+                        table_grad_block<G::SKEW_ROWS>(skew, dist, dp, lane, s0 - (w_lo + P), sat, sum_lo, sum_hi);
                     }
                 }
             }
@@ -760,26 +744,9 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
             }
     }
     if constexpr (!KV) {
-        if (has_bias && p.dtable != nullptr) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                sum_lo += __shfl_xor(sum_lo, off, 64);
-                sum_hi += __shfl_xor(sum_hi, off, 64);
-            }
-            float* const hist = reinterpret_cast<float*>(bwd_smem);     // (the tiles are done with)
-            __syncthreads();
-            for (int x = tid; x < p.n_buckets; x += kBwdThreads) hist[x] = 0.f;
-            __syncthreads();
-            if (lane == 0) {
-                if (sum_lo != 0.f) atomicAdd(&hist[bucket_of(p.bs, -sat)], sum_lo);
-                if (sum_hi != 0.f) atomicAdd(&hist[bucket_of(p.bs, sat)], sum_hi);
-            }
-            for (int x = tid; x <= 2 * sat; x += kBwdThreads)     // distances -> buckets
-                if (hist_rel[x] != 0.f) atomicAdd(&hist[bucket_of(p.bs, x - sat)], hist_rel[x]);
-            __syncthreads();
-            for (int x = tid; x < p.n_buckets; x += kBwdThreads)
-                if (hist[x] != 0.f) atomicAdd(&p.dtable[(int64_t)x * p.H + h], hist[x]);
-        }
+        // (the tiles are done with)
+        if (has_bias && p.dtable != nullptr)
+            table_grad_finish(p, h, slot, reinterpret_cast<const float*>(bwd_smem + G::hist(sat)), reinterpret_cast<float*>(bwd_smem), sat, sum_lo, sum_hi);
     }
 }
 
@@ -823,14 +790,19 @@ hipError_t launch_bwd16_rows(const BwdParams& p, hipStream_t stream) {
 }
 
 template <typename T, int D, bool CAUSAL>
-hipError_t launch_bwd16(const BwdParams& p, hipStream_t stream) {
+hipError_t launch_bwd16(BwdParams p, hipStream_t stream) {
+    p.slots_per_head = p.B * (bwd16_split(p, D, CAUSAL, false) ? (p.M + 63) / 64 : (p.M + 127) / 128);
+    if (p.N <= 0) p.slots = nullptr;      // (no pass that would add them)
     hipError_t e = launch_bwd16_rows<T, D, CAUSAL, 0>(p, stream);
     if (e != hipSuccess) return e;
-    if constexpr (D == 64) return launch_bwd16_rows<T, D, CAUSAL, 1>(p, stream);
-    // head_dim 128: a row's head_dim twice and two gradients of it do not fit 256 registers next to the scores
-    // (the joint pass spills and takes 721 us where the two take 592: B4 H6 L4096)
-    if ((e = launch_bwd16_rows<T, D, CAUSAL, 2>(p, stream)) != hipSuccess) return e;
-    return launch_bwd16_rows<T, D, CAUSAL, 3>(p, stream);
+    if constexpr (D == 64) {
+        return launch_bwd16_rows<T, D, CAUSAL, 1>(p, stream);
+    } else {
+        // head_dim 128: a row's head_dim twice and two gradients of it do not fit 256 registers next to the scores
+        // (the joint pass spills and takes 721 us where the two take 592: B4 H6 L4096)
+        if ((e = launch_bwd16_rows<T, D, CAUSAL, 2>(p, stream)) != hipSuccess) return e;
+        return launch_bwd16_rows<T, D, CAUSAL, 3>(p, stream);
+    }
 }
 
 template <typename T, int D>

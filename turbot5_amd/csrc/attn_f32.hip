@@ -19,6 +19,7 @@
 // or of a value close to the largest, are no numbers.
 #include "split_device.h"
 #include "t5a_internal.h"
+#include "table_grad_device.h"
 
 namespace t5a {
 
@@ -27,9 +28,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int HD = 64, KS = HD / 16, DT = HD / 32;
 constexpr int kPad = 64;                 // a 32 x 32 block spans 63 distances
-constexpr int kSkewRows = 8;             // queries per round of the table gradient
 constexpr int RSTR = HD + 1;             // RAW: fp32 rows padded by one float
-constexpr int kMaxBuckets = 4 * kMaxThresholds;
 
 // SPLIT 1: four groups of 32 own rows, tiles of 32 rows.  SPLIT 2: two groups of own rows, tiles of 64 whose halves go to
 // different wavefronts; what the two hold of a row is put together through LDS at the end.
@@ -44,8 +43,9 @@ template <int SPLIT> struct Geom {
     static_assert(RSTR * OTHER * 4 <= TENSOR, "");
     static __host__ __device__ int lut_floats(int sat) { return (2 * (sat + kPad) + 4) & ~3; }
     static __host__ __device__ int hist(int sat) { return LUT + 4 * lut_floats(sat); }
-    static __host__ __device__ int skew(int sat) { return hist(sat) + 4 * ((2 * sat + 4) & ~3); }
-    static __host__ __device__ int bytes(int sat, bool table_grad) { return table_grad ? skew(sat) + 4 * kSkewRows * 64 * 4 : hist(sat); }
+    static constexpr int SKEW_ROWS = SPLIT == 2 ? 32 : 16;       // queries per round of the table gradient (two workgroups share the LDS with SPLIT 1)
+    static __host__ __device__ int skew(int sat) { return hist(sat) + 4 * kTableGradWaves * table_grad_floats(sat); }
+    static __host__ __device__ int bytes(int sat, bool table_grad) { return table_grad ? skew(sat) + kTableGradWaves * SKEW_ROWS * 64 * 4 : hist(sat); }
 };
 
 // the tiles of the two tensors of the other kind
@@ -249,13 +249,21 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     int own_block, h, b;
     bwd_place<CAUSAL, KV>(p.H, p.B, nblk, own_block, h, b);
     const int own_base = own_block * G::OWN, w_lo = own_base + ow * 32, own_row = w_lo + lr;
+    const int64_t slot = ((int64_t)h * p.B + b) * nblk + own_block;     // (of the table gradient)
+    if constexpr (KV && !RAW) {
+        // (the last block: the shortest of a causal launch)
+        if (p.slots != nullptr && p.table != nullptr && own_block == nblk - 1 && b == 0) table_grad_reduce(p, h, reinterpret_cast<float*>(smem));
+    }
     int M = p.M, N = p.N;
     int64_t q_first = 0, k_first = 0;
     if (p.cu_q != nullptr) {
         q_first = p.cu_q[b]; k_first = p.cu_k[b];
         M = p.len_q != nullptr ? p.len_q[b] : p.cu_q[b + 1] - (int)q_first;
         N = p.len_k != nullptr ? p.len_k[b] : p.cu_k[b + 1] - (int)k_first;
-        if (own_base >= (KV ? N : M)) return false;     // (the grid is sized for the longest sequence)
+        if (own_base >= (KV ? N : M)) {     // (the grid is sized for the longest sequence)
+            if constexpr (!KV) table_grad_none(p, slot);
+            return false;
+        }
     }
     const int n_own = KV ? N : M, n_other = KV ? M : N, P = N - M;
     const bool has_bias = p.table != nullptr;
@@ -263,8 +271,8 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     float* const stats = reinterpret_cast<float*>(smem + G::STAT);
     int* const flag = reinterpret_cast<int*>(smem + G::LUT - 16);
     float* const lut = reinterpret_cast<float*>(smem + G::LUT);
-    float* const hist_rel = reinterpret_cast<float*>(smem + G::hist(sat));
-    float* const skew = reinterpret_cast<float*>(smem + G::skew(sat)) + wave * kSkewRows * 64;
+    float* const dist = reinterpret_cast<float*>(smem + G::hist(sat)) + wave * table_grad_floats(sat);   // dS per distance
+    float* const skew = reinterpret_cast<float*>(smem + G::skew(sat)) + wave * G::SKEW_ROWS * 64;
 
     auto slice = [&](const void* t, int64_t sb, int64_t sh, int64_t sr, int64_t first) {
         return reinterpret_cast<const float*>(t) + (int64_t)b * sb + (int64_t)h * sh + first * sr;
@@ -310,8 +318,8 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     if (has_bias) {
         bias_lo = bias.at(-sat); bias_hi = bias.at(sat);
         if constexpr (!KV) {
-            for (int x = tid; x <= 2 * sat; x += kThreads) hist_rel[x] = 0.f;
-            for (int x = lane; x < kSkewRows * 64; x += 64) skew[x] = 0.f;
+            for (int x = lane; x <= 2 * sat; x += 64) dist[x] = 0.f;
+            for (int x = lane; x < G::SKEW_ROWS * 64; x += 64) skew[x] = 0.f;
         }
     }
     const Reads<SPLIT, RAW> reads(sub0, lane);
@@ -395,23 +403,7 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
                                           ((dp[8] + dp[9]) + (dp[10] + dp[11])) + ((dp[12] + dp[13]) + (dp[14] + dp[15]));
                         if (sat_lo) sum_lo += sum; else sum_hi += sum;
                     } else {
-                        // dS summed per distance: the pair of key kk and query lr at row lr, column kk - lr + R - 1 (attn_bwd.hip)
-                        constexpr int R = kSkewRows;
-#pragma unroll
-                        for (int round = 0; round < 32 / R; ++round) {
-                            if (lr / R == round) {
-                                float* w = skew + (lr % R) * 63 + (R - 1) + 4 * hh;
-#pragma unroll
-                                for (int r = 0; r < 16; ++r) w[8 * (r >> 2) + (r & 3)] = dp[r];
-                            }
-                            asm volatile("" ::: "memory");     // (LDS accesses of a wavefront keep their order)
-                            float c0 = 0.f, c2 = 0.f;
-#pragma unroll
-                            for (int q = 0; q < R; q += 2) { c0 += skew[q * 64 + lane]; c2 += skew[(q + 1) * 64 + lane]; }
-                            asm volatile("" ::: "memory");
-                            const int rel = rel_min + 31 - R * round + lane - (R - 1);
-                            if (lane < 31 + R) atomicAdd(&hist_rel[min(max(rel, -sat), sat) + sat], c0 + c2);
-                        }
+                        table_grad_block<G::SKEW_ROWS>(skew, dist, dp, lane, rel_min + 31, sat, sum_lo, sum_hi);
                     }
                 }
             }
@@ -464,26 +456,9 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
             }
     }
     if constexpr (!KV) {
-        if (has_bias && p.dtable != nullptr) {
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) {
-                sum_lo += __shfl_xor(sum_lo, off, 64);
-                sum_hi += __shfl_xor(sum_hi, off, 64);
-            }
-            float* const hist = reinterpret_cast<float*>(smem);     // (the tiles are done with)
-            __syncthreads();
-            for (int x = tid; x < p.n_buckets; x += kThreads) hist[x] = 0.f;
-            __syncthreads();
-            if (lane == 0) {
-                if (sum_lo != 0.f) atomicAdd(&hist[bucket_of(p.bs, -sat)], sum_lo);
-                if (sum_hi != 0.f) atomicAdd(&hist[bucket_of(p.bs, sat)], sum_hi);
-            }
-            for (int x = tid; x <= 2 * sat; x += kThreads)     // distances -> buckets
-                if (hist_rel[x] != 0.f) atomicAdd(&hist[bucket_of(p.bs, x - sat)], hist_rel[x]);
-            __syncthreads();
-            for (int x = tid; x < p.n_buckets; x += kThreads)
-                if (hist[x] != 0.f) atomicAdd(&p.dtable[(int64_t)x * p.H + h], hist[x]);
-        }
+        // (the tiles are done with)
+        if (has_bias && p.dtable != nullptr)
+            table_grad_finish(p, h, slot, reinterpret_cast<const float*>(smem + G::hist(sat)), reinterpret_cast<float*>(smem), sat, sum_lo, sum_hi);
     }
     return false;
 }
@@ -681,12 +656,17 @@ hipError_t launch_fwd_f32_64(const FwdParams& p, bool causal, hipStream_t stream
     return split ? launch_fwd<false, 2>(p, stream) : launch_fwd<false, 1>(p, stream);
 }
 
-template <bool CAUSAL> static hipError_t launch_passes(const BwdParams& p, hipStream_t stream) {
+template <bool CAUSAL> static hipError_t launch_passes(BwdParams p, hipStream_t stream) {
     const int64_t pairs = (int64_t)p.H * p.B;
-    const hipError_t e = few(p.M, pairs, CAUSAL) ? launch_bwd<CAUSAL, false, 2>(p, stream) : launch_bwd<CAUSAL, false, 1>(p, stream);
+    // (bucketings that reach past some 900 distances leave no room for the larger tiles next to the table gradient's sums)
+    const bool room = Geom<2>::bytes(p.table != nullptr ? p.bs.sat : 0, p.table != nullptr) <= 160 * 1024;
+    const bool split = room && few(p.M, pairs, CAUSAL);
+    p.slots_per_head = p.B * (split ? (p.M + 63) / 64 : (p.M + 127) / 128);
+    if (p.N <= 0) p.slots = nullptr;      // (no pass that would add them)
+    const hipError_t e = split ? launch_bwd<CAUSAL, false, 2>(p, stream) : launch_bwd<CAUSAL, false, 1>(p, stream);
     if (e != hipSuccess) return e;
     return few(p.N, pairs, CAUSAL) ? launch_bwd<CAUSAL, true, 2>(p, stream) : launch_bwd<CAUSAL, true, 1>(p, stream);
 }
-hipError_t launch_bwd_f32_64(const BwdParams& p, bool causal, hipStream_t stream) { return causal ? launch_passes<true>(p, stream) : launch_passes<false>(p, stream); }
+hipError_t launch_bwd_f32_64(BwdParams p, bool causal, hipStream_t stream) { return causal ? launch_passes<true>(p, stream) : launch_passes<false>(p, stream); }
 
 }  // namespace t5a

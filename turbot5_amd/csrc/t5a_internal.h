@@ -163,6 +163,9 @@ struct BwdParams {
     void* dq; void* dk; void* dv;
     float* dtable;                    // (n_buckets, H) fp32, or null
     float* delta; float* lse2;        // workspace, (B,H,M) each
+    // optional workspace of the table gradient, one slot of n_buckets floats (at most kMaxSlotBuckets) per head, sequence and
+    // block of query rows; slots_per_head is filled in by the launch
+    float* slots; int slots_per_head;
     int64_t q_sb, q_sh, q_sr, k_sb, k_sh, k_sr, v_sb, v_sh, v_sr, o_sb, o_sh, o_sr, do_sb, do_sh, do_sr;
     int64_t dq_sb, dq_sh, dq_sr, dk_sb, dk_sh, dk_sr, dv_sb, dv_sh, dv_sr;
     int B, H, M, N;                   // packed: M, N are the longest sequence's lengths
@@ -175,11 +178,13 @@ struct BwdParams {
     const void* table; int table_dtype; int64_t t_sbucket, t_shead;
     BucketSpec bs;
 };
+constexpr int kMaxSlotBuckets = 64;
+constexpr int64_t kMaxSlotBytes = 64 << 20;     // of a launch
 hipError_t launch_bwd_dense(const BwdParams& p, int dtype, int D, bool causal, hipStream_t stream);
 
 // fp32 tensors at head_dim 64 (attn_f32.hip): the dense forward, and the backward's passes behind bwd_rows_kernel
 hipError_t launch_fwd_f32_64(const FwdParams& p, bool causal, hipStream_t stream);
-hipError_t launch_bwd_f32_64(const BwdParams& p, bool causal, hipStream_t stream);
+hipError_t launch_bwd_f32_64(BwdParams p, bool causal, hipStream_t stream);
 
 struct RmsParams {
     const void* x; const void* weight; void* y;

@@ -237,6 +237,14 @@ def _backward_bias_struct(bias, NUM_BUCKETS, MAX_DISTANCE):
     return L.T5ABias(table.data_ptr(), _DTYPES[table.dtype], NUM_BUCKETS, MAX_DISTANCE, 0, *table.stride()), table
 
 
+def _backward_workspace(lib, need, B, H, rows, bias, NUM_BUCKETS, device):
+    """Row statistics, and with a table the slots its gradient is added from in a fixed order."""
+    need = max((need + 15) & ~15, 16)
+    if bias is not None:
+        need += lib.t5a_bwd_table_workspace_bytes(B, H, rows, NUM_BUCKETS)
+    return torch.empty(need, device=device, dtype=torch.uint8)
+
+
 def _dense_backward(q, k, v, bias, o, lse, dout, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, exact_scores):
     """-> dq, dk, dv, dbias (fp32 (NUM_BUCKETS, H), or None without a table); t5a_bwd_dense"""
     B, H, M, D = q.shape
@@ -249,7 +257,7 @@ def _dense_backward(q, k, v, bias, o, lse, dout, causal, sm_scale, NUM_BUCKETS, 
     dq, dk, dv = torch.empty_like(q_), torch.empty_like(k_), torch.empty_like(v_)
     dtable = torch.empty((NUM_BUCKETS, H), device=q.device, dtype=torch.float32) if bias is not None else None
     lib = L.load()
-    ws = torch.empty(max(int(lib.t5a_bwd_workspace_bytes(B, H, M)), 16), device=q.device, dtype=torch.uint8)
+    ws = _backward_workspace(lib, lib.t5a_bwd_workspace_bytes(B, H, M), B, H, M, bias, NUM_BUCKETS, q.device)
     bias_args, keep = _backward_bias_struct(bias, NUM_BUCKETS, MAX_DISTANCE)
     a = L.T5ADenseBwdArgs(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(), g_.data_ptr(), lse.data_ptr(),
                           dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dtable.data_ptr() if dtable is not None else None,
@@ -426,7 +434,7 @@ def _varlen_backward(q, k, v, bias, o, lse, dout, cu_seqlens_q, cu_seqlens_k, ma
     dv = (torch.empty_like if lens[1] is None else torch.zeros_like)(v_)
     dtable = torch.empty((NUM_BUCKETS, H), device=q.device, dtype=torch.float32) if bias is not None else None
     lib = L.load()
-    ws = torch.empty(max(int(lib.t5a_bwd_varlen_workspace_bytes(total_q, H)), 16), device=q.device, dtype=torch.uint8)
+    ws = _backward_workspace(lib, lib.t5a_bwd_varlen_workspace_bytes(total_q, H), B, H, int(max_seqlen_q), bias, NUM_BUCKETS, q.device)
     bias_args, keep = _backward_bias_struct(bias, NUM_BUCKETS, MAX_DISTANCE)
     a = L.T5AVarlenBwdArgs(q_.data_ptr(), k_.data_ptr(), v_.data_ptr(), o_.data_ptr(), g_.data_ptr(), lse.data_ptr(),
                            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dtable.data_ptr() if dtable is not None else None,

@@ -57,9 +57,9 @@ class T5LayerNorm(nn.Module):
             return rms_norm(x, self.weight, self.eps, group, seq_lens=seq_lens, seq_starts=seq_starts,
                             key_bits=key_bits, group_counts=group_counts)
         if group == 1 and differentiated and seq_lens is None and key_bits is None:
-            from .ops import RmsNorm, rms_norm_differentiable
+            from .ops import rms_norm_differentiable, rms_norm_train
             if rms_norm_differentiable(x, self.weight):
-                return RmsNorm.apply(x, self.weight, self.eps, None)[1]
+                return rms_norm_train(x, self.weight, self.eps)[1]
         if group > 1:
             B, L, d = x.shape
             n = L // group
@@ -85,9 +85,9 @@ class T5LayerNorm(nn.Module):
             from .ops import rms_norm
             return rms_norm(x, self.weight, self.eps, 1, residual)
         if self.training and differentiated:
-            from .ops import RmsNorm, rms_norm_differentiable
+            from .ops import rms_norm_differentiable, rms_norm_train
             if rms_norm_differentiable(x, self.weight, residual):
-                return RmsNorm.apply(x, self.weight, self.eps, residual)
+                return rms_norm_train(x, self.weight, self.eps, residual)
         total = x + residual
         return total, self.forward(total)
 

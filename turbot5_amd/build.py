@@ -1,4 +1,5 @@
-"""Builds libt5attn.so (hand-written HIP for gfx950) in-tree with hipcc.
+"""Builds libt5attn.so (hand-written HIP for gfx950) in-tree with hipcc, and _native.so (the backward nodes for torch's
+autograd, host code) with the host compiler.
 
     python -m turbot5_amd.build            # or: from turbot5_amd.build import build; build()
 """
@@ -53,6 +54,19 @@ def _run(cmd, verbose):
         print(out, flush=True)
 
 
+NATIVE = os.path.join(HERE, "_native.so")
+
+
+def _native_cmd():
+    import sysconfig
+    from torch.utils import cpp_extension
+    torch_lib = os.path.join(os.path.dirname(os.path.dirname(cpp_extension.__file__)), "lib")
+    includes = [*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    return [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-DTORCH_API_INCLUDE_EXTENSION_H", *(f"-I{p}" for p in includes), os.path.join(CSRC, "autograd.cpp"), "-o", NATIVE,
+            f"-L{torch_lib}", "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 TRACE_LIB = os.path.join(HERE, "libt5attn_trace.so")
 
 
@@ -68,6 +82,8 @@ def build(verbose: bool = False, jobs: int = 8, extra_flags=(), trace: bool = Fa
     cmds = []
     for obj, src, defs in UNITS:
         cmds.append([hipcc, *flags, *defs, "-c", os.path.join(CSRC, src), "-o", os.path.join(obj_dir, obj)])
+    if not trace:
+        cmds.append(_native_cmd())
     with ThreadPoolExecutor(max_workers=jobs) as ex:
         list(ex.map(lambda c: _run(c, verbose), cmds))
     objs = [os.path.join(obj_dir, o) for o, _, _ in UNITS]

@@ -13,18 +13,19 @@ import torch
 from torch import nn
 
 from . import _lib as L
-from .ops import _DTYPES, _on_device, _plain, _stream
+from .ops import _DTYPES, _nodes, _on_device, _plain, _stream
 
 MAX_BYTES = 0x7fe00000      # of an operand, which the kernel reads with 32-bit offsets
 
 
 def _gemm(a, b, out, a_trans=False, b_trans=False, sum_groups=False, alpha=1.0, relu=False, positive=None):
-    """out[g] = alpha_g a[g] b[g]^T over lists of two-dimensional contiguous tensors; see include/t5attn.h."""
+    """out[g] = alpha_g a[g] b[g]^T over lists of two-dimensional contiguous tensors; see include/t5attn.h.  (What the nodes of
+    ``project`` and ``feed_forward_relu`` call from native code.)"""
     n = len(a)
     args = L.T5AGemmF32Args((C.c_void_p * 3)(*(t.data_ptr() for t in a)), (C.c_void_p * 3)(*(t.data_ptr() for t in b)),
-                            (C.c_void_p * 3)(*(t.data_ptr() for t in out)), a[0].stride(0), b[0].stride(0), out[0].stride(0),
+                            (C.c_void_p * 3)(*(t.data_ptr() for t in out)), a[0].shape[1], b[0].shape[1], out[0].shape[1],
                             positive.data_ptr() if positive is not None else None,
-                            positive.stride(0) if positive is not None else 0, None, 0,
+                            positive.shape[1] if positive is not None else 0, None, 0,
                             out[0].shape[0], out[0].shape[1], a[0].shape[0 if a_trans else 1], n, int(sum_groups),
                             _DTYPES[a[0].dtype], _DTYPES[b[0].dtype], _DTYPES[out[0].dtype], int(a_trans), int(b_trans),
                             int(relu), float(alpha))
@@ -37,100 +38,6 @@ def _gemm(a, b, out, a_trans=False, b_trans=False, sum_groups=False, alpha=1.0, 
     with _on_device(out[0]):
         L.check(lib.t5a_gemm_f32(C.byref(args), _stream(out[0])))
     return out
-
-
-def _rows(t: torch.Tensor, wide: bool = False) -> torch.Tensor:
-    """Detached contiguous aligned rows, fp32 or bf16 (``wide``: fp32)."""
-    t = t.detach()
-    if t.dtype == torch.float16 or (wide and t.dtype != torch.float32):
-        t = t.float()
-    t = t.contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
-
-
-class Projections(torch.autograd.Function):
-    """x W_0^T * factor, x W_1^T, ...: products of the same rows with up to three weights of one shape, each result
-    rounded to ``dtype`` once."""
-
-    @staticmethod
-    def forward(ctx, x, dtype, factor, *weights):
-        rows = _rows(x)
-        out = tuple(torch.empty((x.shape[0], w.shape[0]), device=x.device, dtype=dtype) for w in weights)
-        _gemm([rows] * len(weights), [_rows(w) for w in weights], out, alpha=factor)
-        ctx.save_for_backward(x, *weights)
-        ctx.factor = factor
-        return out
-
-    @staticmethod
-    def backward(ctx, *grads):
-        x, *weights = ctx.saved_tensors
-        need_x, need_w = ctx.needs_input_grad[0], ctx.needs_input_grad[3:]
-        dx, dw = None, [None] * len(weights)
-        if torch.is_grad_enabled() or not _plain(x, *weights, *grads):
-            wide = x.float()
-            for i, (g, w) in enumerate(zip(grads, weights)):
-                g = g.float() * ctx.factor if i == 0 else g.float()
-                if need_x:
-                    part = torch.matmul(g, w)
-                    dx = part if dx is None else dx + part
-                if need_w[i]:
-                    dw[i] = torch.matmul(g.transpose(-1, -2), wide)
-            return (None if dx is None else dx.to(x.dtype), None, None, *dw)
-        g = [_rows(t) for t in grads]
-        if need_x:
-            dx = torch.empty(x.shape, device=x.device, dtype=x.dtype)
-            _gemm(g, [_rows(w) for w in weights], [dx], b_trans=True, sum_groups=True, alpha=ctx.factor)
-        todo = [i for i, n in enumerate(need_w) if n]
-        if todo:
-            rows = _rows(x, wide=g[0].dtype == torch.bfloat16)
-            for i in todo:
-                dw[i] = torch.empty(weights[i].shape, device=x.device, dtype=torch.float32)
-            _gemm([g[i] for i in todo], [rows] * len(todo), [dw[i] for i in todo], a_trans=True, b_trans=True,
-                  alpha=ctx.factor if todo[0] == 0 else 1.0)
-        return (dx, None, None, *dw)
-
-
-class FeedForwardRelu(torch.autograd.Function):
-    """relu(x W_i^T) W_o^T: ReLU and its derivative are part of the products that make their operand."""
-
-    @staticmethod
-    def forward(ctx, x, wi, wo):
-        mid = torch.empty((x.shape[0], wi.shape[0]), device=x.device, dtype=torch.float32)
-        out = torch.empty((x.shape[0], wo.shape[0]), device=x.device, dtype=torch.float32)
-        _gemm([_rows(x)], [_rows(wi)], [mid], relu=True)
-        _gemm([mid], [_rows(wo)], [out])
-        ctx.save_for_backward(x, wi, wo, mid)
-        return out
-
-    @staticmethod
-    def backward(ctx, dy):
-        x, wi, wo, mid = ctx.saved_tensors
-        need_x, need_wi, need_wo = ctx.needs_input_grad
-        dx = dwi = dwo = None
-        if torch.is_grad_enabled() or not _plain(x, wi, wo, dy):
-            mid = torch.relu(torch.matmul(x, wi.t()))      # (differentiable in its turn)
-            dmid = torch.matmul(dy, wo) * (mid > 0)
-            if need_x:
-                dx = torch.matmul(dmid, wi)
-            if need_wi:
-                dwi = torch.matmul(dmid.transpose(-1, -2), x)
-            if need_wo:
-                dwo = torch.matmul(dy.transpose(-1, -2), mid)
-            return dx, dwi, dwo
-        rows, dy = _rows(x), _rows(dy)
-        if need_wo:
-            dwo = torch.empty(wo.shape, device=x.device, dtype=torch.float32)
-            _gemm([dy], [mid], [dwo], a_trans=True, b_trans=True)
-        if need_x or need_wi:
-            dmid = torch.empty_like(mid)
-            _gemm([dy], [_rows(wo)], [dmid], b_trans=True, positive=mid)
-            if need_wi:
-                dwi = torch.empty(wi.shape, device=x.device, dtype=torch.float32)
-                _gemm([dmid], [rows], [dwi], a_trans=True, b_trans=True)
-            if need_x:
-                dx = torch.empty(x.shape, device=x.device, dtype=torch.float32)
-                _gemm([dmid], [_rows(wi)], [dx], b_trans=True)
-        return dx, dwi, dwo
 
 
 def _full_precision() -> bool:
@@ -151,7 +58,7 @@ def _bare(m: nn.Module) -> bool:
 
 def takes(x: torch.Tensor, *layers: nn.Module) -> bool:
     """Whether these layers' products over ``x`` (fp32, or bf16 that torch would widen) are part of a training step that
-    ``Projections`` takes: fp32 weights of one shape on x's device and plain reverse-mode autograd.  Any number of rows: at 8 a product of a T5-small
+    ``project`` takes: fp32 weights of one shape on x's device and plain reverse-mode autograd.  Any number of rows: at 8 a product of a T5-small
     layer takes 4 to 12 us, the library's fp32 one 19 to 25; at 4500 all of a layer's take 600 us, the library's 900."""
     if not x.is_cuda or not torch.is_grad_enabled() or not all(_bare(m) for m in layers):
         return False
@@ -175,12 +82,13 @@ def widths_chain(wi: nn.Module, wo: nn.Module) -> bool:
 
 
 def project(x, dtype, factor, *layers):
-    """The layers' products over the rows of x (see ``Projections``), in x's shape; ``takes`` has said yes."""
-    rows = x.reshape(-1, x.shape[-1])
-    out = Projections.apply(rows, dtype, float(factor), *(m.weight for m in layers))
+    """x W_0^T * factor, x W_1^T, ...: products of the same rows with up to three weights of one shape, each result rounded to
+    ``dtype`` once, in x's shape; ``takes`` has said yes."""
+    out = _nodes().project(x.reshape(-1, x.shape[-1]), dtype, float(factor), [m.weight for m in layers])
     return [t.view(*x.shape[:-1], t.shape[-1]) for t in out]
 
 
 def feed_forward_relu(x, wi: nn.Linear, wo: nn.Linear):
-    """relu(wi(x)) through wo; ``takes`` and ``widths_chain`` have said yes."""
-    return FeedForwardRelu.apply(x.reshape(-1, x.shape[-1]), wi.weight, wo.weight).view(*x.shape[:-1], wo.weight.shape[0])
+    """relu(wi(x)) through wo, ReLU and its derivative part of the products that make their operand; ``takes`` and
+    ``widths_chain`` have said yes."""
+    return _nodes().feed_forward_relu(x.reshape(-1, x.shape[-1]), wi.weight, wo.weight).view(*x.shape[:-1], wo.weight.shape[0])

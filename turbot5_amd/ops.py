@@ -270,6 +270,34 @@ def _dense_backward(q, k, v, bias, o, lse, dout, causal, sm_scale, NUM_BUCKETS, 
     return dq, dk, dv, dtable
 
 
+_NODES = None
+
+
+def _nodes():
+    """The autograd nodes in native code (csrc/autograd.cpp), bound to the loaded library."""
+    global _NODES
+    if _NODES is None:
+        lib = L.load()
+        try:
+            from . import _native
+        except ImportError as e:
+            raise ImportError(f"turbot5_amd/_native.so is not built or does not match this torch (run `python -m turbot5_amd.build`): {e}") from e
+        if _native.abi_version != L.ABI_VERSION:
+            raise ImportError(f"turbot5_amd/_native.so has ABI version {_native.abi_version}, expected {L.ABI_VERSION}: rebuild it")
+        _native.bind(*(C.cast(getattr(lib, name), C.c_void_p).value for name in (
+            "t5a_bwd_dense", "t5a_bwd_varlen", "t5a_bwd_workspace_bytes", "t5a_bwd_varlen_workspace_bytes",
+            "t5a_bwd_table_workspace_bytes", "t5a_last_error", "t5a_gemm_f32", "t5a_gemm_f32_workspace_bytes", "t5a_rmsnorm_train",
+            "t5a_rmsnorm_bwd_workspace_bytes")))
+        _NODES = _native
+    return _NODES
+
+
+def _takes_node(q, k, v, bias) -> bool:
+    """Whether a differentiated call gets the native node: plain tensors and plain reverse-mode autograd.  Compilation, tracing,
+    function transforms, forward mode, dispatch modes and tensor subclasses meet the autograd.Function below."""
+    return not torch.compiler.is_compiling() and q.is_cuda and _nodes().takes([q, k, v, bias])
+
+
 class FlashAttentionBias(torch.autograd.Function):
     """The dense fused-bias forward with its backward (reference fused_bias_attention.py:821-873): gradients for q,
     k, v and the (NUM_BUCKETS, H) table."""
@@ -306,6 +334,11 @@ def flash_attention_with_fusing_bias(q, k, v, bias, causal=False, sm_scale=None,
     """
     needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
                                               or (bias is not None and bias.requires_grad))
+    if needs_grad and _takes_node(q, k, v, bias):
+        o, lse = _dense_forward(q, k, v, bias, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, True, exact_scores)
+        _nodes().attach_dense(o, lse, q, k, v, bias, bool(causal), 1.0 / math.sqrt(q.shape[-1]) if sm_scale is None else float(sm_scale),
+                              NUM_BUCKETS, MAX_DISTANCE, _exact(exact_scores))
+        return (o, lse) if return_lse else o
     if needs_grad:
         o, lse = FlashAttentionBias.apply(q, k, v, bias, causal, sm_scale, NUM_BUCKETS, MAX_DISTANCE, exact_scores)
         return (o, lse) if return_lse else o
@@ -495,6 +528,16 @@ def flash_attention_with_fusing_bias_varlen(q, k, v, bias, cu_seqlens_q, cu_seql
     """
     needs_grad = torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad
                                               or (bias is not None and bias.requires_grad))
+    if needs_grad and _takes_node(q, k, v, bias):
+        cq, ck, lq, lk = (t if t is None or (t.dtype == torch.int32 and t.device == q.device and t.is_contiguous())
+                          else t.to(device=q.device, dtype=torch.int32).contiguous()
+                          for t in (cu_seqlens_q, cu_seqlens_k, seq_lens_q, seq_lens_k))
+        o, lse = _varlen_forward(q, k, v, bias, cq, cq if cu_seqlens_k is cu_seqlens_q else ck, max_seqlen_q, max_seqlen_k, causal, sm_scale,
+                                 NUM_BUCKETS, MAX_DISTANCE, True, lq, lk, launch_plan, exact_scores)
+        _nodes().attach_varlen(o, lse, q, k, v, bias, cq, ck, int(max_seqlen_q), int(max_seqlen_k), lq, lk, bool(causal),
+                               1.0 / math.sqrt(q.shape[-1]) if sm_scale is None else float(sm_scale), NUM_BUCKETS, MAX_DISTANCE,
+                               _exact(exact_scores))
+        return (o, lse) if return_lse else o
     if needs_grad:
         o, lse = FlashAttentionBiasVarlen.apply(q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k, causal,
                                                 sm_scale, NUM_BUCKETS, MAX_DISTANCE, seq_lens_q, seq_lens_k, launch_plan,
@@ -739,96 +782,24 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6, group: in
     return y if total is None else (total, y)
 
 
-def _rms_norm_backward_ops(x, weight, eps, dy, dsum):
-    """The kernel's backward in torch's operations, for whatever needs those: gradients that are differentiated in their
-    turn, batches of gradients, forward-mode levels, tracing."""
-    x32 = x.to(torch.float32)
-    rstd = torch.rsqrt(x32.pow(2).mean(-1, keepdim=True) + eps)
-    n = x32 * rstd
-    if weight.dtype in (torch.float16, torch.bfloat16):
-        n = n.to(weight.dtype)
-    g = (dy * weight).to(torch.float32)
-    dx = rstd * g - x32 * (rstd.pow(3) * (g * x32).mean(-1, keepdim=True))
-    if dsum is not None:
-        dx = dx + dsum
-    dw = (dy.to(torch.float32) * n).sum(tuple(range(dy.dim() - 1)))
-    return dx.to(x.dtype), dw.to(weight.dtype)
-
-
-def _rms_norm_train(x, weight, rstd, dy=None, dsum=None):
-    """t5a_rmsnorm_train over contiguous rows: y, or with ``dy`` (dx, dweight)."""
-    d = x.shape[-1]
-    lib = L.load()
-    a = L.T5ARmsNormTrainArgs()
-    a.x, a.weight, a.rstd = x.data_ptr(), weight.data_ptr(), rstd.data_ptr()
-    a.rows, a.dim = x.numel() // d, d
-    a.x_dtype, a.weight_dtype = _dtype_code(x), _dtype_code(weight)
-    if dy is None:
-        out = torch.empty(x.shape, device=x.device, dtype=weight.dtype if weight.dtype in (torch.float16, torch.bfloat16) else torch.float32)
-        a.y = out.data_ptr()
-    else:
-        out = torch.empty_like(x), torch.empty_like(weight)
-        ws = torch.empty(int(lib.t5a_rmsnorm_bwd_workspace_bytes(a.rows, d)), device=x.device, dtype=torch.uint8)
-        a.dy, a.dx, a.dweight = dy.data_ptr(), out[0].data_ptr(), out[1].data_ptr()
-        a.dsum = dsum.data_ptr() if dsum is not None else None
-        a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    with _on_device(x):
-        L.check(lib.t5a_rmsnorm_train(C.byref(a), _stream(x)))
-    return out
-
-
-def _rows16(t: torch.Tensor) -> torch.Tensor:
-    t = t.detach().contiguous()
-    return t if t.data_ptr() % 16 == 0 else t.clone()
-
-
-class RmsNorm(torch.autograd.Function):
-    """The norm of x, or of x + residual, with its backward: (x + residual, norm), or (None, norm)."""
-
-    @staticmethod
-    def forward(ctx, x, weight, eps, residual):
-        total = x if residual is None else x + residual
-        rstd = torch.rsqrt(total.to(torch.float32).pow(2).mean(-1, keepdim=True) + eps).contiguous()
-        y = _rms_norm_train(_rows16(total), weight.detach().contiguous(), rstd)
-        ctx.save_for_backward(total, weight, rstd)
-        ctx.eps = eps
-        ctx.set_materialize_grads(False)
-        if residual is not None and not (ctx.needs_input_grad[0] or ctx.needs_input_grad[3]):
-            ctx.mark_non_differentiable(total)      # (only the weight is trained: the residual stream carries no graph)
-        return None if residual is None else total, y
-
-    @staticmethod
-    def backward(ctx, dsum, dy):
-        x, weight, rstd = ctx.saved_tensors
-        need = ctx.needs_input_grad
-        if dy is None:
-            dx, dw = dsum, None
-        elif torch.is_grad_enabled() or not _plain(x, weight, dy, dsum):
-            dx, dw = _rms_norm_backward_ops(x, weight, ctx.eps, dy, dsum)
-        else:
-            dx, dw = _rms_norm_train(_rows16(x), weight.detach().contiguous(), rstd, _rows16(dy),
-                                     _rows16(dsum) if dsum is not None else None)
-            dw = dw.view_as(weight)
-        return dx if need[0] else None, dw if need[1] else None, None, dx if need[3] else None
+def rms_norm_train(x, weight, eps, residual=None):
+    """The norm of x, or of x + residual, with its backward: (x + residual, norm), or (None, norm);
+    ``rms_norm_differentiable`` has said yes.  Scaling and backward are ``t5a_rmsnorm_train``."""
+    return _nodes().rms_norm_train(x, weight, float(eps), residual)
 
 
 def _plain(*tensors) -> bool:
     """Plain tensors and plain reverse-mode autograd: no batch of gradients, no tracing, function transform, forward-mode level
     or dispatch mode, for which a formula in torch's own operations is the one that works."""
-    # (what is being compiled or traced is not asked further)
-    if torch.compiler.is_compiling() or torch.jit.is_tracing():
-        return False
-    f = torch._C._functorch
-    return (all(type(t) in (torch.Tensor, torch.nn.Parameter) and not f.is_batchedtensor(t) and not f.is_legacy_batchedtensor(t)
-                for t in tensors if t is not None)
-            and torch.autograd.forward_ad._current_level < 0 and f.peek_interpreter_stack() is None
-            and torch._C._len_torch_dispatch_stack() == 0)
+    # (what is being compiled is not asked further)
+    return (not torch.compiler.is_compiling() and torch.autograd.forward_ad._current_level < 0
+            and _nodes().takes([*tensors]))
 
 
 def rms_norm_differentiable(x, weight, residual=None) -> bool:
-    """Whether ``RmsNorm`` takes this call: plain tensors of the kernels' types on one ROCm device, rows that stay in
+    """Whether ``rms_norm_train`` takes this call: plain tensors of the kernels' types on one ROCm device, rows that stay in
     registers, and plain reverse-mode autograd."""
-    return (_plain(x, weight, residual) and x.is_cuda and weight.device == x.device and x.dtype in _DTYPES
+    return (x.is_cuda and _plain(x, weight, residual) and weight.device == x.device and x.dtype in _DTYPES
             and weight.dtype in _DTYPES and x.numel() > 0
             and weight.shape == x.shape[-1:] and x.shape[-1] % 8 == 0 and x.shape[-1] <= L.RMSNORM_TRAIN_MAX_DIM
             and (residual is None or (type(residual) is torch.Tensor and residual.shape == x.shape

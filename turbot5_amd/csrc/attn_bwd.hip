@@ -418,33 +418,36 @@ __global__ __launch_bounds__(kBwdThreads, 2) void bwd_kernel(const BwdParams p) 
 // head_dim 128 (the T5-3B / 11B head shape): rows of 256 bytes, sixteen chunks
 __device__ __forceinline__ int tile_swz128(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
 
-// Geometry of a 16-bit backward workgroup: four wavefronts, each on 32 own rows and 32 rows of the tile at a time (one
+// Geometry of a 16-bit backward workgroup: wavefronts each on 32 own rows and 32 rows of the tile at a time (one
 // 32 x 32 block of scores: 32 score registers, which is what lets three wavefronts share a SIMD at head_dim 64).
 // SPLIT 1: four groups of own rows, tiles of 32.  SPLIT 2: two groups of own rows, tiles of 64 whose halves go to
-// different wavefronts; the two partial gradients of a row are added through LDS at the end.
+// different wavefronts; the two partial gradients of a row are added through LDS at the end.  SPLIT 4: the same with eight
+// wavefronts and tiles of 128, which halves the chain of tiles behind a block once more.
 template <int D, int PASS, int SPLIT>
 struct Bwd16Geom {
     static constexpr bool KV = PASS != 0;
-    static constexpr int OWNW = 4 / SPLIT, OWN = 32 * OWNW, OTHER = 32 * SPLIT;
+    static constexpr int WAVES = SPLIT == 4 ? 8 : 4, THREADS = 64 * WAVES;
+    static constexpr int OWNW = WAVES / SPLIT, OWN = 32 * OWNW, OTHER = 32 * SPLIT;
     static constexpr int TILE = OTHER * D * 2;                    // bytes of one staged tile
-    static constexpr int SLABS = TILE / 1024 / 4;                 // 1 KB requests per wavefront and tile
+    static constexpr int SLABS = TILE / 1024 / WAVES;               // 1 KB requests per wavefront and tile
     static constexpr int RPS = 1024 / (2 * D);                    // rows per request
     static constexpr int STAGES = 2;                               // tile buffers
     static constexpr int REQS = 2 * SLABS + (KV ? 1 : 0);         // requests per wavefront and tile
-    static constexpr int SKEW_ROWS = (D == 128 && SPLIT == 2) ? 8 : 32;   // queries per round of the table gradient
+    static constexpr int SKEW_ROWS = D == 128 && SPLIT >= 2 ? 8 : SPLIT == 4 ? 16 : 32;   // queries per round of the table gradient
+    static constexpr int STAT_ROWS = OTHER > 64 ? OTHER : 64;      // of one statistic of a tile
     static constexpr int LUT_PAD16 = 64;                          // a 32 x 32 block spans 63 distances
     static constexpr int STAT = STAGES * 2 * TILE;                // byte offsets
-    static constexpr int LUT = STAT + (KV ? STAGES * 2 * 64 * 4 : 0);
+    static constexpr int LUT = STAT + (KV ? STAGES * 2 * STAT_ROWS * 4 : 0);
     static __host__ __device__ int lut_floats(int sat) { return (2 * (sat + LUT_PAD16) + 4) & ~3; }
     static __host__ __device__ int hist(int sat) { return LUT + 4 * lut_floats(sat); }
-    static __host__ __device__ int skew(int sat) { return hist(sat) + (KV ? 0 : 4 * kTableGradWaves * table_grad_floats(sat)); }
-    static __host__ __device__ int bytes(int sat, bool bias) { return skew(sat) + (KV || !bias ? 0 : 4 * SKEW_ROWS * 64 * 4); }
+    static __host__ __device__ int skew(int sat) { return hist(sat) + (KV ? 0 : 4 * WAVES * table_grad_floats(sat)); }
+    static __host__ __device__ int bytes(int sat, bool bias) { return skew(sat) + (KV || !bias ? 0 : WAVES * SKEW_ROWS * 64 * 4); }
 };
 
 template <int D> __device__ __forceinline__ int row_swz(int row) { return D == 64 ? tile_swz(row) : tile_swz128(row); }
 
 template <typename T, int D, bool CAUSAL, int PASS, int SPLIT>
-__global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ? 3 : 2) void bwd16_kernel(const BwdParams p, int nblk) {
+__global__ __launch_bounds__(SPLIT == 4 ? 512 : kBwdThreads, SPLIT != 4 && (D == 64 || (PASS == 3 && SPLIT == 1)) ? 3 : 2) void bwd16_kernel(const BwdParams p, int nblk) {
     constexpr bool KV = PASS != 0, DS = PASS != 3, DA = PASS != 3, DV = PASS == 1 || PASS == 3;   // dS; dq or dk; dv
     using G = Bwd16Geom<D, PASS, SPLIT>;
     constexpr int DT = D / 32, KS = D / 16, OTHER = G::OTHER, CH = D / 8;
@@ -460,7 +463,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
     const int64_t slot = ((int64_t)h * p.B + b) * nblk + own_block;     // (of the table gradient)
     if constexpr (PASS == 1 || PASS == 2) {
         // (the last block: the shortest of a causal launch)
-        if (p.slots != nullptr && p.table != nullptr && own_block == nblk - 1 && b == 0) table_grad_reduce(p, h, reinterpret_cast<float*>(bwd_smem));
+        if (p.slots != nullptr && p.table != nullptr && own_block == nblk - 1 && b == 0) table_grad_reduce<G::WAVES>(p, h, reinterpret_cast<float*>(bwd_smem));
     }
     const int w_lo = own_base + ow * 32, own_row = w_lo + lr;     // this wavefront's, this lane's own rows
     int M = p.M, N = p.N;
@@ -470,7 +473,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
         M = p.len_q != nullptr ? p.len_q[b] : p.cu_q[b + 1] - (int)q_first;
         N = p.len_k != nullptr ? p.len_k[b] : p.cu_k[b + 1] - (int)k_first;
         if (own_base >= (KV ? N : M)) {     // (the grid is sized for the longest sequence)
-            if constexpr (PASS == 0) table_grad_none(p, slot);
+            if constexpr (PASS == 0) table_grad_none<G::WAVES>(p, slot);
             return;
         }
     }
@@ -518,7 +521,10 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
             dma_16(rs_a, lds0 + at, other * a_srb + ch * 16);
             dma_16(rs_b, lds0 + at + G::TILE, other * b_srb + ch * 16);
         }
-        if constexpr (KV) dma_4(rs_s, lds0 + G::STAT + buf * 512 + (wave & 1) * 256, (t * OTHER + lane) * (int)stat_sr * 4);
+        if constexpr (KV) {
+            const int half = G::STAT_ROWS > 64 ? (wave >> 1 & 1) * 64 : 0;
+            dma_4(rs_s, lds0 + G::STAT + (buf * 2 + (wave & 1)) * (G::STAT_ROWS * 4) + half * 4, (t * OTHER + half + lane) * (int)stat_sr * 4);
+        }
     };
     const BiasColumn bias(p, h, lane);
     // Tile t + STAGES - 1 is requested when the barrier at the top of tile t has shown that every wavefront is done with
@@ -552,7 +558,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
     float bias_lo = 0.f, bias_hi = 0.f;     // ... and of the two saturated sides
     {
         const int mid = sat + G::LUT_PAD16;
-        for (int x0 = 0; x0 <= 2 * mid; x0 += kBwdThreads) {
+        for (int x0 = 0; x0 <= 2 * mid; x0 += G::THREADS) {
             const int x = x0 + tid;
             const float v = bias.at(KV ? mid - x : x - mid);
             if (x <= 2 * mid) lut[x] = v;
@@ -604,7 +610,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
         if (t + G::STAGES - 1 < t_hi) request(t + G::STAGES - 1, buf == 0 ? G::STAGES - 1 : buf - 1);
         const T* ta = reinterpret_cast<const T*>(bwd_smem + buf * 2 * G::TILE);
         const T* tb = reinterpret_cast<const T*>(bwd_smem + buf * 2 * G::TILE + G::TILE);
-        const float* rowstat = reinterpret_cast<const float*>(bwd_smem + G::STAT) + buf * 128 + sub0 + 4 * hh;
+        const float* rowstat = reinterpret_cast<const float*>(bwd_smem + G::STAT) + buf * 2 * G::STAT_ROWS + sub0 + 4 * hh;
         (void)rowstat;
 
         const int s0 = t * OTHER + sub0;        // first tile row of this wavefront's block
@@ -617,7 +623,7 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
             if constexpr (KV && DS) {      // (dP starts at -delta: the matrix core subtracts it for free)
 #pragma unroll
                 for (int r4 = 0; r4 < 4; ++r4) {
-                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(rowstat + 64 + 8 * r4);
+                    const f32x4 d4 = *reinterpret_cast<const f32x4*>(rowstat + G::STAT_ROWS + 8 * r4);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) dp[4 * r4 + e] = d4[e];
                 }
@@ -702,28 +708,33 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
     }
 
     if constexpr (SPLIT > 1) {
-        // the partial gradients of the second half's wavefronts, in lane order through the tile buffers
-        float* const red = reinterpret_cast<float*>(bwd_smem) + ow * (((DA ? 1 : 0) + (DV ? 1 : 0)) * DT * 16 * 64) + lane;
-        constexpr int AT_B = DA ? DT * 16 : 0;
-        __syncthreads();
-        if (sub0 != 0) {
+        // the partial gradients of the other wavefronts on the same rows, in lane order through the tile buffers
+        constexpr int AT_B = DA ? DT * 16 : 0, REGS = ((DA ? 1 : 0) + (DV ? 1 : 0)) * DT * 16;
+        const int part = wave / G::OWNW;
+        static_assert(SPLIT / 2 * G::OWNW * REGS * 256 <= G::STAGES * 2 * G::TILE, "");
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+        for (int n = SPLIT / 2; n > 0; n /= 2) {
+            float* const red = reinterpret_cast<float*>(bwd_smem) + ((part & (n - 1)) * G::OWNW + ow) * (REGS * 64) + lane;
+            __syncthreads();
+            if (part >= n && part < 2 * n) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    if constexpr (DA) red[(dt * 16 + r) * 64] = acc_a[dt][r];
-                    if constexpr (DV) red[(AT_B + dt * 16 + r) * 64] = acc_b[dt][r];
-                }
-        }
-        __syncthreads();
-        if (sub0 == 0) {
+                for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
+                    for (int r = 0; r < 16; ++r) {
+                        if constexpr (DA) red[(dt * 16 + r) * 64] = acc_a[dt][r];
+                        if constexpr (DV) red[(AT_B + dt * 16 + r) * 64] = acc_b[dt][r];
+                    }
+            }
+            __syncthreads();
+            if (part < n) {
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    if constexpr (DA) acc_a[dt][r] += red[(dt * 16 + r) * 64];
-                    if constexpr (DV) acc_b[dt][r] += red[(AT_B + dt * 16 + r) * 64];
-                }
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        if constexpr (DA) acc_a[dt][r] += red[(dt * 16 + r) * 64];
+                        if constexpr (DV) acc_b[dt][r] += red[(AT_B + dt * 16 + r) * 64];
+                    }
+            }
         }
     }
     const float scale = p.c1 * 0.6931471805599453f;     // d score / d (q . k), natural units; dv has none
@@ -746,12 +757,12 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
     if constexpr (!KV) {
         // (the tiles are done with)
         if (has_bias && p.dtable != nullptr)
-            table_grad_finish(p, h, slot, reinterpret_cast<const float*>(bwd_smem + G::hist(sat)), reinterpret_cast<float*>(bwd_smem), sat, sum_lo, sum_hi);
+            table_grad_finish<G::WAVES>(p, h, slot, reinterpret_cast<const float*>(bwd_smem + G::hist(sat)), reinterpret_cast<float*>(bwd_smem), sat, sum_lo, sum_hi);
     }
 }
 
-// Whether a pass runs with SPLIT 2: own blocks of 64 instead of 128 rows, each block of scores walked by two wavefronts.
-// It halves the longest chain and doubles the workgroups, at twice the fetches per product, so it pays where 128-row
+// A pass's SPLIT.  2 (own blocks of 64 instead of 128 rows, each block of scores walked by two wavefronts) halves the longest
+// chain and doubles the workgroups, at twice the fetches per product, so it pays where 128-row
 // blocks leave the chip idle (256 compute units with room for three workgroups at head_dim 64, two at 128).  Both
 // sides, us, three kernels, bf16: head_dim 64 full attention, 256 workgroups 245 / 190 (SPLIT 1 / 2), 384 294 / 276, 512
 // 302 / 333; causal, where the longest block counts, 512 233 / 182, 1536 181 / 228; head_dim 128 256 440 / 325, 384
@@ -759,10 +770,18 @@ __global__ __launch_bounds__(kBwdThreads, D == 64 || (PASS == 3 && SPLIT == 1) ?
 // tokens of the pass's own kind): 424 67 / 73, causal 58 / 58, 564 186 / 183, 1464 212 / 222; cross-attention of 16 x 32
 // queries over 16 x 2048 keys, 12 heads, where only the key pass fills the chip: 115 us with both passes by the queries'
 // count, 94 each by its own (head_dim 128, 8 heads 175 / 135; 2048 queries over 32 keys 136 / 111).
-bool bwd16_split(const BwdParams& p, int D, bool causal, bool keys) {
+// 4 (eight wavefronts, tiles of 128) where blocks of 64 rows are one round of one workgroup per compute unit, which is what its
+// LDS allows, and with a causal mask up to one and a half.  us, SPLIT 2 / 4: 64-row blocks of unpacked tensors, head_dim 64 128 (B1 H8 L1000)
+// 46 / 39, 256 (B1 H8 L2000) 72 / 59, causal 71 / 55, 320 (B20 H8 L128) 28 / 41, causal 512 75 / 74, 864 82 / 116; head_dim 128
+// 256 122 / 111, causal 378 (B1 H6 L4000) 226 / 178, 512 139 / 137, 1024 216 / 268.
+// It needs more than one tile to walk: 8 heads of D128 B8 L47 25.9 / 31.4, B5 L128 causal 30.3 / 34.1, D64 B5 L100 20.6 / 21.0, B1 L200
+// 24.2 / 23.5, 2000 queries over 128 keys 47.6 / 37.9.
+int bwd16_split(const BwdParams& p, int D, bool causal, bool keys) {
     const int rows = keys ? p.N : p.M;
-    const int64_t blocks = p.cu_q != nullptr ? ((int64_t)(keys ? p.total_k : p.total_q) / 128 + p.B) * p.H : (int64_t)((rows + 127) / 128) * p.H * p.B;
-    return blocks < (p.cu_q != nullptr ? 320 : causal ? 768 : D == 64 ? 512 : 320);
+    const int64_t pairs = (int64_t)p.H * p.B;
+    if (p.cu_q == nullptr && (keys ? p.M : p.N) > 128 && (rows + 63) / 64 * pairs <= (causal ? 384 : 256)) return 4;
+    const int64_t blocks = p.cu_q != nullptr ? ((int64_t)(keys ? p.total_k : p.total_q) / 128 + p.B) * p.H : (rows + 127) / 128 * pairs;
+    return blocks < (p.cu_q != nullptr ? 320 : causal ? 768 : D == 64 ? 512 : 320) ? 2 : 1;
 }
 
 template <typename T, int D, bool CAUSAL, int PASS, int SPLIT>
@@ -779,19 +798,22 @@ hipError_t launch_bwd16_pass(const BwdParams& p, hipStream_t stream) {
     static LdsLimit limit;     // (per instantiation; 67 KB and more at head_dim 128 with SPLIT 2, 90.6 with the widest bucketing)
     const hipError_t e = limit.allow(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kBwdThreads), lds, stream, p, nblk);
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(G::THREADS), lds, stream, p, nblk);
     return hipGetLastError();
 }
 
 template <typename T, int D, bool CAUSAL, int PASS>
 hipError_t launch_bwd16_rows(const BwdParams& p, hipStream_t stream) {
-    return bwd16_split(p, D, CAUSAL, PASS != 0) ? launch_bwd16_pass<T, D, CAUSAL, PASS, 2>(p, stream)
-                                                            : launch_bwd16_pass<T, D, CAUSAL, PASS, 1>(p, stream);
+    const int split = bwd16_split(p, D, CAUSAL, PASS != 0);
+    // (bucketings that reach past some hundred distances leave no room for the largest tiles next to the table gradient's sums)
+    if (split == 4 && Bwd16Geom<D, PASS, 4>::bytes(p.table != nullptr ? p.bs.sat : 0, p.table != nullptr) <= 160 * 1024)
+        return launch_bwd16_pass<T, D, CAUSAL, PASS, 4>(p, stream);
+    return split > 1 ? launch_bwd16_pass<T, D, CAUSAL, PASS, 2>(p, stream) : launch_bwd16_pass<T, D, CAUSAL, PASS, 1>(p, stream);
 }
 
 template <typename T, int D, bool CAUSAL>
 hipError_t launch_bwd16(BwdParams p, hipStream_t stream) {
-    p.slots_per_head = p.B * (bwd16_split(p, D, CAUSAL, false) ? (p.M + 63) / 64 : (p.M + 127) / 128);
+    p.slots_per_head = p.B * (bwd16_split(p, D, CAUSAL, false) > 1 ? (p.M + 63) / 64 : (p.M + 127) / 128);
     if (p.N <= 0) p.slots = nullptr;      // (no pass that would add them)
     hipError_t e = launch_bwd16_rows<T, D, CAUSAL, 0>(p, stream);
     if (e != hipSuccess) return e;

@@ -44,8 +44,8 @@ template <int SPLIT> struct Geom {
     static __host__ __device__ int lut_floats(int sat) { return (2 * (sat + kPad) + 4) & ~3; }
     static __host__ __device__ int hist(int sat) { return LUT + 4 * lut_floats(sat); }
     static constexpr int SKEW_ROWS = SPLIT == 2 ? 32 : 16;       // queries per round of the table gradient (two workgroups share the LDS with SPLIT 1)
-    static __host__ __device__ int skew(int sat) { return hist(sat) + 4 * kTableGradWaves * table_grad_floats(sat); }
-    static __host__ __device__ int bytes(int sat, bool table_grad) { return table_grad ? skew(sat) + kTableGradWaves * SKEW_ROWS * 64 * 4 : hist(sat); }
+    static __host__ __device__ int skew(int sat) { return hist(sat) + 4 * 4 * table_grad_floats(sat); }
+    static __host__ __device__ int bytes(int sat, bool table_grad) { return table_grad ? skew(sat) + 4 * SKEW_ROWS * 64 * 4 : hist(sat); }
 };
 
 // the tiles of the two tensors of the other kind
@@ -252,7 +252,7 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     const int64_t slot = ((int64_t)h * p.B + b) * nblk + own_block;     // (of the table gradient)
     if constexpr (KV && !RAW) {
         // (the last block: the shortest of a causal launch)
-        if (p.slots != nullptr && p.table != nullptr && own_block == nblk - 1 && b == 0) table_grad_reduce(p, h, reinterpret_cast<float*>(smem));
+        if (p.slots != nullptr && p.table != nullptr && own_block == nblk - 1 && b == 0) table_grad_reduce<4>(p, h, reinterpret_cast<float*>(smem));
     }
     int M = p.M, N = p.N;
     int64_t q_first = 0, k_first = 0;
@@ -261,7 +261,7 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
         M = p.len_q != nullptr ? p.len_q[b] : p.cu_q[b + 1] - (int)q_first;
         N = p.len_k != nullptr ? p.len_k[b] : p.cu_k[b + 1] - (int)k_first;
         if (own_base >= (KV ? N : M)) {     // (the grid is sized for the longest sequence)
-            if constexpr (!KV) table_grad_none(p, slot);
+            if constexpr (!KV) table_grad_none<4>(p, slot);
             return false;
         }
     }
@@ -458,7 +458,7 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     if constexpr (!KV) {
         // (the tiles are done with)
         if (has_bias && p.dtable != nullptr)
-            table_grad_finish(p, h, slot, reinterpret_cast<const float*>(smem + G::hist(sat)), reinterpret_cast<float*>(smem), sat, sum_lo, sum_hi);
+            table_grad_finish<4>(p, h, slot, reinterpret_cast<const float*>(smem + G::hist(sat)), reinterpret_cast<float*>(smem), sat, sum_lo, sum_hi);
     }
     return false;
 }

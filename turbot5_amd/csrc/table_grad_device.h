@@ -1,6 +1,6 @@
 // The bias table's gradient in a backward pass over query rows: dS summed per distance, distances summed per bucket.
 //
-// A wavefront keeps sums of its own for the distances below saturation in LDS and in two registers for the rest; the four
+// A wavefront keeps sums of its own for the distances below saturation in LDS and in two registers for the rest; the
 // wavefronts' sums meet once, at the end.  A workgroup's buckets then go to a slot of the workspace, and the pass over the keys, which
 // follows in the stream, adds the slots of a head in a fixed order.  Atomics, on LDS per distance and on the table per bucket and
 // workgroup, are what this avoids; all workgroups of a head met at the same 32 addresses.  us, the backward's kernels with
@@ -12,7 +12,6 @@
 
 namespace t5a {
 
-constexpr int kTableGradWaves = 4;
 // floats of a wavefront's sums, index distance + sat
 __host__ __device__ inline int table_grad_floats(int sat) { return (2 * sat + 4) & ~3; }
 
@@ -49,7 +48,8 @@ __device__ __forceinline__ void table_grad_block(float* skew, float* sums, const
 }
 
 // All threads: the wavefronts' sums into the workgroup's slot, or without slots into the head's column of the table's gradient.
-// `scratch`: 2 x kTableGradWaves floats.  Eight lanes share a bucket, whose distances are one run on one side of the diagonal.
+// `scratch`: 2 WAVES floats.  Eight lanes share a bucket, whose distances are one run on one side of the diagonal.
+template <int WAVES>
 __device__ __forceinline__ void table_grad_finish(const BwdParams& p, int h, int64_t slot, const float* sums, float* scratch, int sat, float lo, float hi) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, stride = table_grad_floats(sat);
     const BucketSpec& bs = p.bs;
@@ -63,7 +63,7 @@ __device__ __forceinline__ void table_grad_finish(const BwdParams& p, int h, int
     __syncthreads();
     const int last_lo = bucket_of(bs, -sat), last_hi = bucket_of(bs, sat);
     const int sub = tid & 7;
-    for (int b0 = 0; b0 < p.n_buckets; b0 += 32) {      // (uniform: the exchange below needs every lane)
+    for (int b0 = 0; b0 < p.n_buckets; b0 += 8 * WAVES) {      // (uniform: the exchange below needs every lane)
         const int b = b0 + (tid >> 3);
         const bool up = bs.bidirectional && b >= bs.nb;
         const int k = up ? b - bs.nb : b, t = k - bs.max_exact;
@@ -75,14 +75,14 @@ __device__ __forceinline__ void table_grad_finish(const BwdParams& p, int h, int
                 if (!up || d > 0) {
                     const float* at = sums + (up ? d : -d) + sat;
 #pragma unroll
-                    for (int w = 0; w < kTableGradWaves; ++w) s += at[w * stride];
+                    for (int w = 0; w < WAVES; ++w) s += at[w * stride];
                 }
         }
 #pragma unroll
         for (int off = 1; off < 8; off <<= 1) s += __shfl_xor(s, off, 64);
         if (sub == 0 && b < p.n_buckets) {
 #pragma unroll
-            for (int w = 0; w < kTableGradWaves; ++w) {
+            for (int w = 0; w < WAVES; ++w) {
                 if (b == last_lo) s += scratch[2 * w];
                 if (b == last_hi) s += scratch[2 * w + 1];
             }
@@ -93,15 +93,17 @@ __device__ __forceinline__ void table_grad_finish(const BwdParams& p, int h, int
 }
 
 // A workgroup without rows: its slot is zero.
+template <int WAVES>
 __device__ __forceinline__ void table_grad_none(const BwdParams& p, int64_t slot) {
     if (p.slots == nullptr || p.table == nullptr || p.dtable == nullptr) return;
-    for (int b = threadIdx.x; b < p.n_buckets; b += 64 * kTableGradWaves) p.slots[slot * p.n_buckets + b] = 0.f;
+    for (int b = threadIdx.x; b < p.n_buckets; b += 64 * WAVES) p.slots[slot * p.n_buckets + b] = 0.f;
 }
 
 // All threads of one workgroup of the pass over the keys: the slots of a head, into its column of the table's gradient.
-// `scratch`: 64 x kTableGradWaves floats, free on return.
+// `scratch`: 64 WAVES floats, free on return.
+template <int WAVES>
 __device__ __forceinline__ void table_grad_reduce(const BwdParams& p, int h, float* scratch) {
-    const int tid = threadIdx.x, shift = p.n_buckets <= 32 ? 5 : 6, b = tid & ((1 << shift) - 1), parts = 64 * kTableGradWaves >> shift;
+    const int tid = threadIdx.x, shift = p.n_buckets <= 32 ? 5 : 6, b = tid & ((1 << shift) - 1), parts = 64 * WAVES >> shift;
     const float* const from = p.slots + (int64_t)h * p.slots_per_head * p.n_buckets + b;
     float s = 0.f;
     if (b < p.n_buckets) {

@@ -795,7 +795,7 @@ hipError_t launch_bwd16_pass(const BwdParams& p, hipStream_t stream) {
     const bool bias = p.table != nullptr;
     const int lds = G::bytes(bias ? p.bs.sat : 0, bias);
     auto kern = bwd16_kernel<T, D, CAUSAL, PASS, SPLIT>;
-    static LdsLimit limit;     // (per instantiation; 67 KB and more at head_dim 128 with SPLIT 2, 90.6 with the widest bucketing)
+    static LdsLimit limit;     // (per instantiation; 67 KB and more at head_dim 128 with SPLIT 2, 90.6 with the widest bucketing, SPLIT 4 up to 160)
     const hipError_t e = limit.allow(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(G::THREADS), lds, stream, p, nblk);

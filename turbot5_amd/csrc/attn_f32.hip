@@ -65,7 +65,7 @@ template <int SPLIT, bool RAW> struct Tiles {
 #pragma unroll
             for (int n = 0; n < G::PASSES; ++n) {
                 const int row = t * G::OTHER + row0 + 32 * n;
-                const int off = row < rows ? row * stride[e] + ch * 32 : 0x7ffffff0;     // (zeros past the end)
+                const int off = row < rows ? row * stride[e] + ch * 32 : 0x7fffffe0;     // (zeros past the end)
                 u32x4* const d = reinterpret_cast<u32x4*>(&x[e][n]);
                 d[0] = __builtin_amdgcn_raw_buffer_load_b128(rs[e], off, 0, 0);
                 d[1] = __builtin_amdgcn_raw_buffer_load_b128(rs[e], off + 16, 0, 0);

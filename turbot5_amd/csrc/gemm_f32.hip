@@ -3,6 +3,7 @@
 // matrix products in bf16 at 990 TFLOP/s, as fast as the card runs any), below that the latency of a workgroup's steps.
 #include <type_traits>
 
+#include "gemm_offsets.h"
 #include "split_device.h"
 #include "t5a_internal.h"
 
@@ -14,7 +15,7 @@ typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
-constexpr int BK = 32;          // depth of a staged tile
+constexpr int BK = kGemmStep;   // depth of a staged tile
 
 // An operand's tile in LDS: planes of bf16.  ROWS values along the output dimension, BK along the contraction.
 // COL false: the matrix is (rows, contraction) with the contraction contiguous; the plane holds rows of 64 bytes, four chunks of
@@ -38,30 +39,32 @@ struct Operand {
     }
 
     // A lane's pieces of a tile, eight values each.  Read through a buffer descriptor, whose scalar offset advances with the
-    // contraction; what lies past the contraction's end is asked for out of the descriptor's range and arrives as zero.
+    // contraction; what lies past the contraction's end is asked for out of the descriptor's range and arrives as zero
+    // (gemm_offsets.h).
     struct Tile { v8 x[PASSES]; };
     __amdgpu_buffer_rsrc_t rs;
     int at[PASSES], k[PASSES], step;
     __device__ __forceinline__ void start(const T* p, int64_t ld, int base, int rows, int K, int tid) {
-        rs = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(((COL ? K : rows) - 1) * ld + (COL ? rows : K)) * (int)sizeof(T), 0x00020000);
-        step = BK * (int)sizeof(T) * (COL ? (int)ld : 1);
+        rs = __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, operand_bytes(COL ? K : rows, COL ? rows : K, ld, (int)sizeof(T)), 0x00020000);
+        step = step_bytes(K, COL ? ld : 1, (int)sizeof(T));
 #pragma unroll
         for (int n = 0; n < PASSES; ++n) {
             const int c = tid + n * kThreads;
             // (rows past the end: the last ones again; their results are not stored)
             const int row = COL ? min(base + (c % CPR) * 8, rows - 8) : min(base + (c >> 2), rows - 1);
             k[n] = COL ? c / CPR : (c & 3) * 8;
-            at[n] = (COL ? k[n] * (int)ld + row : row * (int)ld + k[n]) * (int)sizeof(T);
+            at[n] = (COL ? min(k[n], K - 1) * (int)ld + row : row * (int)ld + k[n]) * (int)sizeof(T);
         }
     }
     // step kk of the contraction, of which K - kk BK indices are left
     __device__ __forceinline__ void fetch(Tile& t, int kk, int K) const {
+        const int from = step_offset(kk, K, step);
 #pragma unroll
         for (int n = 0; n < PASSES; ++n) {
-            const int off = k[n] < K - kk * BK ? at[n] : 0x7ffffff0;
+            const int off = lane_offset(k[n], kk, K, at[n]);
             u32x4* const d = reinterpret_cast<u32x4*>(&t.x[n]);
 #pragma unroll
-            for (int e = 0; e < (int)sizeof(v8) / 16; ++e) d[e] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * e, kk * step, 0);
+            for (int e = 0; e < (int)sizeof(v8) / 16; ++e) d[e] = __builtin_amdgcn_raw_buffer_load_b128(rs, off + 16 * e, from, 0);
         }
     }
     static __device__ __forceinline__ void store(const Tile& t, __bf16* plane, int tid) {

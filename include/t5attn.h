@@ -439,8 +439,9 @@ int t5a_rmsnorm_train(const t5a_rmsnorm_train_args* args, t5a_stream_t stream);
 
 /*
  * c = a b of fp32 matrices (a linear layer of a training step and its gradients): fp32 sums of products formed on the bf16
- * matrix cores from operands split into three bf16 parts, which carry all 24 bits; results are as accurate as fp32 products
- * added in fp32.  The reference leaves its linear layers to torch (src/turbot5/model/attentions.py:59-62).
+ * matrix cores from operands split into three bf16 parts, which carry all bits of every finite value, denormal ones too; results are as
+ * accurate as fp32 products added in fp32.  Where an operand's magnitude is 2^112 or more, or a sum's 2^96, the products are
+ * formed on the fp32 matrix cores (a slower path of the same call).  The reference leaves its linear layers to torch (src/turbot5/model/attentions.py:59-62).
  * Group g multiplies a[g] (M, K) and b[g] (N, K) over K; trans: the matrix lies in memory as (K, M) / (K, N).  Rows lda / ldb /
  * ldc elements apart, contiguous inside.  sum_groups 0: c[g] = the product of group g; 1: c[0] = the sum over the groups.
  * alpha: a factor of group 0's product.  relu: negative results become 0.  positive (optional, (M, N) fp32, rows ld_positive

@@ -116,6 +116,26 @@ def test_small_magnitudes_keep_their_bits(gpu_device, scale):
     assert (out.double() - want).norm() <= 1e-6 * want.norm()
 
 
+# results from 2^-70 to 2^-125; operands with bf16 parts below the smallest such number, the last two denormal themselves
+@pytest.mark.parametrize("form", ["nn", "nt", "tt"])
+@pytest.mark.parametrize("small,large", [(2.0 ** -112, 2.0 ** 20), (2.0 ** -118, 2.0 ** 48), (2.0 ** -124, 2.0 ** 30), (2.0 ** -124, 2.0 ** 100),
+                                         (2.0 ** -134, 2.0 ** 60), (2.0 ** -146, 2.0 ** 21)])
+def test_small_operands_against_large_ones(gpu_device, form, small, large):
+    """Numbers of which an unscaled bf16 part would lose bits, in products that are no small numbers, on either side."""
+    from turbot5_amd.linear import _gemm
+    g = torch.Generator(device=gpu_device).manual_seed(12)
+    M, N, K = 136, 72, 520
+    a, b = _rand(g, M, K) * small, _rand(g, N, K) * large
+    a[5], b[9, 3] = 0.0, 0.0
+    for x, y in ((a, b), (b, a)):
+        out = torch.full((x.shape[0], y.shape[0]), 7.0, device=gpu_device)
+        _gemm([x.t().contiguous() if form[0] == "t" else x], [y.t().contiguous() if form[1] == "t" else y], [out],
+              a_trans=form[0] == "t", b_trans=form[1] == "t")
+        X, Y = x.double(), y.double()
+        # (a step of the denormal numbers for each of the sums)
+        assert ((out.double() - X @ Y.t()).abs() <= _bound(X, Y, K) + K * 2.0 ** -149).all()
+
+
 def _layers(g, dev, n, d_in, d_out):
     out = []
     for _ in range(n):

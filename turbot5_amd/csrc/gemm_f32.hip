@@ -1,6 +1,10 @@
 // Products of fp32 matrices on the 16-bit matrix cores: the linear layers of a training step with fp32 weights and their
-// gradients.  What bounds them: at thousands of rows the matrix cores at the power the card allows (8192 x 2048 x 512: 104 us, 6
-// matrix products in bf16 at 990 TFLOP/s, as fast as the card runs any), below that the latency of a workgroup's steps.
+// gradients.  What bounds them: at thousands of rows the matrix cores and, next to them, the vector instructions that split the
+// operands, some 160 of a thread beside 24 products per step of the larger tile (8192 x 2048 x 512: 112 us, 6 matrix products in
+// bf16 at 920 TFLOP/s; a library product in bf16 reaches 1214), below that the latency of a workgroup's steps.
+// The factor 2^16 on the operands (split_device.h), one of those instructions per value, takes 1 to 3 %: 65.3 / 67.1 us without / with it at 4500 x 2048 x 512,
+// 108 / 112 at 8192 x 2048 x 512.  A test for lost bits in its place, half an instruction per value, with the scaled products
+// as its way out: 66.5 and 110, a training step of the T5-small encoder the same, for a second copy of the loop.
 #include <type_traits>
 
 #include "gemm_offsets.h"
@@ -76,7 +80,7 @@ struct Operand {
             else { const int row = plane_row(c / CPR); to = row * ROWS + ((c % CPR) ^ swz(row)) * 8; }
             if constexpr (NP == 3) {
                 bf16x8 s[3];
-                split3(t.x[n], s);
+                split3(t.x[n] * kSplitScale, s);
 #pragma unroll
                 for (int q = 0; q < 3; ++q) *reinterpret_cast<bf16x8*>(plane + q * PLANE + to) = s[q];
             } else {
@@ -149,8 +153,8 @@ template <typename Fn> __device__ __forceinline__ void with_finish(const GemmPar
 // A workgroup of 2 x 2 wavefronts forms BM x 64 results in steps of 32 of the contraction: the step's products on one LDS
 // buffer while the next step's values, fetched DEPTH steps ahead into registers, are split into the other.  With tens of steps
 // per workgroup the latency of a step counts as much as its products: one barrier per step, and more steps ahead for the smaller
-// tile.  4500 x 2048 x 512: 64 us = 147 TFLOP/s in fp32 terms, 880 on the bf16 matrix cores (a single buffer and two
-// barriers 71; the fp32 library product 87); 1000 x 512 x 2048 25 us in four splits.
+// tile.  4500 x 2048 x 512: 67 us = 141 TFLOP/s in fp32 terms, 845 on the bf16 matrix cores (before the operands were scaled 65, with
+// a single buffer and two barriers 71; the fp32 library product 87); 1000 x 512 x 2048 25 us in four splits.
 template <typename TA, typename TB, bool ACOL, bool BCOL, int BM>
 __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 3) void gemm_kernel(const GemmParams p) {
     constexpr int BN = 64, DEPTH = BM == 128 ? 2 : 4;
@@ -244,16 +248,10 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 3) void gemm_kernel(const
         it += n;
     }
 
-    // A sum that is not finite, or is so small that the parts of what it was made from may have lost bits (split_device.h): the
-    // products again on the fp32 matrix cores, straight from memory.
+    // A sum that is not finite (split_device.h): the products again on the fp32 matrix cores, straight from memory.
     float odd = 0.f;                     // NaN if any is not finite
-    unsigned least = 0xffffffffu;        // smallest magnitude but zero: twice the bits, less one
-    each([&](float x) {
-        odd += x * 0.f;
-        least = min(least, (__builtin_bit_cast(unsigned, x) << 1) - 1u);
-        return x;
-    });
-    if (__any(odd != odd || least < 2u * __builtin_bit_cast(unsigned, 0x1p-104f))) {
+    each([&](float x) { odd += x * 0.f; return x; });
+    if (__any(odd != odd)) {
         each([](float) { return 0.f; });
         for (int it = it0; it < it_end; ++it) {
             const int g = it / p.steps, kk = it - g * p.steps;
@@ -273,6 +271,9 @@ __global__ __launch_bounds__(kThreads, BM == 128 ? 2 : 3) void gemm_kernel(const
             }
             if (p.groups_k > 1 && g == 0 && (kk + 1 == p.steps || it + 1 == it_end)) each([&](float x) { return x * p.alpha; });
         }
+    } else {
+        constexpr float back = (OA::NP == 3 ? kSplitBack : 1.f) * (OB::NP == 3 ? kSplitBack : 1.f);
+        each([](float x) { return x * back; });
     }
 
     // lane (lr, hh): row lr of the block, columns 8 (r >> 2) + 4 hh + (r & 3)

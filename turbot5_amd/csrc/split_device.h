@@ -5,11 +5,14 @@
 // left out are at most 2^-24 of the product.  v_mfma_f32_32x32x16_bf16 does sixteen times the multiply-adds of
 // v_mfma_f32_32x32x2_f32 per cycle, so six of them take 3/8 of the time.
 //
-// (A part holds multiples of 2^-133: values below 2^-110 keep fewer bits, to an absolute error of 2^-134.)
+// A part holds multiples of 2^-133 and an fp32 number is one of 2^-149, so kernels split x times kSplitScale = 2^16: its parts
+// are exact for every x down to the smallest denormal one (unscaled, numbers below 2^-110 lose bits: 2^-17 of themselves at
+// 2^-117).  The scales of a product's operands are taken out of its fp32 sum, exactly.
 //
-// An infinity, or a value that rounds to one in bf16, gives infinity minus infinity in m and l: what fp32 arithmetic would
-// leave finite or infinite may come out as NaN.  Every such case leaves a value in the result that is not finite (h takes part
-// in a product of its own), which is what the kernels test before they store, to form the result again in fp32.
+// An infinity, or a value that times 2^16 rounds to one in bf16 (2^112 and more), gives infinity minus infinity in m and l: what fp32
+// arithmetic would leave finite or infinite may come out as NaN, and so may a scaled sum past the largest number.  Every such
+// case leaves a value in the result that is not finite (h takes part in a product of its own), which is what the kernels test
+// before they store, to form the result again in fp32.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -20,6 +23,7 @@ namespace t5a {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kPlanes = 3;
+constexpr float kSplitScale = 0x1p16f, kSplitBack = 0x1p-16f;
 
 // (two values at a time: a packed pair is widened with a shift and a mask)
 __device__ __forceinline__ void split3(const f32x8 x, bf16x8 (&out)[kPlanes]) {

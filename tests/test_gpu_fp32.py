@@ -96,6 +96,61 @@ def test_values_that_have_no_bf16_parts(gpu_device, B):
             assert (out[before] - clean[before]).norm() <= 2e-6 * clean[before].norm()
 
 
+# operands of which unscaled bf16 parts would lose bits: all of v (down to denormal ones), of dout, of k or of q, a factor of the scores, and products
+# of dout and v that leave no room for a factor
+@pytest.mark.parametrize("B,causal", [(1, False), (40, True)])
+@pytest.mark.parametrize("small,by", [("v", 2.0 ** -112), ("v", 2.0 ** -124), ("v", 2.0 ** -138), ("d", 2.0 ** -112), ("d", 2.0 ** -124), ("k", 2.0 ** -112),
+                                      ("k", 2.0 ** -124), ("q", 2.0 ** -124), ("s", 2.0 ** -100), ("vd", 2.0 ** 50)])
+def test_small_operands_keep_their_bits(gpu_device, B, causal, small, by):
+    import turbot5_amd as t5
+    H, L = 8, 130
+    g = torch.Generator().manual_seed(B + len(small))
+    q, k, v, d = (0.5 * torch.randn(B, H, L, 64, generator=g) for _ in range(4))
+    table = torch.randn(32, H, generator=g)
+    scale = 1.0
+    if small == "v":
+        v *= by
+    elif small == "d":
+        d *= by
+    elif small == "vd":
+        v, d = v * by, d * by
+    elif small == "k":
+        k *= by
+    elif small == "q":
+        q *= by
+    else:
+        scale, q, k = by, q * 2.0 ** 60, k * 2.0 ** 40
+    ins = [t.to(gpu_device).requires_grad_() for t in (q, k, v, table)]
+    o = t5.flash_attention_with_fusing_bias(*ins, causal=causal, sm_scale=scale)
+    got = [o, *torch.autograd.grad(o, ins, d.to(gpu_device))]
+    # relative as in the test of ordinary sizes (a gradient's terms cancel to a few per cent of their size); half a step of the denormal numbers for each
+    # term of a sum, and a result that is rounded to one
+    for t, r, tol in zip(got, _exact(*ins, causal, scale, d), (2e-6, 7e-6, 7e-6, 7e-6, 7e-6)):
+        assert (t.double().cpu() - r).norm() <= tol * r.norm() + L * 2.0 ** -149 * r.numel() ** 0.5, small
+
+
+@pytest.mark.parametrize("B", [1, 48])
+def test_scores_of_the_smallest_and_the_largest_numbers(gpu_device, B):
+    """Scores of some 6 to 13 from numbers of 2e-38 and 3.3e38 (finite in bf16)."""
+    import turbot5_amd as t5
+    H, L = 8, 96
+    g = torch.Generator().manual_seed(7)
+    q, k, v, d = (0.5 * torch.randn(B, H, L, 64, generator=g) for _ in range(4))
+    table = torch.randn(32, H, generator=g)
+    q[..., 0] = 2e-38 * (1.0 + torch.rand(B, H, L, generator=g))
+    k[:, :, 5, 0] = 3.3e38
+    d *= 0.1                       # (dq holds a tenth of the largest number)
+    ins = [t.to(gpu_device).requires_grad_() for t in (q, k, v, table)]
+    o = t5.flash_attention_with_fusing_bias(*ins, causal=False, sm_scale=1.0)
+    got = [o, *torch.autograd.grad(o, ins, d.to(gpu_device))]
+    # (the first column of dq and dk is far from the others.  Scores that reach 15 carry the roundings of their sums into probabilities: 1e-5
+    # to 6e-5 of a head's largest value; scores off by 5e-3, as lost bits make them, are above)
+    for i, (t, r) in enumerate(zip(got, _exact(*ins, False, 1.0, d))):
+        for columns in (slice(0, 1), slice(1, None)) if i in (1, 2) else (slice(None),):
+            a, b = t.double().cpu()[..., columns], r[..., columns]
+            assert ((a - b).abs() <= 1e-4 * b.abs().amax(dim=(-2, -1), keepdim=True) + L * 2.0 ** -149).all()
+
+
 def test_lut_of_a_table_is_not_marked_built_by_an_fp32_call(gpu_device):
     """The fp32 kernel reads no distance image: a 16-bit call with the same table builds its own."""
     import turbot5_amd as t5

@@ -15,8 +15,14 @@
 // kernels: B4 H8 L512 47 / 26 and 127 / 77, B2 H6 L1999 causal 155 / 74 and 552 / 196, B8 H12 L1024 222 / 141 and 920 / 540, B3 H16
 // L2000 424 / 262 and 1715 / 980.  Errors against 64 bits are smaller: 4.2e-7 for 6.1e-7 (o, B4 H8 L512), 8e-7 for 1.05e-6 (dq, dk, dv).
 //
-// Results that are not finite are formed again by the same workgroup on the fp32 matrix cores (RAW): the parts of an infinity,
-// or of a value close to the largest, are no numbers.
+// What is split is scaled (split_device.h), by exact powers of two that leave the sums again: a tile's rows and the probabilities by 2^16; own
+// rows of a score's product by 2^-16, so that scores carry no factor and nothing is paid per score; own rows of dP's by 2^16, whose 2^32
+// then stays on dS.  Without / with the scales, us, forward and backward (three kernels): B4 H8 L512 24.4 / 24.9 and 69 / 73,
+// B2 H6 L1999 causal 67 / 62 (the bias is at hand ahead of the tile now) and 189 / 199, B8 H12 L1024 141 / 145 and 543 / 560.
+// Scores scaled like dP, with 2^-32 in the factor of their bias's sum: the same times, and errors of o 5 % larger.
+//
+// Results that are not finite, and rows whose own values below 2^-94 the factor 2^-16 would take out of reach, are formed
+// again by the same workgroup on the fp32 matrix cores (RAW): the parts of an infinity, or of a value close to the largest, are no numbers.
 #include "split_device.h"
 #include "t5a_internal.h"
 #include "table_grad_device.h"
@@ -46,6 +52,12 @@ template <int SPLIT> struct Geom {
     static constexpr int SKEW_ROWS = SPLIT == 2 ? 32 : 16;       // queries per round of the table gradient (two workgroups share the LDS with SPLIT 1)
     static __host__ __device__ int skew(int sat) { return hist(sat) + 4 * 4 * table_grad_floats(sat); }
     static __host__ __device__ int bytes(int sat, bool table_grad) { return table_grad ? skew(sat) + 4 * SKEW_ROWS * 64 * 4 : hist(sat); }
+};
+
+// dP and dS carry `ds`; the sums of P or dS times rows are multiplied by back_b and back_a
+template <bool RAW> struct Scale {
+    static constexpr float up = RAW ? 1.f : kSplitScale, down = RAW ? 1.f : kSplitBack;
+    static constexpr float ds = up * up, ds_back = down * down, back_a = ds_back * down, back_b = ds_back;
 };
 
 // the tiles of the two tensors of the other kind
@@ -84,7 +96,7 @@ template <int SPLIT, bool RAW> struct Tiles {
                 } else {
                     __bf16* const to = reinterpret_cast<__bf16*>(buf + e * G::TENSOR) + row * HD + (ch ^ tile_swz(row)) * 8;
                     bf16x8 s[kPlanes];
-                    split3(x[e][n], s);
+                    split3(x[e][n] * kSplitScale, s);
 #pragma unroll
                     for (int q = 0; q < kPlanes; ++q) *reinterpret_cast<bf16x8*>(to + q * G::PLANE) = s[q];
                 }
@@ -96,22 +108,30 @@ template <int SPLIT, bool RAW> struct Tiles {
 template <int SPLIT, bool RAW> struct Own;
 template <int SPLIT> struct Own<SPLIT, false> {
     bf16x8 f[KS][kPlanes];
-    __device__ __forceinline__ void load(const float* row, bool ok, int hh, float factor) {
+    // rows times factor, held times `scale`; the smallest magnitude but zero
+    __device__ __forceinline__ unsigned load(const float* row, bool ok, int hh, float factor, float scale) {
+        unsigned least = 0xffffffffu;        // twice a magnitude's bits, less one
 #pragma unroll
         for (int s = 0; s < KS; ++s) {
             f32x8 x = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
             if (ok) x = *reinterpret_cast<const f32x8*>(row + 16 * s + 8 * hh);
-            split3(x * factor, f[s]);
+            x *= factor;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) least = min(least, (__builtin_bit_cast(unsigned, (float)x[e]) << 1) - 1u);
+            split3(x * scale, f[s]);
         }
+        return least;
     }
 };
 template <int SPLIT> struct Own<SPLIT, true> {
     float f[HD / 2];
-    __device__ __forceinline__ void load(const float* row, bool ok, int hh, float factor) {
+    __device__ __forceinline__ unsigned load(const float* row, bool ok, int hh, float factor, float) {
 #pragma unroll
         for (int s = 0; s < HD / 2; ++s) f[s] = ok ? row[2 * s + hh] * factor : 0.f;
+        return 0xffffffffu;
     }
 };
+constexpr unsigned kTiny = 2u * 0x10800000u;      // 2^-94 as `least` counts
 
 // lane constants of the tile reads of a block whose first tile row is sub0
 template <int SPLIT, bool RAW> struct Reads;
@@ -265,6 +285,7 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
             return false;
         }
     }
+    using X = Scale<RAW>;
     const int n_own = KV ? N : M, n_other = KV ? M : N, P = N - M;
     const bool has_bias = p.table != nullptr;
     const int sat = has_bias ? p.bs.sat : 0;
@@ -301,15 +322,15 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     };
     auto store = [&](int buf) {
         tiles.store(smem + buf * G::BUF);
-        if (KV && tid < 2 * OTHER) stats[buf * 2 * OTHER + tid] = stat;
+        if (KV && tid < 2 * OTHER) stats[buf * 2 * OTHER + tid] = tid < OTHER ? stat : stat * X::ds;
     };
     const BiasColumn bias(p, h, lane);
     if (t_lo < t_hi) fetch(t_lo);
 
     const bool own_ok = own_row < n_own;
     Own<SPLIT, RAW> fa, fb;
-    fa.load(KV ? kp + (int64_t)own_row * p.k_sr : qp + (int64_t)own_row * p.q_sr, own_ok, hh, 1.f);
-    fb.load(KV ? vp + (int64_t)own_row * p.v_sr : gp + (int64_t)own_row * p.do_sr, own_ok, hh, 1.f);
+    unsigned least = fa.load(KV ? kp + (int64_t)own_row * p.k_sr : qp + (int64_t)own_row * p.q_sr, own_ok, hh, 1.f, X::down);
+    fb.load(KV ? vp + (int64_t)own_row * p.v_sr : gp + (int64_t)own_row * p.do_sr, own_ok, hh, 1.f, X::up);
     float nlse2_own = -INFINITY, ndelta_own = 0.f;      // (rows past the end: every probability is 0)
     if (!KV && own_ok) { nlse2_own = p.lse2[stat_base + own_row * stat_sr]; ndelta_own = p.delta[stat_base + own_row * stat_sr]; }
 
@@ -329,6 +350,8 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     const float c1 = p.c1;
 
     if (t_lo < t_hi) { store(0); fetch(t_lo + 1); }
+    asm volatile("" : "+v"(least));      // (formed here and not at the end, which would keep the rows in registers)
+    ndelta_own *= X::ds;                 // (here and not where it is asked for, which would wait for it)
     for (int t = t_lo; t < t_hi; ++t) {
         const int buf = (t - t_lo) & 1;
         __syncthreads();      // tile t is written (and the LUT), the other buffer read
@@ -394,7 +417,10 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
                 dp[r] = pair ? dp[r] * pv : 0.f;
                 s[r] = pv;
             }
-            if constexpr (KV) reads.over_rows(tb, s, acc_b);
+            if constexpr (KV) {
+                if constexpr (!RAW) s *= X::up;
+                reads.over_rows(tb, s, acc_b);
+            }
             reads.over_rows(ta, dp, acc_a);
             if constexpr (!KV) {
                 if (has_bias) {
@@ -437,7 +463,11 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
     if constexpr (!RAW) {
         float x = odd(acc_a);
         if constexpr (KV) x += odd(acc_b);
-        if (anybody(flag, x != x)) return true;
+        else if (has_bias) {
+            x += (sum_lo + sum_hi) * 0.f;
+            for (int y = lane; y <= 2 * sat; y += 64) x += dist[y] * 0.f;
+        }
+        if (anybody(flag, least < kTiny || x != x)) return true;
     }
     const float scale = p.c1 * 0.6931471805599453f;     // d score / d (q . k), natural units; dv has none
     if (own_ok && sub0 == 0) {
@@ -449,16 +479,15 @@ __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigne
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int d0 = 32 * dt + 8 * g + 4 * hh;
-                *reinterpret_cast<f32x4*>(oa + d0) = f32x4{acc_a[dt][4 * g] * scale, acc_a[dt][4 * g + 1] * scale,
-                                                          acc_a[dt][4 * g + 2] * scale, acc_a[dt][4 * g + 3] * scale};
-                if constexpr (KV)
-                    *reinterpret_cast<f32x4*>(ob + d0) = f32x4{acc_b[dt][4 * g], acc_b[dt][4 * g + 1], acc_b[dt][4 * g + 2], acc_b[dt][4 * g + 3]};
+                auto four = [&](const f32x16& acc) { return f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]}; };
+                *reinterpret_cast<f32x4*>(oa + d0) = four(acc_a[dt]) * X::back_a * scale;
+                if constexpr (KV) *reinterpret_cast<f32x4*>(ob + d0) = four(acc_b[dt]) * X::back_b;
             }
     }
     if constexpr (!KV) {
         // (the tiles are done with)
         if (has_bias && p.dtable != nullptr)
-            table_grad_finish<4>(p, h, slot, reinterpret_cast<const float*>(smem + G::hist(sat)), reinterpret_cast<float*>(smem), sat, sum_lo, sum_hi);
+            table_grad_finish<4>(p, h, slot, reinterpret_cast<const float*>(smem + G::hist(sat)), reinterpret_cast<float*>(smem), sat, sum_lo, sum_hi, X::ds_back);
     }
     return false;
 }
@@ -482,6 +511,7 @@ __device__ __forceinline__ bool fwd32_body(const FwdParams& p, int nblk, unsigne
     int own_block, h, b;
     bwd_place<CAUSAL, false>(p.H, p.B, nblk, own_block, h, b);
     const int own_base = own_block * G::OWN, w_lo = own_base + ow * 32, own_row = w_lo + lr;
+    using X = Scale<RAW>;
     const int M = p.M, N = p.N, P = N - M;
     const bool has_bias = p.table != nullptr;
     const int sat = has_bias ? p.bs.sat : 0;
@@ -496,7 +526,7 @@ __device__ __forceinline__ bool fwd32_body(const FwdParams& p, int nblk, unsigne
     if (t_hi > 0) tiles.fetch(0);
     const bool own_ok = own_row < M;
     Own<SPLIT, RAW> own;
-    own.load(slice(p.q, p.q_sb, p.q_sh) + (int64_t)own_row * p.q_sr, own_ok, hh, p.c1);
+    unsigned least = own.load(slice(p.q, p.q_sb, p.q_sh) + (int64_t)own_row * p.q_sr, own_ok, hh, p.c1, X::down);
     fill_bias<false>(bias, lut, sat, tid);
     const float bias_lo = has_bias ? bias.at(-sat) : 0.f, bias_hi = has_bias ? bias.at(sat) : 0.f;
     const Reads<SPLIT, RAW> reads(sub0, lane);
@@ -505,19 +535,18 @@ __device__ __forceinline__ bool fwd32_body(const FwdParams& p, int nblk, unsigne
     float top = -INFINITY, sum = 0.f;     // running maximum of the row (base-2 units), this lane's share of the sum
 
     if (t_hi > 0) { tiles.store(smem); tiles.fetch(1); }
+    asm volatile("" : "+v"(least));
+    __syncthreads();      // (the LUT is written)
     for (int t = 0; t < t_hi; ++t) {
-        __syncthreads();
         const unsigned char* const tk = smem + (t & 1) * G::BUF;
         const int s0 = t * OTHER + sub0;
         const int rel_min = s0 - (w_lo + 31 + P), rel_max = rel_min + 62;
-        auto next = [&]() { tiles.store(smem + ((t + 1) & 1) * G::BUF); tiles.fetch(t + 2); };
-        if (!(s0 < N && (!CAUSAL || rel_min <= 0))) {
-            next();
-        } else {
+        const bool active = s0 < N && (!CAUSAL || rel_min <= 0);
+        // (the products start at bias - running maximum, which is at hand ahead of the tile)
+        const float ref = top > -INFINITY ? top : 0.f;
+        f32x16 s;
+        if (active) {
             const bool sat_lo = rel_max <= -sat, sat_hi = rel_min >= sat;
-            // (the products start at bias - running maximum)
-            f32x16 s;
-            const float ref = top > -INFINITY ? top : 0.f;
             if (sat_lo || sat_hi) {
                 const float c = (sat_lo ? bias_lo : bias_hi) - ref;
 #pragma unroll
@@ -527,6 +556,12 @@ __device__ __forceinline__ bool fwd32_body(const FwdParams& p, int nblk, unsigne
 #pragma unroll
                 for (int r = 0; r < 16; ++r) s[r] = lp[8 * (r >> 2) + (r & 3)] - ref;
             }
+        }
+        __syncthreads();      // (tile t is written, the other buffer read)
+        auto next = [&]() { tiles.store(smem + ((t + 1) & 1) * G::BUF); tiles.fetch(t + 2); };
+        if (!active) {
+            next();
+        } else {
             reads.template over_dim<1>({tk}, {&own}, {&s});
             next();
             if (s0 + 32 > N || (CAUSAL && rel_max > 0)) {
@@ -556,6 +591,7 @@ __device__ __forceinline__ bool fwd32_body(const FwdParams& p, int nblk, unsigne
 #pragma unroll
             for (int r = 0; r < 16; ++r) { s[r] = __builtin_amdgcn_exp2f(s[r]); part += s[r]; }
             sum += part;
+            if constexpr (!RAW) s *= X::up;
             reads.over_rows(tk + G::TENSOR, s, acc);
         }
     }
@@ -585,10 +621,10 @@ __device__ __forceinline__ bool fwd32_body(const FwdParams& p, int nblk, unsigne
     sum += __shfl_xor(sum, 32, 64);
     if constexpr (!RAW) {
         const float x = odd(acc) + sum * 0.f;
-        if (anybody(flag, x != x)) return true;
+        if (anybody(flag, least < kTiny || x != x)) return true;
     }
     if (own_ok && sub0 == 0) {
-        const float inv = sum == 0.f ? 0.f : 1.0f / sum;      // (a row without a visible key: zeros)
+        const float inv = (sum == 0.f ? 0.f : 1.0f / sum) * X::back_b;      // (a row without a visible key: zeros)
         float* const o = reinterpret_cast<float*>(p.o) + (int64_t)b * p.o_sb + (int64_t)h * p.o_sh + (int64_t)own_row * p.o_sr;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)

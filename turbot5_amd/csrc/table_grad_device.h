@@ -48,9 +48,9 @@ __device__ __forceinline__ void table_grad_block(float* skew, float* sums, const
 }
 
 // All threads: the wavefronts' sums into the workgroup's slot, or without slots into the head's column of the table's gradient.
-// `scratch`: 2 WAVES floats.  Eight lanes share a bucket, whose distances are one run on one side of the diagonal.
+// `scratch`: 2 WAVES floats; `unit`: what the sums are multiplied by.  Eight lanes share a bucket, whose distances are one run on one side of the diagonal.
 template <int WAVES>
-__device__ __forceinline__ void table_grad_finish(const BwdParams& p, int h, int64_t slot, const float* sums, float* scratch, int sat, float lo, float hi) {
+__device__ __forceinline__ void table_grad_finish(const BwdParams& p, int h, int64_t slot, const float* sums, float* scratch, int sat, float lo, float hi, float unit = 1.f) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, stride = table_grad_floats(sat);
     const BucketSpec& bs = p.bs;
 #pragma unroll
@@ -86,6 +86,7 @@ __device__ __forceinline__ void table_grad_finish(const BwdParams& p, int h, int
                 if (b == last_lo) s += scratch[2 * w];
                 if (b == last_hi) s += scratch[2 * w + 1];
             }
+            s *= unit;
             if (p.slots != nullptr) p.slots[slot * p.n_buckets + b] = s;
             else if (s != 0.f) atomicAdd(&p.dtable[(int64_t)b * p.H + h], s);
         }

@@ -100,6 +100,30 @@ def test_refusals_and_switches_at_the_time_of_the_backward(gpu_device, monkeypat
     assert all(torch.equal(a, b) for a, b in zip(wide[:3], want))                   # (the table's gradient by atomics there)
 
 
+def test_a_copy_of_the_package_under_another_name(gpu_device, tmp_path, monkeypatch):
+    """Its nodes read its own switch, whatever the other copy's says."""
+    import importlib
+    import os
+    import shutil
+    import turbot5_amd as t5
+    from turbot5_amd import ops
+    shutil.copytree(os.path.dirname(t5.__file__), tmp_path / "vendored_attention", ignore=shutil.ignore_patterns("csrc", "__pycache__"))
+    monkeypatch.syspath_prepend(str(tmp_path))
+    copy = importlib.import_module("vendored_attention")
+    copy_ops = importlib.import_module("vendored_attention.ops")
+    ins, dout = _inputs(gpu_device)
+
+    def grads(package):
+        return torch.autograd.grad(package.flash_attention_with_fusing_bias(*ins, sm_scale=1.0), ins[:3], dout)
+
+    assert copy_ops._nodes() is not ops._nodes()
+    fast = grads(t5)
+    assert all(torch.equal(a, b) for a, b in zip(fast, grads(copy)))
+    monkeypatch.setattr(copy_ops, "BACKWARD_FP32_MATH", True)
+    wide = grads(copy)
+    assert all(torch.equal(a, b) for a, b in zip(fast, grads(t5))) and not torch.equal(fast[0], wide[0])
+
+
 def test_calls_that_keep_the_python_function(gpu_device):
     from turbot5_amd import ops
     ins, _ = _inputs(gpu_device)

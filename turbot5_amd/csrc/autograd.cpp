@@ -39,9 +39,11 @@ struct Library {
     decltype(&t5a_rmsnorm_train) norm;
     decltype(&t5a_rmsnorm_bwd_workspace_bytes) norm_bytes;
 } lib;
+PyObject* switches = nullptr;      // the names of the Python module that binds this one, kept for good
 
-void bind(uintptr_t bwd_dense, uintptr_t bwd_varlen, uintptr_t bwd_bytes, uintptr_t bwd_varlen_bytes, uintptr_t table_bytes, uintptr_t last_error,
+void bind(pybind11::dict names, uintptr_t bwd_dense, uintptr_t bwd_varlen, uintptr_t bwd_bytes, uintptr_t bwd_varlen_bytes, uintptr_t table_bytes, uintptr_t last_error,
           uintptr_t gemm, uintptr_t gemm_bytes, uintptr_t norm, uintptr_t norm_bytes) {
+    switches = names.release().ptr();
     lib.gemm = reinterpret_cast<decltype(lib.gemm)>(gemm);
     lib.gemm_bytes = reinterpret_cast<decltype(lib.gemm_bytes)>(gemm_bytes);
     lib.norm = reinterpret_cast<decltype(lib.norm)>(norm);
@@ -103,7 +105,10 @@ void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device
 bool fp32_math(const Tensor& q) {
     if (q.scalar_type() == at::kFloat) return false;
     pybind11::gil_scoped_acquire gil;
-    return pybind11::cast<bool>(pybind11::module_::import("turbot5_amd.ops").attr("BACKWARD_FP32_MATH"));
+    PyObject* const value = PyDict_GetItemString(switches, "BACKWARD_FP32_MATH");
+    const int on = value != nullptr ? PyObject_IsTrue(value) : 0;
+    if (on < 0) throw pybind11::error_already_set();
+    return on != 0;
 }
 
 template <typename N> std::shared_ptr<N> make_node() { return std::shared_ptr<N>(new N(), torch::autograd::deleteNode); }

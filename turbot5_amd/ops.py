@@ -284,7 +284,7 @@ def _nodes():
             raise ImportError(f"turbot5_amd/_native.so is not built or does not match this torch (run `python -m turbot5_amd.build`): {e}") from e
         if _native.abi_version != L.ABI_VERSION:
             raise ImportError(f"turbot5_amd/_native.so has ABI version {_native.abi_version}, expected {L.ABI_VERSION}: rebuild it")
-        _native.bind(*(C.cast(getattr(lib, name), C.c_void_p).value for name in (
+        _native.bind(globals(), *(C.cast(getattr(lib, name), C.c_void_p).value for name in (
             "t5a_bwd_dense", "t5a_bwd_varlen", "t5a_bwd_workspace_bytes", "t5a_bwd_varlen_workspace_bytes",
             "t5a_bwd_table_workspace_bytes", "t5a_last_error", "t5a_gemm_f32", "t5a_gemm_f32_workspace_bytes", "t5a_rmsnorm_train",
             "t5a_rmsnorm_bwd_workspace_bytes")))

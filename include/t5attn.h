@@ -152,7 +152,7 @@ int t5a_fwd_dense(const t5a_dense_args* args, t5a_stream_t stream);
  * workgroups.
  * Arithmetic of the backward.  fp32 tensors at head_dim 64: fp32 products formed on the bf16 matrix cores from operands split in
  * three, which carry all bits of every finite value (workgroups that meet values of 2^112 and more, sums of 2^80 and more, or own rows
- * with values below 2^-94 form theirs on the fp32 matrix cores).  Head_dim 16 and 32, and 16-bit tensors with fp32_math != 0: every product on
+ * with values below 2^-94 form theirs on the fp32 matrix cores).  Head_dim 16 and 32, and any call with fp32_math != 0: every product on
  * the fp32 matrix cores, inputs widened on their way in (head_dim up to 64).  16-bit tensors at head_dim 64 and 128
  * with fp32_math == 0: the
  * 16-bit matrix cores -- the score and dP products take the inputs as they are, and the probabilities and dS are

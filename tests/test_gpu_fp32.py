@@ -151,6 +151,35 @@ def test_scores_of_the_smallest_and_the_largest_numbers(gpu_device, B):
             assert ((a - b).abs() <= 1e-4 * b.abs().amax(dim=(-2, -1), keepdim=True) + L * 2.0 ** -149).all()
 
 
+# (a block of 64 rows and one more; packed sequences with an empty one)
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("causal", [False, True])
+def test_products_on_the_fp32_matrix_cores_on_demand(gpu_device, monkeypatch, packed, causal):
+    """BACKWARD_FP32_MATH, fp32_math of the C entry points: the kernels of the other head sizes."""
+    import turbot5_amd as t5
+    from turbot5_amd import ops
+    g = torch.Generator().manual_seed(9)
+    shape = (195, 4, 64) if packed else (2, 4, 130, 64)
+    q, k, v, d = (0.5 * torch.randn(*shape, generator=g) for _ in range(4))
+    table = torch.randn(32, 4, generator=g)
+    ins = [t.to(gpu_device).requires_grad_() for t in (q, k, v, table)]
+    if packed:
+        cu = torch.tensor([0, 65, 65, 195], dtype=torch.int32, device=gpu_device)
+        o = t5.flash_attention_with_fusing_bias_varlen(*ins, cu, cu, 130, 130, causal=causal, sm_scale=1.0)
+        parts = [_exact(*(t[a:b].transpose(0, 1)[None] for t in (q, k, v)), table, causal, 1.0, d[a:b].transpose(0, 1)[None]) for a, b in ((0, 65), (65, 195))]
+        want = [torch.cat([p[i][0].transpose(0, 1) for p in parts]) for i in range(1, 4)] + [parts[0][4] + parts[1][4]]
+    else:
+        o = t5.flash_attention_with_fusing_bias(*ins, causal=causal, sm_scale=1.0)
+        want = _exact(q, k, v, table, causal, 1.0, d)[1:]
+    dout = d.to(gpu_device)
+    split = torch.autograd.grad(o, ins, dout, retain_graph=True)
+    monkeypatch.setattr(ops, "BACKWARD_FP32_MATH", True)
+    cores = torch.autograd.grad(o, ins, dout)
+    assert not any(torch.equal(a, b) for a, b in zip(split[:3], cores))
+    for a, b, r in zip(split, cores, want):
+        assert all((t.double().cpu() - r).norm() <= 7e-6 * r.norm() for t in (a, b))
+
+
 def test_lut_of_a_table_is_not_marked_built_by_an_fp32_call(gpu_device):
     """The fp32 kernel reads no distance image: a 16-bit call with the same table builds its own."""
     import turbot5_amd as t5

@@ -6,8 +6,8 @@
 // The general kernels do all arithmetic in fp32 (inputs of any of the three types are widened on their
 // way into LDS; the products run on the fp32 matrix cores, v_mfma_f32_32x32x2_f32), so one code path serves fp32 and
 // 16-bit tensors at head_dim 16, 32 and 64; 16-bit tensors at head_dim 64 and 128 have kernels of their own on the 16-bit
-// matrix cores (bwd16_kernel, further down) unless the caller asks for fp32 arithmetic, and fp32 tensors at head_dim 64 theirs
-// (attn_f32.hip).  The general kernels:
+// matrix cores (bwd16_kernel, further down), and fp32 tensors at head_dim 64 theirs (attn_f32.hip), unless the caller asks
+// for products on the fp32 matrix cores.  The general kernels:
 //
 //   bwd_rows_kernel   delta_i = sum_d o_id do_id and the log-sum-exp in base-2 units, per query row, both negated; also
 //                     clears the table gradient
@@ -123,8 +123,8 @@ __global__ __launch_bounds__(256) void bwd_rows_kernel(const BwdParams p) {
 
 // A workgroup owns 64 rows and walks tiles of 64, whose halves go to different wavefronts; their partial gradients are
 // added through LDS at the end.  One 32 x 32 block of scores per wavefront leaves registers to fetch the next tile's rows
-// under the current tile's products.  The fp32 matrix cores (64 cycles per product) bound it.  fp32 at head_dim 64: 128 own rows and no
-// prefetch took, with every table-gradient pair added to LDS by an atomic, 259 us where this takes 135 (B4 H8 L512 D64, the
+// under the current tile's products.  The fp32 matrix cores (64 cycles per product) bound it.  128 own rows and no
+// prefetch took, with every table-gradient pair added to LDS by an atomic, 259 us where this takes 135 (fp32, B4 H8 L512 D64, the
 // three kernels: 64-row blocks fill 256 compute units, 128-row blocks half of them), 674 / 515 at B4 H12 L1024 and
 // 1210 / 925 at B8 H12 L1024; without the atomics 219, 615 and 1004, so the small blocks are the better at every size.
 template <typename T, int D, bool CAUSAL, bool KV>
@@ -836,8 +836,10 @@ hipError_t launch_bwd_d(const BwdParams& p, bool causal, hipStream_t stream) {
     if constexpr (sizeof(T) == 2 && (D == 64 || D == 128)) {
         if (p.fp32_math == 0) return causal ? launch_bwd16<T, D, true>(p, stream) : launch_bwd16<T, D, false>(p, stream);
     }
-    if constexpr (sizeof(T) == 4 && D == 64) return launch_bwd_f32_64(p, causal, stream);
-    else if constexpr (D == 128) {
+    if constexpr (sizeof(T) == 4 && D == 64) {
+        if (p.fp32_math == 0) return launch_bwd_f32_64(p, causal, stream);
+    }
+    if constexpr (D == 128) {
         return hipErrorInvalidValue;     // (the fp32 kernels hold a row's head_dim in registers: up to 64)
     } else {
         const dim3 gq((p.M + kBwdOwn - 1) / kBwdOwn, p.H, p.B), gk((p.N + kBwdOwn - 1) / kBwdOwn, p.H, p.B);

@@ -102,8 +102,7 @@ void check(int rc) { TORCH_CHECK(rc == T5A_OK, "libt5attn error ", rc, ": ", lib
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 // `BACKWARD_FP32_MATH` of the Python module, as the Python backward reads it: when it runs
-bool fp32_math(const Tensor& q) {
-    if (q.scalar_type() == at::kFloat) return false;
+bool fp32_math() {
     pybind11::gil_scoped_acquire gil;
     PyObject* const value = PyDict_GetItemString(switches, "BACKWARD_FP32_MATH");
     const int on = value != nullptr ? PyObject_IsTrue(value) : 0;
@@ -136,7 +135,7 @@ struct AttentionBackward : public Node {
         if (!grads[0].defined()) return out;
         const auto self = getptr();
         Tensor q0 = q_.unpack(), k0 = k_.unpack(), v0 = v_.unpack(), o0 = o_.unpack(self), lse = lse_.unpack(), table = has_table ? table_.unpack() : Tensor();
-        const bool wide_math = fp32_math(q0);
+        const bool wide_math = fp32_math();
         TORCH_CHECK_NOT_IMPLEMENTED(q0.size(-1) != 128 || (q0.scalar_type() != at::kFloat && !wide_math),
                                     "backward at head_dim 128: bf16 / fp16 tensors only (the fp32 kernels cover head_dim 16, 32 and 64)");
         at::NoGradGuard no_grad;

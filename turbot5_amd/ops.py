@@ -34,7 +34,8 @@ LOG2E = 1.4426950408889634
 # depend on it; tests pin every path of the run logic with it.
 RUN_LEN = 0
 
-# Backward of 16-bit tensors at head_dim 64 (and 128, which has no fp32 path).  False: the 16-bit matrix cores, probabilities and dS rounded to the
+# Backward of fp32 tensors at head_dim 64 (True: products on the fp32 matrix cores, False: on the bf16 ones, from operands split in
+# three, as accurate and in about half the time) and of 16-bit tensors at head_dim 64 (and 128, which has no fp32 path).  False: the 16-bit matrix cores, probabilities and dS rounded to the
 # tensors' type before the products that form dq, dk and dv, as the reference's kernels round them
 # (fused_bias_attention.py:575-590).  True: every product on the fp32 matrix cores (about five times slower).
 BACKWARD_FP32_MATH = False

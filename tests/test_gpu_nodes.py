@@ -100,6 +100,24 @@ def test_refusals_and_switches_at_the_time_of_the_backward(gpu_device, monkeypat
     assert all(torch.equal(a, b) for a, b in zip(wide[:3], want))                   # (the table's gradient by atomics there)
 
 
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("node", [True, False])
+def test_second_derivatives_raise(gpu_device, monkeypatch, packed, node):
+    """A kept graph gives the same first derivatives; what would lack the terms through the attention is an error."""
+    if not node:
+        _function(monkeypatch)
+    ins, dout = _inputs(gpu_device, packed)
+    want = torch.autograd.grad(_call(ins, packed), ins, dout)
+    got = torch.autograd.grad(_call(ins, packed), ins, dout, create_graph=True)
+    assert all(torch.equal(a, b) and a.dtype == b.dtype for a, b in zip(want, got))
+    x = ins[0].detach().float().requires_grad_()
+    first = torch.autograd.grad(_call([(x * x).bfloat16(), *ins[1:]], packed).float().square().sum(), x, create_graph=True)[0]
+    with pytest.raises(RuntimeError, match="second derivative"):
+        torch.autograd.grad(first.square().sum(), x)
+    frozen = torch.autograd.grad(_call([*ins[:3], ins[3].detach()], packed), ins[0], dout, create_graph=True)
+    assert torch.equal(frozen[0], want[0])
+
+
 def test_a_copy_of_the_package_under_another_name(gpu_device, tmp_path, monkeypatch):
     """Its nodes read its own switch, whatever the other copy's says."""
     import importlib

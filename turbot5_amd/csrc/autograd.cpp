@@ -5,12 +5,13 @@
 // (saved variables, so hooks on them work and a changed tensor is noticed) and call the entry points of libt5attn.so, whose
 // addresses the binding passes in.  Attention's forward stays in Python, which hands over its result; norms and linear layers are
 // native both ways.  Gradients that are differentiated in their turn, or come in batches, take formulas in torch's operations
-// (norms and linear layers; the attention kernels have no second derivative).
+// (norms and linear layers; the attention kernels have no second derivative, and asking for one raises).
 //
 // us, a pass of small training calls bound by the host, Python functions / nodes: attention B4 H8 L512 fp32 162 / 95; T5-small encoder,
 // 60 to 500 tokens 3 780 to 4 600 / 2 800.
 #include <torch/extension.h>
 #include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
@@ -112,6 +113,15 @@ bool fp32_math() {
 
 template <typename N> std::shared_ptr<N> make_node() { return std::shared_ptr<N>(new N(), torch::autograd::deleteNode); }
 
+// Gradients of an attention call whose graph is kept: good as they are, an error where one is differentiated in its turn (and not a
+// derivative that silently lacks the terms through the attention).  `of`: what they depend on, so that the error lies on the way to it.
+void first_order_only(variable_list& grads, const variable_list& of) {
+    auto error = std::shared_ptr<torch::autograd::Error>(
+        new torch::autograd::Error("the fused-bias attention has no second derivative", torch::autograd::collect_next_edges(of)), torch::autograd::deleteNode);
+    for (const Tensor& g : grads)
+        if (g.defined()) torch::autograd::set_history(g, error);
+}
+
 struct Params {
     bool causal; double scale; int buckets, max_distance, exact;
     int64_t max_q = 0, max_k = 0;
@@ -138,6 +148,7 @@ struct AttentionBackward : public Node {
         const bool wide_math = fp32_math();
         TORCH_CHECK_NOT_IMPLEMENTED(q0.size(-1) != 128 || (q0.scalar_type() != at::kFloat && !wide_math),
                                     "backward at head_dim 128: bf16 / fp16 tensors only (the fp32 kernels cover head_dim 16, 32 and 64)");
+        const bool graph_kept = at::GradMode::is_enabled();
         at::NoGradGuard no_grad;
         const c10::OptionalDeviceGuard device(q0.device());
         const Tensor g0 = grads[0];
@@ -179,6 +190,11 @@ struct AttentionBackward : public Node {
         }
         out[0] = dq; out[1] = dk; out[2] = dv;
         if (has_table && task_should_compute_output(3)) out[3] = dtable.scalar_type() == table.scalar_type() ? dtable : dtable.to(table.scalar_type());
+        if (graph_kept) {
+            variable_list of = {q0, k0, v0, g0};
+            if (has_table) of.push_back(table);
+            first_order_only(out, of);
+        }
         return out;
     }
 };
@@ -507,6 +523,16 @@ PYBIND11_MODULE(_native, m) {
     m.attr("abi_version") = T5A_ABI_VERSION;
     m.def("bind", &bind);
     m.def("takes", &takes);
+    m.def("first_order_only", [](const std::vector<c10::optional<Tensor>>& grads, const std::vector<c10::optional<Tensor>>& of) {
+        auto defined = [](const std::vector<c10::optional<Tensor>>& ts) {
+            variable_list out;
+            for (const auto& t : ts)
+                if (t) out.push_back(*t);
+            return out;
+        };
+        variable_list g = defined(grads);
+        first_order_only(g, defined(of));
+    });
     m.def("project", &project);
     m.def("feed_forward_relu", &feed_forward_relu);
     m.def("rms_norm_train", &rms_norm_train);

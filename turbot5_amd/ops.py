@@ -299,6 +299,13 @@ def _takes_node(q, k, v, bias) -> bool:
     return not torch.compiler.is_compiling() and q.is_cuda and _nodes().takes([q, k, v, bias])
 
 
+def _first_order_only(grads, of):
+    """An attention's gradients: where their graph is kept, differentiating them raises."""
+    if torch.is_grad_enabled():
+        _nodes().first_order_only(grads, of)
+    return grads
+
+
 class FlashAttentionBias(torch.autograd.Function):
     """The dense fused-bias forward with its backward (reference fused_bias_attention.py:821-873): gradients for q,
     k, v and the (NUM_BUCKETS, H) table."""
@@ -319,7 +326,7 @@ class FlashAttentionBias(torch.autograd.Function):
         causal, sm_scale, nb, md, exact = ctx.args
         dq, dk, dv, dtable = _dense_backward(q, k, v, bias, o, lse, dout, causal, sm_scale, nb, md, exact)
         dbias = dtable.to(bias.dtype) if bias is not None and ctx.needs_input_grad[3] else None
-        return dq, dk, dv, dbias, None, None, None, None, None
+        return (*_first_order_only((dq, dk, dv, dbias), (q, k, v, bias, dout)), None, None, None, None, None)
 
 
 def flash_attention_with_fusing_bias(q, k, v, bias, causal=False, sm_scale=None, NUM_BUCKETS=32, MAX_DISTANCE=128,
@@ -505,7 +512,7 @@ class FlashAttentionBiasVarlen(torch.autograd.Function):
         cq, ck, mq, mk, causal, sm_scale, nb, md, lq, lk, exact = ctx.args
         dq, dk, dv, dtable = _varlen_backward(q, k, v, bias, o, lse, dout, cq, ck, mq, mk, causal, sm_scale, nb, md, lq, lk, exact)
         dbias = dtable.to(bias.dtype) if bias is not None and ctx.needs_input_grad[3] else None
-        return (dq, dk, dv, dbias) + (None,) * 12
+        return (*_first_order_only((dq, dk, dv, dbias), (q, k, v, bias, dout)), *(None,) * 12)
 
 
 def flash_attention_with_fusing_bias_varlen(q, k, v, bias, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,

@@ -106,7 +106,7 @@ int64_t t5a_bias_lut_bytes_windowed(int32_t H, int32_t num_buckets, int32_t max_
 
 /* Layout of the argument structs and set of entry points; a binding compares it with t5a_version() before
  * it passes a struct (a stale library would read pointers from the wrong offsets). */
-#define T5A_ABI_VERSION 118
+#define T5A_ABI_VERSION 119
 int t5a_version(void);
 const char* t5a_last_error(void);
 

@@ -5,6 +5,7 @@ import ctypes as C
 import inspect
 import os
 import re
+import zlib
 
 import pytest
 import torch
@@ -28,6 +29,11 @@ def test_header_symbols_are_exported(lib):
     for name in declared:
         assert getattr(handle, name) is not None
     assert handle.t5a_version() == lib.ABI_VERSION == int(re.search(r"#define T5A_ABI_VERSION (\d+)", header).group(1))
+
+
+def test_a_set_of_entry_points_has_one_version(lib):
+    """A name that is added or taken away changes the sum: raise T5A_ABI_VERSION with it, and write the new pair here."""
+    assert (lib.ABI_VERSION, zlib.crc32(" ".join(sorted(lib.EXPORTS)).encode())) == (119, 0x2567289a)
 
 
 def test_struct_sizes_follow_the_header(lib):

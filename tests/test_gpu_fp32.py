@@ -151,6 +151,35 @@ def test_scores_of_the_smallest_and_the_largest_numbers(gpu_device, B):
             assert ((a - b).abs() <= 1e-4 * b.abs().amax(dim=(-2, -1), keepdim=True) + L * 2.0 ** -149).all()
 
 
+@pytest.mark.parametrize("B", [1, 48])
+@pytest.mark.parametrize("fp32_math", [False, True])
+@pytest.mark.parametrize("what", ["k", "v"])
+def test_a_row_that_is_not_finite_stays_within_its_blocks(gpu_device, monkeypatch, B, fp32_math, what):
+    """Causal backward, key 70 infinite (or its value NaN): dq of queries before its block of 32 keys and queries is that without it, and
+    queries behind it that see it are NaN; queries 64 to 69, in one block with some that see it, may be either."""
+    import turbot5_amd as t5
+    from turbot5_amd import ops
+    monkeypatch.setattr(ops, "BACKWARD_FP32_MATH", fp32_math)
+    H, L = 8, 160
+    g = torch.Generator().manual_seed(13)
+    q, k, v, d = (0.5 * torch.randn(B, H, L, 64, generator=g) for _ in range(4))
+    q[..., 0] = q[..., 0].abs() + 0.1         # (a score of plus infinity)
+    table = torch.randn(32, H, generator=g)
+
+    def dq(k, v):
+        ins = [t.to(gpu_device).requires_grad_() for t in (q, k, v, table)]
+        return torch.autograd.grad(t5.flash_attention_with_fusing_bias(*ins, causal=True, sm_scale=1.0), ins[0], d.to(gpu_device))[0]
+
+    clean = dq(k, v)
+    if what == "k":
+        k[:, :, 70, 0] = math.inf
+    else:
+        v[:, :, 70, 5] = math.nan
+    got = dq(k, v)
+    assert got[:, :, 70:].isnan().all()
+    assert (got[:, :, :64] - clean[:, :, :64]).norm() <= 7e-6 * clean[:, :, :64].norm()
+
+
 # (a block of 64 rows and one more; packed sequences with an empty one)
 @pytest.mark.parametrize("packed", [False, True])
 @pytest.mark.parametrize("causal", [False, True])

@@ -1,4 +1,4 @@
-// Dense and packed attention of fp32 tensors at head_dim 64 on the 16-bit matrix cores: forward and backward.
+// Attention of fp32 tensors at head_dim 64 on the 16-bit matrix cores: the dense forward, the dense and the packed backward.
 //
 // Every product of fp32 numbers is formed from operands split into three bf16 parts (split_device.h): six
 // v_mfma_f32_32x32x16_bf16 for sixteen indices in place of eight v_mfma_f32_32x32x2_f32, 192 cycles for 512.  Scores,
@@ -259,7 +259,8 @@ template <bool DOWN> __device__ __forceinline__ void fill_bias(const BiasColumn&
 // ------------------------------------------------------------------------------------------------------------ backward
 // KV false: a workgroup owns query rows and walks the keys: dq and the table gradient.  KV true: it owns keys and walks the
 // query rows: dk and dv.  Formulas, classes of block and the table gradient as in attn_bwd.hip; RAW leaves what is no pair out of
-// every sum, so that a NaN or infinity reaches exactly the results that see it.
+// the scores, dS and the table gradient.  (A row of the tile that is not finite still reaches every own row that shares a 32 x 32 block of
+// pairs with one that sees it, by a product with zero, as in the general kernels.)
 template <bool CAUSAL, bool KV, int SPLIT, bool RAW>
 __device__ __forceinline__ bool bwd32_body(const BwdParams& p, int nblk, unsigned char* smem) {
     using G = Geom<SPLIT>;

@@ -3,10 +3,16 @@
 Independent of oracle/t5_basic.py's blocked evaluation: each row's live keys and
 bias buckets are enumerated from the index formulas, the softmax is done in
 numpy.  Only for tiny inputs.
+
+``dense_64_bits``: dense attention and its gradients as torch's operations give them in 64 bits, for inputs of some
+thousand rows.
 """
 import math
 
 import numpy as np
+import torch
+
+from oracle import t5_basic as O
 
 
 def bucket(rel, bidirectional=True, nb=32, md=128):
@@ -112,3 +118,17 @@ def tglobal(q, k, v, sk, sv, table, Bl, gbs, nb=32, md=128):
             bs += [0.0 if table is None else table[bucket(g - i // gbs, True, nb, md), h] for g in range(Gn)]
             out[h, i] = _row(q[h, i], ks, vs, bs)
     return out
+
+
+def dense_64_bits(q, k, v, table, causal, scale, far, dout=None):
+    """o, and with ``dout`` the gradients of q, k, v and the table; rows without a key are zero."""
+    q, k, v, table = (t.detach().double().cpu().requires_grad_() for t in (q, k, v, table))
+    M, N = q.shape[2], k.shape[2]
+    rel = torch.arange(N)[None, :] - (torch.arange(M)[:, None] + N - M)
+    s = q @ k.transpose(2, 3) * scale + table[O.relative_position_bucket(rel, not causal, table.shape[0], far)].permute(2, 0, 1)
+    seen = (rel <= 0) if causal else torch.ones_like(rel, dtype=torch.bool)
+    s = torch.where(seen.any(1)[:, None], s.masked_fill(~seen, -math.inf), torch.zeros_like(s))
+    o = (torch.softmax(s, -1) * seen.any(1)[:, None]) @ v
+    if dout is None:
+        return o.detach()
+    return [o.detach(), *torch.autograd.grad(o, (q, k, v, table), dout.double().cpu())]

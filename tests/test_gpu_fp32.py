@@ -6,23 +6,14 @@ import pytest
 import torch
 
 from oracle import t5_basic as O
+from tests.closed_forms import dense_64_bits
 
 pytestmark = pytest.mark.gpu
 
 
-def _exact(q, k, v, table, causal, scale, dout=None):
-    """o and the gradients of q, k, v and the table in 64 bits, rows without a key zero."""
-    q, k, v, table = (t.detach().double().cpu().requires_grad_() for t in (q, k, v, table))
-    M, N = q.shape[2], k.shape[2]
-    rel = torch.arange(N)[None, :] - (torch.arange(M)[:, None] + N - M)
-    s = q @ k.transpose(2, 3) * scale + table[O.relative_position_bucket(rel, not causal, table.shape[0], 128)].permute(2, 0, 1)
-    seen = (rel <= 0) if causal else torch.ones_like(rel, dtype=torch.bool)
-    s = s.masked_fill(~seen, -math.inf)
-    p = torch.softmax(torch.where(seen.any(1)[:, None], s, torch.zeros_like(s)), -1) * seen.any(1)[:, None]
-    o = p @ v
-    if dout is None:
-        return o.detach()
-    return [o.detach(), *torch.autograd.grad(o, (q, k, v, table), dout.double().cpu())]
+def _exact(q, k, v, table, causal, scale, dout=None, far=128):
+    """o and the gradients of q, k, v and the table."""
+    return dense_64_bits(q, k, v, table, causal, scale, far, dout)
 
 
 # (blocks of 64 rows: up to 256, causal 640; of 128 beyond) x tile edges, one row, rows without keys, more keys than rows
@@ -43,6 +34,19 @@ def test_forward_and_gradients_against_64_bits(gpu_device, B, H, M, N, causal):
     # (with one key the gradients are differences of equal terms, of norm 1 and more)
     for t, r, tol in zip(got, want, (2e-6, 7e-6, 7e-6, 7e-6, 7e-6)):
         assert (t.double().cpu() - r).norm() <= tol * r.norm().clamp(min=1.0)
+
+
+@pytest.mark.parametrize("nb,far", [(64, 1000), (64, 1250)])
+def test_bucketings_with_and_without_room_for_the_larger_tiles(gpu_device, nb, far):
+    """Saturated at 773 and 952, either side of 779: blocks of 64 rows for both passes, and of 128 for dq."""
+    import turbot5_amd as t5
+    g = torch.Generator().manual_seed(far)
+    q, k, v, d = (0.5 * torch.randn(1, 2, 1000, 64, generator=g) for _ in range(4))
+    ins = [t.to(gpu_device).requires_grad_() for t in (q, k, v, torch.randn(nb, 2, generator=g))]
+    o = t5.flash_attention_with_fusing_bias(*ins, causal=False, sm_scale=1.0, NUM_BUCKETS=nb, MAX_DISTANCE=far)
+    got = [o, *torch.autograd.grad(o, ins, d.to(gpu_device))]
+    for t, r, tol in zip(got, _exact(*ins, False, 1.0, d, far), (2e-6, 7e-6, 7e-6, 7e-6, 7e-6)):
+        assert (t.double().cpu() - r).norm() <= tol * r.norm()
 
 
 @pytest.mark.parametrize("B", [1, 48])

@@ -795,7 +795,7 @@ hipError_t launch_bwd16_pass(const BwdParams& p, hipStream_t stream) {
     const bool bias = p.table != nullptr;
     const int lds = G::bytes(bias ? p.bs.sat : 0, bias);
     auto kern = bwd16_kernel<T, D, CAUSAL, PASS, SPLIT>;
-    static LdsLimit limit;     // (per instantiation; 67 KB and more at head_dim 128 with SPLIT 2, 90.6 with the widest bucketing, SPLIT 4 up to 160)
+    static LdsLimit limit;     // (per instantiation; bytes with the widest bucketing, saturated at 1024: 115 280 at head_dim 128, 107 088 at 64; SPLIT 4 up to 160 KB)
     const hipError_t e = limit.allow(reinterpret_cast<const void*>(kern), lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(G::THREADS), lds, stream, p, nblk);
@@ -805,7 +805,7 @@ hipError_t launch_bwd16_pass(const BwdParams& p, hipStream_t stream) {
 template <typename T, int D, bool CAUSAL, int PASS>
 hipError_t launch_bwd16_rows(const BwdParams& p, hipStream_t stream) {
     const int split = bwd16_split(p, D, CAUSAL, PASS != 0);
-    // (bucketings that reach past some hundred distances leave no room for the largest tiles next to the table gradient's sums)
+    // (bucketings that saturate past distance 901, 219 at head_dim 128, leave no room for the largest tiles next to the table gradient's sums)
     if (split == 4 && Bwd16Geom<D, PASS, 4>::bytes(p.table != nullptr ? p.bs.sat : 0, p.table != nullptr) <= 160 * 1024)
         return launch_bwd16_pass<T, D, CAUSAL, PASS, 4>(p, stream);
     return split > 1 ? launch_bwd16_pass<T, D, CAUSAL, PASS, 2>(p, stream) : launch_bwd16_pass<T, D, CAUSAL, PASS, 1>(p, stream);

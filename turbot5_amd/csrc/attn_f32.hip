@@ -695,7 +695,7 @@ hipError_t launch_fwd_f32_64(const FwdParams& p, bool causal, hipStream_t stream
 
 template <bool CAUSAL> static hipError_t launch_passes(BwdParams p, hipStream_t stream) {
     const int64_t pairs = (int64_t)p.H * p.B;
-    // (bucketings that reach past some 900 distances leave no room for the larger tiles next to the table gradient's sums)
+    // (bucketings that saturate past distance 779 leave no room for the larger tiles next to the table gradient's sums)
     const bool room = Geom<2>::bytes(p.table != nullptr ? p.bs.sat : 0, p.table != nullptr) <= 160 * 1024;
     const bool split = room && few(p.M, pairs, CAUSAL);
     p.slots_per_head = p.B * (split ? (p.M + 63) / 64 : (p.M + 127) / 128);

@@ -533,6 +533,15 @@ PYBIND11_MODULE(_native, m) {
         variable_list g = defined(grads);
         first_order_only(g, defined(of));
     });
+    m.def("gemm", [](const variable_list& a, const variable_list& b, const variable_list& c, bool a_trans, bool b_trans, bool sum, bool relu, double alpha,
+                     const c10::optional<Tensor>& positive) {
+        at::NoGradGuard no_grad;
+        const c10::OptionalDeviceGuard device(c.at(0).device());
+        Gemm how;
+        how.a_trans = a_trans; how.b_trans = b_trans; how.sum = sum; how.relu = relu; how.alpha = alpha;
+        if (positive) how.positive = *positive;
+        gemm(a, b, c, how);
+    });
     m.def("project", &project);
     m.def("feed_forward_relu", &feed_forward_relu);
     m.def("rms_norm_train", &rms_norm_train);

@@ -7,36 +7,18 @@ result to the attention's type, applies ReLU or its derivative on the way out.
 """
 from __future__ import annotations
 
-import ctypes as C
-
 import torch
 from torch import nn
 
-from . import _lib as L
-from .ops import _DTYPES, _nodes, _on_device, _plain, _stream
+from .ops import _nodes, _plain
 
 MAX_BYTES = 0x7fe00000      # of an operand, which the kernel reads with 32-bit offsets
 
 
 def _gemm(a, b, out, a_trans=False, b_trans=False, sum_groups=False, alpha=1.0, relu=False, positive=None):
-    """out[g] = alpha_g a[g] b[g]^T over lists of two-dimensional contiguous tensors; see include/t5attn.h.  (What the nodes of
-    ``project`` and ``feed_forward_relu`` call from native code.)"""
-    n = len(a)
-    args = L.T5AGemmF32Args((C.c_void_p * 3)(*(t.data_ptr() for t in a)), (C.c_void_p * 3)(*(t.data_ptr() for t in b)),
-                            (C.c_void_p * 3)(*(t.data_ptr() for t in out)), a[0].shape[1], b[0].shape[1], out[0].shape[1],
-                            positive.data_ptr() if positive is not None else None,
-                            positive.shape[1] if positive is not None else 0, None, 0,
-                            out[0].shape[0], out[0].shape[1], a[0].shape[0 if a_trans else 1], n, int(sum_groups),
-                            _DTYPES[a[0].dtype], _DTYPES[b[0].dtype], _DTYPES[out[0].dtype], int(a_trans), int(b_trans),
-                            int(relu), float(alpha))
-    lib = L.load()
-    nbytes = lib.t5a_gemm_f32_workspace_bytes(C.byref(args))
-    ws = None
-    if nbytes > 0:
-        ws = torch.empty(nbytes, device=out[0].device, dtype=torch.uint8)
-        args.workspace, args.workspace_bytes = ws.data_ptr(), nbytes
-    with _on_device(out[0]):
-        L.check(lib.t5a_gemm_f32(C.byref(args), _stream(out[0])))
+    """out[g] = alpha_g a[g] b[g]^T over lists of two-dimensional contiguous tensors (see include/t5attn.h): the call that the nodes of
+    ``project`` and ``feed_forward_relu`` make."""
+    _nodes().gemm(a, b, out, bool(a_trans), bool(b_trans), bool(sum_groups), bool(relu), float(alpha), positive)
     return out
 
 

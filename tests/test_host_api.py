@@ -82,6 +82,18 @@ def test_fp32_products_are_checked_without_gpu(lib):
             assert need % (M * N * 4) == 0 and 0 <= need // (M * N * 4) <= 16 and need // (M * N * 4) != 1
 
 
+def test_feed_forward_takes_no_second_layer_that_outgrows_the_first():
+    """A product's operands are below 2 GiB: a second layer wider than the first one's input, whose weight or results may not be, stays
+    with torch (its backward was refused by the library)."""
+    from torch import nn
+    from turbot5_amd import linear
+    wi = nn.Linear(64, 1 << 20, bias=False, device="meta")
+    assert linear.widths_chain(wi, nn.Linear(1 << 20, 64, bias=False, device="meta"))
+    assert linear.widths_chain(wi, nn.Linear(1 << 20, 32, bias=False, device="meta"))
+    for width in (72, 4096):
+        assert not linear.widths_chain(wi, nn.Linear(1 << 20, width, bias=False, device="meta"))
+
+
 def test_key_bits_layout_and_size(lib):
     """Token j is bit (j & 31) of word 8 + (j >> 5); zero words in front and behind, as many as the kernels' tiles
     may look at; the side-token count is the number of valid block ENDs."""

@@ -58,9 +58,10 @@ def takes(x: torch.Tensor, *layers: nn.Module) -> bool:
 
 
 def widths_chain(wi: nn.Module, wo: nn.Module) -> bool:
-    """wo is a layer of the same kind over wi's output (which ``takes`` has said yes to)."""
+    """wo is a layer of the same kind over wi's output (which ``takes`` has said yes to), no wider than wi's input: then its weight and its
+    results are no larger than what ``takes`` has measured."""
     return (_bare(wo) and _plain(wo.weight) and wo.weight.dtype == torch.float32 and wo.weight.device == wi.weight.device
-            and wo.weight.shape[1] == wi.weight.shape[0] and wo.weight.shape[0] % 8 == 0 and wo.weight.numel() > 0)
+            and wo.weight.shape[1] == wi.weight.shape[0] and wo.weight.shape[0] % 8 == 0 and 0 < wo.weight.shape[0] <= wi.weight.shape[1])
 
 
 def project(x, dtype, factor, *layers):

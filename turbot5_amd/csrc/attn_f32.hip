@@ -9,11 +9,11 @@
 // products over the tile's rows (transposing reads).  A tile is fetched into registers a step ahead and split into the other of
 // two LDS buffers beside the products: one barrier per tile.
 //
-// What bounds it: large launches the matrix cores at the clock the card's power allows them (B3 H16 L2000, forward 262 us: 1120
+// What bounds it: large launches the matrix cores at the clock the card's power allows them (B3 H16 L2000, forward 265 us: 1110
 // TFLOP/s of bf16 products, where a loop of nothing but such products on random numbers runs at 1870), small ones the chain of one
 // wavefront per SIMD: products, exponentials, splits.  us, products on the fp32 matrix cores / this, forward and the backward's
-// kernels: B4 H8 L512 47 / 26 and 127 / 77, B2 H6 L1999 causal 155 / 74 and 552 / 196, B8 H12 L1024 222 / 141 and 920 / 540, B3 H16
-// L2000 424 / 262 and 1715 / 980.  Errors against 64 bits are smaller: 4.2e-7 for 6.1e-7 (o, B4 H8 L512), 8e-7 for 1.05e-6 (dq, dk, dv).
+// kernels: B4 H8 L512 47 / 25 and 127 / 73, B2 H6 L1999 causal 155 / 62 and 552 / 199, B8 H12 L1024 222 / 145 and 920 / 560, B3 H16
+// L2000 424 / 265 and 1715 / 1020.  Errors against 64 bits are smaller: 4.5e-7 for 6.1e-7 (o, B4 H8 L512), 8.5e-7 for 1.05e-6 (dq, dk, dv).
 //
 // What is split is scaled (split_device.h), by exact powers of two that leave the sums again: a tile's rows and the probabilities by 2^16; own
 // rows of a score's product by 2^-16, so that scores carry no factor and nothing is paid per score; own rows of dP's by 2^16, whose 2^32
@@ -680,7 +680,7 @@ hipError_t launch_fwd(const FwdParams& p, hipStream_t stream) {
 
 // Whether blocks of 64 rows are taken (SPLIT 2) in place of 128: where they are one round of one workgroup per compute unit
 // (what their LDS allows), and with a causal mask, where the longest block counts, up to two and a half.  us, SPLIT 2 / 1,
-// forward and backward: blocks of 64 rows 256 (B4 H8 L512) 26 / 33 and 77 / 114; 320 (B5 H8 L512) 44 / 31 and 132 / 116; 384 (B2 H8
+// forward and backward (before the operands were scaled): blocks of 64 rows 256 (B4 H8 L512) 26 / 33 and 77 / 114; 320 (B5 H8 L512) 44 / 31 and 132 / 116; 384 (B2 H8
 // L1500) 102 / 77 and 292 / 276; 192 (B32 H6 L64) 14 / 16 and 34 / 39; causal 512 (B4 H8 L1000) 46 / 54 and 142 / 198, 576 (B3 H6
 // L2000) 96 / 98 and 284 / 362, 768 (B4 H12 L1000) 71 / 59 and 216 / 203.
 bool few(int rows, int64_t pairs, bool causal) { return ((int64_t)(rows + 63) / 64) * pairs <= (causal ? 640 : 256); }
